@@ -296,7 +296,8 @@ def tolerance(case):
     and as the largest single difference: decode in float16 2.4e-4 and 1.2e-3, in bfloat16 1.7e-3 and 3.9e-3 (the
     rounding of the output); causal calls over plain rows 2.6e-4 and 5.7e-3; prefill over the packed cache, whose rows
     are rounded to float16 once reconstructed, 8.9e-4 (bfloat16 1.85e-3) and 1.8e-2; VecInfer's reconstruction
-    3.4e-4 and, where two centroids are equally near, 0.1."""
+    3.4e-4 and, where two centroids are equally near, 0.1; decode over VecInfer indices with the transform's sums in
+    another order, which moves a few indices between equally near centroids, 2.6e-4 and 5.3e-3."""
     kind, half = case["kind"], case.get("dtype", "float16") == "float16"
     if kind == "fill":
         return {"rel": 1.4e-3 if half else 7e-3, "max": 0.4} if case["method"] == "vecinfer" else "exact"
@@ -304,4 +305,5 @@ def tolerance(case):
         return {"rel": 3.6e-3 if half else 7.4e-3, "max": 0.075}
     if kind == "flash":
         return {"rel": 1e-3, "max": 2.3e-2}
-    return {"rel": 1e-3, "max": 5e-3} if half else {"rel": 7e-3, "max": 1.6e-2}
+    most = 2.1e-2 if kind == "vecstep" else 5e-3 if half else 1.6e-2
+    return {"rel": 1e-3 if half else 7e-3, "max": most}
