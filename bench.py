@@ -650,7 +650,7 @@ def _extras(torch, K, dev):
     flops4 = 2 * 524288 * 4096 * 4
     ex["vq_assign_4096_centroids_sub4"] = {"ms": round(ms4, 5), "TFLOPs_gemm_form": round(flops4 / ms4 / 1e9, 2),
                                            "frac_mfma_f16_peak": round(flops4 / ms4 / 1e9 / MFMA_F16_PEAK_TFLOPS, 5),
-                                           "note": "codebook tiles streamed from LDS, 16 chunks of 256 centroids"}
+                                           "note": "codebook as operand tiles in LDS"}
     ex["vq_assign_4096_centroids_sub4"].update(_vq_census(torch, x4d[:1, :1024], cb4, fn4()[:1, :1024]))
     del x4d, cb4
     # Kitty keys (mixed 4/2-bit by channel variance): two launches of the key-axis round trip plus the ranking

@@ -244,7 +244,7 @@ int vq_vecinfer_assign(const void *x, int x_dtype, int64_t N, const void *codebo
  * float32 [smooth_rows, D] with smooth_rows 1 or H, or NULL.  k_hat, when not NULL, receives
  * the reconstruction (codebook[idx] @ Hd^T) * smooth in the dtype of keys; k_tilde, when not
  * NULL, receives k~ as float32.  Covers sub_dim 4 or 8, D / sub_dim in {8, 16, 32, 64},
- * n_centroids <= 256, 16-byte aligned buffers; VQ_ERR_UNSUPPORTED otherwise (callers then
+ * n_centroids * sub_dim <= 16384, 16-byte aligned buffers; VQ_ERR_UNSUPPORTED otherwise (callers then
  * transform with a matrix product and call vq_vecinfer_assign).  Replaces
  * vecinfer_encode_decode_metal (veloxquant_mlx/metal/_vecinfer.py:225-293,
  * metal/src/vecinfer_encode_decode_full.metal) and the encode half of

@@ -136,6 +136,40 @@ def test_mfma_filter_near_ties_follow_the_exact_rule(sub, nc, dtype):
     np.testing.assert_array_equal(got, ref)
 
 
+@pytest.mark.parametrize("sub,nc", [(4, 513), (4, 1000), (4, 4095), (4, 4096), (8, 545), (8, 2047), (8, 2048)])
+@pytest.mark.parametrize("n", [1, 65, 32768, 32769, 70001])
+def test_large_codebooks_split_and_image_forms(sub, nc, n):
+    """Codebooks above 512 centroids on both sides of the sub-vector count where the two forms of the kernel meet, with a
+    partly filled last tile, duplicated and clustered centroids, sub-vectors on centroids and on bisectors, far outside the
+    codebook, zeros and a NaN row (no distance below infinity: index 0)."""
+    require_gpu()
+    rng = np.random.default_rng(nc * 3 + n)
+    cb = (rng.standard_normal((nc, sub)) * 3).astype(np.float32)
+    cb[nc - 1] = cb[7]; cb[300] = cb[7]; cb[17] = cb[16] + np.float32(2.0 ** -12); cb[18] = cb[16]
+    x = (rng.standard_normal((n, sub)) * 3).astype(np.float32)
+    a, b = rng.integers(0, nc, n), rng.integers(0, nc, n)
+    x[::7] = 0.5 * (cb[a[::7]] + cb[b[::7]])
+    x[3::11] = cb[a[3::11]]
+    x[5::1009] *= np.float32(3000)                   # outside the filter's range
+    x[6::4001] = 0
+    x[2::2003] = cb[7] + np.float32(1e-4)
+    got = host(K.vecinfer_quantize_metal(to_dev(x), to_dev(cb), sub)).reshape(-1)
+    np.testing.assert_array_equal(got, cref.vq_assign(x, cb, sub).reshape(-1))
+    x[0, 1] = np.nan
+    assert host(K.vecinfer_quantize_metal(to_dev(x[:2]), to_dev(cb), sub)).reshape(-1)[0] == 0
+
+
+@pytest.mark.parametrize("scale", [1e-6, 1e-3, 1e3, 1e6])
+def test_assignment_follows_the_exact_rule_at_any_scale(scale):
+    require_gpu()
+    rng = np.random.default_rng(3)
+    for sub, nc, n in ((4, 4096, 500), (8, 256, 3000), (4, 1024, 40000)):
+        cb = (rng.standard_normal((nc, sub)) * scale).astype(np.float32)
+        x = (rng.standard_normal((n, sub)) * scale * np.exp(rng.standard_normal((n, 1)))).astype(np.float32)
+        got = host(K.vecinfer_quantize_metal(to_dev(x), to_dev(cb), sub)).reshape(-1)
+        np.testing.assert_array_equal(got, cref.vq_assign(x, cb, sub).reshape(-1))
+
+
 def test_mfma_filter_large_magnitudes_and_ragged_count():
     require_gpu()
     rng = np.random.default_rng(11)

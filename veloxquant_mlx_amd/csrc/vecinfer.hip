@@ -158,7 +158,7 @@ extern "C" int vq_vecinfer_encode_keys(const void *keys, int k_dtype, int64_t B,
     VQ_REQUIRE(launch_encode_keys_mfma(keys, k_dtype, B, H, S, D, smooth, smooth_rows, hadamard_scale, codebook, cb_dtype,
                                        n_centroids, sub_dim, idx, idx_dtype, k_hat, k_tilde, (hipStream_t)stream),
                VQ_ERR_UNSUPPORTED,
-               "%s: needs sub_dim 4 or 8, D / sub_dim in {8, 16, 32, 64}, n_centroids <= 256 and 16-byte aligned buffers", fn);
+               "%s: needs sub_dim 4 or 8, D / sub_dim in {8, 16, 32, 64}, n_centroids * sub_dim <= 16384 and 16-byte aligned buffers", fn);
     VQ_HIP_CHECK_LAUNCH(fn);
     return VQ_OK;
 }

@@ -2,31 +2,30 @@
 // identical to the sequential float32 rule of veloxquant_mlx/metal/src/vecinfer_quantize.metal:8-28
 // (squares rounded separately, dimensions added left to right, strict '<').
 //
-// The matrix unit cannot reproduce that rounding order, so it is used as a filter whose error
-// is bounded, and every decision the bound cannot settle is re-taken with the exact rule:
+// The matrix unit cannot reproduce that rounding order, so it only names the few centroids that can win,
+// and the exact rule chooses among them:
 //
-//   t[c, v] = |c|^2 - 2 c.v     v_mfma_f32_16x16x32_f16: A = -2c (16 centroids), B = v (16
-//                               sub-vectors), accumulator input = |c|^2 in float32.
-//                               c and v travel as fp16 high part + fp16 remainder in separate
-//                               k-slots (all four cross terms), so t is good to ~2^-20 for
-//                               fp16, bf16 and float32 inputs alike.
-//   per lane and column the two smallest t are tracked at 2.5 vector operations a score: the
-//   position of the score (centroid tile, accumulator register) replaces its low mantissa bits
-//   (one and-or), and a PAIR of new keys a, b updates the sorted pair k1 <= k2 in three:
-//   m = med3(k1, a, b), k1 = min3(k1, a, b), k2 = min(k2, m);
-//   if second - first > eps (eps = 2^-14 (|v|^2 + max|c|^2): four times what the six replaced
-//   mantissa bits can move a score, far above filter error and the rounding of the exact
-//   rule) the first is the answer;
-//   otherwise, if the two leaders come from different trackers (lanes) and no other tracked
-//   score lies within eps, the exact rule decides between the two; in the remaining (rare) case
-//   the column's scores are recomputed and every centroid with t <= first + eps is evaluated with
-//   the exact rule, lowest index winning ties.
+//   d2[c, v] = |c|^2 - 2 c.v + |v|^2   v_mfma_f32_32x32x16_f16, 32 centroids x 32 sub-vectors a product.  c and v
+//       travel as fp16 high part + fp16 remainder, |c|^2 and |v|^2 as two fp16 parts in k-slots of their own, so the
+//       accumulator input is the constant zero.  Codebook and sub-vectors are first multiplied by one power of two that
+//       puts max|c|^2 in [256, 1024) (remainders stay out of the subnormals); d2 is then good to 2^-19 (|c|^2 + |v|^2):
+//       3 2^-22 from the parts of c and v and the product of remainders that is left out, 2^-22 from those of |c|^2, 2^-21
+//       from the accumulation (16 terms: 5e-7 of the largest measured).
+//   A *cell* is the 16 scores one lane holds of a product: 16 centroids, one sub-vector.  |v|^2 carries a small surplus
+//       that keeps every score positive, so float bits order as integers: the smallest of a cell costs eight min3, the
+//       tile number goes into its seven low bits (one and-or), and the two smallest cells of the lane are kept in two
+//       more operations: 11 vector operations for 16 scores (0.69 a score; tracking the two smallest scores
+//       themselves with their positions took 2.5).
+//   If the second cell is farther than eps (2^-16 |v|^2 + 2^-14 d2: filter error of both sides, |c|^2 <= 2 |v|^2 + 2 d2, plus the tag bits) the
+//       exact rule runs over the 16 centroids of the first; else, if both leaders come from different lanes and nothing
+//       else lies within eps, over the 32 of both; else over the whole codebook (rare: a wave does it together).
 //
-// The codebook lives in LDS as ready-made operand tiles (16 or 32 bytes a centroid, |c|^2
-// beside them), 4096 centroids of four dimensions or 2048 of eight at most; a wave keeps 64
-// sub-vectors in registers as four B operands and walks the tiles, four products and forty
-// tracking operations a tile.  Sixteen waves to a CU (four per SIMD, 128 registers each): the
-// loop is bound by vector issue, which one or two waves a SIMD do not fill.
+// Two forms.  IMAGE: the block builds the codebook once in LDS as operand tiles (24 bytes a centroid of four dimensions,
+// 48 of eight) and its waves walk all tiles for 64 sub-vectors at a time; four waves a SIMD, because a
+// product keeps the vector unit waiting for its 16 results.  SPLIT, for few sub-vectors: a block takes 64 sub-vectors and
+// its waves share out the *tiles*, straight from memory; their cells are merged through LDS and the exact rule runs
+// with one lane a centroid.  SPLIT spends twice the vector work a sub-vector (every wave forms its operands from float
+// rows) but fills the chip from a few dozen blocks on.  Where the line lies: see kSplitMax.
 #include <atomic>
 
 #include "vecinfer.hpp"
@@ -34,62 +33,62 @@
 namespace vq {
 
 typedef uint32_t u32;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int VM_MAXC = 4096;
+constexpr int VM_MAXC = 4096;   // tile numbers have seven bits
+// SPLIT up to this many sub-vectors and above kSplitC centroids: two rounds of its blocks (one to a CU).  Measured, us a call,
+// SPLIT / IMAGE: 4096 centroids of four dimensions, 512 sub-vectors 9.9 / 19.3, 16384 10.7 / 27.5, 65536 42 / 26.6; 2048 of
+// eight 9.8 / 18.0, 9.5 / 21.3, 38 / 24.0; 1024 of four 8.1 / 8.1, 8.1 / 9.2, 26.9 / 12.3.
+constexpr int64_t kSplitMax = 32768;
+constexpr int kSplitC = 1024;
+// codebooks up to this size track quarter cells (seven bits: 16 tiles and four runs, with room)
+constexpr int kFineC = 512;
 
-// Bare min / median-of-three: the scores are never NaN, so the canonicalising moves the
-// compiler wraps around fminf would only cost issue slots in the hottest loop.
-__device__ __forceinline__ float vmin(float a, float b) {
-    float d;
-    asm("v_min_f32 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
+__device__ __forceinline__ u32 umin3(u32 a, u32 b, u32 c) { return min(min(a, b), c); }
+__device__ __forceinline__ u32 umed3(u32 a, u32 b, u32 c) {
+    u32 d;
+    asm("v_med3_u32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
     return d;
 }
-__device__ __forceinline__ float vmax(float a, float b) {
-    float d;
-    asm("v_max_f32 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
-    return d;
-}
-__device__ __forceinline__ float vmin3(float a, float b, float c) {
-    float d;
-    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
-    return d;
-}
-__device__ __forceinline__ float vmed3(float a, float b, float c) {
-    float d;
-    asm("v_med3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
-    return d;
-}
-// two new keys into the sorted pair k1 <= k2
-__device__ __forceinline__ void track2(float &k1, float &k2, float a, float b) {
-    const float m = vmed3(k1, a, b);
-    k1 = vmin3(k1, a, b);
-    k2 = vmin(k2, m);
-}
-// a score with its low six mantissa bits replaced by `tag` (0..63 once the tile loop is unrolled: mask and
-// tag are inline constants of one v_and_or_b32)
-__device__ __forceinline__ float tagged(float d, int tag) {
-    return __uint_as_float((__float_as_uint(d) & 0xFFFFFFC0u) | (u32)tag);
-}
-// the exact rule against centroid c: from the operand image when the codebook is 16-bit (its high parts are the
-// centroid itself, times -2), from memory when it is float32
-template <int SUB>
-__device__ __forceinline__ float exact_dist_c(const float *x, const char *tiles, const void *cb, int ct, int c) {
-    float cv[SUB];
-    if (ct != VQ_F32) {
-        const f16 *img = reinterpret_cast<const f16 *>(tiles + (size_t)c * (4 * SUB));
+// the smallest of a lane's 16 scores of a product, with the tile number in its low bits
+__device__ __forceinline__ u32 cell_key(const f32x16 &d, u32 mask, int tile) {
+    u32 s[16];
 #pragma unroll
-        for (int i = 0; i < SUB; ++i) cv[i] = (float)img[i] * -0.5f;
-    } else {
+    for (int i = 0; i < 16; ++i) s[i] = __float_as_uint(d[i]);
+    const u32 a = umin3(s[0], s[1], s[2]), b = umin3(s[3], s[4], s[5]), c = umin3(s[6], s[7], s[8]);
+    const u32 e = umin3(s[9], s[10], s[11]), f = umin3(s[12], s[13], s[14]);
+    const u32 m = min(umin3(a, b, c), umin3(e, f, s[15]));
+    u32 r;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(m), "v"(mask), "s"(tile));
+    return r;
+}
+// The same at a quarter of the cell: the four runs of four scores apart, run number below the tile number.  Eighteen
+// operations for 16 scores, but the exact rule then runs over four centroids: for small codebooks, where it is most of the work.
+__device__ __forceinline__ void keep_quarters(u32 &k1, u32 &k2, const f32x16 &d, u32 mask, int tile) {
+    u32 q[4];
 #pragma unroll
-        for (int i = 0; i < SUB; ++i) cv[i] = ((const float *)cb)[(int64_t)c * SUB + i];
+    for (int g = 0; g < 4; ++g) {
+        const u32 a = __float_as_uint(d[4 * g]), b = __float_as_uint(d[4 * g + 1]), c = __float_as_uint(d[4 * g + 2]);
+        const u32 m = min(umin3(a, b, c), __float_as_uint(d[4 * g + 3]));
+        asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(q[g]) : "v"(m), "v"(mask), "s"(4 * tile + g));
     }
-    float dist = 0.0f;
 #pragma unroll
-    for (int i = 0; i < SUB; ++i) {
-        const float d = __fsub_rn(x[i], cv[i]);
-        dist = __fadd_rn(dist, __fmul_rn(d, d));
+    for (int g = 0; g < 4; g += 2) {   // two new keys into the sorted pair
+        const u32 m = umed3(k1, q[g], q[g + 1]);
+        k1 = umin3(k1, q[g], q[g + 1]);
+        k2 = min(k2, m);
     }
-    return dist;
+}
+// a new key into the sorted pair k1 <= k2
+__device__ __forceinline__ void keep_two(u32 &k1, u32 &k2, u32 key) {
+    k2 = umed3(k1, k2, key);
+    k1 = min(k1, key);
+}
+// lanes 0..31 of a with lanes 32..63 of b: a = [a.low, b.low], b = [a.high, b.high]
+__device__ __forceinline__ void swap_halves(u32 &a, u32 &b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
 }
 
 // ---- the key transform in front of the assignment, and the reconstruction behind it --------
@@ -152,393 +151,620 @@ template <int SUB, int LT> __device__ __forceinline__ void wht_lanes(float (&x)[
     if constexpr (LT > 32) lane_butterfly<SUB, 32>(x, lane);
 }
 
+// ---- rows of the codebook ---------------------------------------------------------------------
 
-// bytes of one centroid's operand image: fp16 high parts, then fp16 remainders, of -2 c
-template <int SUB> constexpr int cent_bytes() { return 4 * SUB; }
-
-// dynamic LDS: [operand tiles: nc16 * cent_bytes][|c|^2: nc16 floats][per wave: 64 x 16 halves, 64 x 8 floats]
-template <int SUB, int LT, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4, 4)))
-void vq_assign_mfma_kernel(const void *__restrict__ x, int xt, int64_t N, const void *__restrict__ cb, int ct, int nc,
-                           void *__restrict__ idx, int it, KeyXform kx) {
-    extern __shared__ __align__(16) char s_dyn[];
-    __shared__ float s_red[WAVES];
-    constexpr int CB = cent_bytes<SUB>();
-    const int ntiles = (nc + 63) / 64 * 4, nc16 = 16 * ntiles;   // whole groups of four tiles (padded with centroids never chosen)
-    char *s_tiles = s_dyn;
-    float *s_c2 = reinterpret_cast<float *>(s_dyn + (size_t)nc16 * CB);
-    char *s_stage = reinterpret_cast<char *>(s_c2 + nc16);
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n = lane & 15, blk = lane >> 4;
-    f16 (*s_xh)[16] = reinterpret_cast<f16 (*)[16]>(s_stage + wave * 4096);          // [64][high 8 | remainder 8]
-    float (*s_xf)[8] = reinterpret_cast<float (*)[8]>(s_stage + wave * 4096 + 2048);   // [64][8] float32 (exact rule)
-
-    // ---- the codebook as operand tiles: thread c splits centroid c (one or two vector loads a row when the
-    // codebook is 16-byte aligned, element by element otherwise)
-    float cmax2 = 0.f;
-    const bool cb_aligned = (reinterpret_cast<uintptr_t>(cb) & 15u) == 0;
-    for (int c = tid; c < nc16; c += 64 * WAVES) {
-        float row[SUB];
-        float c2 = 3.0e38f;   // past the end: never the nearest
-        if (c < nc) {
-            if (!cb_aligned) {
+// N rows at once: every load is on its way before the first is used
+template <int SUB, int N>
+__device__ __forceinline__ void load_centroids(const void *cb, int ct, bool aligned, const int (&c)[N], float (&row)[N][SUB]) {
+    if (!aligned) {
 #pragma unroll
-                for (int e = 0; e < SUB; ++e) row[e] = ld_any(cb, ct, (int64_t)c * SUB + e);
-            } else if (ct == VQ_F32) {
+        for (int i = 0; i < N; ++i)
 #pragma unroll
-                for (int e = 0; e < SUB; e += 4) {
-                    const float4 v = *reinterpret_cast<const float4 *>((const float *)cb + (int64_t)c * SUB + e);
-                    row[e] = v.x; row[e + 1] = v.y; row[e + 2] = v.z; row[e + 3] = v.w;
-                }
+            for (int e = 0; e < SUB; ++e) row[i][e] = ld_any(cb, ct, (int64_t)c[i] * SUB + e);
+    } else if (ct == VQ_F32) {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+            for (int e = 0; e < SUB; e += 4) {
+                const float4 v = *reinterpret_cast<const float4 *>((const float *)cb + (int64_t)c[i] * SUB + e);
+                row[i][e] = v.x; row[i][e + 1] = v.y; row[i][e + 2] = v.z; row[i][e + 3] = v.w;
+            }
+    } else {
+        u32 w[N][SUB / 2];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if constexpr (SUB == 8) {
+                const uint4 v = *reinterpret_cast<const uint4 *>((const u16 *)cb + (int64_t)c[i] * 8);
+                w[i][0] = v.x; w[i][1] = v.y; w[i][2] = v.z; w[i][3] = v.w;
             } else {
-                u32 w[SUB / 2];
-                if constexpr (SUB == 8) {
-                    const uint4 v = *reinterpret_cast<const uint4 *>((const u16 *)cb + (int64_t)c * 8);
-                    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
-                } else {
-                    const uint2 v = *reinterpret_cast<const uint2 *>((const u16 *)cb + (int64_t)c * 4);
-                    w[0] = v.x; w[1] = v.y;
-                }
+                const uint2 v = *reinterpret_cast<const uint2 *>((const u16 *)cb + (int64_t)c[i] * 4);
+                w[i][0] = v.x; w[i][1] = v.y;
+            }
+        }
 #pragma unroll
-                for (int e = 0; e < SUB / 2; ++e) {
-                    if (ct == VQ_F16) {
-                        const f16x2 h = __builtin_bit_cast(f16x2, w[e]);
-                        row[2 * e] = (float)h[0]; row[2 * e + 1] = (float)h[1];
-                    } else {
-                        row[2 * e] = __uint_as_float(w[e] << 16); row[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+            for (int e = 0; e < SUB / 2; ++e) {
+                const f16x2 h = __builtin_bit_cast(f16x2, w[i][e]);
+                row[i][2 * e] = ct == VQ_F16 ? (float)h[0] : __uint_as_float(w[i][e] << 16);
+                row[i][2 * e + 1] = ct == VQ_F16 ? (float)h[1] : __uint_as_float(w[i][e] & 0xffff0000u);
+            }
+    }
+}
+template <int SUB>
+__device__ __forceinline__ void load_centroid(const void *cb, int ct, bool aligned, int c, float (&row)[SUB]) {
+    const int cc[1] = {c};
+    float r[1][SUB];
+    load_centroids<SUB, 1>(cb, ct, aligned, cc, r);
+#pragma unroll
+    for (int e = 0; e < SUB; ++e) row[e] = r[0][e];
+}
+template <int SUB> __device__ __forceinline__ float norm2(const float *row) {
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < SUB; ++e) s = __builtin_fmaf(row[e], row[e], s);
+    return s;
+}
+// the exact rule
+template <int SUB> __device__ __forceinline__ float exact_dist(const float *x, const float *c) {
+    float dist = 0.0f;
+#pragma unroll
+    for (int i = 0; i < SUB; ++i) {
+        const float d = __fsub_rn(x[i], c[i]);
+        dist = __fadd_rn(dist, __fmul_rn(d, d));
+    }
+    return dist;
+}
+// A float as fp16 high part and remainder.  The value is pinned first: left alone, the compiler forms the high part of a
+// fused product once from the rounded float and once from the exact product, and at fp16 ties the two differ.
+__device__ __forceinline__ u32 high_and_rest(float v) {
+    asm("" : "+v"(v));
+    const f16 h = (f16)v;
+    return __builtin_bit_cast(u32, f16x2{h, (f16)(v - (float)h)});
+}
+__device__ __forceinline__ u32 pack_h2(float a, float b) { return __builtin_bit_cast(u32, f16x2{(f16)a, (f16)b}); }
+// floats (products with powers of two: exact) as fp16 high parts and remainders, packed in pairs
+template <int SUB> __device__ __forceinline__ void split_h(const float *v, u32 *hi, u32 *lo) {
+#pragma unroll
+    for (int e = 0; e < SUB; e += 2) {
+        const f16 a = (f16)v[e], b = (f16)v[e + 1];
+        hi[e / 2] = __builtin_bit_cast(u32, f16x2{a, b});
+        lo[e / 2] = pack_h2(v[e] - (float)a, v[e + 1] - (float)b);
+    }
+}
+// the power of two that puts cmax2 = max |c|^2 into [256, 1024)
+__device__ __forceinline__ float codebook_scale(float cmax2) {
+    if (!(cmax2 > 1e-30f) || !(cmax2 < 1e30f)) return 1.f;
+    const int e = (int)((__float_as_uint(cmax2) >> 23) & 255u) - 127;   // 2^e <= cmax2 < 2^(e+1)
+    const int k = (e - 8) >> 1;                                         // floor
+    return __uint_as_float((u32)(127 - k) << 23);
+}
+
+// Operand image of a centroid, in words.  SUB 4: [remainder 4 | high 4 | |c|^2 parts, 2^15 2^15]; lanes 0..31 read words
+// 0..3 against [high | high] of the sub-vector, lanes 32..63 words 2..5 against [remainder | 1 1 | |v|^2 2^-15 parts].
+// SUB 8: [high 8][remainder 8][|c|^2 parts, 2^15 2^15, 0 0 0 0]: a first product of high and remainder against the
+// sub-vector's high part, a second of high and the last block against [remainder | 1 1, |v|^2 2^-15 parts, 0 ..].
+template <int SUB> constexpr int image_words() { return SUB == 4 ? 6 : 12; }
+constexpr u32 kTwo15 = 0x78007800u;   // fp16 2^15, twice
+
+template <int SUB> __device__ __forceinline__ void centroid_image(const float *row, float cs, u32 *img) {
+    float s[SUB], c2 = 0.f;
+#pragma unroll
+    for (int e = 0; e < SUB; ++e) {
+        const float t = row[e] * cs;
+        c2 = __builtin_fmaf(t, t, c2);
+        s[e] = -2.f * t;
+    }
+    u32 hi[SUB / 2], lo[SUB / 2];
+    split_h<SUB>(s, hi, lo);
+    const u32 cc = high_and_rest(c2);
+    if constexpr (SUB == 4) {
+        img[0] = lo[0]; img[1] = lo[1]; img[2] = hi[0]; img[3] = hi[1]; img[4] = cc; img[5] = kTwo15;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { img[e] = hi[e]; img[4 + e] = lo[e]; }
+        img[8] = cc; img[9] = kTwo15; img[10] = 0; img[11] = 0;
+    }
+}
+
+// ---- sub-vectors -----------------------------------------------------------------------------
+
+// where the index of sub-vector sv goes: `rows_out` rows of a (sequence, head) in the output for the S of the input
+struct IndexDst {
+    int shift;          // log2(sub-vectors a token), or -1: densely, in order
+    u32 S;
+    int64_t rows_out;
+    __device__ __forceinline__ int64_t at(int64_t sv) const {
+        if (shift < 0) return sv;
+        const u32 token = (u32)(sv >> shift), bh = token / S;   // (dense otherwise: fewer than 2^32 tokens)
+        return (((int64_t)bh * rows_out + (token - bh * S)) << shift) + (sv & ((1 << shift) - 1));
+    }
+};
+
+// One lane's sub-vector and the operands of the wave's 64: column block b holds sub-vectors 32 b + (lane & 31).
+template <int SUB> struct SubVec {
+    float xf[SUB];
+    float sm[SUB];
+    float x2;      // |v|^2, scaled
+    bool far;      // out of the filter's range (NaN, infinities, far outside the codebook): the exact rule alone
+    f16x8 B1[2], B2[2];
+};
+
+__device__ __forceinline__ f16x8 h8(u32 a, u32 b, u32 c, u32 d) { return __builtin_bit_cast(f16x8, make_uint4(a, b, c, d)); }
+
+template <int SUB>
+__device__ __forceinline__ uint4 load_raw(const void *x, int xt, int64_t sv, bool live) {
+    uint4 r = make_uint4(0, 0, 0, 0);
+    if (!live || xt == VQ_F32) return r;
+    if constexpr (SUB == 8) r = *reinterpret_cast<const uint4 *>((const u16 *)x + sv * 8);
+    else { const uint2 t = *reinterpret_cast<const uint2 *>((const u16 *)x + sv * 4); r.x = t.x; r.y = t.y; }
+    return r;
+}
+
+template <int SUB, int LT>
+__device__ __forceinline__ void take_subvec(SubVec<SUB> &s, const void *x, int xt, uint4 raw, int64_t sv, bool live, int lane,
+                                            const KeyXform &kx) {
+    float xf[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) xf[e] = 0.f;
+    if (xt != VQ_F32) {
+        const u32 w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+        for (int e = 0; e < SUB / 2; ++e) {
+            if (xt == VQ_F16) {
+                const f16x2 h = __builtin_bit_cast(f16x2, w[e]);
+                xf[2 * e] = (float)h[0]; xf[2 * e + 1] = (float)h[1];
+            } else {
+                xf[2 * e] = __uint_as_float(w[e] << 16); xf[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
+            }
+        }
+    } else if (live) {
+#pragma unroll
+        for (int e = 0; e < SUB; ++e) xf[e] = ((const float *)x)[sv * SUB + e];
+    }
+    if constexpr (LT > 0) {
+        // the lane's channels of its token: divide by the smoothing factors, transform, scale
+#pragma unroll
+        for (int e = 0; e < SUB; ++e) s.sm[e] = 1.f;
+        if (kx.smooth != nullptr && live) {
+            const u32 token = (u32)(sv / LT);
+            const u32 srow = kx.smooth_rows > 1 ? (token / (u32)kx.S) % (u32)kx.heads : 0;
+            const float *sp = kx.smooth + ((int64_t)srow * LT + (lane & (LT - 1))) * SUB;
+#pragma unroll
+            for (int e = 0; e < SUB; ++e) { s.sm[e] = sp[e]; xf[e] = xf[e] / s.sm[e]; }
+        }
+        wht_lanes<SUB, LT>(xf, lane);
+#pragma unroll
+        for (int e = 0; e < SUB; ++e) xf[e] *= kx.h;
+    }
+#pragma unroll
+    for (int e = 0; e < SUB; ++e) s.xf[e] = xf[e];
+}
+
+template <int SUB> __device__ __forceinline__ void make_operands(SubVec<SUB> &s, float cs) {
+    float v[SUB];
+    s.x2 = 0.f;
+#pragma unroll
+    for (int e = 0; e < SUB; ++e) {
+        v[e] = s.xf[e] * cs;
+        s.x2 = __builtin_fmaf(v[e], v[e], s.x2);
+    }
+    s.far = !(s.x2 <= 6.7e7f);   // 256 to 512 times the largest centroid; a NaN ends here too
+    if (s.far) {
+        s.x2 = 0.f;
+#pragma unroll
+        for (int e = 0; e < SUB; ++e) v[e] = 0.f;
+    }
+    // |v|^2 and the surplus that keeps every score positive: above the filter's error and the rounding of the two parts
+    const float vv = __builtin_fmaf(s.x2, 1.52587890625e-05f, s.x2 + 0.03125f) * 3.0517578125e-05f;
+    u32 hi[SUB / 2], lo[SUB / 2];
+    split_h<SUB>(v, hi, lo);
+    u32 ones = 0x3c003c00u, parts = high_and_rest(vv);
+    if constexpr (SUB == 4) {
+        u32 a0 = hi[0], a1 = hi[1], a2 = hi[0], a3 = hi[1];
+        u32 b0 = lo[0], b1 = lo[1], b2 = ones, b3 = parts;
+        swap_halves(a0, b0); swap_halves(a1, b1); swap_halves(a2, b2); swap_halves(a3, b3);
+        s.B1[0] = h8(a0, a1, a2, a3);
+        s.B1[1] = h8(b0, b1, b2, b3);
+    } else {
+        u32 a[4], b[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { a[e] = hi[e]; b[e] = hi[e]; swap_halves(a[e], b[e]); }
+        s.B1[0] = h8(a[0], a[1], a[2], a[3]);
+        s.B1[1] = h8(b[0], b[1], b[2], b[3]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            a[e] = lo[e];
+            b[e] = e == 0 ? ones : e == 1 ? parts : 0u;
+            swap_halves(a[e], b[e]);
+        }
+        s.B2[0] = h8(a[0], a[1], a[2], a[3]);
+        s.B2[1] = h8(b[0], b[1], b[2], b[3]);
+    }
+}
+
+template <int SUB> __device__ __forceinline__ float margin(const SubVec<SUB> &s, u32 f1) {
+    return __builtin_fmaf(6.103515625e-05f, __uint_as_float(f1), __builtin_fmaf(1.52587890625e-05f, s.x2, 2.44140625e-04f));
+}
+// first centroid of a cell's run g: a lane holds four runs of four rows of its tile
+__device__ __forceinline__ int cell_centroid(u32 key, int half, int g) { return (int)(key & 127u) * 32 + 8 * g + 4 * half; }
+
+__device__ __forceinline__ void take_nearer(float &d, int &i, float od, int oi) {
+    if (od < d || (od == d && oi < i)) { d = od; i = oi; }
+}
+// The whole codebook by the exact rule for the sub-vectors of the lanes in `m`, one after the other by the whole wave:
+// `x` is the lane's sub-vector, `my_idx` its result.
+template <int SUB>
+__device__ __forceinline__ void scan_all(unsigned long long m, const float (&x)[SUB], const void *cb, int ct, bool aligned, int nc, int lane,
+                                         int &my_idx) {
+    constexpr int N = SUB == 4 ? 8 : 2;   // rows in flight: more would spill
+    while (m != 0) {
+        const int src = __builtin_ctzll(m);
+        m &= m - 1;
+        float xs[SUB], d = INFINITY;
+        int i = 0;   // (no distance below infinity: index 0)
+#pragma unroll
+        for (int e = 0; e < SUB; ++e) xs[e] = __shfl(x[e], src);
+#pragma unroll 1
+        for (int c0 = lane; c0 < nc; c0 += 64 * N) {
+            int c[N];
+            float row[N][SUB];
+#pragma unroll
+            for (int r = 0; r < N; ++r) c[r] = min(c0 + 64 * r, nc - 1);
+            load_centroids<SUB, N>(cb, ct, aligned, c, row);
+#pragma unroll
+            for (int r = 0; r < N; ++r) {
+                const float t = exact_dist<SUB>(xs, row[r]);
+                if (t < d) { d = t; i = c[r]; }
+            }
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) take_nearer(d, i, __shfl_xor(d, o), __shfl_xor(i, o));
+        if (lane == src) my_idx = i;
+    }
+}
+
+
+template <int SUB, int LT>
+__device__ __forceinline__ void store_result(int64_t sv, int my_idx, const SubVec<SUB> &s, const void *cb, int ct, bool aligned, void *idx,
+                                             int it, const IndexDst &dst, const KeyXform &kx, int lane, bool live) {
+    if (live) st_idx(idx, it, dst.at(sv), my_idx);
+    if constexpr (LT > 0) {
+        if (kx.k_tilde != nullptr && live) {
+#pragma unroll
+            for (int e = 0; e < SUB; e += 4)
+                *reinterpret_cast<float4 *>(kx.k_tilde + sv * SUB + e) = make_float4(s.xf[e], s.xf[e + 1], s.xf[e + 2], s.xf[e + 3]);
+        }
+        if (kx.k_hat != nullptr) {   // block-uniform
+            float row[SUB], c[8];
+            load_centroid<SUB>(cb, ct, aligned, my_idx, row);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) c[e] = e < SUB ? row[e] : 0.f;
+            wht_lanes<SUB, LT>(c, lane);
+#pragma unroll
+            for (int e = 0; e < SUB; ++e) c[e] = c[e] * kx.h * s.sm[e];
+            if (live) {
+                if (kx.hat_dtype == VQ_F32) {
+#pragma unroll
+                    for (int e = 0; e < SUB; e += 4)
+                        *reinterpret_cast<float4 *>((float *)kx.k_hat + sv * SUB + e) = make_float4(c[e], c[e + 1], c[e + 2], c[e + 3]);
+                } else {
+                    u32 w[4];
+#pragma unroll
+                    for (int e = 0; e < SUB; e += 2) {
+                        if (kx.hat_dtype == VQ_F16) w[e / 2] = pack_h2(c[e], c[e + 1]);
+                        else w[e / 2] = (u32)f32_to_bf16(c[e]) | ((u32)f32_to_bf16(c[e + 1]) << 16);
                     }
+                    if constexpr (SUB == 8) *reinterpret_cast<uint4 *>((u16 *)kx.k_hat + sv * 8) = make_uint4(w[0], w[1], w[2], w[3]);
+                    else *reinterpret_cast<uint2 *>((u16 *)kx.k_hat + sv * 4) = make_uint2(w[0], w[1]);
                 }
             }
-            c2 = 0.f;
-#pragma unroll
-            for (int e = 0; e < SUB; ++e) c2 += row[e] * row[e];
-            cmax2 = fmaxf(cmax2, c2);
-        } else {
-#pragma unroll
-            for (int e = 0; e < SUB; ++e) row[e] = 0.f;
         }
-        f16 *img = reinterpret_cast<f16 *>(s_tiles + (size_t)c * CB);
-#pragma unroll
-        for (int e = 0; e < SUB; ++e) {
-            const f16 hi = (f16)row[e];
-            const f16 lo = (f16)(row[e] - (float)hi);
-            img[e] = (f16)(-2.f) * hi;
-            img[SUB + e] = (f16)(-2.f) * lo;
-        }
-        s_c2[c] = c2;
+    }
+}
+
+// What one assignment works on.
+struct AssignJob {
+    const void *x;
+    int xt;
+    int64_t N;        // sub-vectors
+    const void *cb;
+    int ct, nc;
+    void *idx;
+    int it;
+    IndexDst dst;
+    KeyXform kx;
+};
+
+// ---- IMAGE: dynamic LDS holds the operand tiles of the whole codebook ---------------------------
+
+template <int SUB, int LT, int WAVES, bool FINE>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void vq_assign_image_kernel(AssignJob j) {
+    extern __shared__ __align__(16) u32 s_img[];
+    __shared__ float s_red[WAVES];
+    constexpr int IW = image_words<SUB>();
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ntiles = (j.nc + 63) / 64 * 2;   // an even number; past the end: the last centroid again
+    const bool aligned = (reinterpret_cast<uintptr_t>(j.cb) & 15u) == 0;
+
+    float cmax2 = 0.f;
+    for (int c = tid; c < j.nc; c += 64 * WAVES) {
+        float row[SUB];
+        load_centroid<SUB>(j.cb, j.ct, aligned, c, row);
+        cmax2 = fmaxf(cmax2, norm2<SUB>(row));
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) cmax2 = fmaxf(cmax2, __shfl_xor(cmax2, o));
     if (lane == 0) s_red[wave] = cmax2;
     __syncthreads();
-    cmax2 = s_red[0];
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w) cmax2 = fmaxf(cmax2, s_red[w]);
+    for (int w = 0; w < WAVES; ++w) cmax2 = fmaxf(cmax2, s_red[w]);
+    const float cs = codebook_scale(cmax2);
+    for (int c = tid; c < ntiles * 32; c += 64 * WAVES) {
+        float row[SUB];
+        load_centroid<SUB>(j.cb, j.ct, aligned, min(c, j.nc - 1), row);
+        u32 img[IW];
+        centroid_image<SUB>(row, cs, img);
+#pragma unroll
+        for (int e = 0; e < IW; e += 2) *reinterpret_cast<uint2 *>(&s_img[c * IW + e]) = make_uint2(img[e], img[e + 1]);
+    }
+    __syncthreads();
 
-    // what a lane reads of a tile.  SUB 8: lane groups 0, 1 the high parts, 2, 3 the remainders of centroid n
-    // (the sub-vector side alternates high part / remainder: all four cross terms).  SUB 4: every lane group
-    // the 16 bytes [high 4 | remainder 4] of centroid n; the sub-vector side carries [high | high] in lane
-    // group 0, [remainder | remainder] in group 1 and zeros in groups 2, 3.
-    const int a_off = SUB == 8 ? n * 32 + (blk >> 1) * 16 : n * 16;
-    const int c_off = 16 * blk;                       // |c|^2 of centroids 4 blk .. 4 blk + 3 of the tile
-    const bool multi = ntiles > 16;                   // more than one chunk of 256 centroids
-
-    const int64_t n_steps = (N + 63) / 64;
-    const int64_t stride = (int64_t)gridDim.x * WAVES;
-    const bool packed16 = SUB == 8 && xt != VQ_F32;   // one 16-byte load per sub-vector, fetched a step ahead
-    const bool packed8 = SUB == 4 && xt != VQ_F32;
-    auto load_raw = [&](int64_t step) {
+    const u32 *a_ptr = s_img + (lane & 31) * IW + half * (SUB == 4 ? 2 : 4);
+    const u32 mask = ~127u;
+    // steps go to the blocks first, then to a block's waves: fewer steps than waves leave every CU its share
+    const int64_t n_steps = (j.N + 63) / 64, stride = (int64_t)gridDim.x * WAVES;
+    int64_t step = (int64_t)wave * gridDim.x + blockIdx.x;
+    uint4 raw = load_raw<SUB>(j.x, j.xt, step * 64 + lane, step * 64 + lane < j.N);
+    for (; step < n_steps; step += stride) {
         const int64_t sv = step * 64 + lane;
-        uint4 r = make_uint4(0, 0, 0, 0);
-        if (step < n_steps && sv < N) {
-            if (packed16) r = *reinterpret_cast<const uint4 *>((const u16 *)x + sv * 8);
-            else if (packed8) { const uint2 t = *reinterpret_cast<const uint2 *>((const u16 *)x + sv * 4); r.x = t.x; r.y = t.y; }
+        const bool live = sv < j.N;
+        SubVec<SUB> s;
+        take_subvec<SUB, LT>(s, j.x, j.xt, raw, sv, live, lane, j.kx);
+        {
+            const int64_t nx = sv + stride * 64;
+            raw = load_raw<SUB>(j.x, j.xt, nx, nx < j.N);
         }
-        return r;
-    };
-    uint4 raw = load_raw((int64_t)blockIdx.x * WAVES + wave);
-    for (int64_t step = (int64_t)blockIdx.x * WAVES + wave; step < n_steps; step += stride) {
-        const int64_t sv = step * 64 + lane;   // this lane's sub-vector
-        const uint4 raw_next = load_raw(step + stride);
-        // ---- convert, split, bounce through LDS
-        float xf[8];
+        make_operands<SUB>(s, cs);
+        u32 k1[2] = {~0u, ~0u}, k2[2] = {~0u, ~0u};
+        auto product = [&](const u32 *ap, f32x16 *D) {
+            const f32x16 zero = {};
+            if constexpr (SUB == 4) {
+                const uint2 p = *reinterpret_cast<const uint2 *>(ap), q = *reinterpret_cast<const uint2 *>(ap + 2);
+                const f16x8 A = h8(p.x, p.y, q.x, q.y);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) xf[e] = 0.f;
-        if (packed16 || packed8) {
-            const u32 w[4] = {raw.x, raw.y, raw.z, raw.w};
+                for (int b = 0; b < 2; ++b) D[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, s.B1[b], zero, 0, 0, 0);
+            } else {
+                // words 0..3 / 4..7 of the first product, 0..3 / 8..11 of the second
+                const f16x8 A1 = *reinterpret_cast<const f16x8 *>(ap), A2 = *reinterpret_cast<const f16x8 *>(ap + half * 4);
 #pragma unroll
-            for (int e = 0; e < SUB / 2; ++e) {
-                if (xt == VQ_F16) {
-                    const f16x2 h = __builtin_bit_cast(f16x2, w[e]);
-                    xf[2 * e] = (float)h[0]; xf[2 * e + 1] = (float)h[1];
-                } else {
-                    xf[2 * e] = __uint_as_float(w[e] << 16); xf[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
+                for (int b = 0; b < 2; ++b) {
+                    D[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A1, s.B1[b], zero, 0, 0, 0);
+                    D[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A2, s.B2[b], D[b], 0, 0, 0);
                 }
+            }
+        };
+        const u32 *ap = a_ptr;
+        auto track = [&](int b, const f32x16 &d, int t) {
+            if constexpr (FINE) keep_quarters(k1[b], k2[b], d, mask, t);
+            else keep_two(k1[b], k2[b], cell_key(d, mask, t));
+        };
+        f32x16 D[2];
+        if constexpr (SUB == 4) {   // one tile's products are on their way while the other's scores are reduced
+            f32x16 E[2];
+            product(ap, D);
+#pragma unroll 1
+            for (int t = 0; t < ntiles; t += 2) {
+                ap += 32 * IW;
+                product(ap, E);
+#pragma unroll
+                for (int b = 0; b < 2; ++b) track(b, D[b], t);
+                if (t + 2 < ntiles) {
+                    ap += 32 * IW;
+                    product(ap, D);
+                }
+#pragma unroll
+                for (int b = 0; b < 2; ++b) track(b, E[b], t + 1);
             }
         } else {
+#pragma unroll 1
+            for (int t = 0; t < ntiles; ++t, ap += 32 * IW) {
+                product(ap, D);
 #pragma unroll
-            for (int e = 0; e < SUB; ++e) xf[e] = sv < N ? ld_any(x, xt, sv * SUB + e) : 0.f;
-        }
-        float sm[8];
-        if constexpr (LT > 0) {
-            // the lane's channels of its token: divide by the smoothing factors, transform, scale
-            const int64_t token = sv / LT;
-            const int64_t srow = kx.smooth_rows > 1 ? (token / kx.S) % kx.heads : 0;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) sm[e] = 1.f;
-            if (kx.smooth != nullptr && sv < N) {
-                const float *sp = kx.smooth + (srow * LT + (lane & (LT - 1))) * SUB;
-#pragma unroll
-                for (int e = 0; e < SUB; ++e) { sm[e] = sp[e]; xf[e] = xf[e] / sm[e]; }
-            }
-            wht_lanes<SUB, LT>(xf, lane);
-#pragma unroll
-            for (int e = 0; e < SUB; ++e) xf[e] *= kx.h;
-            if (kx.k_tilde != nullptr && sv < N) {
-#pragma unroll
-                for (int e = 0; e < SUB; e += 4)
-                    *reinterpret_cast<float4 *>(kx.k_tilde + sv * SUB + e) = make_float4(xf[e], xf[e + 1], xf[e + 2], xf[e + 3]);
+                for (int b = 0; b < 2; ++b) track(b, D[b], t);
             }
         }
-        f16x8 xh, xl;
-        float x2 = 0.f;   // |v|^2 for the margin only: fused multiply-adds will do
+        // both halves' cells of the lane's own sub-vector: column block = lane / 32
+        swap_halves(k1[0], k1[1]);
+        swap_halves(k2[0], k2[1]);
+        const bool low_first = k1[0] <= k1[1];   // [0]: rows of lanes 0..31, [1]: of lanes 32..63
+        const u32 f1 = low_first ? k1[0] : k1[1], o1 = low_first ? k1[1] : k1[0];
+        const u32 n1 = low_first ? k2[0] : k2[1], n2 = low_first ? k2[1] : k2[0];
+        const int h1 = low_first ? 0 : 1;
+        const float lim = __uint_as_float(f1) + margin<SUB>(s, f1);
+        const bool second = !(__uint_as_float(o1) > lim);             // a cell of the other half may hold the winner
+        const bool all = s.far || !(__uint_as_float(n1) > lim) || (second && !(__uint_as_float(n2) > lim));
+        float dbest = INFINITY;
+        int my_idx = 0;
+        auto eval_cell = [&](u32 key, int hf) {
+            constexpr int ALL = FINE ? 4 : 16, N = FINE || SUB == 8 ? 4 : 8;   // rows, and rows in flight: more would spill
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x2 = __builtin_fmaf(xf[e], xf[e], x2);
-        if (LT == 0 && packed16 && xt == VQ_F16) {
-            // fp16 sub-vectors as they came: they are their own high part, the remainder is zero
-            xh = __builtin_bit_cast(f16x8, raw);
-            xl = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        } else {
+            for (int g = 0; g < ALL; g += N) {
+                int c[N];
+                float row[N][SUB];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                xh[e] = (f16)xf[e];
-                xl[e] = (f16)(xf[e] - (float)xh[e]);
+                for (int r = 0; r < N; ++r) {
+                    const int first = FINE ? cell_centroid((key & 127u) >> 2, hf, key & 3u) : cell_centroid(key, hf, (g + r) >> 2);
+                    c[r] = min(first + (r & 3), j.nc - 1);
+                }
+                load_centroids<SUB, N>(j.cb, j.ct, aligned, c, row);
+#pragma unroll
+                for (int r = 0; r < N; ++r) take_nearer(dbest, my_idx, exact_dist<SUB>(s.xf, row[r]), c[r]);
             }
-        }
-        if constexpr (SUB == 4) {   // [high | high] and [remainder | remainder]
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { xh[4 + e] = xh[e]; xl[4 + e] = xl[e]; }
-        }
-        auto stage = [&]() {   // the lane's sub-vector into the wave's staging rows
-            *reinterpret_cast<f16x8 *>(&s_xh[lane][0]) = xh;
-            *reinterpret_cast<f16x8 *>(&s_xh[lane][8]) = xl;
-            *reinterpret_cast<float4 *>(&s_xf[lane][0]) = make_float4(xf[0], xf[1], xf[2], xf[3]);
-            *reinterpret_cast<float4 *>(&s_xf[lane][4]) = make_float4(xf[4], xf[5], xf[6], xf[7]);
-            // the wave reads what its own lanes wrote: LDS serves a wave's requests in order
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         };
-        stage();
-
-        // B operands of the four column groups: sub-vector 16 t + n
-        f16x8 B[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            B[t] = *reinterpret_cast<const f16x8 *>(&s_xh[16 * t + n][8 * (blk & 1)]);
-            if (SUB == 4 && blk >= 2) B[t] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        }
-        // the lane's sorted pair of every column group, over all chunks: key and chunk number
-        float K1[4], K2[4];
-        int Q1[4], Q2[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) { K1[t] = INFINITY; K2[t] = INFINITY; Q1[t] = 0; Q2[t] = 0; }
-
-#pragma unroll 1
-        for (int t0 = 0; t0 < ntiles; t0 += 16) {
-            // two sorted pairs a lane and column group: accumulator registers 0, 1 feed one, 2, 3 the other (twice
-            // the trackers at the same cost: the leaders of a column less often share one)
-            float k1[4], k2[4], m1[4], m2[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) { k1[t] = INFINITY; k2[t] = INFINITY; m1[t] = INFINITY; m2[t] = INFINITY; }
-            const char *tp = s_tiles + (size_t)t0 * 16 * CB + a_off;
-            const char *cp = reinterpret_cast<const char *>(s_c2 + t0 * 16) + c_off;
-            const int left = ntiles - t0;   // tiles of this chunk (tiles past the codebook's end do not exist in LDS)
-#pragma unroll
-            for (int j4 = 0; j4 < 16; j4 += 4) {
-                if (j4 < left) {
-#pragma unroll
-                    for (int j = j4; j < j4 + 4; ++j) {
-                        const f16x8 A = *reinterpret_cast<const f16x8 *>(tp + j * 16 * CB);
-                        const float4 c4 = *reinterpret_cast<const float4 *>(cp + j * 64);
-                        const f32x4 C = {c4.x, c4.y, c4.z, c4.w};
-                        f32x4 D[4];
-#pragma unroll
-                        for (int t = 0; t < 4; ++t) D[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[t], C, 0, 0, 0);
-#pragma unroll
-                        for (int t = 0; t < 4; ++t) {
-                            track2(k1[t], k2[t], tagged(D[t][0], 4 * j), tagged(D[t][1], 4 * j + 1));
-                            track2(m1[t], m2[t], tagged(D[t][2], 4 * j + 2), tagged(D[t][3], 4 * j + 3));
-                        }
-                    }
-                }
-            }
-            // fold the chunk into the lane's pair (an earlier chunk keeps its place on equal keys)
-            const int q = t0 >> 4;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                {   // the lane's two pairs into one (keys are distinct: they carry their register)
-                    const float hi = vmax(k1[t], m1[t]);
-                    k1[t] = vmin(k1[t], m1[t]);
-                    k2[t] = vmin3(hi, k2[t], m2[t]);
-                }
-                if (!multi) { K1[t] = k1[t]; K2[t] = k2[t]; continue; }
-                const bool first = k1[t] < K1[t];
-                const float o1 = K1[t], o2 = K2[t];
-                const int p1 = Q1[t], p2 = Q2[t];
-                K1[t] = first ? k1[t] : o1;
-                Q1[t] = first ? q : p1;
-                // the second: of (old first, new second) when the new first leads, else of (old second, new first)
-                const float sa = first ? o1 : o2, sb = first ? k2[t] : k1[t];
-                const int pa = first ? p1 : p2;
-                const bool keep = !(sb < sa);
-                K2[t] = keep ? sa : sb;
-                Q2[t] = keep ? pa : q;
-            }
-        }
-
-        // ---- the pairs change hands through the staging rows (whose sub-vectors sit in registers as well): lane
-        // (n, blk) collects the four lanes' pairs of column group blk -- the group its own sub-vector 16 blk + n
-        // belongs to -- and decides that one column by itself: one decision a lane instead of four.
-        __builtin_amdgcn_wave_barrier();   // every B operand has been read
-        {
-            uint4 *ex = reinterpret_cast<uint4 *>(s_stage + wave * 4096);   // [group][n][source lane group]
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-                ex[(t * 16 + n) * 4 + blk] = make_uint4(__float_as_uint(K1[t]), __float_as_uint(K2[t]), (u32)Q1[t], (u32)Q2[t]);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        // smallest three of the eight tracked scores of the column, the first two with their origin (source lane
-        // group, chunk); equal keys of different origins are different centroids: the earlier source comes first
-        float f1 = INFINITY, f2 = INFINITY, g3 = INFINITY;
-        int o1 = 0, o2 = 0;
-        {
-            const uint4 *ex = reinterpret_cast<const uint4 *>(s_stage + wave * 4096) + (blk * 16 + n) * 4;
-#pragma unroll
-            for (int src = 0; src < 4; ++src) {
-                const uint4 e = ex[src];
-                const float a[2] = {__uint_as_float(e.x), __uint_as_float(e.y)};
-                const int q[2] = {(int)e.z * 4 + src, (int)e.w * 4 + src};
-#pragma unroll
-                for (int k = 0; k < 2; ++k) {   // insert a[k] into the sorted triple
-                    const bool b1 = a[k] < f1, b2 = a[k] < f2;
-                    g3 = b2 ? f2 : vmin(g3, a[k]);
-                    f2 = b1 ? f1 : (b2 ? a[k] : f2);
-                    o2 = b1 ? o1 : (b2 ? q[k] : o2);
-                    f1 = b1 ? a[k] : f1;
-                    o1 = b1 ? q[k] : o1;
-                }
-            }
-        }
-        const float eps = 6.103515625e-05f * (x2 + cmax2);   // 2^-14 (|v|^2 + max |c|^2)
-        // centroid of a key: chunk * 256 + 16 * tile + 4 * lane group + register
-        auto centroid = [&](float key, int org) {
-            const u32 b = __float_as_uint(key) & 63u;
-            return (org >> 2) * 256 + (int)((b >> 2) * 16u + (u32)(org & 3) * 4u + (b & 3u));
-        };
-        const int i1 = centroid(f1, o1), i2 = centroid(f2, o2);
-        int my_idx = i1;
-        const bool unsure = !(f2 - f1 > eps);
-        if (__any(unsure)) {
-            // Whatever a lane dropped (inside a tracker, or when its trackers and chunks were merged into one pair)
-            // is at least that lane's second entry, so when the leading two come from different lanes nothing
-            // untracked lies below g3, the third smallest tracked score.
-            const bool other_lane = ((o1 ^ o2) & 3) != 0;
-            const bool two = unsure && other_lane && (g3 - f1 > eps) && i1 < nc && i2 < nc;
-            if (two) {   // exactly two contenders: the exact rule on both
-                const float d1 = exact_dist_c<SUB>(xf, s_tiles, cb, ct, i1), d2 = exact_dist_c<SUB>(xf, s_tiles, cb, ct, i2);
-                my_idx = (d2 < d1 || (d2 == d1 && i2 < i1)) ? i2 : i1;
-            }
-            const bool many = unsure && !two;
-            const unsigned long long many_mask = __ballot(many);
-            if (many_mask != 0) {
-                // Recompute the scores of every such column and apply the exact rule to every centroid the filter
-                // cannot exclude: the four lanes of a column work together again, so the sub-vectors go back into
-                // the staging rows first.  A tile without such a centroid (nearly all) costs one product and four
-                // compares.
-                __builtin_amdgcn_wave_barrier();   // the exchanged pairs have been read
-                stage();
-                const float thr_own = f1 + eps;
-#pragma unroll 1
-                for (int t = 0; t < 4; ++t) {
-                    if (((many_mask >> (16 * t)) & 0xFFFFull) == 0) continue;
-                    const bool col = ((many_mask >> (16 * t + n)) & 1ull) != 0;   // this lane's column of group t
-                    const float thr = __shfl(thr_own, 16 * t + n);
-                    const float *xv = &s_xf[16 * t + n][0];
-                    const f16x8 Bt = *reinterpret_cast<const f16x8 *>(&s_xh[16 * t + n][8 * (blk & 1)]);
-                    const f16x8 Bz = (SUB == 4 && blk >= 2) ? f16x8{0, 0, 0, 0, 0, 0, 0, 0} : Bt;
-                    float dbest = INFINITY;
-                    int ibest = 0x7fffffff;
-#pragma unroll 1
-                    for (int j = 0; j < ntiles; ++j) {
-                        const f16x8 A = *reinterpret_cast<const f16x8 *>(s_tiles + (size_t)j * 16 * CB + a_off);
-                        const float4 c4 = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(s_c2 + j * 16) + c_off);
-                        const f32x4 D = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, Bz, f32x4{c4.x, c4.y, c4.z, c4.w}, 0, 0, 0);
-                        const int c0 = 16 * j + 4 * blk;
-                        const bool h0 = col && c0 < nc && D[0] <= thr, h1 = col && c0 + 1 < nc && D[1] <= thr;
-                        const bool h2 = col && c0 + 2 < nc && D[2] <= thr, h3 = col && c0 + 3 < nc && D[3] <= thr;
-                        if (!__any(h0 || h1 || h2 || h3)) continue;
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const bool h = r == 0 ? h0 : r == 1 ? h1 : r == 2 ? h2 : h3;
-                            if (h) {
-                                const float d = exact_dist_c<SUB>(xv, s_tiles, cb, ct, c0 + r);
-                                if (d < dbest || (d == dbest && c0 + r < ibest)) { dbest = d; ibest = c0 + r; }
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int o = 16; o <= 32; o <<= 1) {
-                        const float d = __shfl_xor(dbest, o);
-                        const int ci = __shfl_xor(ibest, o);
-                        if (d < dbest || (d == dbest && ci < ibest)) { dbest = d; ibest = ci; }
-                    }
-                    if (blk == t && many) my_idx = ibest;
-                }
-            }
-        }
-        if (sv < N) st_idx(idx, it, sv, my_idx);
-        if constexpr (LT > 0) {
-            if (kx.k_hat != nullptr) {   // block-uniform
-                float c[8];
-                const int ci = my_idx < nc ? my_idx : nc - 1;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) c[e] = e < SUB ? ld_any(cb, ct, (int64_t)ci * SUB + e) : 0.f;
-                wht_lanes<SUB, LT>(c, lane);
-#pragma unroll
-                for (int e = 0; e < SUB; ++e) c[e] = c[e] * kx.h * sm[e];
-                if (sv < N) {
-                    if (kx.hat_dtype == VQ_F32) {
-#pragma unroll
-                        for (int e = 0; e < SUB; e += 4)
-                            *reinterpret_cast<float4 *>((float *)kx.k_hat + sv * SUB + e) = make_float4(c[e], c[e + 1], c[e + 2], c[e + 3]);
-                    } else {
-                        u32 w[4];
-#pragma unroll
-                        for (int e = 0; e < SUB; e += 2) {
-                            if (kx.hat_dtype == VQ_F16) w[e / 2] = __builtin_bit_cast(u32, f16x2{(f16)c[e], (f16)c[e + 1]});
-                            else w[e / 2] = (u32)f32_to_bf16(c[e]) | ((u32)f32_to_bf16(c[e + 1]) << 16);
-                        }
-                        if constexpr (SUB == 8) *reinterpret_cast<uint4 *>((u16 *)kx.k_hat + sv * 8) = make_uint4(w[0], w[1], w[2], w[3]);
-                        else *reinterpret_cast<uint2 *>((u16 *)kx.k_hat + sv * 4) = make_uint2(w[0], w[1]);
-                    }
-                }
-            }
-        }
-        raw = raw_next;
-        __builtin_amdgcn_wave_barrier();   // the next step overwrites this wave's LDS slots
+        my_idx = 0x7fffffff;
+        eval_cell(f1, h1);
+        if (__any(second)) { if (second) eval_cell(o1, 1 - h1); }
+        const unsigned long long m = __ballot(all);
+        if (m != 0) scan_all<SUB>(m, s.xf, j.cb, j.ct, aligned, j.nc, lane, my_idx);
+        store_result<SUB, LT>(sv, my_idx, s, j.cb, j.ct, aligned, j.idx, j.it, j.dst, j.kx, lane, live);
     }
 }
 
-// ---- launch: sixteen waves to a CU, as two blocks of eight or, when the codebook image is large, one of sixteen
-template <int SUB, int LT, int WAVES>
-static void launch_tiles_waves(const void *x, int xt, int64_t N, const void *cb, int ct, int nc, void *idx, int it,
-                               const KeyXform &kx, size_t image, int blocks_per_cu, hipStream_t st) {
-    auto kernel = vq_assign_mfma_kernel<SUB, LT, WAVES>;
+// ---- SPLIT: one block for 64 sub-vectors, the tiles shared out over its waves -------------------
+
+template <int WAVES> struct SplitLds {
+    float red[WAVES];
+    u32 keys[64][WAVES][4];   // of a sub-vector, wave by wave: two smallest cells of each half
+    float xf[64][8];
+    float x2[64];
+    int idx[64];
+};
+
+// TW: tiles a wave takes at most
+template <int SUB, int LT, int WAVES, int TW>
+__device__ __forceinline__ void assign_split(const AssignJob &j, int64_t block, SplitLds<WAVES> &lds) {
+    constexpr int IW = image_words<SUB>();
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ntiles = (j.nc + 31) / 32;
+    const bool aligned = (reinterpret_cast<uintptr_t>(j.cb) & 15u) == 0;
+    const int64_t sv = block * 64 + lane;
+    const bool live = sv < j.N;
+    const uint4 raw = load_raw<SUB>(j.x, j.xt, sv, live);
+    int rc[TW];
+    float row[TW][SUB];
+    float cmax2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < TW; ++i) rc[i] = min((wave + i * WAVES) * 32 + (lane & 31), j.nc - 1);   // tiles wave, wave + WAVES, ..; past the end: the last centroid again
+    load_centroids<SUB, TW>(j.cb, j.ct, aligned, rc, row);
+#pragma unroll
+    for (int i = 0; i < TW; ++i) cmax2 = fmaxf(cmax2, norm2<SUB>(row[i]));
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) cmax2 = fmaxf(cmax2, __shfl_xor(cmax2, o));
+    if (lane == 0) lds.red[wave] = cmax2;
+    SubVec<SUB> s;
+    take_subvec<SUB, LT>(s, j.x, j.xt, raw, sv, live, lane, j.kx);
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) cmax2 = fmaxf(cmax2, lds.red[w]);
+    const float cs = codebook_scale(cmax2);
+    make_operands<SUB>(s, cs);
+    if (wave == 0) {
+#pragma unroll
+        for (int e = 0; e < SUB; e += 4) *reinterpret_cast<float4 *>(&lds.xf[lane][e]) = make_float4(s.xf[e], s.xf[e + 1], s.xf[e + 2], s.xf[e + 3]);
+        lds.x2[lane] = s.far ? -1.f : s.x2;
+    }
+    u32 k1[2] = {~0u, ~0u}, k2[2] = {~0u, ~0u};
+    const u32 mask = ~127u;
+#pragma unroll
+    for (int i = 0; i < TW; ++i) {
+        const int t = wave + i * WAVES;
+        if (t < ntiles) {   // wave-uniform
+            u32 img[IW];
+            centroid_image<SUB>(row[i], cs, img);
+            f32x16 D[2];
+            const f32x16 zero = {};
+            if constexpr (SUB == 4) {
+                const f16x8 A = h8(half ? img[2] : img[0], half ? img[3] : img[1], half ? img[4] : img[2], half ? img[5] : img[3]);
+#pragma unroll
+                for (int b = 0; b < 2; ++b) D[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, s.B1[b], zero, 0, 0, 0);
+            } else {
+                const f16x8 A1 = h8(half ? img[4] : img[0], half ? img[5] : img[1], half ? img[6] : img[2], half ? img[7] : img[3]);
+                const f16x8 A2 = h8(half ? img[8] : img[0], half ? img[9] : img[1], half ? 0u : img[2], half ? 0u : img[3]);
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    D[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A1, s.B1[b], zero, 0, 0, 0);
+                    D[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A2, s.B2[b], D[b], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < 2; ++b) keep_two(k1[b], k2[b], cell_key(D[b], mask, t));
+        }
+    }
+    swap_halves(k1[0], k1[1]);
+    swap_halves(k2[0], k2[1]);
+    *reinterpret_cast<uint4 *>(&lds.keys[lane][wave][0]) = make_uint4(k1[0], k2[0], k1[1], k2[1]);
+    __syncthreads();
+
+    // merge: WAVES lanes a sub-vector, each with one wave's four cells
+    const int g = tid / WAVES, l = tid % WAVES;   // sub-vector of the block, lane of its group
+    {
+        const uint4 e = *reinterpret_cast<const uint4 *>(&lds.keys[g][l][0]);
+        // a tracker is (wave, half); of its two cells the first can lead, the second bounds what it dropped
+        u32 f1 = min(e.x, e.z), f2 = max(e.x, e.z), bound = min(e.y, e.w);
+        int o1 = 2 * l + (e.z < e.x), o2 = 2 * l + !(e.z < e.x);
+#pragma unroll
+        for (int o = 1; o < WAVES; o <<= 1) {
+            const u32 g1 = __shfl_xor(f1, o), g2 = __shfl_xor(f2, o);
+            const int p1 = __shfl_xor(o1, o), p2 = __shfl_xor(o2, o);
+            bound = min(bound, (u32)__shfl_xor(bound, o));
+            const bool mine = f1 < g1 || (f1 == g1 && o1 < p1);
+            // the second of the pair, and what falls out joins the bound
+            const u32 a = mine ? f2 : g2, b = mine ? g1 : f1, c = mine ? g2 : f2;
+            const int pa = mine ? o2 : p2, pb = mine ? p1 : o1;
+            f1 = mine ? f1 : g1;
+            o1 = mine ? o1 : p1;
+            const bool keep = a < b || (a == b && pa < pb);
+            f2 = keep ? a : b;
+            o2 = keep ? pa : pb;
+            bound = min(bound, min(keep ? b : a, c));
+        }
+        SubVec<SUB> v;
+        v.x2 = lds.x2[g];
+        const bool far = v.x2 < 0.f;
+        float xs[SUB];
+#pragma unroll
+        for (int e = 0; e < SUB; e += 4) {
+            const float4 t = *reinterpret_cast<const float4 *>(&lds.xf[g][e]);
+            xs[e] = t.x; xs[e + 1] = t.y; xs[e + 2] = t.z; xs[e + 3] = t.w;
+        }
+        const float lim = __uint_as_float(f1) + margin<SUB>(v, f1);
+        const bool second = !(__uint_as_float(f2) > lim), all = far || !(__uint_as_float(bound) > lim);
+        float d = INFINITY;
+        int i = 0x7fffffff;
+        // sixteen rows of a cell, 16 / WAVES a lane
+#pragma unroll
+        for (int k = 0; k < 16 / WAVES; ++k) {
+            const int r = l * (16 / WAVES) + k, c = min(cell_centroid(f1, o1 & 1, r >> 2) + (r & 3), j.nc - 1);
+            float rw[SUB];
+            load_centroid<SUB>(j.cb, j.ct, aligned, c, rw);
+            take_nearer(d, i, exact_dist<SUB>(xs, rw), c);
+        }
+        if (__any(second)) {
+            if (second) {
+#pragma unroll
+                for (int k = 0; k < 16 / WAVES; ++k) {
+                    const int r = l * (16 / WAVES) + k, c = min(cell_centroid(f2, o2 & 1, r >> 2) + (r & 3), j.nc - 1);
+                    float rw[SUB];
+                    load_centroid<SUB>(j.cb, j.ct, aligned, c, rw);
+                    take_nearer(d, i, exact_dist<SUB>(xs, rw), c);
+                }
+            }
+        }
+#pragma unroll
+        for (int o = 1; o < WAVES; o <<= 1) take_nearer(d, i, __shfl_xor(d, o), __shfl_xor(i, o));
+        const unsigned long long m = __ballot(all && l == 0);   // one lane of each group
+        if (m != 0) scan_all<SUB>(m, xs, j.cb, j.ct, aligned, j.nc, lane, i);
+        if (l == 0) lds.idx[g] = i;
+    }
+    __syncthreads();
+    if (wave == 0) store_result<SUB, LT>(sv, lds.idx[lane], s, j.cb, j.ct, aligned, j.idx, j.it, j.dst, j.kx, lane, live);
+}
+
+template <int SUB, int LT, int WAVES, int TW>
+__global__ __launch_bounds__(64 * WAVES) void vq_assign_split_kernel(AssignJob j) {
+    __shared__ SplitLds<WAVES> lds;
+    assign_split<SUB, LT, WAVES, TW>(j, blockIdx.x, lds);
+}
+
+// ---- launch -----------------------------------------------------------------------------------
+
+template <int SUB, int LT, int WAVES, bool FINE>
+static void launch_image(const AssignJob &j, size_t image, int blocks_per_cu, hipStream_t st) {
+    auto kernel = vq_assign_image_kernel<SUB, LT, WAVES, FINE>;
     // more than 64 KB of block-shared memory has to be allowed per kernel and device, once (a second
     // thread that gets here first repeats the same call)
     static std::atomic<bool> allowed[64] = {};
@@ -548,43 +774,39 @@ static void launch_tiles_waves(const void *x, int xt, int64_t N, const void *cb,
         (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256);
         if (dev >= 0 && dev < 64) allowed[dev].store(true, std::memory_order_release);
     }
-    int64_t blocks = cdiv(cdiv(N, 64), WAVES);
+    int64_t blocks = cdiv(j.N, 64);
     if (blocks > 256 * blocks_per_cu) blocks = 256 * blocks_per_cu;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(64 * WAVES), image + (size_t)WAVES * 4096, st, x, xt, N, cb, ct, nc,
-                       idx, it, kx);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(64 * WAVES), image, st, j);
 }
 
-template <int SUB, int LT>
-static bool launch_tiles(const void *x, int xt, int64_t N, const void *cb, int ct, int nc, void *idx, int it, const KeyXform &kx,
-                         hipStream_t st) {
-    const int nc16 = (nc + 63) / 64 * 64;
-    const size_t image = (size_t)nc16 * (cent_bytes<SUB>() + 4);
-    if (image + 8 * 4096 <= 78 * 1024) launch_tiles_waves<SUB, LT, 8>(x, xt, N, cb, ct, nc, idx, it, kx, image, 2, st);
-    else if (image + 16 * 4096 <= 159 * 1024) launch_tiles_waves<SUB, LT, 16>(x, xt, N, cb, ct, nc, idx, it, kx, image, 1, st);
-    else return false;
+template <int SUB, int LT> static bool launch_job(const AssignJob &j, hipStream_t st) {
+    if (j.nc > (SUB == 8 ? VM_MAXC / 2 : VM_MAXC)) return false;
+    const size_t image = (size_t)((j.nc + 63) / 64) * 64 * image_words<SUB>() * 4;
+    if (j.nc <= kFineC) launch_image<SUB, LT, 8, true>(j, image, 2, st);
+    else if (j.nc > kSplitC && j.N <= kSplitMax)
+        hipLaunchKernelGGL((vq_assign_split_kernel<SUB, LT, 16, (SUB == 8 ? 4 : 8)>), dim3((unsigned)cdiv(j.N, 64)), dim3(1024), 0, st, j);
+    else if (image <= 78 * 1024) launch_image<SUB, LT, 8, false>(j, image, 2, st);
+    else launch_image<SUB, LT, 16, false>(j, image, 1, st);
     return true;
 }
 
 bool launch_assign_mfma(const void *x, int xt, int64_t N, const void *cb, int ct, int nc, int sub, void *idx, int it,
                         hipStream_t st) {
-    if (nc > VM_MAXC || !(sub == 4 || sub == 8)) return false;
+    if (!(sub == 4 || sub == 8)) return false;
     if (xt != VQ_F32 && ((uintptr_t)x & (sub == 8 ? 15u : 7u))) return false;
-    const KeyXform none = {};
-    return sub == 8 ? launch_tiles<8, 0>(x, xt, N, cb, ct, nc, idx, it, none, st)
-                    : launch_tiles<4, 0>(x, xt, N, cb, ct, nc, idx, it, none, st);
+    const AssignJob j = {x, xt, N, cb, ct, nc, idx, it, {-1, 1, 0}, {}};
+    return sub == 8 ? launch_job<8, 0>(j, st) : launch_job<4, 0>(j, st);
 }
 
 bool launch_encode_keys_mfma(const void *keys, int kt, int64_t B, int64_t heads, int64_t S, int64_t D, const float *smooth,
                              int smooth_rows, float h, const void *cb, int ct, int nc, int sub, void *idx, int it, void *k_hat,
                              float *k_tilde, hipStream_t st) {
-    if (nc > VM_MAXC || !(sub == 4 || sub == 8) || D % sub != 0) return false;
+    if (!(sub == 4 || sub == 8) || D % sub != 0 || B * heads * S > 0x7fffffff) return false;
     const int64_t lt = D / sub;
     if (!(lt == 8 || lt == 16 || lt == 32 || lt == 64)) return false;
     if (((uintptr_t)keys | (uintptr_t)k_hat | (uintptr_t)k_tilde | (uintptr_t)smooth) & 15u) return false;
-    const int64_t N = B * heads * S * lt;
-    const KeyXform kx = {smooth, smooth_rows, heads, S, h, k_hat, kt, k_tilde};
-#define VQ_ENC(SUB, LT) return launch_tiles<SUB, LT>(keys, kt, N, cb, ct, nc, idx, it, kx, st)
+    const AssignJob j = {keys, kt, B * heads * S * lt, cb, ct, nc, idx, it, {-1, 1, 0}, {smooth, smooth_rows, heads, S, h, k_hat, kt, k_tilde}};
+#define VQ_ENC(SUB, LT) return launch_job<SUB, LT>(j, st)
     if (sub == 8) { if (lt == 8) VQ_ENC(8, 8); else if (lt == 16) VQ_ENC(8, 16); else if (lt == 32) VQ_ENC(8, 32); else VQ_ENC(8, 64); }
     else { if (lt == 8) VQ_ENC(4, 8); else if (lt == 16) VQ_ENC(4, 16); else if (lt == 32) VQ_ENC(4, 32); else VQ_ENC(4, 64); }
 #undef VQ_ENC

@@ -736,7 +736,7 @@ def vecinfer_encode_decode_metal(keys: torch.Tensor, k_codebook: torch.Tensor, s
         sm = sm.contiguous()
     n_sub = D // sub_dim
     h = _sylvester_scale(H_mat)
-    fused = h > 0 and sub_dim in (4, 8) and n_sub in (8, 16, 32, 64) and cb.shape[0] <= 256
+    fused = h > 0 and sub_dim in (4, 8) and n_sub in (8, 16, 32, 64) and cb.shape[0] * sub_dim <= 16384
     if fused:
         idx = torch.empty((B, Hh, S, n_sub), dtype=index_dtype, device=keys.device)
         k_hat = torch.empty_like(kk) if want_k_hat else None
