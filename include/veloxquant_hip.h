@@ -176,6 +176,13 @@ int vq_kv_tail_append(const void *k_new, const void *v_new, const int64_t k_stri
                       void *k_tail, void *v_tail, int elem_bytes, int64_t B, int64_t H, int64_t S, int64_t D,
                       int64_t tail_cap, int64_t pos, void *stream);
 
+/* The first tokens of a plain cache: rows [0, S) of the contiguous buffers [B, H, cap, D] from
+ * k_new / v_new, rows [S, cap) zeroed, both buffers in one launch (arguments as above; the
+ * zeroed buffer a cache starts from and the assignment into it, veloxquant_mlx/cache/kivi_cache.py:248). */
+int vq_kv_fill(const void *k_new, const void *v_new, const int64_t k_strides[3], const int64_t v_strides[3],
+               void *k_buf, void *v_buf, int elem_bytes, int64_t B, int64_t H, int64_t S, int64_t D, int64_t cap,
+               void *stream);
+
 /* A whole chunk of a packed KIVI cache in one call: the concatenation, the quantisation of
  * the tokens that aged out of the fp16 residual window and the start of the next tail
  * (KIVIKVCache.update_and_fetch, veloxquant_mlx/cache/kivi_cache.py:206-262, on packed
@@ -472,6 +479,16 @@ int vq_vecinfer_attend(const vq_lut_attend_args *a);
 int vq_skvq_clipped_roundtrip(const void *x, void *out, int dtype, int64_t B, int64_t H, int64_t r, int64_t D,
                               int64_t x_stride_bh, int64_t out_stride_bh, const int32_t *perm, const int32_t *inv,
                               int bits, int group, const float *alphas, int n_alphas, void *stream);
+
+/* Channel order per head from a chunk of rows (SKVQKVCache._per_head_perms,
+ * veloxquant_mlx/cache/skvq_cache.py:186-224): the channels by their range (largest minus smallest value over
+ * the chunk, equal ranges in channel order) where that order has the lower mean squared float32 round-trip error, else
+ * the stored order.  perm / inv: device int32 [H, D], written.  x as for vq_skvq_clipped_roundtrip.
+ * workspace: vq_skvq_channel_orders_workspace bytes. */
+size_t vq_skvq_channel_orders_workspace(int64_t B, int64_t H, int64_t r, int64_t D, int group);
+int vq_skvq_channel_orders(const void *x, int dtype, int64_t B, int64_t H, int64_t r, int64_t D, int64_t x_stride_bh,
+                           int bits, int group, const float *alphas, int n_alphas, int32_t *perm, int32_t *inv,
+                           void *workspace, size_t workspace_bytes, void *stream);
 
 #ifdef __cplusplus
 }

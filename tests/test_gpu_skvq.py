@@ -206,3 +206,65 @@ def test_reorder_beats_identity_on_heterogeneous_channels():   # test_skvq_cache
         return float(np.mean((host(ko)[:, :, :q].astype(np.float32) - k[:, :, :q].astype(np.float32)) ** 2))
 
     assert mse(True) < mse(False)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("B,H,r,D,bits,g", [
+    (1, 1, 1, 8, 2, 8),          # one row, one piece
+    (2, 3, 123, 128, 4, 32),     # the cache's default chunk without its sinks
+    (1, 2, 37, 50, 3, 16),       # channels that do not move as 16-byte pieces, a ragged last group
+    (3, 2, 21, 80, 2, 32),
+    (1, 2, 9, 2056, 4, 64),      # more channels than a block has threads
+])
+def test_channel_orders_match_the_stated_rule(dtype, B, H, r, D, bits, g):
+    """Channels by range (stable), kept where the mean squared error of the float32 round trip is lower; heads whose two
+    errors are within 1e-9 of each other (the double sums differ by order, 1e-13 at most) may go either way."""
+    require_gpu()
+    rng = np.random.default_rng(D + bits)
+    x = to_dev((rng.standard_normal((B, H, r + 3, D)) * _het_scales(D, seed=D)).astype(np.float32)).to(dtype)
+    x[..., 5] = x[..., 2]                                    # equal ranges: channel order decides
+    rows = x[:, :, 3:]                                       # a token slice of a larger buffer
+    perm, inv = K.skvq_channel_orders(rows, bits, g, o.DEFAULT_ALPHA_GRID)
+    xn = rows.float().cpu().numpy()
+    span = xn.max(axis=(0, 2)) - xn.min(axis=(0, 2))
+    cand = np.argsort(span, axis=-1, kind="stable").astype(np.int32)
+    err = [np.square((o.round_trip(xn, p, None if p is None else np.argsort(p, axis=-1).astype(np.int32), bits, g, o.DEFAULT_ALPHA_GRID)
+                      - xn).astype(np.float64)).mean(axis=(0, 2, 3)) for p in (None, cand)]
+    for h in range(H):
+        clear = abs(err[1][h] - err[0][h]) > 1e-9 * err[0][h]
+        want = cand[h] if err[1][h] < err[0][h] else np.arange(D)
+        got = host(perm[h])
+        assert np.array_equal(got, want) or (not clear and (np.array_equal(got, cand[h]) or np.array_equal(got, np.arange(D))))
+        assert np.array_equal(host(inv[h])[got], np.arange(D))
+
+
+def test_channel_orders_put_ranges_that_are_not_numbers_last():
+    require_gpu()
+    x = torch.randn((1, 2, 16, 64), device="cuda:0") * torch.linspace(3.0, 0.1, 64, device="cuda:0")
+    x[0, 0, 4, 10] = float("nan")
+    x[0, 0, 4, 20] = float("inf")
+    perm, inv = K.skvq_channel_orders(x, 4, 64, (1.0,))      # the error of that head is not a number: the stored order stays
+    assert np.array_equal(host(perm[0]), np.arange(64)) and np.array_equal(host(inv[0]), np.arange(64))
+    with pytest.raises(ValueError, match="non-empty"):
+        K.skvq_channel_orders(x[:, :, :0], 4, 64, (1.0,))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,S,D,layout", [(1, 1, 1, 8, "bhsd"), (2, 3, 257, 128, "bhsd"), (2, 5, 130, 64, "bshd"), (1, 2, 19, 80, "slice"),
+                                            (1, 2, 5, 2056, "bhsd"), (1, 2, 7, 50, "bhsd")])
+def test_first_tokens_of_a_plain_cache(dtype, B, H, S, D, layout):
+    """The buffers a cache starts from: the tokens, then zeros, for rows that go through the one-launch copy and for
+    rows (50 channels) that do not."""
+    from veloxquant_mlx_amd.cache._fp16_cache import FP16KVCache
+    require_gpu()
+    torch.empty(1 << 22, device="cuda:0").fill_(float("nan"))    # recycled memory is not zero
+    make = {"bhsd": lambda: torch.randn((B, H, S, D), device="cuda:0").to(dtype),
+            "bshd": lambda: torch.randn((B, S, H, D), device="cuda:0").to(dtype).transpose(1, 2),
+            "slice": lambda: torch.randn((B, H, S + 8, D), device="cuda:0").to(dtype)[:, :, 8:]}[layout]
+    k, v = make(), make()
+    c = FP16KVCache()
+    ko, vo = c.update_and_fetch(k, v)
+    assert torch.equal(ko, k) and torch.equal(vo, v) and c.offset == S
+    assert c.keys.shape[2] == -(-S // 256) * 256 and not c.keys[:, :, S:].any() and not c.values[:, :, S:].any()
+    ko, vo = c.update_and_fetch(k[:, :, :1], v[:, :, :1])
+    assert torch.equal(ko[:, :, S:], k[:, :, :1]) and torch.equal(vo[:, :, :S], v)

@@ -22,6 +22,7 @@ namespace vq {
 
 constexpr int SK_THREADS = 256;
 constexpr int SK_MAX_ALPHAS = 8;
+constexpr int SK_AHEAD = 4;    // rows a thread requests at a time
 
 struct SkAlphas { float a[SK_MAX_ALPHAS]; int n; };
 
@@ -62,6 +63,18 @@ __device__ __forceinline__ void sk_codes8(const float *x, float (&q)[8], float l
 
 // eight consecutive elements as one (16-bit types) or two (float32) 16-byte accesses
 template <typename T> struct Vec8 {
+    struct Raw { uint4 w[sizeof(T) / 2]; };   // as loaded
+    static __device__ __forceinline__ Raw request(const T *p) {
+        Raw r;
+#pragma unroll
+        for (int i = 0; i < (int)sizeof(T) / 2; ++i) r.w[i] = reinterpret_cast<const uint4 *>(p)[i];
+        return r;
+    }
+    static __device__ __forceinline__ void unpack(const Raw &r, float (&v)[8]) {
+        const T *e = reinterpret_cast<const T *>(&r);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = Elem<T>::ld(e + k);
+    }
     static __device__ __forceinline__ void ld(const T *p, float (&v)[8]) {
         if constexpr (sizeof(T) == 4) {
             const float4 a = *reinterpret_cast<const float4 *>(p), b = *reinterpret_cast<const float4 *>(p + 4);
@@ -86,12 +99,16 @@ template <typename T> struct Vec8 {
     }
 };
 
-template <typename T, int GROUP>   // GROUP > 0: the group size, known at compile time; 0: any
+// ERR: the squared error of the float32 reconstruction instead of the reconstruction, the stored channel order
+// (blockIdx.y 0) against the order `perm` (1): err[(y n_rows + row) tpr + piece] takes the double-precision sum over
+// the channels of one thread's pieces, in stored channel order for both.
+template <typename T, int GROUP, bool ERR>   // GROUP > 0: the group size, known at compile time; 0: any
 __global__ __launch_bounds__(SK_THREADS)
-void skvq_roundtrip_kernel(const T *__restrict__ x, T *out, int64_t n_bh, int64_t H, int64_t r, int64_t D,
+void skvq_roundtrip_kernel(const T *x, T *out, double *__restrict__ err, int64_t n_bh, int64_t H, int64_t r, int64_t D,
                            int64_t x_stride_bh, int64_t out_stride_bh, const int32_t *__restrict__ perm, const int32_t *__restrict__ inv,
                            int group, uint64_t group_magic, int G, int rows_pb, int tpr, bool vec, float levels, SkAlphas al) {
     extern __shared__ float s_x[];
+    if (ERR && blockIdx.y == 0) perm = inv = nullptr;
     const int tid = threadIdx.x;
     const int gstride = group + 1, Dp = G * group;
     const int64_t row0 = (int64_t)blockIdx.x * rows_pb, n_rows = n_bh * r;   // n_rows < 2^31 (checked by the caller)
@@ -137,7 +154,40 @@ void skvq_roundtrip_kernel(const T *__restrict__ x, T *out, int64_t n_bh, int64_
             if (iv && j == (int)D - 1 && Dp > (int)D) fill_k = k;   // the order's last channel also fills a ragged last group
         }
     };
-    for (int lr = lr_base; lr < rows_pb && lr_base < rpp; lr += rpp) {
+    // Rows of one piece a thread: SK_AHEAD of them are requested before the first is put in its place (8 x 8 heads of 4091
+    // rows, in place, five factors and orders: 80 us, 83 us with one request at a time; stored order 69 and 74 us).
+    const bool ahead = vec && one_piece && cq * 8 < (int)D;
+    if (ahead) {
+        const int c0 = cq * 8;
+        for (int lr0 = lr_base; lr0 < rows_pb && lr_base < rpp; lr0 += SK_AHEAD * rpp) {
+            typename Vec8<T>::Raw raw[SK_AHEAD];
+            uint32_t head[SK_AHEAD];
+#pragma unroll
+            for (int i = 0; i < SK_AHEAD; ++i) {
+                const int lr = lr0 + i * rpp;
+                if (lr >= rows_pb || row0 + lr >= n_rows) continue;
+                const Where w = where(lr);
+                head[i] = w.head;
+                raw[i] = Vec8<T>::request(x + (int64_t)w.bh * x_stride_bh + (int64_t)w.t * D + c0);
+            }
+#pragma unroll
+            for (int i = 0; i < SK_AHEAD; ++i) {
+                const int lr = lr0 + i * rpp;
+                if (lr >= rows_pb || row0 + lr >= n_rows) continue;
+                float v[8];
+                Vec8<T>::unpack(raw[i], v);
+                place(head[i], c0);
+                float *dst = s_x + lr * G * gstride;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    dst[off[k]] = v[k];
+                    if (k == fill_k)
+                        for (int jp = (int)D; jp < Dp; ++jp) dst[pos(jp)] = v[k];
+                }
+            }
+        }
+    }
+    for (int lr = lr_base; !(ahead || (scatter && one_piece)) && lr < rows_pb && lr_base < rpp; lr += rpp) {
         if (row0 + lr >= n_rows) continue;
         const Where w = where(lr);
         const T *src = x + (int64_t)w.bh * x_stride_bh + (int64_t)w.t * D;
@@ -243,6 +293,29 @@ void skvq_roundtrip_kernel(const T *__restrict__ x, T *out, int64_t n_bh, int64_
     }
     __syncthreads();
 
+    if constexpr (ERR) {
+        for (int lr = lr_base; lr < rows_pb && lr_base < rpp; lr += rpp) {
+            if (row0 + lr >= n_rows) continue;
+            const Where w = where(lr);
+            const T *src = x + (int64_t)w.bh * x_stride_bh + (int64_t)w.t * D;
+            const int32_t *iv = inv ? inv + (int64_t)w.head * D : nullptr;
+            const float *srcl = s_x + lr * G * gstride;
+            double sum = 0.0;
+            for (int c0 = cq * 8; c0 < (int)D; c0 += tpr * 8) {
+                float v[8];
+                if (vec) Vec8<T>::ld(src + c0, v);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const int c = c0 + k;
+                    if (c >= (int)D) continue;
+                    const double d = (double)__fsub_rn(srcl[pos(iv ? iv[c] : c)], vec ? v[k] : Elem<T>::ld(src + c));
+                    sum += d * d;
+                }
+            }
+            err[((int64_t)blockIdx.y * n_rows + row0 + lr) * tpr + cq] = sum;
+        }
+        return;
+    }
     for (int lr = lr_base; lr < rows_pb && lr_base < rpp; lr += rpp) {
         if (row0 + lr >= n_rows) continue;
         const Where w = where(lr);
@@ -265,14 +338,132 @@ void skvq_roundtrip_kernel(const T *__restrict__ x, T *out, int64_t n_bh, int64_
     }
 }
 
-}  // namespace vq
+// ---- channel orders of the first flushed chunk (veloxquant_mlx/cache/skvq_cache.py:186-224) ----
+//
+// Three launches a tensor: the candidate order of every head (channels by their range over the chunk's rows, equal
+// ranges in channel order), the squared round-trip error of the stored and of the candidate order (the ERR form of the
+// kernel above), and the choice per head (the candidate only where its mean error is lower).  Latency is all there is
+// to them: 8 x 8 heads of 123 rows of 128 channels took 0.21 ms a tensor as library reductions and sorts.
+constexpr int SK_ORD_THREADS = 1024;
 
-using namespace vq;
+// floats as unsigned numbers in the same order (NaNs are kept apart)
+__device__ __forceinline__ uint32_t sk_key(float f) {
+    const uint32_t u = __float_as_uint(f);
+    return u & 0x80000000u ? ~u : u | 0x80000000u;
+}
+__device__ __forceinline__ float sk_unkey(uint32_t k) { return __uint_as_float(k & 0x80000000u ? k & 0x7fffffffu : ~k); }
 
-extern "C" int vq_skvq_clipped_roundtrip(const void *x, void *out, int dtype, int64_t B, int64_t H, int64_t r,
-                                         int64_t D, int64_t x_stride_bh, int64_t out_stride_bh, const int32_t *perm,
-                                         const int32_t *inv, int bits, int group, const float *alphas, int n_alphas, void *stream) {
-    const char *fn = "vq_skvq_clipped_roundtrip";
+// One block per head; W channels (8 where rows move as 16-byte pieces, else 1) a thread, so that the block reads
+// SK_ORD_THREADS / (D / W) rows at a time.  LDS: smallest, largest, NaN mark of every channel, then the ranges.
+template <typename T, int W>
+__global__ __launch_bounds__(SK_ORD_THREADS)
+void skvq_order_kernel(const T *__restrict__ x, int64_t B, int64_t H, int64_t r, int D, int64_t x_stride_bh,
+                       int32_t *__restrict__ perm, int32_t *__restrict__ inv) {
+    extern __shared__ uint32_t s_ord[];
+    uint32_t *s_mn = s_ord, *s_mx = s_ord + D, *s_nan = s_ord + 2 * D;
+    float *s_rng = reinterpret_cast<float *>(s_ord);
+    const int tid = threadIdx.x;
+    const int64_t h = blockIdx.x, n = B * r;
+    for (int c = tid; c < D; c += SK_ORD_THREADS) { s_mn[c] = ~0u; s_mx[c] = 0u; s_nan[c] = 0u; }
+    __syncthreads();
+    const int pieces = D / W, width = pieces < SK_ORD_THREADS ? pieces : SK_ORD_THREADS, rows = SK_ORD_THREADS / width;
+    const int p0 = tid % width, row0 = tid / width;
+    for (int p = p0; p < pieces && row0 < rows; p += width) {
+        float mn[W], mx[W];
+        uint32_t nan = 0u;
+#pragma unroll
+        for (int k = 0; k < W; ++k) { mn[k] = INFINITY; mx[k] = -INFINITY; }
+        int64_t b = row0 / r, t = row0 - b * r;   // the thread's next row, carried along: no division in the loop
+#pragma unroll 1
+        for (int64_t i = row0; i < n; i += SK_AHEAD * rows) {
+            typename Vec8<T>::Raw raw[SK_AHEAD];
+            float one[SK_AHEAD];
+#pragma unroll
+            for (int j = 0; j < SK_AHEAD; ++j) {
+                if (i + j * rows >= n) continue;
+                const T *src = x + (b * H + h) * x_stride_bh + t * D + (int64_t)p * W;
+                if constexpr (W == 8) raw[j] = Vec8<T>::request(src);
+                else one[j] = Elem<T>::ld(src);
+                for (t += rows; t >= r; t -= r) ++b;
+            }
+#pragma unroll
+            for (int j = 0; j < SK_AHEAD; ++j) {
+                if (i + j * rows >= n) continue;
+                float v[8];
+                if constexpr (W == 8) Vec8<T>::unpack(raw[j], v);
+                else v[0] = one[j];
+#pragma unroll
+                for (int k = 0; k < W; ++k) {
+                    mn[k] = fminf(mn[k], v[k]);
+                    mx[k] = fmaxf(mx[k], v[k]);
+                    nan |= v[k] != v[k] ? 1u << k : 0u;
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            atomicMin(&s_mn[p * W + k], sk_key(mn[k]));
+            atomicMax(&s_mx[p * W + k], sk_key(mx[k]));
+            if (nan >> k & 1u) s_nan[p * W + k] = 1u;
+        }
+    }
+    __syncthreads();
+    for (int c = tid; c < D; c += SK_ORD_THREADS)   // each thread its own words: the range takes the place of the smallest value
+        s_rng[c] = s_nan[c] ? NAN : __fsub_rn(sk_unkey(s_mx[c]), sk_unkey(s_mn[c]));
+    __syncthreads();
+    for (int c = tid; c < D; c += SK_ORD_THREADS) {   // place = channels before this one; a NaN comes after every number
+        const float mine = s_rng[c];
+        const bool mine_nan = mine != mine;
+        int place = 0;
+        for (int j = 0; j < D; ++j) {
+            const float o = s_rng[j];
+            const bool o_nan = o != o;
+            const bool before = mine_nan ? !o_nan : o < mine, same = mine_nan ? o_nan : o == mine;
+            place += (before || (same && j < c)) ? 1 : 0;
+        }
+        perm[h * D + place] = c;
+        inv[h * D + c] = place;
+    }
+}
+
+// One block per head: both orders' errors summed in one fixed order, and the head's order kept or replaced by the stored one.
+__global__ __launch_bounds__(SK_ORD_THREADS)
+void skvq_choose_kernel(const double *__restrict__ err, int64_t B, int64_t H, int64_t r, int tpr, int D,
+                        int32_t *__restrict__ perm, int32_t *__restrict__ inv) {
+    __shared__ double s_sum[2][SK_ORD_THREADS];
+    const int tid = threadIdx.x;
+    const int64_t h = blockIdx.x, n_rows = B * H * r, per_bh = r * tpr;
+    double a[2] = {0.0, 0.0};
+    int64_t b = tid / per_bh, i = tid - b * per_bh;   // the errors of the head, sequence after sequence
+    const double *e = err + h * per_bh, *e1 = e + n_rows * tpr;
+    const int64_t step = H * per_bh;
+#pragma unroll 8
+    for (int64_t n = tid; n < B * per_bh; n += SK_ORD_THREADS) {
+        a[0] += e[b * step + i];
+        a[1] += e1[b * step + i];
+        for (i += SK_ORD_THREADS; i >= per_bh; i -= per_bh) ++b;
+    }
+    s_sum[0][tid] = a[0];
+    s_sum[1][tid] = a[1];
+    for (int w = SK_ORD_THREADS / 2; w > 0; w >>= 1) {
+        __syncthreads();
+        if (tid < w) { s_sum[0][tid] += s_sum[0][tid + w]; s_sum[1][tid] += s_sum[1][tid + w]; }
+    }
+    __syncthreads();
+    const double count = (double)(B * r * D);
+    if (s_sum[1][0] / count < s_sum[0][0] / count) return;   // (an error that is not a number keeps the stored order)
+    for (int c = tid; c < D; c += SK_ORD_THREADS) perm[h * D + c] = inv[h * D + c] = c;
+}
+
+// how a round-trip launch covers its rows
+struct SkPlan {
+    int threads, tpr;
+    int64_t G, rows_pb, n_rows, blocks;
+    uint64_t group_magic;
+    size_t lds;
+};
+static int plan_skvq(const char *fn, int64_t B, int64_t H, int64_t r, int64_t D, int bits, int group, const float *alphas, int n_alphas,
+                     SkPlan &p, SkAlphas &al) {
     VQ_REQUIRE(bits >= 1 && bits <= 8, VQ_ERR_INVALID, "%s: bits must be in [1, 8], got %d", fn, bits);
     VQ_REQUIRE(group >= 1, VQ_ERR_INVALID, "%s: group_size must be >= 1, got %d", fn, group);
     VQ_REQUIRE(alphas && n_alphas >= 1 && n_alphas <= SK_MAX_ALPHAS, VQ_ERR_INVALID,
@@ -281,45 +472,102 @@ extern "C" int vq_skvq_clipped_roundtrip(const void *x, void *out, int dtype, in
         VQ_REQUIRE(alphas[k] > 0.f && alphas[k] <= 1.f, VQ_ERR_INVALID, "%s: alphas must lie in (0, 1], got %g", fn,
                    (double)alphas[k]);
     VQ_REQUIRE(B >= 0 && H >= 0 && r >= 0 && D >= 0, VQ_ERR_INVALID, "%s: negative dimension", fn);
+    al.n = n_alphas;
+    for (int k = 0; k < SK_MAX_ALPHAS; ++k) al.a[k] = k < n_alphas ? alphas[k] : 1.f;
+    p.G = (D + group - 1) / group;
+    const int64_t row_words = p.G * (group + 1);
+    VQ_REQUIRE(p.G <= SK_THREADS && row_words * 4 <= 48 * 1024 && group < 65536, VQ_ERR_UNSUPPORTED,
+               "%s: head_dim %lld with group %d does not fit a block (at most %d groups, 48 KB per row)", fn,
+               (long long)D, group, SK_THREADS);
+    if (B * H * r * D == 0) return VQ_OK;
+    // one wave per block where a wave covers whole rows: blocks then interleave freely on a CU (the
+    // phases of a block do not overlap each other, those of different blocks do)
+    p.threads = (p.G <= 64 && (p.G * group + 7) / 8 <= 64) ? 64 : SK_THREADS;
+    p.rows_pb = p.threads / p.G;
+    if (p.rows_pb * row_words * 4 > 48 * 1024) p.rows_pb = 48 * 1024 / (row_words * 4);
+    p.n_rows = B * H * r;
+    p.blocks = (p.n_rows + p.rows_pb - 1) / p.rows_pb;
+    VQ_REQUIRE(p.n_rows <= 0x7fffffff, VQ_ERR_UNSUPPORTED, "%s: too many rows (%lld)", fn, (long long)p.n_rows);
+    // floor(j / group) == (j * magic) >> 32 for j, group < 2^16 (a row holds at most 12288 words in LDS)
+    p.group_magic = (1ull << 32) / (uint64_t)group + 1;
+    const int64_t pieces = (p.G * group + 7) / 8;   // threads side by side on a row (eight channels each)
+    p.tpr = (int)(pieces < p.threads ? pieces : p.threads);
+    p.lds = (size_t)(p.rows_pb * row_words * 4);
+    return VQ_OK;
+}
+
+template <typename T, bool ERR>
+static void launch_skvq(const SkPlan &p, const SkAlphas &al, const void *x, void *out, double *err, int64_t B, int64_t H, int64_t r, int64_t D,
+                        int64_t xs, int64_t os, const int32_t *perm, const int32_t *inv, int bits, int group, bool vec, hipStream_t st) {
+    const dim3 grid((unsigned)p.blocks, ERR ? 2 : 1);
+    const float levels = (float)((1 << bits) - 1);
+#define VQ_SK_LAUNCH(GROUP)                                                                                                   \
+    hipLaunchKernelGGL((skvq_roundtrip_kernel<T, GROUP, ERR>), grid, dim3(p.threads), p.lds, st, (const T *)x, (T *)out, err, B * H, H, \
+                       r, D, xs, os, perm, inv, group, p.group_magic, (int)p.G, (int)p.rows_pb, p.tpr, vec, levels, al)
+    if (group == 32) VQ_SK_LAUNCH(32);
+    else if (group == 64) VQ_SK_LAUNCH(64);
+    else VQ_SK_LAUNCH(0);
+#undef VQ_SK_LAUNCH
+}
+
+}  // namespace vq
+
+using namespace vq;
+
+extern "C" int vq_skvq_clipped_roundtrip(const void *x, void *out, int dtype, int64_t B, int64_t H, int64_t r,
+                                         int64_t D, int64_t x_stride_bh, int64_t out_stride_bh, const int32_t *perm,
+                                         const int32_t *inv, int bits, int group, const float *alphas, int n_alphas, void *stream) {
+    const char *fn = "vq_skvq_clipped_roundtrip";
+    SkPlan p;
+    SkAlphas al;
     VQ_REQUIRE(is_float_tag(dtype), VQ_ERR_INVALID, "%s: unsupported dtype tag %d", fn, dtype);
+    const int rc = plan_skvq(fn, B, H, r, D, bits, group, alphas, n_alphas, p, al);
+    if (rc != VQ_OK) return rc;
     if (B * H * r * D == 0) return VQ_OK;
     VQ_REQUIRE(x && out, VQ_ERR_INVALID, "%s: null pointer", fn);
     VQ_REQUIRE(x_stride_bh >= r * D && out_stride_bh >= r * D, VQ_ERR_INVALID, "%s: stride below r * D", fn);
-    const int64_t G = (D + group - 1) / group;
-    const int64_t row_words = G * (group + 1);
-    VQ_REQUIRE(G <= SK_THREADS && row_words * 4 <= 48 * 1024 && group < 65536, VQ_ERR_UNSUPPORTED,
-               "%s: head_dim %lld with group %d does not fit a block (at most %d groups, 48 KB per row)", fn,
-               (long long)D, group, SK_THREADS);
-    // one wave per block where a wave covers whole rows: blocks then interleave freely on a CU (the
-    // phases of a block do not overlap each other, those of different blocks do)
-    const int threads = (G <= 64 && (G * group + 7) / 8 <= 64) ? 64 : SK_THREADS;
-    int64_t rows_pb = threads / G;
-    if (rows_pb * row_words * 4 > 48 * 1024) rows_pb = 48 * 1024 / (row_words * 4);
-    const int64_t n_rows = B * H * r, blocks = (n_rows + rows_pb - 1) / rows_pb;
-    VQ_REQUIRE(n_rows <= 0x7fffffff, VQ_ERR_UNSUPPORTED, "%s: too many rows (%lld)", fn, (long long)n_rows);
-    // floor(j / group) == (j * magic) >> 32 for j, group < 2^16 (a row holds at most 12288 words in LDS)
-    const uint64_t group_magic = (1ull << 32) / (uint64_t)group + 1;
-    // threads side by side on a row (eight channels each), and whether rows can move as 16-byte pieces
-    const int64_t pieces = (G * group + 7) / 8;
-    const int tpr = (int)(pieces < threads ? pieces : threads);
     VQ_REQUIRE(perm || !inv, VQ_ERR_INVALID, "%s: inv given without perm", fn);
+    // whether rows can move as 16-byte pieces
     const bool vec = (perm == nullptr || inv != nullptr) && D % 8 == 0 && x_stride_bh % 8 == 0 && out_stride_bh % 8 == 0 &&
                      ((uintptr_t)x % 16 == 0) && ((uintptr_t)out % 16 == 0);
-    SkAlphas al;
-    al.n = n_alphas;
-    for (int k = 0; k < SK_MAX_ALPHAS; ++k) al.a[k] = k < n_alphas ? alphas[k] : 1.f;
-    hipStream_t st = (hipStream_t)stream;
-    const size_t lds = (size_t)(rows_pb * row_words * 4);
-#define VQ_SK_LAUNCH(GROUP)                                                                                              \
-    VQ_DISPATCH_FLOAT(dtype, T, {                                                                                      \
-        hipLaunchKernelGGL((skvq_roundtrip_kernel<T, GROUP>), dim3((unsigned)blocks), dim3(threads), lds, st,          \
-                           (const T *)x, (T *)out, B * H, H, r, D, x_stride_bh, out_stride_bh, perm, inv, group,       \
-                           group_magic, (int)G, (int)rows_pb, tpr, vec, (float)((1 << bits) - 1), al);                 \
+    VQ_DISPATCH_FLOAT(dtype, T, {
+        launch_skvq<T, false>(p, al, x, out, nullptr, B, H, r, D, x_stride_bh, out_stride_bh, perm, inv, bits, group, vec, (hipStream_t)stream);
     })
-    if (group == 32) { VQ_SK_LAUNCH(32); }
-    else if (group == 64) { VQ_SK_LAUNCH(64); }
-    else { VQ_SK_LAUNCH(0); }
-#undef VQ_SK_LAUNCH
+    VQ_HIP_CHECK_LAUNCH(fn);
+    return VQ_OK;
+}
+
+extern "C" size_t vq_skvq_channel_orders_workspace(int64_t B, int64_t H, int64_t r, int64_t D, int group) {
+    if (B < 1 || H < 1 || r < 1 || D < 1 || group < 1) return 0;
+    const int64_t pieces = ((D + group - 1) / group * group + 7) / 8, tpr = pieces < SK_THREADS ? pieces : SK_THREADS;
+    return (size_t)(2 * B * H * r * tpr) * sizeof(double);
+}
+
+extern "C" int vq_skvq_channel_orders(const void *x, int dtype, int64_t B, int64_t H, int64_t r, int64_t D, int64_t x_stride_bh,
+                                      int bits, int group, const float *alphas, int n_alphas, int32_t *perm, int32_t *inv,
+                                      void *workspace, size_t workspace_bytes, void *stream) {
+    const char *fn = "vq_skvq_channel_orders";
+    SkPlan p;
+    SkAlphas al;
+    VQ_REQUIRE(is_float_tag(dtype), VQ_ERR_INVALID, "%s: unsupported dtype tag %d", fn, dtype);
+    VQ_REQUIRE(B >= 1 && H >= 1 && r >= 1 && D >= 1, VQ_ERR_INVALID, "%s: empty chunk", fn);
+    const int rc = plan_skvq(fn, B, H, r, D, bits, group, alphas, n_alphas, p, al);
+    if (rc != VQ_OK) return rc;
+    VQ_REQUIRE(x && perm && inv && workspace, VQ_ERR_INVALID, "%s: null pointer", fn);
+    VQ_REQUIRE(x_stride_bh >= r * D, VQ_ERR_INVALID, "%s: stride below r * D", fn);
+    VQ_REQUIRE(H <= 0x7fffffff, VQ_ERR_UNSUPPORTED, "%s: too many heads", fn);
+    VQ_REQUIRE(workspace_bytes >= vq_skvq_channel_orders_workspace(B, H, r, D, group), VQ_ERR_WORKSPACE, "%s: workspace too small", fn);
+    const bool vec = D % 8 == 0 && x_stride_bh % 8 == 0 && (uintptr_t)x % 16 == 0;
+    double *err = (double *)workspace;
+    hipStream_t st = (hipStream_t)stream;
+    VQ_DISPATCH_FLOAT(dtype, T, {
+        const size_t lds = (size_t)D * 12;   // D <= 12288 words of a row, so at most 144 KB
+        auto kernel = vec ? skvq_order_kernel<T, 8> : skvq_order_kernel<T, 1>;
+        if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)H), dim3(SK_ORD_THREADS), lds, st, (const T *)x, B, H, r, (int)D, x_stride_bh, perm, inv);
+        launch_skvq<T, true>(p, al, x, nullptr, err, B, H, r, D, x_stride_bh, x_stride_bh, perm, inv, bits, group, vec, st);
+    })
+    hipLaunchKernelGGL(skvq_choose_kernel, dim3((unsigned)H), dim3(SK_ORD_THREADS), 0, st, err, B, H, r, p.tpr, (int)D, perm, inv);
     VQ_HIP_CHECK_LAUNCH(fn);
     return VQ_OK;
 }

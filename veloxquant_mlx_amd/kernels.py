@@ -107,6 +107,17 @@ def kivi_group_quant_dequant(x: torch.Tensor, axis: int, group_size: int, levels
     return out.view(x.shape)
 
 
+def _slab(name: str, t: torch.Tensor, what: str) -> int:
+    """Elements between consecutive (b, h) slabs of a token slice of a contiguous [B, H, cap, D] buffer."""
+    (B, H, r, D), st = t.shape, t.stride()
+    step = st[1] if H > 1 else (st[0] if B > 1 else r * D)
+    ok = (D == 1 or st[3] == 1) and (r == 1 or st[2] == D) and (B == 1 or H == 1 or st[0] == H * st[1]) \
+        and step >= r * D
+    if not ok:
+        raise ValueError(f"{name}: {what} must be a token slice of a contiguous [B, H, cap, D] buffer, strides {st}")
+    return step
+
+
 def skvq_clipped_round_trip(x: torch.Tensor, bits: int, group_size: int, alphas, perm: torch.Tensor | None = None,
                             out: torch.Tensor | None = None, inv: torch.Tensor | None = None) -> torch.Tensor:
     """Round-trip ``x [B, H, r, D]`` through SKVQ's clipped group quantisation.
@@ -130,17 +141,6 @@ def skvq_clipped_round_trip(x: torch.Tensor, bits: int, group_size: int, alphas,
         raise ValueError(f"{name}: alphas must be 1..8 values in (0, 1], got {al}")
     tag = _ftag(name, x)
     B, H, r, D = x.shape
-
-    def slab(t: torch.Tensor, what: str) -> int:
-        """Elements between consecutive (b, h) slabs of a token slice of a contiguous [B, H, cap, D] buffer."""
-        st = t.stride()
-        step = st[1] if H > 1 else (st[0] if B > 1 else r * D)
-        ok = (D == 1 or st[3] == 1) and (r == 1 or st[2] == D) and (B == 1 or H == 1 or st[0] == H * st[1]) \
-            and step >= r * D
-        if not ok:
-            raise ValueError(f"{name}: {what} must be a token slice of a contiguous [B, H, cap, D] buffer, strides {st}")
-        return step
-
     if out is None:
         out = torch.empty((B, H, r, D), dtype=x.dtype, device=x.device)
     elif out.shape != x.shape or out.dtype != x.dtype:
@@ -148,7 +148,7 @@ def skvq_clipped_round_trip(x: torch.Tensor, bits: int, group_size: int, alphas,
     if x.numel() == 0:
         return out
     _need_gpu(name, x, out)
-    xs, os_ = slab(x, "x"), slab(out, "out")
+    xs, os_ = _slab(name, x, "x"), _slab(name, out, "out")
     pp = None
     if perm is not None:
         if perm.shape != (H, D) or perm.dtype != torch.int32:
@@ -163,11 +163,34 @@ def skvq_clipped_round_trip(x: torch.Tensor, bits: int, group_size: int, alphas,
         _need_gpu(name, inv)
         inv = inv.contiguous()
         ip = inv.data_ptr()
-    arr = (_lib.C.c_float * len(al))(*al)
+    arr = (C.c_float * len(al))(*al)
     rc = _lib.load().vq_skvq_clipped_roundtrip(x.data_ptr(), out.data_ptr(), tag, B, H, r, D, xs, os_, pp, ip, int(bits),
                                                int(group_size), arr, len(al), _stream(x))
     _lib.check(rc)
     return out
+
+
+def skvq_channel_orders(x: torch.Tensor, bits: int, group_size: int, alphas):
+    """Channel order per head and its inverse, int32 ``[H, D]`` each, from a chunk ``x [B, H, r, D]`` (a token slice of
+    a larger ``[B, H, cap, D]`` buffer): channels sorted by range, kept only on heads where that lowers the mean squared
+    round-trip error (``SKVQKVCache._per_head_perms``, veloxquant_mlx/cache/skvq_cache.py:186-224)."""
+    name = "skvq_channel_orders"
+    if x.ndim != 4 or x.numel() == 0:
+        raise ValueError(f"{name}: x must be a non-empty [B, H, r, D], got {tuple(x.shape)}")
+    tag = _ftag(name, x)
+    _need_gpu(name, x)
+    B, H, r, D = x.shape
+    xs = _slab(name, x, "x")
+    al = [float(a) for a in alphas]
+    perm = torch.empty((H, D), dtype=torch.int32, device=x.device)
+    inv = torch.empty_like(perm)
+    lib = _lib.load()
+    n = lib.vq_skvq_channel_orders_workspace(B, H, r, D, int(group_size))
+    ws = torch.empty((n,), dtype=torch.uint8, device=x.device)
+    _lib.check(lib.vq_skvq_channel_orders(x.data_ptr(), tag, B, H, r, D, xs, int(bits), int(group_size),
+                                          (C.c_float * len(al))(*al), len(al), perm.data_ptr(), inv.data_ptr(),
+                                          ws.data_ptr(), n, _stream(x)))
+    return perm, inv
 
 
 def row_norms(x: torch.Tensor) -> torch.Tensor:
@@ -463,6 +486,48 @@ def kv_tail_append(k_new: torch.Tensor, v_new: torch.Tensor, k_tail: torch.Tenso
     v_new, vs = strides(v_new)
     _lib.check(_lib.load().vq_kv_tail_append(k_new.data_ptr(), v_new.data_ptr(), ks, vs, k_tail.data_ptr(),
                                              v_tail.data_ptr(), es, B, H, S, D, cap, pos, _stream(k_new)))
+
+
+def _plain_eager() -> bool:
+    """Outside tracing, function transforms, forward-mode levels and dispatch modes: a call that hands raw pointers
+    to a kernel sees what the torch operation in its place would."""
+    return not (torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None
+                or torch._C._len_torch_dispatch_stack() > 0 or torch.autograd.forward_ad._current_level >= 0
+                or torch.compiler.is_compiling())
+
+
+def kv_rows_copyable(k_new: torch.Tensor, v_new: torch.Tensor) -> bool:
+    """Whether :func:`kv_fill` (and :func:`kv_tail_append` without a copy) takes these new tokens: plain tensors of one
+    shape and 16- or 32-bit float type on the current device, outside autograd and function transforms, whose rows
+    lie 16-byte aligned."""
+    if not (type(k_new) is type(v_new) is torch.Tensor and k_new.is_cuda and k_new.ndim == 4 and k_new.shape == v_new.shape
+            and k_new.dtype == v_new.dtype and k_new.dtype in _FLOAT_TAG and k_new.device == v_new.device
+            and k_new.device.index == torch.cuda.current_device()):
+        return False
+    if k_new.requires_grad or v_new.requires_grad or k_new.numel() == 0 or not _plain_eager():
+        return False
+    es = k_new.element_size()
+    if k_new.shape[3] * es % 16:
+        return False
+    for t in (k_new, v_new):
+        st = t.stride()
+        if st[3] != 1 or st[0] * es % 16 or st[1] * es % 16 or st[2] * es % 16 or t.data_ptr() % 16:
+            return False
+    return True
+
+
+def kv_fill(k_new: torch.Tensor, v_new: torch.Tensor, cap: int):
+    """Buffers ``[B, H, cap, D]`` that start with ``k_new, v_new [B, H, S, D]`` and are zero from there on, in one
+    launch; the tokens are ones that :func:`kv_rows_copyable` accepts."""
+    B, H, S, D = k_new.shape
+    if cap < S:
+        raise ValueError(f"kv_fill: {S} tokens exceed the capacity {cap}")
+    kb, vb = (torch.empty((B, H, cap, D), dtype=k_new.dtype, device=k_new.device) for _ in range(2))
+    ks, vs = k_new.stride(), v_new.stride()
+    _lib.check(_lib.load().vq_kv_fill(k_new.data_ptr(), v_new.data_ptr(), (C.c_int64 * 3)(ks[0], ks[1], ks[2]),
+                                      (C.c_int64 * 3)(vs[0], vs[1], vs[2]), kb.data_ptr(), vb.data_ptr(), k_new.element_size(),
+                                      B, H, S, D, cap, _stream(k_new)))
+    return kb, vb
 
 
 def kivi_cache_append(k_new: torch.Tensor, v_new: torch.Tensor, k_tail: torch.Tensor, v_tail: torch.Tensor,
