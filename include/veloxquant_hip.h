@@ -64,6 +64,13 @@ int vq_device_count(void);
 int vq_kivi_quant_dequant(const void *x, void *out, int dtype, int64_t BH, int64_t S, int64_t D,
                           int axis, int group, int levels, float eps, void *stream);
 
+/* The flush of a plain cache (KIVIKVCache.update_and_fetch, veloxquant_mlx/cache/kivi_cache.py:245-260): keys
+ * through groups along tokens, values through groups along channels, both in place on rows [B*H slabs, S, D] whose slabs
+ * lie stride_bh elements apart (the same layout for both).  head_dim 64, 128 or 256, groups of 8 2^n channels up to the
+ * head_dim; VQ_ERR_UNSUPPORTED, with nothing changed, for other shapes (vq_kivi_quant_dequant into a copy takes those). */
+int vq_kivi_round_trip_kv(void *k, void *v, int dtype, int64_t BH, int64_t S, int64_t D, int64_t stride_bh, int group,
+                          int levels, float eps, void *stream);
+
 /* The same round trip along the token axis with a level count per channel: channel c of slab bh has
  * levels_hi levels where hi_mask[bh * D + c] != 0 and levels_lo otherwise.  One launch for
  * quantize_mixed_channels (veloxquant_mlx/quantizers/kitty.py:138-169), which forms the hi-bit and the

@@ -312,3 +312,29 @@ def test_keys_and_values_in_one_call_equal_the_single_calls(dtype, b, g, D, S, v
             assert torch.equal(bufs[1][0][:, :, off // per:], vp) and torch.equal(bufs[1][1][..., off:], vs)
         else:
             assert torch.equal(bufs[1][0][:, :, off:], vp) and torch.equal(bufs[1][2][:, :, off:], vz)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,lo,n,cap,D,g", [
+    (1, 1, 0, 32, 64, 128, 32), (2, 3, 64, 1920, 2048, 128, 32), (1, 2, 64, 320, 512, 128, 64), (1, 2, 0, 100, 256, 128, 32),
+    (2, 2, 16, 48, 256, 128, 16), (1, 3, 32, 96, 256, 64, 32), (1, 2, 128, 256, 512, 256, 64), (1, 1, 0, 8, 256, 64, 8),
+])
+def test_round_trip_in_place_equals_the_two_round_trips(dtype, B, H, lo, n, cap, D, g):
+    """Keys and values of a slice of two buffers in place: the bits of the two separate round trips, and no other row changes."""
+    require_gpu()
+    k, v = (torch.randn((B, H, cap, D), device="cuda:0").to(dtype) for _ in range(2))
+    k0, v0 = k.clone(), v.clone()
+    want_k, want_v = K.kivi_group_quant_dequant(k[:, :, lo:lo + n], -2, g, 3), K.kivi_group_quant_dequant(v[:, :, lo:lo + n], -1, g, 3)
+    assert K.kivi_round_trip_kv(k[:, :, lo:lo + n], v[:, :, lo:lo + n], g, 3)
+    k0[:, :, lo:lo + n], v0[:, :, lo:lo + n] = want_k, want_v
+    assert torch.equal(k, k0) and torch.equal(v, v0)
+
+
+def test_round_trip_in_place_leaves_other_shapes_alone():
+    require_gpu()
+    for D, g in ((80, 16), (128, 24), (64, 128), (128, 256)):
+        k = torch.randn((1, 2, 256, D), device="cuda:0").half()
+        k0 = k.clone()
+        assert not K.kivi_round_trip_kv(k, k.clone(), g, 3) and torch.equal(k, k0)
+    k = torch.randn((1, 256, 2, 64), device="cuda:0").half().transpose(1, 2)
+    assert not K.kivi_round_trip_kv(k, k.clone(memory_format=torch.preserve_format), 32, 3)

@@ -89,6 +89,7 @@ _SIGNATURES = {
     "vq_kivi_quant_pack": (i32, [vp, i32, i64, i64, i64, i64, i32, i32, i32, f32, i32, i32, vp, vp, vp, i32, i64, i64, vp]),
     "vq_zip_route": (i32, [vp, i64, i64, i64, vp, vp]),
     "vq_row_norms": (i32, [vp, i32, i64, i64, vp, vp]),
+    "vq_kivi_round_trip_kv": (i32, [vp, vp, i32, i64, i64, i64, i64, i32, i32, f32, vp]),
     "vq_kivi_quant_dequant_mixed": (i32, [vp, vp, i32, i64, i64, i64, i32, i32, i32, vp, f32, vp]),
     "vq_channel_moments": (i32, [vp, i32, i64, i64, i64, i64, vp, i32, vp]),
     "vq_channel_variance": (i32, [vp, i64, i32, i64, i64, vp, vp]),

@@ -284,8 +284,10 @@ class KIVIKVCache(FP16KVCache):
             if self._fused_enabled:
                 # pack from the still-exact fp16 rows before they are overwritten
                 self._pack_block(self.keys[:, :, lo:hi], self.values[:, :, lo:hi], lo)
-            self.keys[:, :, lo:hi] = self._quant_dequant_along(self.keys[:, :, lo:hi], axis=-2)
-            self.values[:, :, lo:hi] = self._quant_dequant_along(self.values[:, :, lo:hi], axis=-1)
+            k_rows, v_rows = self.keys[:, :, lo:hi], self.values[:, :, lo:hi]
+            if not K.kivi_round_trip_kv(k_rows, v_rows, self._group_size, self._levels, self._eps):
+                self.keys[:, :, lo:hi] = self._quant_dequant_along(k_rows, axis=-2)
+                self.values[:, :, lo:hi] = self._quant_dequant_along(v_rows, axis=-1)
             self._n_quantized = new_boundary
             k_all, v_all = self.keys[:, :, : self.offset], self.values[:, :, : self.offset]
         self._account_bytes(B, H, S, D, n_quant_now)

@@ -326,7 +326,7 @@ constexpr int KT_MAXP = 8;
 
 template <typename T, typename M, int LPR, int MODE, int NP>
 __device__ __forceinline__ void kivi_key_tile_body(int bx, int64_t bh,
-    const T *__restrict__ x, T *__restrict__ out, int64_t S, int64_t x_stride_bh, int group, float levels,
+    const T *x, T *out, int64_t S, int64_t x_stride_bh, int group, float levels,
     float eps, int bits, uint32_t *__restrict__ packed, M *__restrict__ scale, M *__restrict__ zero,
     int64_t cap_tokens, int64_t dst_tok0, int W, const int32_t *__restrict__ rows = nullptr, int64_t rows_stride = 0) {
     constexpr int D = LPR * 8;
@@ -418,7 +418,7 @@ __device__ __forceinline__ void kivi_key_tile_body(int bx, int64_t bh,
                 float y[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) y[i] = recon(q[i], sc[i], mn[i]);
-                store8<T>(rows != nullptr ? out + bh * x_stride_bh + src[p] * D + 8 * o : out + (bh * S + s) * D + 8 * o, y);
+                store8<T>(out + bh * x_stride_bh + src[p] * D + 8 * o, y);
             }
         } else {
             uint32_t *row = packed + (bh * cap_tokens + dst_tok0 + (valid ? s : 0)) * W;
@@ -429,7 +429,7 @@ __device__ __forceinline__ void kivi_key_tile_body(int bx, int64_t bh,
 
 template <typename T, typename M, int LPR, int MODE, int NP>
 __global__ __launch_bounds__(256) void kivi_key_tile_kernel(
-    const T *__restrict__ x, T *__restrict__ out, int64_t S, int64_t x_stride_bh, int group, float levels,
+    const T *x, T *out, int64_t S, int64_t x_stride_bh, int group, float levels,
     float eps, int bits, uint32_t *__restrict__ packed, M *__restrict__ scale, M *__restrict__ zero,
     int64_t cap_tokens, int64_t dst_tok0, int W, const int32_t *__restrict__ rows, int64_t rows_stride) {
     kivi_key_tile_body<T, M, LPR, MODE, NP>((int)blockIdx.x, (int64_t)blockIdx.y, x, out, S, x_stride_bh, group, levels, eps,
@@ -445,7 +445,7 @@ constexpr int VT_TILES = 4;   // row tiles of 256 / LPR rows one block of the va
 
 template <typename T, typename M, int LPR, int MODE>
 __device__ __forceinline__ void kivi_value_tile_body(int bx, int64_t bh,
-    const T *__restrict__ x, T *__restrict__ out, int64_t S, int64_t x_stride_bh, int group, float levels,
+    const T *x, T *out, int64_t S, int64_t x_stride_bh, int group, float levels,
     float eps, int bits, uint32_t *__restrict__ packed, M *__restrict__ scale, M *__restrict__ zero,
     int64_t cap_tokens, int64_t dst_tok0, int W) {
     constexpr int D = LPR * 8;
@@ -515,7 +515,7 @@ __device__ __forceinline__ void kivi_value_tile_body(int bx, int64_t bh,
                 float y[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) y[i] = recon(q[i], sc, mn);
-                store8<T>(out + (bh * S + s) * D + 8 * o, y);
+                store8<T>(out + bh * x_stride_bh + s * D + 8 * o, y);
             }
             continue;
         }
@@ -559,7 +559,7 @@ __device__ __forceinline__ void kivi_value_tile_body(int bx, int64_t bh,
 
 template <typename T, typename M, int LPR, int MODE>
 __global__ __launch_bounds__(256) void kivi_value_tile_kernel(
-    const T *__restrict__ x, T *__restrict__ out, int64_t S, int64_t x_stride_bh, int group, float levels,
+    const T *x, T *out, int64_t S, int64_t x_stride_bh, int group, float levels,
     float eps, int bits, uint32_t *__restrict__ packed, M *__restrict__ scale, M *__restrict__ zero,
     int64_t cap_tokens, int64_t dst_tok0, int W) {
     kivi_value_tile_body<T, M, LPR, MODE>((int)blockIdx.x, (int64_t)blockIdx.y, x, out, S, x_stride_bh, group, levels, eps,
@@ -599,15 +599,14 @@ constexpr int VP_STRETCHES = 16;   // stretches of PER tokens per block of 256 t
 // The same walk writing the reconstruction instead (the round trip): stretches of 8 tokens, the last one of a
 // sequence may be short.
 template <typename T, int GL>
-__global__ __launch_bounds__(256) void kivi_value_roundtrip_kernel(const T *__restrict__ x, T *__restrict__ out, int64_t S,
-                                                                   int64_t x_stride_bh, float levels, float eps) {
+__device__ __forceinline__ void kivi_value_roundtrip_body(int bx, int64_t bh, const T *x, T *out, int64_t S, int64_t x_stride_bh,
+                                                          float levels, float eps) {
     constexpr int D = 128, PER = 8;
     const int tid = threadIdx.x, o = tid & 15;
-    const int64_t bh = blockIdx.y;
-    const int64_t t0 = ((int64_t)blockIdx.x * VP_STRETCHES + (tid >> 4)) * PER;
+    const int64_t t0 = ((int64_t)bx * VP_STRETCHES + (tid >> 4)) * PER;
     if (t0 >= S) return;
     const T *xb = x + bh * x_stride_bh + t0 * D + 8 * o;
-    T *ob = out + (bh * S + t0) * D + 8 * o;
+    T *ob = out + bh * x_stride_bh + t0 * D + 8 * o;
     const LevelDiv ld = level_div(levels);
     Raw8<T> v[PER];
 #pragma unroll
@@ -627,6 +626,11 @@ __global__ __launch_bounds__(256) void kivi_value_roundtrip_kernel(const T *__re
         for (int c = 0; c < 8; ++c) y[c] = recon(q[c], sc, mn);
         if (t0 + i < S) store8<T>(ob + (int64_t)i * D, y);
     }
+}
+template <typename T, int GL>
+__global__ __launch_bounds__(256) void kivi_value_roundtrip_kernel(const T *x, T *out, int64_t S, int64_t x_stride_bh, float levels,
+                                                                   float eps) {
+    kivi_value_roundtrip_body<T, GL>((int)blockIdx.x, (int64_t)blockIdx.y, x, out, S, x_stride_bh, levels, eps);
 }
 
 // The GL lanes of a channel group hold the same (token, group) extrema after the fold: with GL = 4 or 8 each of them
@@ -827,7 +831,7 @@ constexpr int KQ_WAVES = 4;   // groups per block
 // alt_first for this (sequence, head) and `alt_rs` its row stride in elements; alt_first is a multiple of the group
 // (or lies at or past S), so a group reads one source.
 template <typename T, typename M, int MODE, int TPL, bool MIXED = false, bool TWO = false>
-__device__ __forceinline__ void kivi_key_quad_body(int gk, int64_t bh, const T *__restrict__ x, T *__restrict__ out, int64_t S,
+__device__ __forceinline__ void kivi_key_quad_body(int gk, int64_t bh, const T *x, T *out, int64_t S,
                                                    int64_t x_stride_bh, float levels, float eps, int bits,
                                                    uint32_t *__restrict__ packed, M *__restrict__ scale, M *__restrict__ zero,
                                                    int64_t cap_tokens, int64_t dst_tok0, int W,
@@ -848,7 +852,7 @@ __device__ __forceinline__ void kivi_key_quad_body(int gk, int64_t bh, const T *
         if (levels == 0.f) {
 #pragma unroll
             for (int i = 0; i < TPL; ++i)
-                if (r0 + i < S) *reinterpret_cast<uint4 *>(out + (bh * S + r0 + i) * D + 8 * o) = *reinterpret_cast<const uint4 *>(xb + (int64_t)i * row_gap);
+                if (r0 + i < S) *reinterpret_cast<uint4 *>(out + bh * x_stride_bh + (r0 + i) * D + 8 * o) = *reinterpret_cast<const uint4 *>(xb + (int64_t)i * row_gap);
             return;
         }
     }
@@ -952,7 +956,7 @@ __device__ __forceinline__ void kivi_key_quad_body(int gk, int64_t bh, const T *
                     float y[8];
 #pragma unroll
                     for (int c = 0; c < 8; ++c) y[c] = recon(q[c], sc[c], mn[c]);
-                    store8<T>(out + (bh * S + srow) * D + 8 * o, y);
+                    store8<T>(out + bh * x_stride_bh + srow * D + 8 * o, y);
                 }
             } else {
                 // (a whole group: one base for the lane's rows, the rows a constant apart)
@@ -978,7 +982,7 @@ __device__ __forceinline__ void kivi_key_quad_body(int gk, int64_t bh, const T *
 
 template <typename T, typename M, int MODE, int TPL>
 __global__ __launch_bounds__(64 * KQ_WAVES) void kivi_key_quad_kernel(
-    const T *__restrict__ x, T *__restrict__ out, int64_t S, int64_t x_stride_bh, float levels, float eps, int bits,
+    const T *x, T *out, int64_t S, int64_t x_stride_bh, float levels, float eps, int bits,
     uint32_t *__restrict__ packed, M *__restrict__ scale, M *__restrict__ zero, int64_t cap_tokens, int64_t dst_tok0, int W) {
     kivi_key_quad_body<T, M, MODE, TPL>((int)blockIdx.x * KQ_WAVES + (int)(threadIdx.x >> 6), (int64_t)blockIdx.y, x, out, S,
                                         x_stride_bh, levels, eps, bits, packed, scale, zero, cap_tokens, dst_tok0, W);
@@ -992,7 +996,7 @@ struct PackDst { uint32_t *packed; void *scale, *zero; };
 // the same for head_dim 128, groups of 32 or 64, 2 or 4 bits, token-packed values: the quad-layout key body and the
 // word-owning value body, neither of which uses block-shared memory
 template <typename T, int TPL>
-__global__ __launch_bounds__(64 * KQ_WAVES) void kivi_key_quad_mixed_kernel(const T *__restrict__ x, T *__restrict__ out, int64_t S,
+__global__ __launch_bounds__(64 * KQ_WAVES) void kivi_key_quad_mixed_kernel(const T *x, T *out, int64_t S,
                                                                            int64_t x_stride_bh, float levels_lo, float levels_hi,
                                                                            const uint8_t *__restrict__ hi_mask, float eps) {
     kivi_key_quad_body<T, float, 0, TPL, true>((int)blockIdx.x * KQ_WAVES + (int)(threadIdx.x >> 6), (int64_t)blockIdx.y, x, out, S,
@@ -1002,11 +1006,26 @@ __global__ __launch_bounds__(64 * KQ_WAVES) void kivi_key_quad_mixed_kernel(cons
 // Round trip with a level count per token group (AgeTieredKV: windows of different ages at different bit widths,
 // veloxquant_mlx/quantizers/age_tiered.py:117-174); fp16 / bf16 rows only (a passing group is copied as 16-byte pieces).
 template <typename T, int TPL>
-__global__ __launch_bounds__(64 * KQ_WAVES) void kivi_key_quad_grouplevels_kernel(const T *__restrict__ x, T *__restrict__ out, int64_t S,
+__global__ __launch_bounds__(64 * KQ_WAVES) void kivi_key_quad_grouplevels_kernel(const T *x, T *out, int64_t S,
                                                                                  int64_t x_stride_bh, const float *__restrict__ group_levels,
                                                                                  float eps) {
     kivi_key_quad_body<T, float, 0, TPL>((int)blockIdx.x * KQ_WAVES + (int)(threadIdx.x >> 6), (int64_t)blockIdx.y, x, out, S, x_stride_bh,
                                          1.f, eps, 0, nullptr, nullptr, nullptr, 0, 0, 0, nullptr, 0.f, group_levels);
+}
+
+// Keys and values of a plain cache's flush, in place, in one launch: the first key_blocks blocks of a (sequence, head)
+// take the key groups, the rest the value rows.  Both bodies hold every row they write before they store the first.
+// A flush of a few MB is bound by its launches: with copies out of and back into the buffer around two round trips it
+// took six of them, 30 us for 2048 tokens of eight heads (17 MB); this one takes 7.
+template <typename T, int TPL>
+__global__ __launch_bounds__(64 * KQ_WAVES) void kivi_kv_roundtrip_kernel(T *k, T *v, int64_t S, int64_t stride_bh, int key_blocks,
+                                                                          float levels, float eps) {
+    const int bx = (int)blockIdx.x;
+    if (bx < key_blocks)
+        kivi_key_quad_body<T, float, 0, TPL>(bx * KQ_WAVES + (int)(threadIdx.x >> 6), (int64_t)blockIdx.y, k, k, S, stride_bh, levels, eps,
+                                             0, nullptr, nullptr, nullptr, 0, 0, 0);
+    else
+        kivi_value_roundtrip_body<T, TPL / 2>(bx - key_blocks, (int64_t)blockIdx.y, v, v, S, stride_bh, levels, eps);
 }
 
 // Sum and sum of squares over the tokens of every channel of x [N, S, D] in double precision: block (chunk, n)
@@ -1869,6 +1888,42 @@ extern "C" int vq_kivi_quant_dequant(const void *x, void *out, int dtype, int64_
                                (const T *)x, (T *)out, BH, S, D, axis, group, (float)levels, eps);
     });
     VQ_HIP_CHECK_LAUNCH("vq_kivi_quant_dequant");
+    return VQ_OK;
+}
+
+extern "C" int vq_kivi_round_trip_kv(void *k, void *v, int dtype, int64_t BH, int64_t S, int64_t D, int64_t stride_bh, int group,
+                                     int levels, float eps, void *stream) {
+    const char *fn = "vq_kivi_round_trip_kv";
+    VQ_REQUIRE(group >= 1, VQ_ERR_INVALID, "%s: group_size must be >= 1, got %d", fn, group);
+    VQ_REQUIRE(levels >= 1, VQ_ERR_INVALID, "%s: levels must be >= 1, got %d", fn, levels);
+    VQ_REQUIRE(BH >= 0 && S >= 0 && D >= 0, VQ_ERR_INVALID, "%s: negative dimension", fn);
+    VQ_REQUIRE(is_float_tag(dtype), VQ_ERR_INVALID, "%s: unsupported dtype tag %d", fn, dtype);
+    // what the tile kernels take on both axes: the generic kernel reads a group again for every element it writes
+    VQ_REQUIRE((D == 64 || D == 128 || D == 256) && stride_bh % 8 == 0 && BH <= 65535 && group <= KT_MAXP * (2048 / (int)D) &&
+                   group % 8 == 0 && pow2(group / 8) && group <= D,
+               VQ_ERR_UNSUPPORTED, "%s: head_dim %lld with groups of %d is not updated in place", fn, (long long)D, group);
+    if (BH * S == 0) return VQ_OK;
+    VQ_REQUIRE(k && v, VQ_ERR_INVALID, "%s: null pointer", fn);
+    VQ_REQUIRE(aligned16(k) && aligned16(v), VQ_ERR_UNSUPPORTED, "%s: rows must be 16-byte aligned", fn);
+    VQ_REQUIRE(stride_bh >= S * D, VQ_ERR_INVALID, "%s: stride below S * D", fn);
+    hipStream_t st = (hipStream_t)stream;
+    VQ_DISPATCH_FLOAT(dtype, T, {
+        if (D == 128 && (group == 32 || group == 64)) {
+            const int key_blocks = (int)cdiv(cdiv(S, group), KQ_WAVES);
+            const dim3 grid((unsigned)(key_blocks + cdiv(S, VP_STRETCHES * 8)), (unsigned)BH);
+            if (group == 32)
+                hipLaunchKernelGGL((kivi_kv_roundtrip_kernel<T, 8>), grid, dim3(64 * KQ_WAVES), 0, st, (T *)k, (T *)v, S, stride_bh, key_blocks,
+                                   (float)levels, eps);
+            else
+                hipLaunchKernelGGL((kivi_kv_roundtrip_kernel<T, 16>), grid, dim3(64 * KQ_WAVES), 0, st, (T *)k, (T *)v, S, stride_bh, key_blocks,
+                                   (float)levels, eps);
+        } else {
+            const bool ok = try_tile_path<T, float>(0, VQ_AXIS_TOKEN, k, k, BH, S, D, stride_bh, group, levels, eps, 0, nullptr, nullptr, nullptr, 0, 0, st) &&
+                            try_tile_path<T, float>(0, VQ_AXIS_CHANNEL, v, v, BH, S, D, stride_bh, group, levels, eps, 0, nullptr, nullptr, nullptr, 0, 0, st);
+            if (!ok) return fail(VQ_ERR_UNSUPPORTED, "%s: head_dim %lld with groups of %d is not updated in place", fn, (long long)D, group);
+        }
+    });
+    VQ_HIP_CHECK_LAUNCH(fn);
     return VQ_OK;
 }
 

@@ -107,6 +107,30 @@ def kivi_group_quant_dequant(x: torch.Tensor, axis: int, group_size: int, levels
     return out.view(x.shape)
 
 
+def kivi_round_trip_kv(k: torch.Tensor, v: torch.Tensor, group_size: int, levels: int, eps: float = 1e-8) -> bool:
+    """The round trips a KIVI cache gives the rows that leave its residual window (``axis=-2`` on keys, ``axis=-1`` on
+    values, veloxquant_mlx/cache/kivi_cache.py:245-260), in place on ``k, v [B, H, S, D]`` -- the same token slice of two
+    contiguous ``[B, H, cap, D]`` buffers -- in one library call.  False, with nothing changed, for rows it does not take
+    (:func:`kivi_group_quant_dequant` takes those)."""
+    if not (k.is_cuda and k.ndim == 4 and k.shape == v.shape and k.dtype == v.dtype and k.dtype in _FLOAT_TAG
+            and k.stride() == v.stride() and k.device == v.device) or k.requires_grad or v.requires_grad or not _plain_eager():
+        return False
+    B, H, S, D = k.shape
+    g = int(group_size)
+    # the shapes whose kernels hold a whole group before they write it, and rows they can move as 16-byte pieces
+    if D not in (64, 128, 256) or not (8 <= g <= min(D, 16384 // D)) or g & (g - 1) or B * H > 65535 or k.numel() == 0:
+        return False
+    try:
+        step = _slab("kivi_round_trip_kv", k, "k")
+    except ValueError:
+        return False
+    if step % 8 or k.data_ptr() % 16 or v.data_ptr() % 16:
+        return False
+    _lib.check(_lib.load().vq_kivi_round_trip_kv(k.data_ptr(), v.data_ptr(), _FLOAT_TAG[k.dtype], B * H, S, D, step, g, int(levels),
+                                                 float(eps), _stream(k)))
+    return True
+
+
 def _slab(name: str, t: torch.Tensor, what: str) -> int:
     """Elements between consecutive (b, h) slabs of a token slice of a contiguous [B, H, cap, D] buffer."""
     (B, H, r, D), st = t.shape, t.stride()
