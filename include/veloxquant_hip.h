@@ -405,7 +405,8 @@ size_t vq_kivi_attend_workspace(const vq_attend_args *a);
 
 /* Reports what vq_kivi_attend would do for these arguments: *path = 0 for the
  * layout-agnostic vector kernel, 1 for the MFMA decode kernel, 2 for the MFMA
- * prefill kernel (16 or more queries per sequence); *nparts = number of partial
+ * prefill kernel (16 or more queries per sequence), 3 and 4 for the vector kernels that share
+ * a kv head's bytes between its query rows (4: byte codes); *nparts = number of partial
  * results per query row.  No counterpart in the reference (its
  * _auto_nsg heuristic, veloxquant_mlx/metal/_scalar_attend.py:337-362, is the
  * nearest thing); used by tests and benchmarks to name the kernel measured. */
@@ -470,6 +471,36 @@ typedef struct vq_lut_attend_args {
  * VecInferKVCache.fused_sdpa (veloxquant_mlx/cache/vecinfer_cache.py:670-731). */
 size_t vq_vecinfer_attend_workspace(const vq_lut_attend_args *a);
 int vq_vecinfer_attend(const vq_lut_attend_args *a);
+
+/* The same without the look-up table, for codebooks of any size that fits LDS (float32, 144 KB in all) and a few query
+ * rows: the centroids are gathered on chip.  q is the plain query: smooth (float32 [smooth_rows, D], one row or one per
+ * kv head, or NULL) and the orthonormal Sylvester-Hadamard matrix of magnitude hadamard_scale (0: none) are applied
+ * inside (apply_dual_transform_queries, veloxquant_mlx/allocators/vecinfer.py:137-184).  Covers D 64 / 128 / 256, key
+ * sub-vectors of 4 or 8 channels, value sub-vectors of 8, Hq / Hkv * Sq <= 255; other shapes return
+ * VQ_ERR_UNSUPPORTED (workspace 0). */
+typedef struct vq_index_attend_args {
+    const void *q;
+    void *out;
+    int32_t q_dtype, out_dtype;
+    int64_t B, Hq, Hkv, Sq, D;
+    const void *k_idx, *v_idx;   /* [B, Hkv, cap_tokens, D / sub_dim], VQ_U8 or VQ_I32, 16-byte aligned */
+    int32_t k_idx_dtype, v_idx_dtype;
+    int64_t n_tokens, cap_tokens;
+    const void *k_codebook, *v_codebook;
+    int32_t k_cb_dtype, v_cb_dtype;
+    int32_t n_k_centroids, n_v_centroids, k_sub_dim, v_sub_dim;
+    const float *smooth;
+    int32_t smooth_rows;
+    float hadamard_scale;
+    float scale;
+    int32_t causal;
+    int64_t sliding_window;
+    void *workspace;
+    size_t workspace_bytes;
+    void *stream;
+} vq_index_attend_args;
+size_t vq_vecinfer_attend_indices_workspace(const vq_index_attend_args *a);
+int vq_vecinfer_attend_indices(const vq_index_attend_args *a);
 
 /* ---- SKVQ clipped group quantisation ------------------------------------- */
 

@@ -1,0 +1,93 @@
+"""Attention with sixteen channels a lane: byte codes with float32 scale / zero against the one-wave-a-row kernel, and
+codebook indices against the composition in float64 (veloxquant_mlx/allocators/vecinfer.py:137-184, 321-335)."""
+
+import math
+
+import pytest
+import torch
+
+from tests._gpu import require_gpu
+from veloxquant_mlx_amd import kernels as K
+from veloxquant_mlx_amd.allocators.vecinfer import walsh_hadamard_matrix
+
+pytestmark = pytest.mark.gpu
+
+
+def _visible(Sq, n, causal, window, device):
+    pos, t = torch.arange(n - Sq, n, device=device)[:, None], torch.arange(n, device=device)[None]
+    keep = t <= pos if causal else torch.ones((Sq, n), dtype=torch.bool, device=device)
+    return keep & (t > pos - window) if window else keep
+
+
+# tokens round the units of 16 / 32, the shortest split (128) and one with several units a wave; GQA groups of one tile and of
+# two; groups of 32 and more; buffers with room to spare
+@pytest.mark.parametrize("B,Hq,Hkv,D,n,group,Sq,causal,window,extra", [
+    (1, 8, 2, 64, 1, 32, 1, False, 0, 31), (2, 7, 1, 64, 129, 32, 1, False, 0, 0), (1, 4, 4, 128, 33, 64, 1, False, 0, 63),
+    (2, 28, 4, 128, 1037, 32, 1, False, 0, 3), (1, 12, 4, 256, 517, 128, 1, False, 0, 0), (1, 2, 1, 256, 95, 32, 3, True, 0, 0),
+    (1, 8, 2, 128, 700, 32, 2, True, 0, 4), (1, 4, 2, 128, 900, 32, 1, False, 77, 0), (3, 16, 1, 128, 4099, 96, 1, False, 0, 0),
+])
+def test_byte_codes_against_the_general_kernel(B, Hq, Hkv, D, n, group, Sq, causal, window, extra):
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(n + D)
+    r = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    cap, codes = n + extra, lambda: torch.randint(0, 2 ** 31 - 1, (B, Hkv, n + extra, D // 4), generator=gen, device="cuda", dtype=torch.int32)
+    ks = r(B, Hkv, -(-cap // group), D).abs() * 0.02
+    vs = r(B, Hkv, cap, -(-D // group)).abs() * 0.02
+    kw = dict(k_packed=codes(), k_scale=ks, k_zero=-128 * ks + r(*ks.shape), v_packed=codes(), v_scale=vs,
+              v_zero=-128 * vs + r(*vs.shape), n_packed=n, bits=8, group_size=group, scale=D ** -0.5, causal=causal,
+              sliding_window=window, out_dtype=torch.float32)
+    q, wide, general = r(B, Hq, Sq, D), {}, {}
+    out = K.kivi_packed_attend(q, _plan_out=wide, **kw)
+    ref = K.kivi_packed_attend(q, num_splits=-1, _plan_out=general, **kw)
+    assert wide["path"] == 4 and general["path"] == 0
+    # both rebuild code * scale + zero in float32 and differ by the order of their sums
+    assert float((out - ref).abs().max()) < 5e-5
+    # one type, group or layout further is the other kernels'
+    other = dict(kw, k_scale=ks.half(), k_zero=kw["k_zero"].half(), v_scale=vs.half(), v_zero=kw["v_zero"].half())
+    K.kivi_packed_attend(q, _plan_out=wide, **other)
+    assert wide["path"] != 4
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,n,Sq,causal,window,nk,sub,rows,cap", [
+    (1, 8, 2, 128, 1, 1, False, 0, 4096, 4, 2, 1), (2, 32, 8, 128, 777, 1, False, 0, 4096, 4, 8, 1024), (1, 7, 1, 64, 129, 2, True, 0, 256, 8, 1, 129),
+    (1, 12, 4, 256, 500, 1, False, 0, 256, 8, 0, 512), (1, 28, 4, 128, 2049, 1, False, 100, 1024, 4, 4, 2050), (1, 3, 3, 64, 33, 1, True, 0, 256, 4, 1, 64),
+    (1, 4, 2, 128, 4100, 4, True, 33, 300, 8, 2, 4100), (1, 4, 2, 64, 300, 21, True, 0, 4096, 4, 2, 300),
+])
+@pytest.mark.parametrize("q_dtype", [torch.float32, torch.bfloat16])
+def test_indices_against_float64(B, Hq, Hkv, D, n, Sq, causal, window, nk, sub, rows, cap, q_dtype):
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(n + nk)
+    r = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    idx = lambda m, s: torch.randint(0, m, (B, Hkv, cap, D // s), generator=gen, device="cuda",
+                                     dtype=torch.uint8 if m <= 256 else torch.int32)
+    q, ki, vi, kcb, vcb = r(B, Hq, Sq, D).to(q_dtype), idx(nk, sub), idx(256, 8), r(nk, sub), r(256, 8)
+    smooth = r(rows, D).exp() if rows else None
+    H = walsh_hadamard_matrix(D, device="cuda")
+    scale = 0.3 / math.sqrt(D)
+    out = K.vecinfer_attend_indices(q, ki, kcb, vi, vcb, scale, n_tokens=n, smooth=smooth, H_mat=H, causal=causal, sliding_window=window)
+    qt = q.double()
+    if rows:
+        qt = qt * smooth.double().repeat_interleave(Hq // rows if rows > 1 else Hq, 0)[None, :, None]
+    qt = qt @ H.double()
+    wide = lambda i, cb: cb.double()[i[:, :, :n].long()].reshape(B, Hkv, n, D).repeat_interleave(Hq // Hkv, 1)
+    s = (qt[..., None, :] * wide(ki, kcb)[:, :, None]).sum(-1) * scale
+    s = s.masked_fill(~_visible(Sq, n, causal, window, "cuda"), -math.inf)
+    p = torch.softmax(s, -1)
+    ref = (p[..., None] * wide(vi, vcb)[:, :, None]).sum(-2)
+    # float32 throughout: a score of |s| carries |s| 2^-24 per addition (D of them at most) into every probability;
+    # bfloat16 rounds the output to 2^-9
+    tol = float(s[s > -math.inf].abs().max()) * D * 2.0 ** -24 * 2 + 1e-5
+    err = (out.double() - ref).abs()
+    assert float((err - ref.abs() * (2.0 ** -8 if q_dtype == torch.bfloat16 else 0)).max()) < tol * float(ref.abs().max())
+
+
+def test_indices_refused_shapes():
+    require_gpu()
+    z = lambda *s, dtype=torch.float32: torch.zeros(s, device="cuda", dtype=dtype)
+    ki, vi, kcb, vcb = z(1, 2, 64, 32, dtype=torch.int32), z(1, 2, 64, 16, dtype=torch.uint8), z(4096, 4), z(256, 8)
+    attend = lambda q, ki=ki, vi=vi, kcb=kcb, vcb=vcb: K.vecinfer_attend_indices(q, ki, kcb, vi, vcb, 0.1, n_tokens=64)
+    assert attend(z(1, 4, 1, 128)) is not None
+    assert attend(z(1, 4, 128, 128)) is None                                # 256 rows a kv head
+    assert attend(z(1, 4, 1, 128, dtype=torch.float64)) is None
+    assert attend(z(1, 4, 1, 128), ki=z(1, 2, 64, 64, dtype=torch.int32)[..., ::2]) is None
+    assert attend(z(1, 4, 1, 128), ki=z(1, 2, 64, 16, dtype=torch.int32), kcb=z(8192, 8)) is None   # codebook past LDS

@@ -61,6 +61,22 @@ class LutAttendArgs(C.Structure):
     ]
 
 
+class IndexAttendArgs(C.Structure):
+    """Mirror of ``vq_index_attend_args``."""
+
+    _fields_ = [
+        ("q", vp), ("out", vp), ("q_dtype", i32), ("out_dtype", i32),
+        ("B", i64), ("Hq", i64), ("Hkv", i64), ("Sq", i64), ("D", i64),
+        ("k_idx", vp), ("v_idx", vp), ("k_idx_dtype", i32), ("v_idx_dtype", i32),
+        ("n_tokens", i64), ("cap_tokens", i64),
+        ("k_codebook", vp), ("v_codebook", vp), ("k_cb_dtype", i32), ("v_cb_dtype", i32),
+        ("n_k_centroids", i32), ("n_v_centroids", i32), ("k_sub_dim", i32), ("v_sub_dim", i32),
+        ("smooth", vp), ("smooth_rows", i32), ("hadamard_scale", f32), ("scale", f32),
+        ("causal", i32), ("sliding_window", i64),
+        ("workspace", vp), ("workspace_bytes", sz), ("stream", vp),
+    ]
+
+
 class KiviAppendArgs(C.Structure):
     """Mirror of ``vq_kivi_append_args``."""
 
@@ -116,6 +132,8 @@ _SIGNATURES = {
     "vq_kivi_prefill_tiles": (i32, [C.POINTER(AttendArgs), i64, i64]),
     "vq_vecinfer_attend_workspace": (sz, [C.POINTER(LutAttendArgs)]),
     "vq_vecinfer_attend": (i32, [C.POINTER(LutAttendArgs)]),
+    "vq_vecinfer_attend_indices_workspace": (sz, [C.POINTER(IndexAttendArgs)]),
+    "vq_vecinfer_attend_indices": (i32, [C.POINTER(IndexAttendArgs)]),
 }
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)

@@ -361,20 +361,29 @@ class VecInferKVCache(FP16KVCache):
             raise RuntimeError("VecInferKVCache.fused_sdpa called before any tokens were cached via update_and_fetch.")
         self._to_device(q)
         n = self._stored_S_kv
-        smooth = self._smooth.float() if self._smooth is not None else torch.ones(
-            (self._head_dim,), dtype=torch.float32, device=q.device)
-        q_tilde = apply_dual_transform_queries(q.float(), smooth, self._H)
         kcb, vcb = self._key_codebook, self._value_codebook
         n_sub_k, n_sub_v = self._head_dim // kcb.shape[1], self._head_dim // vcb.shape[1]
         table_kernel = (kcb.shape[0] == vcb.shape[0] <= 256 and max(n_sub_k, n_sub_v) <= 32
                         and (n_sub_k + n_sub_v) * kcb.shape[0] * 4 <= 65536
                         and (self._stored_k_indices.dtype != torch.uint8 or (n_sub_k % 4 == 0 and n_sub_v % 4 == 0)))
+        # Few query rows: straight from the indices, centroids gathered on chip.  Each four rows of a kv head read the indices
+        # again; a table kernel that takes the codebooks reads them less often, which shows from nine rows on (32 / 8 heads of 128
+        # channels, 4 x 16384 tokens, 8-bit codebooks: 47 / 60 us from the table with 4 rows, 83 / 82 with 8, 157 / 90 with 16).
+        H_kv = self._stored_k_indices.shape[1]
+        if q.shape[1] % H_kv == 0 and (q.shape[1] // H_kv) * q.shape[2] <= (8 if table_kernel else 255):
+            out = K.vecinfer_attend_indices(q, self._stored_k_indices, kcb, self._stored_v_indices, vcb, float(scale), n_tokens=n,
+                                            smooth=None if self._smooth is None else self._smooth.float(), H_mat=self._H,
+                                            causal=bool(causal) and q.shape[2] > 1, sliding_window=int(sliding_window or 0))
+            if out is not None:
+                return out
+        smooth = self._smooth.float() if self._smooth is not None else torch.ones(
+            (self._head_dim,), dtype=torch.float32, device=q.device)
+        q_tilde = apply_dual_transform_queries(q.float(), smooth, self._H)
         # A prefill-sized call (256 query rows or more per kv head at a head size the matrix-unit prefill blocks take)
         # gathers the centroids once into a transient copy in the queries' 16-bit type -- what update_and_fetch hands
         # a host that attends by itself (vecinfer_cache.py:336-379: the reconstruction cast to the input dtype) -- and
         # attends over it with those blocks: the table kernel builds a table per query row, which pays for a few rows
         # per kv head only (512 queries over 4.6k tokens, 32 / 8 heads: 0.64 ms from the tables, 0.09 ms this way).
-        H_kv = self._stored_k_indices.shape[1]
         prefill_sized = (self._head_dim in (128, 256) and q.shape[1] % H_kv == 0 and (q.shape[1] // H_kv) * q.shape[2] >= 256
                          and q.dtype in (torch.float16, torch.bfloat16))
         if table_kernel and not prefill_sized:

@@ -37,6 +37,11 @@ AttendPlan plan_attend(const vq_attend_args &a) {
         p.nparts = p.nsplit;
         return p;
     }
+    if (p.path == 0 && wide_kernel_supported(a)) {
+        p.path = 4;
+        plan_attend_wide(a, p);
+        return p;
+    }
     if (p.path == 0 && a.num_splits >= 0 && rows_kernel_supported(a)) {
         // four query rows of a kv head per block; splits until the grid holds four blocks per compute unit,
         // of at least 256 tokens each
@@ -376,13 +381,20 @@ extern "C" int vq_kivi_attend(const vq_attend_args *a_in) {
         rc = launch_attend_rows(*a, p);
         if (rc != VQ_OK) return rc;
         VQ_HIP_CHECK_LAUNCH(fn);
+    } else if (p.path == 4) {
+        launch_attend_wide(*a, p);
+        VQ_HIP_CHECK_LAUNCH(fn);
     } else {
         rc = launch_attend_generic(*a, p.nsplit, p.split_len);
         if (rc != VQ_OK) return rc;
         VQ_HIP_CHECK_LAUNCH(fn);
     }
     if (a_in->sink_k != nullptr) return finish();   // the patch pass does the merge as well
-    rc = launch_attend_merge(*a, p.nparts);
+    if (p.path == 1 || p.path == 2) {
+        rc = launch_attend_merge(*a, p.nparts);
+    } else {
+        launch_merge_splits((const float *)a->workspace, a->B * a->Hq * a->Sq, p.nparts, a->D, a->out, a->out_dtype, (hipStream_t)a->stream);
+    }
     VQ_HIP_CHECK_LAUNCH(fn);
     return rc;
 }

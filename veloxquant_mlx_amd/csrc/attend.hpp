@@ -22,7 +22,8 @@ __device__ __host__ __forceinline__ int64_t window_first(const vq_attend_args &a
 
 struct AttendPlan {
     int path;           // 0 generic waves, 1 MFMA decode (row tiles of <= 8), 2 MFMA prefill (LDS-staged, 64-row blocks),
-                        // 3 vector-unit rows kernel (any head_dim / bit width, four query rows a block)
+                        // 3 vector-unit rows kernel (any head_dim / bit width, four query rows a block),
+                        // 4 the same over byte codes, sixteen channels a lane (attend_wide.hip)
     int nsplit;         // splits along the tokens the main kernel covers
     int nparts;         // partials per query row handed to the merge kernel
     int64_t split_len;  // tokens per split (multiple of 64)
@@ -105,12 +106,19 @@ void rows_tiling(const vq_attend_args &a, int &pq, int &tiles);
 int launch_attend_rows(const vq_attend_args &a, const AttendPlan &p);
 // the same kernel over the tail tokens only, into partial `part0` of `nparts` per query row
 int launch_attend_rows_tail(const vq_attend_args &a, int part0, int nparts);
+// byte codes, sixteen channels a lane (attend_wide.hip): whether it takes the shapes, its splits, the launch
+bool wide_kernel_supported(const vq_attend_args &a);
+void plan_attend_wide(const vq_attend_args &a, AttendPlan &p);
+void launch_attend_wide(const vq_attend_args &a, const AttendPlan &p);
 int launch_attend_merge(const vq_attend_args &a, int nparts);
 // protected rows (vq_attend_args.sink_k): rewrites every output row from the partials in the
 // workspace, with the stand-ins' weights taken out and the exact rows put in
 void launch_sink_patch(const vq_attend_args &a, int nparts);
 // merges partials [rows][nparts][D + 2] of (max, sum, accumulator) into out [rows][D]
 void launch_merge_rows(const float *ws, int64_t rows, int nparts, int64_t D, void *out, int out_dtype, hipStream_t st);
+// the same with a block a row where rows are few and partials many (sums in another order: not for launches whose
+// other form merges inside the kernel)
+void launch_merge_splits(const float *ws, int64_t rows, int nparts, int64_t D, void *out, int out_dtype, hipStream_t st);
 
 // MFMA decode path (attend_mfma.hip)
 bool mfma_decode_supported(const vq_attend_args &a);

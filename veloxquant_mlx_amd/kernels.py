@@ -16,7 +16,7 @@ import torch
 
 from . import _lib
 from ._lib import (VQ_AXIS_CHANNEL, VQ_AXIS_TOKEN, VQ_BF16, VQ_F16, VQ_F32, VQ_I32, VQ_U8,
-                   VQ_V_CHANNEL_PACKED, VQ_V_TOKEN_PACKED, AttendArgs, LutAttendArgs)
+                   VQ_V_CHANNEL_PACKED, VQ_V_TOKEN_PACKED, AttendArgs, IndexAttendArgs, LutAttendArgs)
 
 _FLOAT_TAG = {torch.float16: VQ_F16, torch.bfloat16: VQ_BF16, torch.float32: VQ_F32}
 _V_LAYOUT = {"channel": VQ_V_CHANNEL_PACKED, "token": VQ_V_TOKEN_PACKED}
@@ -1281,6 +1281,54 @@ __all__ = [
 # ---------------------------------------------------------------------------
 # attention over VecInfer indices
 # ---------------------------------------------------------------------------
+
+def vecinfer_attend_indices(q: torch.Tensor, k_indices: torch.Tensor, k_codebook: torch.Tensor, v_indices: torch.Tensor,
+                            v_codebook: torch.Tensor, scale: float, *, n_tokens: int, smooth: torch.Tensor | None = None,
+                            H_mat: torch.Tensor | None = None, causal: bool = False, sliding_window: int = 0):
+    """Attention of a few query rows over the first ``n_tokens`` rows of codebook indices ``[B,H_kv,cap,n_sub]``, the
+    centroids gathered on chip and the query transform ``(q * smooth) @ H_mat`` (allocators/vecinfer.py:137-184) done
+    inside.  Returns ``None`` for shapes, types, orders or alignments that the kernel does not take."""
+    if (q.dtype not in _FLOAT_TAG or k_codebook.dtype not in _FLOAT_TAG or v_codebook.dtype not in _FLOAT_TAG
+            or k_indices.dtype not in (torch.uint8, torch.int32) or v_indices.dtype not in (torch.uint8, torch.int32)
+            or q.ndim != 4 or k_indices.ndim != 4 or v_indices.shape[:3] != k_indices.shape[:3] or q.shape[0] != k_indices.shape[0]
+            or not (k_indices.is_contiguous() and v_indices.is_contiguous() and k_codebook.is_contiguous() and v_codebook.is_contiguous())
+            or not (q.is_cuda and q.device == k_indices.device == v_indices.device == k_codebook.device == v_codebook.device)
+            or (k_indices.data_ptr() | v_indices.data_ptr()) % 16):
+        return None
+    B, H_q, S_q, D = q.shape
+    _, H_kv, cap, n_sub = k_indices.shape
+    if n_sub * k_codebook.shape[1] != D or v_indices.shape[3] * v_codebook.shape[1] != D:
+        return None
+    h, rows = 0.0, 1
+    if H_mat is not None:
+        h = _sylvester_scale(H_mat) if tuple(H_mat.shape) == (D, D) and H_mat.dtype == torch.float32 else 0.0
+        if h == 0.0:
+            return None
+    if smooth is not None:
+        if smooth.dtype != torch.float32 or smooth.device != q.device or smooth.shape[-1] != D or smooth.ndim > 2:
+            return None
+        smooth, rows = smooth.contiguous(), smooth.shape[0] if smooth.ndim == 2 else 1
+        if rows not in (1, H_kv):
+            return None
+    q = q.contiguous()
+    a = IndexAttendArgs(
+        q=q.data_ptr(), q_dtype=_FLOAT_TAG[q.dtype], out_dtype=_FLOAT_TAG[q.dtype], B=B, Hq=H_q, Hkv=H_kv, Sq=S_q, D=D,
+        k_idx=k_indices.data_ptr(), v_idx=v_indices.data_ptr(), k_idx_dtype=VQ_U8 if k_indices.dtype == torch.uint8 else VQ_I32,
+        v_idx_dtype=VQ_U8 if v_indices.dtype == torch.uint8 else VQ_I32, n_tokens=n_tokens, cap_tokens=cap,
+        k_codebook=k_codebook.data_ptr(), v_codebook=v_codebook.data_ptr(), k_cb_dtype=_FLOAT_TAG[k_codebook.dtype],
+        v_cb_dtype=_FLOAT_TAG[v_codebook.dtype], n_k_centroids=k_codebook.shape[0], n_v_centroids=v_codebook.shape[0],
+        k_sub_dim=k_codebook.shape[1], v_sub_dim=v_codebook.shape[1], smooth=None if smooth is None else smooth.data_ptr(),
+        smooth_rows=rows, hadamard_scale=h, scale=float(scale), causal=1 if causal else 0, sliding_window=int(sliding_window or 0))
+    lib = _lib.load()
+    need = lib.vq_vecinfer_attend_indices_workspace(C.byref(a))
+    if need == 0:
+        return None
+    out = torch.empty_like(q)
+    ws = _workspace(q.device, need)
+    a.out, a.workspace, a.workspace_bytes, a.stream = out.data_ptr(), ws.data_ptr(), ws.numel(), _stream(q)
+    _lib.check(lib.vq_vecinfer_attend_indices(C.byref(a)))
+    return out
+
 
 def metal_fused_sdpa(q_tilde: torch.Tensor, k_indices: torch.Tensor, k_codebook: torch.Tensor,
                      v_indices: torch.Tensor, v_codebook: torch.Tensor, scale: float, *, causal: bool = True,
