@@ -145,3 +145,10 @@ def test_fp16_large_magnitudes_match_fp32_assignment():
     idx16 = host(A.quantize_vq(to_dev(x, torch.float16), cb, 8))
     assert float((idx32 == idx16).mean()) > 0.99
     np.testing.assert_array_equal(idx32, ov.quantize_vq(x, host(cb), 8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [1, 2, 64, 128, 512])
+def test_hadamard_matrix_made_on_the_gpu_is_the_host_one(d):
+    require_gpu()
+    assert torch.equal(A.walsh_hadamard_matrix(d, device="cuda").cpu(), A.walsh_hadamard_matrix(d))

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import math
 
+import numpy as np
 import torch
 
 from .. import kernels as K
@@ -27,8 +28,13 @@ def walsh_hadamard_matrix(d: int, dtype=torch.float32, device=None) -> torch.Ten
     """Orthonormal Sylvester-Hadamard matrix ``[d, d]`` (vecinfer.py:60-87)."""
     if d < 1 or (d & (d - 1)) != 0:
         raise ValueError(f"walsh_hadamard_matrix: d={d} must be a power of 2.")
-    H = torch.ones((1, 1), dtype=torch.float32)
     r = 1.0 / math.sqrt(2.0)
+    if dtype == torch.float32 and device is not None and torch.device(device).type == "cuda" and K._plain_eager():
+        magnitude = np.float32(1.0)
+        for _ in range(d.bit_length() - 1):   # the products below, one rounding each
+            magnitude = np.float32(magnitude * np.float32(r))
+        return K.hadamard_matrix(d, float(magnitude), torch.device(device))
+    H = torch.ones((1, 1), dtype=torch.float32)
     while H.shape[0] < d:
         H = torch.cat([torch.cat([H, H], dim=1), torch.cat([H, -H], dim=1)], dim=0) * r
     return H.to(dtype=dtype, device=device)

@@ -81,7 +81,7 @@ class VecInferKVCache(FP16KVCache):
         sm = getattr(config, "smooth_factors", None)
         self._smooth = None if sm is None else torch.as_tensor(sm)
         self._validate_smooth()
-        self._H = walsh_hadamard_matrix(D, dtype=torch.float32)
+        self._H: torch.Tensor | None = None   # made on the device of the first keys
 
         n_kc, n_vc = 2 ** self._key_bits, 2 ** self._value_bits
         seed = opt["seed"]
@@ -136,7 +136,7 @@ class VecInferKVCache(FP16KVCache):
         sm = self._smooth
         if sm is None:
             return
-        sm32 = sm.float()
+        sm32 = sm.float().cpu()   # a few KB: one copy, not a row of kernels and a copy of their sum
         bad = ~(torch.isfinite(sm32) & (sm32 > _SMOOTH_FLOOR))
         n_bad = int(bad.sum())
         if n_bad:
@@ -163,8 +163,8 @@ class VecInferKVCache(FP16KVCache):
 
     def _to_device(self, ref: torch.Tensor) -> None:
         dev = ref.device
-        if self._H.device != dev:
-            self._H = self._H.to(dev)
+        if self._H is None or self._H.device != dev:
+            self._H = walsh_hadamard_matrix(self._head_dim, device=dev)
             self._key_codebook = self._key_codebook.to(dev)
             self._value_codebook = self._value_codebook.to(dev)
             if self._smooth is not None:

@@ -163,6 +163,23 @@ extern "C" int vq_vecinfer_encode_keys(const void *keys, int k_dtype, int64_t B,
     return VQ_OK;
 }
 
+namespace vq {
+// 64 KB at D = 128: the launch is all it costs (built on the host and copied: 300 us and a synchronisation)
+__global__ void hadamard_kernel(float *__restrict__ out, int64_t D, float magnitude) {
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < D * D; e += (int64_t)gridDim.x * blockDim.x)
+        out[e] = __popcll((unsigned long long)((e / D) & (e % D))) & 1 ? -magnitude : magnitude;
+}
+}  // namespace vq
+
+extern "C" int vq_hadamard(float *out, int64_t D, float magnitude, void *stream) {
+    const char *fn = "vq_hadamard";
+    VQ_REQUIRE(out != nullptr && D >= 1 && D <= (1 << 20) && (D & (D - 1)) == 0, VQ_ERR_INVALID, "%s: D=%lld must be a power of 2", fn, (long long)D);
+    const int64_t g = cdiv(D * D, 256);
+    hipLaunchKernelGGL(hadamard_kernel, dim3((unsigned)(g < 4096 ? g : 4096)), dim3(256), 0, (hipStream_t)stream, out, D, magnitude);
+    VQ_HIP_CHECK_LAUNCH(fn);
+    return VQ_OK;
+}
+
 extern "C" int vq_vecinfer_dequant(const void *idx, int idx_dtype, int64_t N, const void *codebook, int cb_dtype,
                                    int n_centroids, int sub_dim, void *out, int out_dtype, void *stream) {
     const char *fn = "vq_vecinfer_dequant";

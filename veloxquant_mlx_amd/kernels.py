@@ -765,6 +765,16 @@ vecinfer_quantize_hip = vecinfer_quantize_metal
 vecinfer_dequant_hip = vecinfer_dequant_metal
 
 
+def hadamard_matrix(D: int, magnitude: float, device: torch.device) -> torch.Tensor:
+    """The Sylvester-Hadamard matrix of entries +-``magnitude`` (a float32 value) made on the GPU, known to be one."""
+    H = torch.empty((D, D), dtype=torch.float32, device=device)
+    with torch.cuda.device(H.device):
+        _lib.check(_lib.load().vq_hadamard(H.data_ptr(), D, magnitude, _stream(H)))
+    if not H.is_inference():   # (such a tensor has no version to hold the verdict against)
+        H._vq_sylvester = (H._version, magnitude)
+    return H
+
+
 def _sylvester_scale(H_mat: torch.Tensor) -> float:
     """``|H[0, 0]|`` if ``H_mat`` is the orthonormal Sylvester-Hadamard matrix in natural order
     (every entry ``(-1)^popcount(a & b)`` times one magnitude), else 0.  Checked once per tensor
