@@ -184,11 +184,12 @@ int vq_kv_tail_append(const void *k_new, const void *v_new, const int64_t k_stri
                       int64_t tail_cap, int64_t pos, void *stream);
 
 /* The first tokens of a plain cache: rows [0, S) of the contiguous buffers [B, H, cap, D] from
- * k_new / v_new, rows [S, cap) zeroed, both buffers in one launch (arguments as above; the
+ * k_new / v_new, rows [S, cap) zeroed, both buffers in one launch; rows [skip0, skip1) of the first S are not written (the caller's
+ * next launch does: a round trip from the input straight into the buffer) (arguments as above; the
  * zeroed buffer a cache starts from and the assignment into it, veloxquant_mlx/cache/kivi_cache.py:248). */
 int vq_kv_fill(const void *k_new, const void *v_new, const int64_t k_strides[3], const int64_t v_strides[3],
                void *k_buf, void *v_buf, int elem_bytes, int64_t B, int64_t H, int64_t S, int64_t D, int64_t cap,
-               void *stream);
+               int64_t skip0, int64_t skip1, void *stream);
 
 /* A whole chunk of a packed KIVI cache in one call: the concatenation, the quantisation of
  * the tokens that aged out of the fp16 residual window and the start of the next tail
@@ -526,10 +527,11 @@ int vq_skvq_clipped_roundtrip(const void *x, void *out, int dtype, int64_t B, in
  * veloxquant_mlx/cache/skvq_cache.py:186-224): the channels by their range (largest minus smallest value over
  * the chunk, equal ranges in channel order) where that order has the lower mean squared float32 round-trip error, else
  * the stored order.  perm / inv: device int32 [H, D], written.  x as for vq_skvq_clipped_roundtrip.
- * workspace: vq_skvq_channel_orders_workspace bytes. */
-size_t vq_skvq_channel_orders_workspace(int64_t B, int64_t H, int64_t r, int64_t D, int group);
-int vq_skvq_channel_orders(const void *x, int dtype, int64_t B, int64_t H, int64_t r, int64_t D, int64_t x_stride_bh,
-                           int bits, int group, const float *alphas, int n_alphas, int32_t *perm, int32_t *inv,
+ * x2: a second tensor of the same shape and strides with bits2 (values beside keys), or NULL; its orders follow the
+ * first's, perm / inv [2, H, D].  workspace: vq_skvq_channel_orders_workspace bytes for 1 or 2 tensors. */
+size_t vq_skvq_channel_orders_workspace(int64_t B, int64_t H, int64_t r, int64_t D, int group, int tensors);
+int vq_skvq_channel_orders(const void *x, const void *x2, int dtype, int64_t B, int64_t H, int64_t r, int64_t D, int64_t x_stride_bh,
+                           int bits, int bits2, int group, const float *alphas, int n_alphas, int32_t *perm, int32_t *inv,
                            void *workspace, size_t workspace_bytes, void *stream);
 
 #ifdef __cplusplus

@@ -268,3 +268,21 @@ def test_first_tokens_of_a_plain_cache(dtype, B, H, S, D, layout):
     assert c.keys.shape[2] == -(-S // 256) * 256 and not c.keys[:, :, S:].any() and not c.values[:, :, S:].any()
     ko, vo = c.update_and_fetch(k[:, :, :1], v[:, :, :1])
     assert torch.equal(ko[:, :, S:], k[:, :, :1]) and torch.equal(vo[:, :, :S], v)
+
+
+@pytest.mark.parametrize("shape,window,n_sink", [((1, 2, 128, 64), 128, 0), ((2, 3, 391, 128), 128, 5), ((1, 1, 96, 256), 32, 31), ((2, 2, 100, 64), 128, 5)])
+def test_first_tokens_in_one_pass_are_the_same_as_in_place(shape, window, n_sink):
+    """Rows that go through the round trip on their way into the buffer, and both tensors' orders from one launch, against a cache
+    whose first tokens come in a layout (rows a multiple of two apart) that takes the copy and the in-place launches."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(shape[2])
+    k = torch.randn(shape, generator=gen, device="cuda").half() * torch.exp(torch.randn(shape[3], generator=gen, device="cuda")).half()
+    v = torch.randn(shape, generator=gen, device="cuda").half()
+    spread = lambda t: torch.stack([t, t], 3).flatten(2, 3)[:, :, ::2]
+    cfg = KVCacheConfig(method="skvq", head_dim=shape[3], skvq_window=window, skvq_n_sink=n_sink)
+    a, b = KVCacheFactory.create(cfg), KVCacheFactory.create(cfg)
+    outs = [c.update_and_fetch(x, y) for c, x, y in ((a, k, v), (b, spread(k), spread(v)))]
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    assert torch.equal(a.keys, b.keys) and torch.equal(a.values, b.values) and a.offset == b.offset
+    for p, q in ((a.key_perms, b.key_perms), (a.value_perms, b.value_perms)):
+        assert (p is None) == (q is None) and (p is None or torch.equal(p, q))

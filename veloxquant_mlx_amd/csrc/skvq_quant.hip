@@ -25,6 +25,9 @@ constexpr int SK_MAX_ALPHAS = 8;
 constexpr int SK_AHEAD = 4;    // rows a thread requests at a time
 
 struct SkAlphas { float a[SK_MAX_ALPHAS]; int n; };
+// what differs between the tensors of a launch (blockIdx.z); perm / inv as void: the order kernel writes them
+struct SkSide { const void *x; void *out; int32_t *perm, *inv; float levels; };
+struct SkSides { SkSide t[2]; };
 
 // clamp(rint((x - lo) / sc), 0, levels) without an IEEE division on the common path.  t = x - lo is
 // rounded once, as in the reference; q0 = t * rcp(sc) lies within 2.5 ulp (1.5e-7 relative) of the
@@ -100,14 +103,19 @@ template <typename T> struct Vec8 {
 };
 
 // ERR: the squared error of the float32 reconstruction instead of the reconstruction, the stored channel order
-// (blockIdx.y 0) against the order `perm` (1): err[(y n_rows + row) tpr + piece] takes the double-precision sum over
+// (blockIdx.y 0) against the order `perm` (1), of the tensor blockIdx.z: err[((2 z + y) n_rows + row) tpr + piece] takes the double-precision sum over
 // the channels of one thread's pieces, in stored channel order for both.
 template <typename T, int GROUP, bool ERR>   // GROUP > 0: the group size, known at compile time; 0: any
 __global__ __launch_bounds__(SK_THREADS)
-void skvq_roundtrip_kernel(const T *x, T *out, double *__restrict__ err, int64_t n_bh, int64_t H, int64_t r, int64_t D,
-                           int64_t x_stride_bh, int64_t out_stride_bh, const int32_t *__restrict__ perm, const int32_t *__restrict__ inv,
-                           int group, uint64_t group_magic, int G, int rows_pb, int tpr, bool vec, float levels, SkAlphas al) {
+void skvq_roundtrip_kernel(SkSides sides, double *__restrict__ err, int64_t n_bh, int64_t H, int64_t r, int64_t D,
+                           int64_t x_stride_bh, int64_t out_stride_bh,
+                           int group, uint64_t group_magic, int G, int rows_pb, int tpr, bool vec, SkAlphas al) {
     extern __shared__ float s_x[];
+    const SkSide side = sides.t[ERR ? blockIdx.z : 0];
+    const T *x = (const T *)side.x;
+    T *out = (T *)side.out;
+    const int32_t *__restrict__ perm = side.perm, *__restrict__ inv = side.inv;
+    const float levels = side.levels;
     if (ERR && blockIdx.y == 0) perm = inv = nullptr;
     const int tid = threadIdx.x;
     const int gstride = group + 1, Dp = G * group;
@@ -312,7 +320,7 @@ void skvq_roundtrip_kernel(const T *x, T *out, double *__restrict__ err, int64_t
                     sum += d * d;
                 }
             }
-            err[((int64_t)blockIdx.y * n_rows + row0 + lr) * tpr + cq] = sum;
+            err[((int64_t)(2 * blockIdx.z + blockIdx.y) * n_rows + row0 + lr) * tpr + cq] = sum;
         }
         return;
     }
@@ -340,7 +348,8 @@ void skvq_roundtrip_kernel(const T *x, T *out, double *__restrict__ err, int64_t
 
 // ---- channel orders of the first flushed chunk (veloxquant_mlx/cache/skvq_cache.py:186-224) ----
 //
-// Three launches a tensor: the candidate order of every head (channels by their range over the chunk's rows, equal
+// Three launches for keys and values together (they take different blocks of the same launches: latency is what they
+// cost, and one after the other they took 105 us instead of 53): the candidate order of every head (channels by their range over the chunk's rows, equal
 // ranges in channel order), the squared round-trip error of the stored and of the candidate order (the ERR form of the
 // kernel above), and the choice per head (the candidate only where its mean error is lower).  Latency is all there is
 // to them: 8 x 8 heads of 123 rows of 128 channels took 0.21 ms a tensor as library reductions and sorts.
@@ -357,8 +366,9 @@ __device__ __forceinline__ float sk_unkey(uint32_t k) { return __uint_as_float(k
 // SK_ORD_THREADS / (D / W) rows at a time.  LDS: smallest, largest, NaN mark of every channel, then the ranges.
 template <typename T, int W>
 __global__ __launch_bounds__(SK_ORD_THREADS)
-void skvq_order_kernel(const T *__restrict__ x, int64_t B, int64_t H, int64_t r, int D, int64_t x_stride_bh,
-                       int32_t *__restrict__ perm, int32_t *__restrict__ inv) {
+void skvq_order_kernel(SkSides sides, int64_t B, int64_t H, int64_t r, int D, int64_t x_stride_bh) {
+    const T *__restrict__ x = (const T *)sides.t[blockIdx.z].x;
+    int32_t *__restrict__ perm = sides.t[blockIdx.z].perm, *__restrict__ inv = sides.t[blockIdx.z].inv;
     extern __shared__ uint32_t s_ord[];
     uint32_t *s_mn = s_ord, *s_mx = s_ord + D, *s_nan = s_ord + 2 * D;
     float *s_rng = reinterpret_cast<float *>(s_ord);
@@ -428,8 +438,9 @@ void skvq_order_kernel(const T *__restrict__ x, int64_t B, int64_t H, int64_t r,
 
 // One block per head: both orders' errors summed in one fixed order, and the head's order kept or replaced by the stored one.
 __global__ __launch_bounds__(SK_ORD_THREADS)
-void skvq_choose_kernel(const double *__restrict__ err, int64_t B, int64_t H, int64_t r, int tpr, int D,
-                        int32_t *__restrict__ perm, int32_t *__restrict__ inv) {
+void skvq_choose_kernel(const double *__restrict__ err, int64_t B, int64_t H, int64_t r, int tpr, int D, SkSides sides) {
+    int32_t *__restrict__ perm = sides.t[blockIdx.z].perm, *__restrict__ inv = sides.t[blockIdx.z].inv;
+    err += (int64_t)blockIdx.z * 2 * B * H * r * tpr;
     __shared__ double s_sum[2][SK_ORD_THREADS];
     const int tid = threadIdx.x;
     const int64_t h = blockIdx.x, n_rows = B * H * r, per_bh = r * tpr;
@@ -497,13 +508,12 @@ static int plan_skvq(const char *fn, int64_t B, int64_t H, int64_t r, int64_t D,
 }
 
 template <typename T, bool ERR>
-static void launch_skvq(const SkPlan &p, const SkAlphas &al, const void *x, void *out, double *err, int64_t B, int64_t H, int64_t r, int64_t D,
-                        int64_t xs, int64_t os, const int32_t *perm, const int32_t *inv, int bits, int group, bool vec, hipStream_t st) {
-    const dim3 grid((unsigned)p.blocks, ERR ? 2 : 1);
-    const float levels = (float)((1 << bits) - 1);
+static void launch_skvq(const SkPlan &p, const SkAlphas &al, const SkSides &sides, int tensors, double *err, int64_t B, int64_t H, int64_t r,
+                        int64_t D, int64_t xs, int64_t os, int group, bool vec, hipStream_t st) {
+    const dim3 grid((unsigned)p.blocks, ERR ? 2 : 1, (unsigned)tensors);
 #define VQ_SK_LAUNCH(GROUP)                                                                                                   \
-    hipLaunchKernelGGL((skvq_roundtrip_kernel<T, GROUP, ERR>), grid, dim3(p.threads), p.lds, st, (const T *)x, (T *)out, err, B * H, H, \
-                       r, D, xs, os, perm, inv, group, p.group_magic, (int)p.G, (int)p.rows_pb, p.tpr, vec, levels, al)
+    hipLaunchKernelGGL((skvq_roundtrip_kernel<T, GROUP, ERR>), grid, dim3(p.threads), p.lds, st, sides, err, B * H, H, r, D, xs, os, \
+                       group, p.group_magic, (int)p.G, (int)p.rows_pb, p.tpr, vec, al)
     if (group == 32) VQ_SK_LAUNCH(32);
     else if (group == 64) VQ_SK_LAUNCH(64);
     else VQ_SK_LAUNCH(0);
@@ -530,44 +540,52 @@ extern "C" int vq_skvq_clipped_roundtrip(const void *x, void *out, int dtype, in
     // whether rows can move as 16-byte pieces
     const bool vec = (perm == nullptr || inv != nullptr) && D % 8 == 0 && x_stride_bh % 8 == 0 && out_stride_bh % 8 == 0 &&
                      ((uintptr_t)x % 16 == 0) && ((uintptr_t)out % 16 == 0);
+    SkSides sides = {};
+    sides.t[0] = {x, out, (int32_t *)perm, (int32_t *)inv, (float)((1 << bits) - 1)};
     VQ_DISPATCH_FLOAT(dtype, T, {
-        launch_skvq<T, false>(p, al, x, out, nullptr, B, H, r, D, x_stride_bh, out_stride_bh, perm, inv, bits, group, vec, (hipStream_t)stream);
+        launch_skvq<T, false>(p, al, sides, 1, nullptr, B, H, r, D, x_stride_bh, out_stride_bh, group, vec, (hipStream_t)stream);
     })
     VQ_HIP_CHECK_LAUNCH(fn);
     return VQ_OK;
 }
 
-extern "C" size_t vq_skvq_channel_orders_workspace(int64_t B, int64_t H, int64_t r, int64_t D, int group) {
-    if (B < 1 || H < 1 || r < 1 || D < 1 || group < 1) return 0;
+extern "C" size_t vq_skvq_channel_orders_workspace(int64_t B, int64_t H, int64_t r, int64_t D, int group, int tensors) {
+    if (B < 1 || H < 1 || r < 1 || D < 1 || group < 1 || tensors < 1 || tensors > 2) return 0;
     const int64_t pieces = ((D + group - 1) / group * group + 7) / 8, tpr = pieces < SK_THREADS ? pieces : SK_THREADS;
-    return (size_t)(2 * B * H * r * tpr) * sizeof(double);
+    return (size_t)(2 * tensors * B * H * r * tpr) * sizeof(double);
 }
 
-extern "C" int vq_skvq_channel_orders(const void *x, int dtype, int64_t B, int64_t H, int64_t r, int64_t D, int64_t x_stride_bh,
-                                      int bits, int group, const float *alphas, int n_alphas, int32_t *perm, int32_t *inv,
+extern "C" int vq_skvq_channel_orders(const void *x, const void *x2, int dtype, int64_t B, int64_t H, int64_t r, int64_t D, int64_t x_stride_bh,
+                                      int bits, int bits2, int group, const float *alphas, int n_alphas, int32_t *perm, int32_t *inv,
                                       void *workspace, size_t workspace_bytes, void *stream) {
     const char *fn = "vq_skvq_channel_orders";
     SkPlan p;
     SkAlphas al;
+    const int tensors = x2 != nullptr ? 2 : 1;
     VQ_REQUIRE(is_float_tag(dtype), VQ_ERR_INVALID, "%s: unsupported dtype tag %d", fn, dtype);
     VQ_REQUIRE(B >= 1 && H >= 1 && r >= 1 && D >= 1, VQ_ERR_INVALID, "%s: empty chunk", fn);
     const int rc = plan_skvq(fn, B, H, r, D, bits, group, alphas, n_alphas, p, al);
     if (rc != VQ_OK) return rc;
+    VQ_REQUIRE(x2 == nullptr || (bits2 >= 1 && bits2 <= 8), VQ_ERR_INVALID, "%s: bits must be in [1, 8], got %d", fn, bits2);
     VQ_REQUIRE(x && perm && inv && workspace, VQ_ERR_INVALID, "%s: null pointer", fn);
     VQ_REQUIRE(x_stride_bh >= r * D, VQ_ERR_INVALID, "%s: stride below r * D", fn);
     VQ_REQUIRE(H <= 0x7fffffff, VQ_ERR_UNSUPPORTED, "%s: too many heads", fn);
-    VQ_REQUIRE(workspace_bytes >= vq_skvq_channel_orders_workspace(B, H, r, D, group), VQ_ERR_WORKSPACE, "%s: workspace too small", fn);
-    const bool vec = D % 8 == 0 && x_stride_bh % 8 == 0 && (uintptr_t)x % 16 == 0;
+    VQ_REQUIRE(workspace_bytes >= vq_skvq_channel_orders_workspace(B, H, r, D, group, tensors), VQ_ERR_WORKSPACE, "%s: workspace too small", fn);
+    const bool vec = D % 8 == 0 && x_stride_bh % 8 == 0 && (((uintptr_t)x | (uintptr_t)x2) & 15u) == 0;
     double *err = (double *)workspace;
     hipStream_t st = (hipStream_t)stream;
+    SkSides sides = {};
+    sides.t[0] = {x, nullptr, perm, inv, (float)((1 << bits) - 1)};
+    if (x2 != nullptr) sides.t[1] = {x2, nullptr, perm + H * D, inv + H * D, (float)((1 << bits2) - 1)};
+    const dim3 heads((unsigned)H, 1, (unsigned)tensors);
     VQ_DISPATCH_FLOAT(dtype, T, {
         const size_t lds = (size_t)D * 12;   // D <= 12288 words of a row, so at most 144 KB
         auto kernel = vec ? skvq_order_kernel<T, 8> : skvq_order_kernel<T, 1>;
         if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        hipLaunchKernelGGL(kernel, dim3((unsigned)H), dim3(SK_ORD_THREADS), lds, st, (const T *)x, B, H, r, (int)D, x_stride_bh, perm, inv);
-        launch_skvq<T, true>(p, al, x, nullptr, err, B, H, r, D, x_stride_bh, x_stride_bh, perm, inv, bits, group, vec, st);
+        hipLaunchKernelGGL(kernel, heads, dim3(SK_ORD_THREADS), lds, st, sides, B, H, r, (int)D, x_stride_bh);
+        launch_skvq<T, true>(p, al, sides, tensors, err, B, H, r, D, x_stride_bh, x_stride_bh, group, vec, st);
     })
-    hipLaunchKernelGGL(skvq_choose_kernel, dim3((unsigned)H), dim3(SK_ORD_THREADS), 0, st, err, B, H, r, p.tpr, (int)D, perm, inv);
+    hipLaunchKernelGGL(skvq_choose_kernel, heads, dim3(SK_ORD_THREADS), 0, st, err, B, H, r, p.tpr, (int)D, sides);
     VQ_HIP_CHECK_LAUNCH(fn);
     return VQ_OK;
 }

@@ -5,20 +5,21 @@ namespace vq {
 
 struct TailSrc { const uint4 *p; int64_t sb, sh, ss; };   // strides in 16-byte vectors
 
-// Rows [pos, pos + S) of every (sequence, head) slab from the new tokens, rows [pos + S, end) zeroed; blockIdx.z = 0 keys,
-// 1 values.  A plain copy, bound by memory: a thread keeps one 16-byte column (the lanes of a wave lie side by side on a row
+// Rows [pos, pos + S) of every (sequence, head) slab from the new tokens, rows [pos + S, end) zeroed, new rows
+// [skip0, skip1) left to another kernel; blockIdx.z = 0 keys, 1 values.  A plain copy, bound by memory: a thread keeps one 16-byte column (the lanes of a wave lie side by side on a row
 // or on neighbouring rows) and walks rows, so that the only divisions are one per thread and one scalar one per slab; with the
 // coordinates of every vector divided out in 64 bits the same copy was bound by those divisions.
 constexpr int KF_PASSES = 8;   // rows a thread takes of a slab: enough loads in flight, and a block is worth its launch
 __global__ __launch_bounds__(256) void kv_fill_kernel(TailSrc k, TailSrc v, uint4 *__restrict__ k_dst, uint4 *__restrict__ v_dst,
                                                       int64_t BH, int64_t H, int64_t S, int row_vecs, int64_t cap, int64_t pos,
-                                                      int64_t end) {
+                                                      int64_t end, int64_t skip0, int64_t skip1) {
     const TailSrc src = blockIdx.z ? v : k;
     uint4 *dst = blockIdx.z ? v_dst : k_dst;
     const int width = row_vecs < 256 ? row_vecs : 256, rows = 256 / width;
     const int c0 = (int)threadIdx.x % width, r0 = (int)threadIdx.x / width;
     if (r0 >= rows) return;
     const int64_t n = end - pos, base = (int64_t)blockIdx.x * (rows * KF_PASSES) + r0;
+    auto skipped = [&](int64_t s) { return s >= skip0 && s < skip1; };
     for (int64_t bh = blockIdx.y; bh < BH; bh += gridDim.y) {
         const uint4 *from = src.p + (bh / H) * src.sb + (bh % H) * src.sh;
         uint4 *to = dst + (bh * cap + pos) * row_vecs;
@@ -28,12 +29,12 @@ __global__ __launch_bounds__(256) void kv_fill_kernel(TailSrc k, TailSrc v, uint
             for (int i = 0; i < KF_PASSES; ++i) {
                 const int64_t s = base + i * rows;
                 x[i] = make_uint4(0, 0, 0, 0);
-                if (s < S) x[i] = from[s * src.ss + c];
+                if (s < S && !skipped(s)) x[i] = from[s * src.ss + c];
             }
 #pragma unroll
             for (int i = 0; i < KF_PASSES; ++i) {
                 const int64_t s = base + i * rows;
-                if (s < n) to[s * row_vecs + c] = x[i];
+                if (s < n && !skipped(s)) to[s * row_vecs + c] = x[i];
             }
         }
     }
@@ -77,7 +78,7 @@ using namespace vq;
 
 static int kv_fill(const char *fn, const void *k_new, const void *v_new, const int64_t k_strides[3], const int64_t v_strides[3],
                    void *k_tail, void *v_tail, int elem_bytes, int64_t B, int64_t H, int64_t S, int64_t D, int64_t tail_cap,
-                   int64_t pos, int64_t end, hipStream_t stream) {
+                   int64_t pos, int64_t end, int64_t skip0, int64_t skip1, hipStream_t stream) {
     VQ_REQUIRE(elem_bytes == 2 || elem_bytes == 4, VQ_ERR_INVALID, "%s: elem_bytes must be 2 or 4, got %d", fn, elem_bytes);
     VQ_REQUIRE(B >= 0 && H >= 0 && S >= 0 && D >= 1, VQ_ERR_INVALID, "%s: negative dimension", fn);
     VQ_REQUIRE(pos >= 0 && pos + S <= tail_cap, VQ_ERR_INVALID, "%s: tokens [%lld, %lld) exceed the tail capacity %lld", fn,
@@ -100,7 +101,7 @@ static int kv_fill(const char *fn, const void *k_new, const void *v_new, const i
     const TailSrc v = {(const uint4 *)v_new, v_strides[0] / vec, v_strides[1] / vec, v_strides[2] / vec};
     const int64_t slabs = B * H < 65535 ? B * H : 65535;
     hipLaunchKernelGGL(kv_fill_kernel, dim3((unsigned)blocks, (unsigned)slabs, 2), dim3(256), 0, stream, k, v, (uint4 *)k_tail,
-                       (uint4 *)v_tail, B * H, H, S, (int)row_vecs, tail_cap, pos, end);
+                       (uint4 *)v_tail, B * H, H, S, (int)row_vecs, tail_cap, pos, end, skip0, skip1);
     VQ_HIP_CHECK_LAUNCH(fn);
     return VQ_OK;
 }
@@ -109,13 +110,16 @@ extern "C" int vq_kv_tail_append(const void *k_new, const void *v_new, const int
                                  const int64_t v_strides[3], void *k_tail, void *v_tail, int elem_bytes, int64_t B,
                                  int64_t H, int64_t S, int64_t D, int64_t tail_cap, int64_t pos, void *stream) {
     return kv_fill("vq_kv_tail_append", k_new, v_new, k_strides, v_strides, k_tail, v_tail, elem_bytes, B, H, S, D, tail_cap, pos,
-                   pos + S, (hipStream_t)stream);
+                   pos + S, 0, 0, (hipStream_t)stream);
 }
 
 extern "C" int vq_kv_fill(const void *k_new, const void *v_new, const int64_t k_strides[3], const int64_t v_strides[3], void *k_buf,
-                          void *v_buf, int elem_bytes, int64_t B, int64_t H, int64_t S, int64_t D, int64_t cap, void *stream) {
+                          void *v_buf, int elem_bytes, int64_t B, int64_t H, int64_t S, int64_t D, int64_t cap, int64_t skip0,
+                          int64_t skip1, void *stream) {
+    VQ_REQUIRE(skip0 >= 0 && skip0 <= skip1 && skip1 <= S, VQ_ERR_INVALID, "vq_kv_fill: rows [%lld, %lld) to leave out of %lld",
+               (long long)skip0, (long long)skip1, (long long)S);
     return kv_fill("vq_kv_fill", k_new, v_new, k_strides, v_strides, k_buf, v_buf, elem_bytes, B, H, S, D, cap, 0, cap,
-                   (hipStream_t)stream);
+                   skip0, skip1, (hipStream_t)stream);
 }
 
 // One call for a whole chunk of a packed KIVI cache: append, quantise what aged out of the

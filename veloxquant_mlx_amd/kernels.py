@@ -142,6 +142,14 @@ def _slab(name: str, t: torch.Tensor, what: str) -> int:
     return step
 
 
+def regular_slabs(t: torch.Tensor) -> bool:
+    """Whether ``t [B, H, r, D]`` is a token slice of a contiguous ``[B, H, cap, D]`` buffer."""
+    try:
+        return _slab("", t, "") >= 0
+    except ValueError:
+        return False
+
+
 def skvq_clipped_round_trip(x: torch.Tensor, bits: int, group_size: int, alphas, perm: torch.Tensor | None = None,
                             out: torch.Tensor | None = None, inv: torch.Tensor | None = None) -> torch.Tensor:
     """Round-trip ``x [B, H, r, D]`` through SKVQ's clipped group quantisation.
@@ -194,10 +202,11 @@ def skvq_clipped_round_trip(x: torch.Tensor, bits: int, group_size: int, alphas,
     return out
 
 
-def skvq_channel_orders(x: torch.Tensor, bits: int, group_size: int, alphas):
+def skvq_channel_orders(x: torch.Tensor, bits: int, group_size: int, alphas, x2: torch.Tensor | None = None, bits2: int = 0):
     """Channel order per head and its inverse, int32 ``[H, D]`` each, from a chunk ``x [B, H, r, D]`` (a token slice of
     a larger ``[B, H, cap, D]`` buffer): channels sorted by range, kept only on heads where that lowers the mean squared
-    round-trip error (``SKVQKVCache._per_head_perms``, veloxquant_mlx/cache/skvq_cache.py:186-224)."""
+    round-trip error (``SKVQKVCache._per_head_perms``, veloxquant_mlx/cache/skvq_cache.py:186-224).  With ``x2`` (a chunk
+    of the same shape, its own ``bits2``) both at once: ``[2, H, D]`` each."""
     name = "skvq_channel_orders"
     if x.ndim != 4 or x.numel() == 0:
         raise ValueError(f"{name}: x must be a non-empty [B, H, r, D], got {tuple(x.shape)}")
@@ -205,16 +214,21 @@ def skvq_channel_orders(x: torch.Tensor, bits: int, group_size: int, alphas):
     _need_gpu(name, x)
     B, H, r, D = x.shape
     xs = _slab(name, x, "x")
+    tensors = 1 if x2 is None else 2
+    if x2 is not None:
+        _need_gpu(name, x2)
+        if x2.shape != x.shape or x2.dtype != x.dtype or x2.device != x.device or _slab(name, x2, "x2") != xs:
+            raise ValueError(f"{name}: x2 must match x in shape, type, device and strides")
     al = [float(a) for a in alphas]
-    perm = torch.empty((H, D), dtype=torch.int32, device=x.device)
+    perm = torch.empty((tensors, H, D), dtype=torch.int32, device=x.device)
     inv = torch.empty_like(perm)
     lib = _lib.load()
-    n = lib.vq_skvq_channel_orders_workspace(B, H, r, D, int(group_size))
+    n = lib.vq_skvq_channel_orders_workspace(B, H, r, D, int(group_size), tensors)
     ws = torch.empty((n,), dtype=torch.uint8, device=x.device)
-    _lib.check(lib.vq_skvq_channel_orders(x.data_ptr(), tag, B, H, r, D, xs, int(bits), int(group_size),
-                                          (C.c_float * len(al))(*al), len(al), perm.data_ptr(), inv.data_ptr(),
-                                          ws.data_ptr(), n, _stream(x)))
-    return perm, inv
+    _lib.check(lib.vq_skvq_channel_orders(x.data_ptr(), None if x2 is None else x2.data_ptr(), tag, B, H, r, D, xs, int(bits),
+                                          int(bits2), int(group_size), (C.c_float * len(al))(*al), len(al), perm.data_ptr(),
+                                          inv.data_ptr(), ws.data_ptr(), n, _stream(x)))
+    return (perm, inv) if tensors == 2 else (perm[0], inv[0])
 
 
 def row_norms(x: torch.Tensor) -> torch.Tensor:
@@ -540,9 +554,10 @@ def kv_rows_copyable(k_new: torch.Tensor, v_new: torch.Tensor) -> bool:
     return True
 
 
-def kv_fill(k_new: torch.Tensor, v_new: torch.Tensor, cap: int):
+def kv_fill(k_new: torch.Tensor, v_new: torch.Tensor, cap: int, skip: tuple[int, int] = (0, 0)):
     """Buffers ``[B, H, cap, D]`` that start with ``k_new, v_new [B, H, S, D]`` and are zero from there on, in one
-    launch; the tokens are ones that :func:`kv_rows_copyable` accepts."""
+    launch; the tokens are ones that :func:`kv_rows_copyable` accepts.  Rows ``skip[0] .. skip[1] - 1`` are left for the
+    caller to write."""
     B, H, S, D = k_new.shape
     if cap < S:
         raise ValueError(f"kv_fill: {S} tokens exceed the capacity {cap}")
@@ -550,7 +565,7 @@ def kv_fill(k_new: torch.Tensor, v_new: torch.Tensor, cap: int):
     ks, vs = k_new.stride(), v_new.stride()
     _lib.check(_lib.load().vq_kv_fill(k_new.data_ptr(), v_new.data_ptr(), (C.c_int64 * 3)(ks[0], ks[1], ks[2]),
                                       (C.c_int64 * 3)(vs[0], vs[1], vs[2]), kb.data_ptr(), vb.data_ptr(), k_new.element_size(),
-                                      B, H, S, D, cap, _stream(k_new)))
+                                      B, H, S, D, cap, skip[0], skip[1], _stream(k_new)))
     return kb, vb
 
 
