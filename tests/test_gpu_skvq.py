@@ -83,6 +83,38 @@ def test_round_trip_kernel_matches_the_oracle_bit_for_bit(dtype, B, H, r, D, bit
         assert not torch.equal(plain, out)
 
 
+@pytest.mark.parametrize("alphas", [o.DEFAULT_ALPHA_GRID, (1.0, 0.999, 0.998, 0.5, 1e-3, 1e-30, 1.0, 0.999)])
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+@pytest.mark.parametrize("group", [32, 64])
+def test_search_narrowed_by_bounds_takes_the_stated_winner(group, bits, alphas):
+    """Groups whose factors' errors lie close together, and values at the ends of what the bounds cover.  Bit for bit: the
+    factors that the bounds leave open are compared by the stated rule."""
+    require_gpu()
+    rng = np.random.default_rng(group + bits + len(alphas))
+    n, D = 24, 128
+    base = rng.standard_normal((n, D)).astype(np.float32)
+    kinds = [
+        base,
+        base.astype(np.float16).astype(np.float32),
+        np.float32(1000) + base * np.float32(1e-3),                 # range far below the magnitude
+        np.float32(1e6) + np.round(base),
+        np.round(base * 2),                                         # few distinct values, many ties
+        np.sign(base),                                              # two values: clipping only adds errors
+        np.full_like(base, 3.25),                                   # no range: every factor alike
+        base * np.float32(1e-7), base * np.float32(1e-18), base * np.float32(1e-30),
+        base * np.float32(1e14), base * np.float32(3e15), base * np.float32(1e25),
+        np.where(rng.random((n, D)) < 0.03, base * np.float32(50), base),
+        np.where(rng.random((n, D)) < 0.03, np.float32(1e15), base),
+        np.where(rng.random((n, D)) < 0.03, np.float32(9e14), np.float32(-9e14)) + base,
+    ]
+    x = np.concatenate(kinds).reshape(1, 1, -1, D).astype(np.float32)
+    with np.errstate(all="ignore"):
+        ref = o.round_trip(x, None, None, bits, group, alphas)
+    out = host(K.skvq_clipped_round_trip(to_dev(x), bits, group, alphas))
+    rows = np.where((_bits(out) != _bits(ref)).any(axis=-1).ravel())[0]
+    assert rows.size == 0, f"kinds {sorted(set((rows // n).tolist()))}"
+
+
 def test_round_trip_in_place_on_a_slice_of_a_larger_buffer():
     require_gpu()
     k, _ = _kv(2, 3, 40, 64, seed=2, channel_scales=_het_scales(64))

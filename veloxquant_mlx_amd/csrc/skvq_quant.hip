@@ -102,6 +102,51 @@ template <typename T> struct Vec8 {
     }
 };
 
+// The clip factors whose error can be the smallest, as bits.  The stated error of a factor -- codes by division, every step
+// rounded, squares added left to right -- costs ten operations a value and a division where a code is near a tie; five give r = sc * sqrt(sum((t - q)^2)) with
+// t = (x - lo) / sc in one fma and q = clamp(rint(t)), which is close enough to rule out
+// all factors but one in 99.6 % of the groups at 4 bits (a 4100-token prompt of 8 x 8 heads, both tensors: 243 -> 230 us; what
+// is left is the exchange of rows with LDS in the head's order and the latency of a wave's one batch of rows).
+// How close (u = 2^-24, W = levels * sc, M the largest |x|, so |lo| <= M and |x - lo| <= rng to within a few u * M):
+//   * the stated difference d = q * sc + lo - x of a code has an error of u (3 W + 3 M);
+//   * t has an error of u (2 rng + M) / sc (1 / sc is good to u after the Newton step), the stated quotient one of 2 u rng / sc;
+//   * codes that differ for that stand on either side of a tie, so their |d| differ by twice the sum of both;
+//   * t - q is rounded where the clamp moved q: u rng.
+// So every |d| is within u (3 W + 6 M + 11 rng) of sc |t - q|, and by the triangle inequality the roots of the two sums differ
+// by at most sqrt(GROUP) times that; the sums' own rounding and the root cost (GROUP + 6) u relative.  The bounds below are these
+// with a fourth to spare.  Errors below 1e-15, where squares lose bits, stay open, and so does everything at magnitudes
+// whose squares could overflow and for values that are not numbers.  `low` is the group's own memory, read before.
+// best_lo / best_sc: of the one factor that is open, if it is one.
+template <int GROUP, class Factor>
+__device__ __forceinline__ uint32_t sk_open_factors(const float *xv, float *low, const SkAlphas &al, const Factor &factor, float M, float rng,
+                                                    float levels, float &best_lo, float &best_sc) {
+    constexpr float U = 5.9604645e-8f, REL = (GROUP + 16) * U, ROOT = GROUP <= 32 ? 5.66f : 8.01f;
+    static_assert(GROUP >= SK_MAX_ALPHAS && GROUP <= 64, "a group has a word for every factor");
+    float high = INFINITY;   // the smallest upper bound of a factor's error
+    for (int k = 0; k < al.n; ++k) {
+        float lo, sc, s0 = 0.f;
+        factor(k, lo, sc);
+        float rs = __builtin_amdgcn_rcpf(sc);
+        rs = __builtin_fmaf(__builtin_fmaf(-sc, rs, 1.f), rs, rs);
+        const float c = -lo * rs;
+#pragma unroll
+        for (int j = 0; j < GROUP; ++j) {
+            const float t = __builtin_fmaf(xv[j], rs, c);
+            const float d = t - __builtin_amdgcn_fmed3f(__builtin_rintf(t), 0.f, levels);
+            s0 = __builtin_fmaf(d, d, s0);
+        }
+        const float r = sc * __builtin_amdgcn_sqrtf(s0);
+        const float off = ROOT * U * (4.f * levels * sc + 8.f * M + 14.f * rng) + 1e-15f;
+        low[k] = s0 < 1e30f ? r * (1.f - REL) - off : -INFINITY;   // (a factor near 0 can overflow the sum)
+        const float up = r * (1.f + REL) + off;
+        if (up < high) { high = up; best_lo = lo; best_sc = sc; }   // (this factor stays open)
+    }
+    if (!(M < 1e15f)) high = INFINITY;
+    uint32_t open = 0;
+    for (int k = 0; k < al.n; ++k) open |= (low[k] > high ? 0u : 1u) << k;
+    return open;
+}
+
 // ERR: the squared error of the float32 reconstruction instead of the reconstruction, the stored channel order
 // (blockIdx.y 0) against the order `perm` (1), of the tensor blockIdx.z: err[((2 z + y) n_rows + row) tpr + piece] takes the double-precision sum over
 // the channels of one thread's pieces, in stored channel order for both.
@@ -245,13 +290,23 @@ void skvq_roundtrip_kernel(SkSides sides, double *__restrict__ err, int64_t n_bh
             for (int j = 1; j < GROUP; ++j) { mn = fminf(mn, xv[j]); mx = fmaxf(mx, xv[j]); }
             const float mid = __fmul_rn(__fadd_rn(mx, mn), 0.5f), rng = __fsub_rn(mx, mn);
             const float tie = 0.5f - 1e-6f * (levels + 2.0f);
-            float best_err = 0.f, best_lo = 0.f, best_sc = 1.f;
-            for (int k = 0; k < al.n; ++k) {
+            auto factor = [&](int k, float &lo, float &sc) {
                 const float ar = __fmul_rn(al.a[k], rng);
-                const float lo = __fsub_rn(mid, __fmul_rn(ar, 0.5f));
-                const float sc = fmaxf(__fdiv_rn(ar, levels), 1e-8f);
+                lo = __fsub_rn(mid, __fmul_rn(ar, 0.5f));
+                sc = fmaxf(__fdiv_rn(ar, levels), 1e-8f);
+            };
+            float best_err = 0.f, best_lo = 0.f, best_sc = 1.f;
+            uint32_t open = 1u;   // the factors that can be the winner
+            if (al.n > 1) open = sk_open_factors<GROUP>(xv, p, al, factor, fmaxf(fabsf(mn), fabsf(mx)), rng, levels, best_lo, best_sc);
+            else factor(0, best_lo, best_sc);
+            const bool several = (open & (open - 1)) != 0;
+            bool first = true;
+            for (int k = 0; k < al.n; ++k) {
+                const bool mine = several && ((open >> k) & 1u);
+                if (__builtin_amdgcn_ballot_w64(mine) == 0) continue;
+                float lo, sc, sum = 0.f;
+                factor(k, lo, sc);
                 const float rs = __builtin_amdgcn_rcpf(sc);
-                float sum = 0.f;
 #pragma unroll
                 for (int j0 = 0; j0 < GROUP; j0 += 8) {
                     float q[8];
@@ -263,7 +318,8 @@ void skvq_roundtrip_kernel(SkSides sides, double *__restrict__ err, int64_t n_bh
                     }
                 }
                 const float err = __fdiv_rn(sum, (float)GROUP);
-                if (k == 0 || err < best_err) { best_err = err; best_lo = lo; best_sc = sc; }
+                if (mine && (first || err < best_err)) { best_err = err; best_lo = lo; best_sc = sc; }
+                if (mine) first = false;
             }
             const float best_rs = __builtin_amdgcn_rcpf(best_sc);
 #pragma unroll
