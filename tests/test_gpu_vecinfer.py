@@ -159,6 +159,23 @@ def test_large_codebooks_split_and_image_forms(sub, nc, n):
     assert host(K.vecinfer_quantize_metal(to_dev(x[:2]), to_dev(cb), sub)).reshape(-1)[0] == 0
 
 
+@pytest.mark.parametrize("far_out", [1e16, 3e19, float("inf")])
+@pytest.mark.parametrize("sub,nc,n", [(4, 256, 200), (8, 300, 200), (4, 1000, 200), (4, 4096, 200), (8, 2048, 200), (4, 4096, 33000)])
+def test_a_diverged_centroid_leaves_the_exact_rule_to_the_others(sub, nc, n, far_out):
+    """One centroid whose square leaves the range the filter can be brought to, beside centroids whose squares pass the
+    largest fp16 number: sub-vectors on and near all of them, in every form of the kernel."""
+    require_gpu()
+    rng = np.random.default_rng(nc + sub)
+    cb = (rng.standard_normal((nc, sub)) * 300).astype(np.float32)
+    cb[nc // 3] = far_out
+    near = cb[rng.integers(0, nc, n)]
+    near[~(np.abs(near[:, 0]) < 1e10)] = 5.0
+    x = (near + rng.standard_normal((n, sub)) * np.float32(20) * (rng.random((n, 1)) < 0.7)).astype(np.float32)
+    with np.errstate(all="ignore"):
+        ref = cref.vq_assign(x, cb, sub).reshape(-1)
+    np.testing.assert_array_equal(host(K.vecinfer_quantize_metal(to_dev(x), to_dev(cb), sub)).reshape(-1), ref)
+
+
 @pytest.mark.parametrize("scale", [1e-6, 1e-3, 1e3, 1e6])
 def test_assignment_follows_the_exact_rule_at_any_scale(scale):
     require_gpu()

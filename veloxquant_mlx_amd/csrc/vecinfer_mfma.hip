@@ -232,9 +232,13 @@ template <int SUB> __device__ __forceinline__ void split_h(const float *v, u32 *
         lo[e / 2] = pack_h2(v[e] - (float)a, v[e + 1] - (float)b);
     }
 }
-// the power of two that puts cmax2 = max |c|^2 into [256, 1024)
+// The power of two that puts cmax2 = max |c|^2 into [256, 1024).  Codebooks that none does this to: of squares near zero, whose
+// scores all lie within the margin; of squares near infinity (a diverged centroid), whose other centroids the fp16 parts of
+// |c|^2 cannot hold -- the scale is not a number then, so that no sub-vector is in the filter's range (make_operands) and the
+// exact rule alone decides.
 __device__ __forceinline__ float codebook_scale(float cmax2) {
-    if (!(cmax2 > 1e-30f) || !(cmax2 < 1e30f)) return 1.f;
+    if (!(cmax2 > 1e-30f)) return 1.f;
+    if (!(cmax2 < 1e30f)) return NAN;
     const int e = (int)((__float_as_uint(cmax2) >> 23) & 255u) - 127;   // 2^e <= cmax2 < 2^(e+1)
     const int k = (e - 8) >> 1;                                         // floor
     return __uint_as_float((u32)(127 - k) << 23);
@@ -349,7 +353,7 @@ template <int SUB> __device__ __forceinline__ void make_operands(SubVec<SUB> &s,
         v[e] = s.xf[e] * cs;
         s.x2 = __builtin_fmaf(v[e], v[e], s.x2);
     }
-    s.far = !(s.x2 <= 6.7e7f);   // 256 to 512 times the largest centroid; a NaN ends here too
+    s.far = !(s.x2 <= 6.7e7f);   // 256 to 512 times the largest centroid; a NaN, of the sub-vector or of the scale, ends here too
     if (s.far) {
         s.x2 = 0.f;
 #pragma unroll
