@@ -10,6 +10,7 @@ import torch
 from oracle import cref, vecinfer as ov
 from tests._gpu import gpu, host, require_gpu, to_dev
 from veloxquant_mlx_amd import kernels as K
+from veloxquant_mlx_amd.cache import KVCacheConfig, KVCacheFactory
 
 pytestmark = gpu
 
@@ -448,3 +449,30 @@ def test_encode_keys_other_shapes_take_the_composition():
         K.vecinfer_encode_decode_metal(to_dev(keys[0]), to_dev(cb), 8, to_dev(Hm))
     with pytest.raises(ValueError, match="not divisible"):
         K.vecinfer_encode_decode_metal(to_dev(keys), to_dev(cb), 7, to_dev(Hm))
+
+
+@pytest.mark.parametrize("modes", [{}, dict(fused_sdpa=True), dict(fused_sdpa=True, fused_sdpa_memory_bound=True)])
+@pytest.mark.parametrize("key_bits,key_sub", [(12, 4), (8, 8), (4, 16)])
+def test_cache_under_inference_mode(modes, key_bits, key_sub):
+    """Filled and attended under ``torch.inference_mode``, from its first keys on and from a restored state on: the values of a
+    cache outside of it."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    r = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    cfg = KVCacheConfig(method="vecinfer", head_dim=64, key_codebook_bits=key_bits, key_sub_dim=key_sub, smooth_factors=r(2, 64).exp(),
+                        key_codebook=r(1 << key_bits, key_sub), value_codebook=r(256, 8), **modes)
+    k, v, q = r(1, 2, 70, 64).half(), r(1, 2, 70, 64).half(), r(1, 4, 1, 64).half()
+
+    def use():
+        c = KVCacheFactory.create(cfg)
+        outs = [*c.update_and_fetch(k, v), *c.update_and_fetch(k[:, :, :1], v[:, :, :1])]
+        if modes:
+            outs.append(c.fused_sdpa(q, 0.1))
+            d = KVCacheFactory.create(cfg)
+            d.state = c.state
+            outs += [d.fused_sdpa(q, 0.1), d.fused_sdpa(q, 0.1)]
+        return outs
+    want = use()
+    with torch.inference_mode():
+        got = use()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

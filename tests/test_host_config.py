@@ -104,6 +104,20 @@ def test_kivi_cache_surface():
     assert KIVIKVCache(KVCacheConfig(method="kivi"))._v_layout == "token"
 
 
+def test_hadamard_check_of_inference_tensors():
+    """A matrix made under ``torch.inference_mode`` has no version to hold the verdict against: it is looked at each time."""
+    import torch
+
+    from veloxquant_mlx_amd.allocators.vecinfer import walsh_hadamard_matrix
+    from veloxquant_mlx_amd.kernels import _sylvester_scale
+    plain = walsh_hadamard_matrix(8)
+    with torch.inference_mode():
+        H = walsh_hadamard_matrix(8)
+        assert H.is_inference() and _sylvester_scale(H) == _sylvester_scale(plain) == float(plain[0, 0])
+        H[3, 4] += 1.0
+        assert _sylvester_scale(H) == 0.0
+
+
 def test_vecinfer_cache_validation():
     import numpy as np
     kw = dict(method="vecinfer", key_codebook=np.zeros((256, 8), np.float32), key_sub_dim=8, key_codebook_bits=8,

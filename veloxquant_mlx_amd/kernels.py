@@ -781,21 +781,24 @@ vecinfer_dequant_hip = vecinfer_dequant_metal
 
 
 def hadamard_matrix(D: int, magnitude: float, device: torch.device) -> torch.Tensor:
-    """The Sylvester-Hadamard matrix of entries +-``magnitude`` (a float32 value) made on the GPU, known to be one."""
-    H = torch.empty((D, D), dtype=torch.float32, device=device)
+    """The Sylvester-Hadamard matrix of entries +-``magnitude`` (a float32 value) made on the GPU, known to be one.  An ordinary
+    tensor under ``torch.inference_mode`` too: it outlives the call, and the verdict is held against its version."""
+    with torch.inference_mode(False):
+        H = torch.empty((D, D), dtype=torch.float32, device=device)
     with torch.cuda.device(H.device):
         _lib.check(_lib.load().vq_hadamard(H.data_ptr(), D, magnitude, _stream(H)))
-    if not H.is_inference():   # (such a tensor has no version to hold the verdict against)
-        H._vq_sylvester = (H._version, magnitude)
+    H._vq_sylvester = (H._version, magnitude)
     return H
 
 
 def _sylvester_scale(H_mat: torch.Tensor) -> float:
     """``|H[0, 0]|`` if ``H_mat`` is the orthonormal Sylvester-Hadamard matrix in natural order
     (every entry ``(-1)^popcount(a & b)`` times one magnitude), else 0.  Checked once per tensor
-    object and version (the verdict rides on the tensor itself)."""
+    object and version (the verdict rides on the tensor itself), on every call where there is no version (a tensor made
+    under ``torch.inference_mode``)."""
+    version = None if H_mat.is_inference() else H_mat._version
     memo = getattr(H_mat, "_vq_sylvester", None)
-    if memo is None or memo[0] != H_mat._version:
+    if memo is None or version is None or memo[0] != version:
         D = H_mat.shape[0]
         ok = H_mat.ndim == 2 and H_mat.shape[1] == D and D >= 1 and (D & (D - 1)) == 0
         h = 0.0
@@ -808,8 +811,9 @@ def _sylvester_scale(H_mat: torch.Tensor) -> float:
             for b in range(max(D.bit_length() - 1, 0)):
                 sign = sign * (1 - 2 * ((par >> b) & 1)).to(Hf.dtype)
             ok = h > 0 and bool(torch.equal(Hf, sign * h))
-        memo = (H_mat._version, h if ok else 0.0)
-        H_mat._vq_sylvester = memo
+        memo = (version, h if ok else 0.0)
+        if version is not None:
+            H_mat._vq_sylvester = memo
     return memo[1]
 
 
