@@ -394,6 +394,23 @@ def test_encode_keys_on_integer_keys_is_exact(D, sub):
     np.testing.assert_array_equal(host(idx8), idx_ref.astype(np.uint8))
 
 
+def test_encode_keys_at_any_storage_offset():
+    """Keys and smoothing factors that are contiguous but start between 16-byte boundaries, at codebooks on both sides of 256
+    centroids: the same values as from aligned memory."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    r = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    keys, smooth, Hm = r(1, 2, 7, 128).half(), r(2, 128).exp(), to_dev(ov.walsh_hadamard_matrix(128))
+    moved = torch.empty(keys.numel() + 1, dtype=keys.dtype, device="cuda")[1:].view(keys.shape).copy_(keys)
+    smooth_moved = torch.empty(smooth.numel() + 3, device="cuda")[3:].view(smooth.shape).copy_(smooth)
+    assert moved.is_contiguous() and moved.data_ptr() % 16 and smooth_moved.data_ptr() % 16
+    for nc, sub in ((4096, 4), (2048, 8), (256, 8)):
+        cb = r(nc, sub)
+        ref = K.vecinfer_encode_decode_metal(keys, cb, sub, Hm, smooth, want_k_tilde=True)
+        for k, sm in ((moved, smooth), (keys, smooth_moved)):
+            assert all(torch.equal(a, b) for a, b in zip(K.vecinfer_encode_decode_metal(k, cb, sub, Hm, sm, want_k_tilde=True), ref))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("smooth_rows", [None, 1, "heads", "vector"])
 def test_encode_keys_random_keys(dtype, smooth_rows):

@@ -856,6 +856,7 @@ def vecinfer_encode_decode_metal(keys: torch.Tensor, k_codebook: torch.Tensor, s
     h = _sylvester_scale(H_mat)
     fused = h > 0 and sub_dim in (4, 8) and n_sub in (8, 16, 32, 64) and cb.shape[0] * sub_dim <= 16384
     if fused:
+        kk, sm = (t if t is None or t.data_ptr() % 16 == 0 else t.clone() for t in (kk, sm))   # contiguous, but off the boundary
         idx = torch.empty((B, Hh, S, n_sub), dtype=index_dtype, device=keys.device)
         k_hat = torch.empty_like(kk) if want_k_hat else None
         k_tilde = torch.empty((B, Hh, S, D), dtype=torch.float32, device=keys.device) if want_k_tilde else None
