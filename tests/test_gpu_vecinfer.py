@@ -411,6 +411,25 @@ def test_encode_keys_at_any_storage_offset():
             assert all(torch.equal(a, b) for a, b in zip(K.vecinfer_encode_decode_metal(k, cb, sub, Hm, sm, want_k_tilde=True), ref))
 
 
+def test_encode_keys_with_a_large_codebook_keeps_the_gradient_of_the_factors():
+    """Above 256 centroids the reconstruction (centroids @ H^T) * smooth carries gradients to the smoothing factors, and the
+    transformed keys to the keys."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    r = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    keys, smooth, cb, Hm = r(1, 2, 9, 64), r(2, 64).exp(), r(1024, 4), to_dev(ov.walsh_hadamard_matrix(64))
+    sm, kk = smooth.clone().requires_grad_(), keys.clone().requires_grad_()
+    k_hat, _, k_tilde = K.vecinfer_encode_decode_metal(keys, cb, 4, Hm, sm, want_k_tilde=True)
+    g, = torch.autograd.grad(k_hat.sum(), sm)
+    torch.testing.assert_close(g, (k_hat.detach() / smooth[None, :, None]).sum(dim=(0, 2)), rtol=1e-4, atol=1e-3)
+    *_, k_tilde = K.vecinfer_encode_decode_metal(kk, cb, 4, Hm, smooth, want_k_tilde=True)
+    g, = torch.autograd.grad(k_tilde.sum(), kk)
+    torch.testing.assert_close(g, (Hm.sum(1) / smooth[:, None])[None].expand_as(g), rtol=1e-4, atol=1e-4)
+    with torch.no_grad():   # nothing to differentiate: the fused launch, at the same values
+        k_fused, _ = K.vecinfer_encode_decode_metal(keys, cb, 4, Hm, sm)
+    torch.testing.assert_close(k_fused, k_hat.detach(), rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("smooth_rows", [None, 1, "heads", "vector"])
 def test_encode_keys_random_keys(dtype, smooth_rows):

@@ -855,6 +855,9 @@ def vecinfer_encode_decode_metal(keys: torch.Tensor, k_codebook: torch.Tensor, s
     n_sub = D // sub_dim
     h = _sylvester_scale(H_mat)
     fused = h > 0 and sub_dim in (4, 8) and n_sub in (8, 16, 32, 64) and cb.shape[0] * sub_dim <= 16384
+    if fused and cb.shape[0] > 256:   # the composition's products carry gradients and tangents: a caller who asks for them keeps them
+        fused = torch.autograd.forward_ad._current_level < 0 and not (torch.is_grad_enabled() and (
+            H_mat.requires_grad or (sm is not None and sm.requires_grad) or (want_k_tilde and keys.requires_grad)))
     if fused:
         kk, sm = (t if t is None or t.data_ptr() % 16 == 0 else t.clone() for t in (kk, sm))   # contiguous, but off the boundary
         idx = torch.empty((B, Hh, S, n_sub), dtype=index_dtype, device=keys.device)
