@@ -91,3 +91,30 @@ def test_indices_refused_shapes():
     assert attend(z(1, 4, 1, 128, dtype=torch.float64)) is None
     assert attend(z(1, 4, 1, 128), ki=z(1, 2, 64, 64, dtype=torch.int32)[..., ::2]) is None
     assert attend(z(1, 4, 1, 128), ki=z(1, 2, 64, 16, dtype=torch.int32), kcb=z(8192, 8)) is None   # codebook past LDS
+
+
+def _byte_call(B, Hkv, D, n, gen, group=32, bits=8, meta=torch.float32):
+    r = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    words = lambda: torch.randint(0, 2 ** 31 - 1, (B, Hkv, n, -(-D // (32 // bits))), generator=gen, device="cuda", dtype=torch.int32)
+    ks, vs = r(B, Hkv, -(-n // group), D).abs() * 0.02, r(B, Hkv, n, -(-D // group)).abs() * 0.02
+    half = 2.0 ** (bits - 1)
+    return dict(k_packed=words(), k_scale=ks.to(meta), k_zero=(-half * ks).to(meta), v_packed=words(), v_scale=vs.to(meta),
+                v_zero=(-half * vs).to(meta), n_packed=n, bits=bits, group_size=group, scale=D ** -0.5)
+
+
+@pytest.mark.parametrize("bits,group,Hq,Hkv,D,path", [(4, 32, 16, 4, 32, 3), (8, 32, 16, 4, 64, 4), (4, 4, 16, 4, 32, 0)])
+def test_a_batch_adds_in_the_order_of_its_parts(bits, group, Hq, Hkv, D, path):
+    """Under ``fixed_order`` with the same cut, sequences of a large batch (more than 8192 query rows) give the bits that they
+    give in a small one: layers stacked into one call against a call a layer."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(bits + D)
+    B = 8192 // Hq + 2
+    kw = _byte_call(B, Hkv, D, 4096, gen, group, bits)
+    q, plan, one = torch.randn((B, Hq, 1, D), generator=gen, device="cuda"), {}, {}
+    out = K.kivi_packed_attend(q, fixed_order=True, num_splits=16, _plan_out=plan, **kw)
+    assert plan["path"] == path and plan["nparts"] > 8
+    at = slice(3, 5)
+    part = {name: t[at].contiguous() if isinstance(t, torch.Tensor) else t for name, t in kw.items()}
+    few = K.kivi_packed_attend(q[at], fixed_order=True, num_splits=16, _plan_out=one, **part)
+    assert one == plan
+    assert torch.equal(out[at], few)

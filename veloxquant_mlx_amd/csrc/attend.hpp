@@ -84,8 +84,9 @@ __device__ __forceinline__ float merge_partials(const float *p, int nparts, int6
     }
     return den > 0.f ? num / den : 0.f;
 }
-// the round size by the number of records: one round of loads when they fit (every caller goes
-// through here, so the in-kernel merge and the merge kernel add in the same order)
+// the round size by the number of records: one round of loads when they fit (the decode kernel's own merge and the launch
+// that does it otherwise both go through here, so they add in the same order; launch_merge_splits, of the vector kernels, has
+// an order of its own)
 template <bool DEVICE_SCOPE>
 __device__ __forceinline__ float merge_records(const float *p, int nparts, int64_t stride, int64_t d) {
     return nparts <= 8 ? merge_partials<DEVICE_SCOPE, 8>(p, nparts, stride, d)
@@ -116,8 +117,8 @@ int launch_attend_merge(const vq_attend_args &a, int nparts);
 void launch_sink_patch(const vq_attend_args &a, int nparts);
 // merges partials [rows][nparts][D + 2] of (max, sum, accumulator) into out [rows][D]
 void launch_merge_rows(const float *ws, int64_t rows, int nparts, int64_t D, void *out, int out_dtype, hipStream_t st);
-// the same with a block a row where rows are few and partials many (sums in another order: not for launches whose
-// other form merges inside the kernel)
+// the same with a block a row where partials are many (sums in another order: not for launches whose other form merges
+// inside the kernel)
 void launch_merge_splits(const float *ws, int64_t rows, int nparts, int64_t D, void *out, int out_dtype, hipStream_t st);
 
 // MFMA decode path (attend_mfma.hip)
