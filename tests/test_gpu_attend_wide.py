@@ -118,3 +118,19 @@ def test_a_batch_adds_in_the_order_of_its_parts(bits, group, Hq, Hkv, D, path):
     few = K.kivi_packed_attend(q[at], fixed_order=True, num_splits=16, _plan_out=one, **part)
     assert one == plan
     assert torch.equal(out[at], few)
+
+
+@pytest.mark.parametrize("bits,D", [(8, 64), (4, 32)])
+def test_an_infinite_value_of_a_run_that_weighs_nothing(bits, D):
+    """Sixteen runs, one of which scores so low that its weight underflows, with an infinite value in it: 0 * inf is not a
+    number, as in a softmax over all tokens in float32."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(bits)
+    kw = _byte_call(1, 1, D, 4096, gen, bits=bits)
+    q = torch.ones((1, 1, 1, D), device="cuda")
+    kw["k_zero"][:, :, 32:40] -= 300.0        # tokens 1024 .. 1279: a run of their own
+    kw["v_zero"][:, :, 1100, 0] = float("inf")
+    plan = {}
+    out = K.kivi_packed_attend(q, num_splits=16, _plan_out=plan, **kw)
+    assert plan["nparts"] == 16
+    assert out[..., :32].isnan().all() and out[..., 32:].isfinite().all()

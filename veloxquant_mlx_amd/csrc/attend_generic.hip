@@ -185,16 +185,18 @@ __global__ __launch_bounds__(MS_THREADS) void attend_merge_splits_kernel(const f
     const bool mine = tid < nsplit;
     const float m = mine ? rec[(int64_t)tid * (D + 2)] : -INFINITY, l = mine ? rec[(int64_t)tid * (D + 2) + 1] : 0.f;
     const float gm = block_reduce(m, true, s_red);
-    const float w = m == -INFINITY ? 0.f : __expf(m - gm);
+    // a record that saw no token is left out; one whose weight underflows is not: 0 times an infinity is not a number
+    const bool there = m != -INFINITY;
+    const float w = there ? __expf(m - gm) : -1.f;
     if (mine) s_w[tid] = w;
-    const float den = block_reduce(w == 0.f ? 0.f : l * w, false, s_red);   // (its barriers publish s_w)
+    const float den = block_reduce(there ? l * w : 0.f, false, s_red);   // (its barriers publish s_w)
     const int slices = MS_THREADS / D, c = tid % D, slice = tid / D;
     float num = 0.f;
     if (slice < slices) {
 #pragma unroll 8
         for (int s = slice; s < nsplit; s += slices) {
             const float ww = s_w[s], o = rec[(int64_t)s * (D + 2) + 2 + c];
-            if (ww != 0.f) num += o * ww;
+            if (ww >= 0.f) num += o * ww;
         }
     }
     s_o[tid] = num;
