@@ -42,6 +42,12 @@ def test_chunk_append_layouts(layout):
     _case(2, 4, 37, 128, 64, 20, torch.float16, layout)
 
 
+@pytest.mark.parametrize("B,H,S,D", [(576, 8, 1, 128), (4681, 7, 1, 256), (3, 5, 4370, 128), (1, 1, 1, 8)])
+def test_many_slabs_of_one_token_and_few_of_many(B, H, S, D):
+    """From a single vector to just past the 4096 blocks of a launch, where a thread takes a second vector."""
+    _case(B, H, S, D, S + 2, 1, torch.float16)
+
+
 def test_odd_head_dim_and_ends_of_the_buffer():
     _case(1, 3, 5, 72, 8, 3, torch.float16)     # last rows of the buffer; 144-byte rows
     _case(1, 3, 8, 72, 8, 0, torch.bfloat16)    # fills the buffer
