@@ -134,3 +134,17 @@ def test_an_infinite_value_of_a_run_that_weighs_nothing(bits, D):
     out = K.kivi_packed_attend(q, num_splits=16, _plan_out=plan, **kw)
     assert plan["nparts"] == 16
     assert out[..., :32].isnan().all() and out[..., 32:].isfinite().all()
+
+
+@pytest.mark.parametrize("n,asked", [(4096, 16), (4096, 32), (1000, 64), (65536, 512), (257, 2)])
+def test_a_given_cut_is_the_same_on_byte_codes(n, asked):
+    """``num_splits`` cuts the tokens alike whichever vector kernel takes them: runs of at least 256 tokens, whole 64s -- and so the
+    partials a caller has set memory aside for."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    kw, q = _byte_call(1, 1, 64, n, gen), torch.randn((1, 4, 1, 64), generator=gen, device="cuda")
+    wide, rows = {}, {}
+    K.kivi_packed_attend(q, num_splits=asked, _plan_out=wide, **kw)
+    half = {name: t.half() if name in ("k_scale", "k_zero", "v_scale", "v_zero") else t for name, t in kw.items()}
+    K.kivi_packed_attend(q, num_splits=asked, _plan_out=rows, **half)
+    assert wide["path"] == 4 and rows["path"] == 3 and wide["nparts"] == rows["nparts"]

@@ -369,15 +369,17 @@ __global__ __launch_bounds__(WD_THREADS) void attend_wide_kernel(WideArgs a, Row
     }
 }
 
-// splits: one block of eight waves a CU (the registers of four rows of sums leave room for one, the codebooks of the
-// defaults in LDS for two), of at least 128 tokens
+// Splits: one block of eight waves a CU (the registers of four rows of sums leave room for one, the codebooks of the
+// defaults in LDS for two), of at least 128 tokens.  A caller's own cut (`want`) is that of the vector kernel in attend_rows.hip, so
+// that it means the same, and takes the same room for partials, whichever of the two runs.
 void wide_splits(int64_t units, int64_t n, int want, int64_t &split_len, int &nsplit) {
+    const int64_t least = want > 0 ? 256 : 128, gran = want > 0 ? 64 : 32;
     int64_t ns = want > 0 ? want : 256 / (units > 0 ? units : 1);
-    const int64_t most = n > 128 ? n / 128 : 1;
+    const int64_t most = n > least ? n / least : 1;
     if (ns > most) ns = most;
     if (ns > 512) ns = 512;
     if (ns < 1) ns = 1;
-    split_len = cdiv(cdiv(n, ns), 32) * 32;
+    split_len = cdiv(cdiv(n, ns), gran) * gran;
     nsplit = (int)cdiv(n, split_len);
 }
 
