@@ -148,3 +148,15 @@ def test_a_given_cut_is_the_same_on_byte_codes(n, asked):
     half = {name: t.half() if name in ("k_scale", "k_zero", "v_scale", "v_zero") else t for name, t in kw.items()}
     K.kivi_packed_attend(q, num_splits=asked, _plan_out=rows, **half)
     assert wide["path"] == 4 and rows["path"] == 3 and wide["nparts"] == rows["nparts"]
+
+
+def test_byte_codes_of_any_batch_take_one_path():
+    """The kernel of a call does not change with the batch while its grid fits: 36 layers of 16 sequences of 8 heads."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    kw = _byte_call(36 * 16, 8, 64, 33, gen)
+    q, plan, one = torch.randn((36 * 16, 8, 1, 64), generator=gen, device="cuda"), {}, {}
+    out = K.kivi_packed_attend(q, fixed_order=True, num_splits=1, _plan_out=plan, **kw)
+    part = {name: t[:2].contiguous() if isinstance(t, torch.Tensor) else t for name, t in kw.items()}
+    few = K.kivi_packed_attend(q[:2], fixed_order=True, num_splits=1, _plan_out=one, **part)
+    assert plan["path"] == one["path"] == 4 and torch.equal(out[:2], few)
