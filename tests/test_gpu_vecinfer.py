@@ -512,3 +512,33 @@ def test_cache_under_inference_mode(modes, key_bits, key_sub):
     with torch.inference_mode():
         got = use()
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,S,n,sub,by_index", [
+    (1, 4, 1, 128, 1, 3000, 8, True), (48, 32, 8, 128, 1, 1537, 8, False), (32, 8, 8, 128, 1, 3072, 8, True), (32, 8, 8, 128, 1, 3073, 8, False),
+    (32, 8, 8, 64, 1, 4096, 8, True), (32, 8, 8, 64, 1, 4097, 8, False), (16, 16, 8, 128, 4, 3073, 8, False), (32, 8, 8, 128, 1, 3073, 4, True),
+    (64, 4, 4, 256, 1, 1537, 8, False), (64, 4, 4, 256, 1, 1536, 8, True), (1, 4, 1, 128, 9, 40, 8, False),
+])
+def test_few_rows_over_small_codebooks_take_the_kernel_of_their_depth(monkeypatch, B, Hq, Hkv, D, S, n, sub, by_index):
+    """Both sides of the rule between the index kernel and the table kernel, which agree."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    r = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    cfg = KVCacheConfig(method="vecinfer", head_dim=D, key_codebook_bits=8, key_sub_dim=sub, key_codebook=r(256, sub),
+                        value_codebook=r(256, 8), fused_sdpa=True, fused_sdpa_memory_bound=True)
+    c = KVCacheFactory.create(cfg)
+    idx = lambda s: torch.randint(0, 256, (B, Hkv, n, D // s), generator=gen, device="cuda", dtype=torch.uint8)
+    c.state, q = (idx(sub), idx(8)), r(B, Hq, S, D)
+    real, calls = K.vecinfer_attend_indices, []
+
+    def spy(*a, **k):
+        calls.append(real(*a, **k))
+        return calls[-1]
+    monkeypatch.setattr(K, "vecinfer_attend_indices", spy)
+    out = c.fused_sdpa(q, 0.1 / D ** 0.5)
+    assert (len(calls) == 1 and calls[0] is not None) == by_index
+    monkeypatch.setattr(K, "vecinfer_attend_indices", (lambda *a, **k: None) if by_index else real)
+    kw = dict(n_tokens=n, H_mat=c._H, causal=S > 1)
+    other = c.fused_sdpa(q, 0.1 / D ** 0.5) if by_index else real(q, *c.state[:1], c._key_codebook, c.state[1], c._value_codebook, 0.1 / D ** 0.5, **kw)
+    # both sum in float32 over at most 4097 tokens of unit variance; scores of a few units, D of them rounded
+    assert other is None or float((out - other).abs().max()) < 2e-4

@@ -366,11 +366,19 @@ class VecInferKVCache(FP16KVCache):
         table_kernel = (kcb.shape[0] == vcb.shape[0] <= 256 and max(n_sub_k, n_sub_v) <= 32
                         and (n_sub_k + n_sub_v) * kcb.shape[0] * 4 <= 65536
                         and (self._stored_k_indices.dtype != torch.uint8 or (n_sub_k % 4 == 0 and n_sub_v % 4 == 0)))
-        # Few query rows: straight from the indices, centroids gathered on chip.  Each four rows of a kv head read the indices
-        # again; a table kernel that takes the codebooks reads them less often, which shows from nine rows on (32 / 8 heads of 128
-        # channels, 4 x 16384 tokens, 8-bit codebooks: 47 / 60 us from the table with 4 rows, 83 / 82 with 8, 157 / 90 with 16).
+        # Few query rows: straight from the indices, centroids gathered on chip.  Each four rows of a kv head read the indices again,
+        # and a CU holds one block: what counts is how many tokens a CU walks (index_attend_depth).  A table kernel that takes the codebooks
+        # reads them less often and fills the chip with many short blocks, but builds its tables first; for key sub-vectors of
+        # eight it is the quicker one from nine rows on (32 / 8 heads of 128 channels, 4 x 16384 tokens, 8-bit codebooks:
+        # 47 / 60 us from the table with 4 rows, 83 / 82 with 8, 157 / 90 with 16) and from a depth on, indices / table:
+        # 128 channels 2048 tokens deep 49 / 60 and 34 / 36 us (GQA groups of 4 and 1), 3008 61 / 63 and 44 / 43, 3296 72 / 69 and
+        # 54 / 41, 8192 162 / 93; 64 channels 4096 49 / 62, 6000 69 / 61, 8192 93 / 72; 256 channels 1504 61 / 115, 1664 69 / 79 and
+        # 62 / 62, 2000 80 / 67, 6000 205 / 123.  (Key sub-vectors of four: 119 / 328 at the deepest measured.)
         H_kv = self._stored_k_indices.shape[1]
-        if q.shape[1] % H_kv == 0 and (q.shape[1] // H_kv) * q.shape[2] <= (8 if table_kernel else 255):
+        rows = (q.shape[1] // H_kv) * q.shape[2] if q.shape[1] % H_kv == 0 else 256
+        if rows <= (8 if table_kernel else 255) and not (
+                table_kernel and kcb.shape[1] == 8 and q.shape[2] > 0
+                and K.index_attend_depth(q.shape[0] * H_kv, rows // q.shape[2], q.shape[2], n) > min(4096, 3072 * 128 // self._head_dim)):
             out = K.vecinfer_attend_indices(q, self._stored_k_indices, kcb, self._stored_v_indices, vcb, float(scale), n_tokens=n,
                                             smooth=None if self._smooth is None else self._smooth.float(), H_mat=self._H,
                                             causal=bool(causal) and q.shape[2] > 1, sliding_window=int(sliding_window or 0))

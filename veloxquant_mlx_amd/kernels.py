@@ -1315,6 +1315,14 @@ __all__ = [
 # attention over VecInfer indices
 # ---------------------------------------------------------------------------
 
+def index_attend_depth(kv_heads: int, group: int, S_q: int, n_tokens: int) -> int:
+    """Tokens that a CU walks in :func:`vecinfer_attend_indices` over ``kv_heads`` kv heads of all sequences, ``group`` query heads
+    each: row tiles of four deal the rows, and a launch has one block of eight waves a CU, each over its run of the tokens."""
+    positions = 4 // group if S_q > 1 and group <= 4 and 4 % group == 0 else 1
+    units = kv_heads * -(-S_q // positions) * (-(-group // 4) if group > 4 else 1)
+    return -(-n_tokens // (256 // units)) if 0 < units <= 256 else -(-units // 256) * n_tokens
+
+
 def vecinfer_attend_indices(q: torch.Tensor, k_indices: torch.Tensor, k_codebook: torch.Tensor, v_indices: torch.Tensor,
                             v_codebook: torch.Tensor, scale: float, *, n_tokens: int, smooth: torch.Tensor | None = None,
                             H_mat: torch.Tensor | None = None, causal: bool = False, sliding_window: int = 0):
