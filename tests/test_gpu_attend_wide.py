@@ -160,3 +160,18 @@ def test_byte_codes_of_any_batch_take_one_path():
     part = {name: t[:2].contiguous() if isinstance(t, torch.Tensor) else t for name, t in kw.items()}
     few = K.kivi_packed_attend(q[:2], fixed_order=True, num_splits=1, _plan_out=one, **part)
     assert plan["path"] == one["path"] == 4 and torch.equal(out[:2], few)
+
+
+def test_indices_of_any_batch_take_one_path():
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(10)
+    B, Hkv, D, n = 40, 8, 128, 130
+    r = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    ki = torch.randint(0, 4096, (B, Hkv, n, 32), generator=gen, device="cuda", dtype=torch.int32)
+    vi = torch.randint(0, 256, (B, Hkv, n, 16), generator=gen, device="cuda", dtype=torch.uint8)
+    q, kcb, vcb = r(B, 2 * Hkv, 1, D), r(4096, 4), r(256, 8)
+    out = K.vecinfer_attend_indices(q, ki, kcb, vi, vcb, 0.02, n_tokens=n)
+    assert out is not None
+    few = K.vecinfer_attend_indices(q[7:9], ki[7:9].contiguous(), kcb, vi[7:9].contiguous(), vcb, 0.02, n_tokens=n)
+    # (the cut follows the batch: the sums' order differs, 130 tokens of unit variance)
+    assert float((out[7:9] - few).abs().max()) < 1e-5

@@ -484,8 +484,13 @@ int validate_index(const vq_index_attend_args *a, const char *fn) {
     VQ_REQUIRE(a->smooth == nullptr || a->smooth_rows == 1 || a->smooth_rows == a->Hkv, VQ_ERR_INVALID, "%s: smooth must have 1 or H_kv rows", fn);
     VQ_REQUIRE(wide_head(a->D) && (a->k_sub_dim == 4 || a->k_sub_dim == 8) && a->v_sub_dim == 8 && a->scale > 0.f &&
                    a->n_k_centroids <= 65536 && a->n_v_centroids <= 65536 && index_tables(*a) <= WD_MAX_LDS &&
-                   (a->Hq / a->Hkv) * a->Sq <= WD_MAX_INDEX_ROWS && a->B * a->Hkv * WD_MAX_INDEX_ROWS <= 65535,
+                   (a->Hq / a->Hkv) * a->Sq <= WD_MAX_INDEX_ROWS,
                VQ_ERR_UNSUPPORTED, "%s: shapes outside what the kernel covers", fn);
+    // the batch counts only where the grid ends (32 / 8 heads of 128 channels, one row, 4096 x 4 codebooks: 40 x 9001 tokens 331 us,
+    // 3426 through a copy of the context; 40 x 300 34 and 158)
+    int pq, tiles;
+    wide_tiling(a->Hq, a->Hkv, a->Sq, pq, tiles);
+    VQ_REQUIRE(a->B * a->Hkv * (int64_t)tiles <= 65535, VQ_ERR_UNSUPPORTED, "%s: too many (sequence, kv head, row tile) blocks", fn);
     return VQ_OK;
 }
 
