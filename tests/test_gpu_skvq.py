@@ -56,6 +56,8 @@ def _bits(a):
     (1, 2, 700, 128, 1, 64, False),
     (2, 2, 21, 80, 4, 32, True),     # ragged last group on the 16-byte path: the order's last channel fills it
     (1, 3, 50, 192, 2, 64, True),    # rows of a block in several heads, groups of 64
+    (2, 2, 21, 64, 4, 128, True),    # a group wider than the row
+    (1, 3, 33, 256, 4, 16, True),    # any group size on the 16-byte path
 ])
 def test_round_trip_kernel_matches_the_oracle_bit_for_bit(dtype, B, H, r, D, bits, g, with_perm):
     require_gpu()

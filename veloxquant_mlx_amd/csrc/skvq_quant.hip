@@ -207,9 +207,12 @@ void skvq_roundtrip_kernel(SkSides sides, double *__restrict__ err, int64_t n_bh
             if (iv && j == (int)D - 1 && Dp > (int)D) fill_k = k;   // the order's last channel also fills a ragged last group
         }
     };
-    // Rows of one piece a thread: SK_AHEAD of them are requested before the first is put in its place (8 x 8 heads of 4091
-    // rows, in place, five factors and orders: 80 us, 83 us with one request at a time; stored order 69 and 74 us).
-    const bool ahead = vec && one_piece && cq * 8 < (int)D;
+    // Rows of one piece a thread and whole groups of 32 or 64: SK_AHEAD of them are requested before the first is put in its
+    // place (8 x 8 heads of 4091 rows, in place, five factors and orders: 80 us, 83 us with one request at a time; stored order
+    // 69 and 74 us).  Elsewhere it costs: a ragged last group leaves its pad to threads that then wait for a second loop
+    // (80 channels, groups of 32, 1024 rows 13.7 -> 16.1 us), and the kernel for any group is no quicker for it (64 x 1024 rows
+    // of 256 channels, groups of 16 32.2 -> 35.5).
+    const bool ahead = GROUP > 0 && vec && one_piece && Dp == (int)D;
     if (ahead) {
         const int c0 = cq * 8;
         for (int lr0 = lr_base; lr0 < rows_pb && lr_base < rpp; lr0 += SK_AHEAD * rpp) {
@@ -240,7 +243,7 @@ void skvq_roundtrip_kernel(SkSides sides, double *__restrict__ err, int64_t n_bh
             }
         }
     }
-    for (int lr = lr_base; !(ahead || (scatter && one_piece)) && lr < rows_pb && lr_base < rpp; lr += rpp) {
+    for (int lr = lr_base; !ahead && lr < rows_pb && lr_base < rpp; lr += rpp) {
         if (row0 + lr >= n_rows) continue;
         const Where w = where(lr);
         const T *src = x + (int64_t)w.bh * x_stride_bh + (int64_t)w.t * D;
