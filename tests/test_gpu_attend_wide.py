@@ -136,6 +136,19 @@ def test_an_infinite_value_of_a_run_that_weighs_nothing(bits, D):
     assert out[..., :32].isnan().all() and out[..., 32:].isfinite().all()
 
 
+@pytest.mark.parametrize("B,D,n,asked,path", [(64, 128, 36, 0, 4), (65, 128, 36, 0, 3), (65, 128, 37, 0, 4), (65, 128, 36, 1, 4),
+                                              (385, 128, 64, 0, 3), (385, 128, 65, 0, 4), (384, 128, 64, 0, 4), (65, 64, 72, 0, 3), (65, 256, 18, 0, 3)])
+def test_many_tiles_over_few_tokens_take_the_smaller_blocks(B, D, n, asked, path):
+    """Both sides of the rule, against the one-wave-a-row kernel."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(B + n)
+    kw, q, plan = _byte_call(B, 4, D, n, gen), torch.randn((B, 8, 1, D), generator=gen, device="cuda"), {}
+    out = K.kivi_packed_attend(q, num_splits=asked, _plan_out=plan, **kw)
+    ref = K.kivi_packed_attend(q, num_splits=-1, **kw)
+    assert plan["path"] == path
+    assert float((out - ref).abs().max()) < 5e-5   # (the order of float32 sums over the same rebuilt rows)
+
+
 @pytest.mark.parametrize("n,asked", [(4096, 16), (4096, 32), (1000, 64), (65536, 512), (257, 2)])
 def test_a_given_cut_is_the_same_on_byte_codes(n, asked):
     """``num_splits`` cuts the tokens alike whichever vector kernel takes them: runs of at least 256 tokens, whole 64s -- and so the

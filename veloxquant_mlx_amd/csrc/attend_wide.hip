@@ -439,9 +439,17 @@ bool wide_kernel_supported(const vq_attend_args &a) {
     if (a.Hkv < 1 || a.Hq % a.Hkv != 0 || (a.Hq / a.Hkv) * a.Sq > WD_MAX_ROWS) return false;
     int pq, tiles;
     rows_tiling(a, pq, tiles);
+    // Many tiles over a few tokens each: a block of eight waves has work for one or two of them, and the four-wave blocks of
+    // attend_rows.hip are done sooner.  us there / here, 128 channels, 1024 tiles: 16 tokens 33 / 41, 33 38 / 41, 48 45 / 42;
+    // 3200: 33 tokens 93 / 126, 64 115 / 122, 80 143 / 130; 512: 16 tokens 21 / 23, 33 23 / 23; 256: 16 tokens 18 / 14.  64 channels
+    // reach it at twice the tokens (1024 tiles: 64 tokens 33 / 34, 80 41 / 35; 3200: 64 tokens 77 / 100, 160 130 / 120), 256 at half
+    // (1600: 16 tokens 45 / 60, 33 67 / 67).
+    // A caller's own cut keeps its kernel whatever the batch.
+    const int64_t blocks = a.B * a.Hkv * (int64_t)tiles;
+    if (a.num_splits == 0 && blocks > 256 && a.n_packed * a.D <= (blocks > 1536 ? 8192 : 4608)) return false;
     return a.num_splits >= 0 && a.n_packed > 0 && a.n_tail == 0 && a.pack_bits == 8 && a.v_layout == VQ_V_CHANNEL_PACKED &&
            a.meta_dtype == VQ_F32 && wide_head(a.D) && a.group % 32 == 0 && a.packed_lens == nullptr && a.k_new == nullptr &&
-           a.sink_k == nullptr && a.scale > 0.f && a.B * a.Hkv * (int64_t)tiles <= 65535 &&
+           a.sink_k == nullptr && a.scale > 0.f && blocks <= 65535 &&
            (((uintptr_t)a.k_packed | (uintptr_t)a.v_packed | (uintptr_t)a.k_scale | (uintptr_t)a.k_zero) & 15u) == 0;
 }
 
