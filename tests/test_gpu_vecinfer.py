@@ -160,6 +160,20 @@ def test_large_codebooks_split_and_image_forms(sub, nc, n):
     assert host(K.vecinfer_quantize_metal(to_dev(x[:2]), to_dev(cb), sub)).reshape(-1)[0] == 0
 
 
+@pytest.mark.parametrize("nc", [1, 2, 16, 31, 33, 63, 65, 97, 500, 513, 577, 1025])
+@pytest.mark.parametrize("sub", [4, 8])
+def test_rows_past_the_end_of_a_codebook_never_count(sub, nc):
+    """Codebooks that end inside a tile, or leave the second tile of a pair empty: sub-vectors at the last centroid, at the origin
+    with the codebook far from it, and out to the end of the filter's range (256 times the largest centroid) and past it."""
+    require_gpu()
+    rng = np.random.default_rng(nc * 10 + sub)
+    cb = (rng.standard_normal((nc, sub)) + (6 if nc % 2 else 0)).astype(np.float32)
+    x = np.concatenate([cb[-1] + rng.standard_normal((300, sub)) * 0.1, np.tile(cb[-1], (5, 1)), np.zeros((5, sub)),
+                        rng.standard_normal((300, sub)) * np.abs(cb).max() * np.exp(rng.uniform(0, 7, (300, 1)))]).astype(np.float32)
+    got = host(K.vecinfer_quantize_metal(to_dev(x), to_dev(cb), sub)).reshape(-1)
+    np.testing.assert_array_equal(got, cref.vq_assign(x, cb, sub).reshape(-1))
+
+
 @pytest.mark.parametrize("far_out", [1e16, 3e19, float("inf")])
 @pytest.mark.parametrize("sub,nc,n", [(4, 256, 200), (8, 300, 200), (4, 1000, 200), (4, 4096, 200), (8, 2048, 200), (4, 4096, 33000)])
 def test_a_diverged_centroid_leaves_the_exact_rule_to_the_others(sub, nc, n, far_out):

@@ -271,6 +271,17 @@ template <int SUB> __device__ __forceinline__ void centroid_image(const float *r
     }
 }
 
+// A row past the end of the codebook: zeros for c, twice 65504 for |c|^2 and 65504 for the factors of |v|^2's parts, so its score
+// 131008 + 2 |v|^2 lies above (32 + |v|)^2, the largest a centroid can have, by more than the margin for every |v| in
+// the filter's range.  It never leads a cell that holds a centroid and never counts as near (the last centroid in its place, again and
+// again, was as near as itself wherever it won, and sent one sub-vector in nc through the whole codebook: 16 centroids of four
+// over 1048576 76 us, 14 since).
+template <int SUB> __device__ __forceinline__ void pad_image(u32 *img) {
+#pragma unroll
+    for (int e = 0; e < image_words<SUB>(); ++e) img[e] = 0;
+    img[SUB == 4 ? 4 : 8] = img[SUB == 4 ? 5 : 9] = 0x7bff7bffu;
+}
+
 // ---- sub-vectors -----------------------------------------------------------------------------
 
 // where the index of sub-vector sv goes: `rows_out` rows of a (sequence, head) in the output for the S of the input
@@ -490,7 +501,7 @@ void vq_assign_image_kernel(AssignJob j) {
     constexpr int IW = image_words<SUB>();
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int ntiles = (j.nc + 63) / 64 * 2;   // an even number; past the end: the last centroid again
+    const int ntiles = (j.nc + 63) / 64 * 2;   // an even number
     const bool aligned = (reinterpret_cast<uintptr_t>(j.cb) & 15u) == 0;
 
     float cmax2 = 0.f;
@@ -507,10 +518,14 @@ void vq_assign_image_kernel(AssignJob j) {
     for (int w = 0; w < WAVES; ++w) cmax2 = fmaxf(cmax2, s_red[w]);
     const float cs = codebook_scale(cmax2);
     for (int c = tid; c < ntiles * 32; c += 64 * WAVES) {
-        float row[SUB];
-        load_centroid<SUB>(j.cb, j.ct, aligned, min(c, j.nc - 1), row);
         u32 img[IW];
-        centroid_image<SUB>(row, cs, img);
+        if (c < j.nc) {
+            float row[SUB];
+            load_centroid<SUB>(j.cb, j.ct, aligned, c, row);
+            centroid_image<SUB>(row, cs, img);
+        } else {
+            pad_image<SUB>(img);
+        }
 #pragma unroll
         for (int e = 0; e < IW; e += 2) *reinterpret_cast<uint2 *>(&s_img[c * IW + e]) = make_uint2(img[e], img[e + 1]);
     }
@@ -642,7 +657,7 @@ __device__ __forceinline__ void assign_split(const AssignJob &j, int64_t block, 
     float row[TW][SUB];
     float cmax2 = 0.f;
 #pragma unroll
-    for (int i = 0; i < TW; ++i) rc[i] = min((wave + i * WAVES) * 32 + (lane & 31), j.nc - 1);   // tiles wave, wave + WAVES, ..; past the end: the last centroid again
+    for (int i = 0; i < TW; ++i) rc[i] = min((wave + i * WAVES) * 32 + (lane & 31), j.nc - 1);   // tiles wave, wave + WAVES, ..; past the end: the last centroid again (in its own tile, whose two cells are both looked at)
     load_centroids<SUB, TW>(j.cb, j.ct, aligned, rc, row);
 #pragma unroll
     for (int i = 0; i < TW; ++i) cmax2 = fmaxf(cmax2, norm2<SUB>(row[i]));
