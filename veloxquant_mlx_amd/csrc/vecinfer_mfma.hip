@@ -504,11 +504,18 @@ void vq_assign_image_kernel(AssignJob j) {
     const int ntiles = (j.nc + 63) / 64 * 2;   // an even number
     const bool aligned = (reinterpret_cast<uintptr_t>(j.cb) & 15u) == 0;
 
-    float cmax2 = 0.f;
-    for (int c = tid; c < j.nc; c += 64 * WAVES) {
-        float row[SUB];
-        load_centroid<SUB>(j.cb, j.ct, aligned, c, row);
-        cmax2 = fmaxf(cmax2, norm2<SUB>(row));
+    float cmax2 = 0.f, kept[FINE ? SUB : 1];
+    static_assert(!FINE || kFineC <= 64 * WAVES, "a thread reads one row");
+    if constexpr (FINE) {   // one row a thread, read once: of a small call the second read's wait shows
+        load_centroid<SUB>(j.cb, j.ct, aligned, min(tid, j.nc - 1), kept);
+        cmax2 = norm2<SUB>(kept);
+        cmax2 = cmax2 == cmax2 ? cmax2 : 0.f;
+    } else {
+        for (int c = tid; c < j.nc; c += 64 * WAVES) {
+            float row[SUB];
+            load_centroid<SUB>(j.cb, j.ct, aligned, c, row);
+            cmax2 = fmaxf(cmax2, norm2<SUB>(row));
+        }
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) cmax2 = fmaxf(cmax2, __shfl_xor(cmax2, o));
@@ -521,7 +528,12 @@ void vq_assign_image_kernel(AssignJob j) {
         u32 img[IW];
         if (c < j.nc) {
             float row[SUB];
-            load_centroid<SUB>(j.cb, j.ct, aligned, c, row);
+            if constexpr (FINE) {
+#pragma unroll
+                for (int e = 0; e < SUB; ++e) row[e] = kept[e];
+            } else {
+                load_centroid<SUB>(j.cb, j.ct, aligned, c, row);
+            }
             centroid_image<SUB>(row, cs, img);
         } else {
             pad_image<SUB>(img);
