@@ -318,6 +318,7 @@ def test_keys_and_values_in_one_call_equal_the_single_calls(dtype, b, g, D, S, v
 @pytest.mark.parametrize("B,H,lo,n,cap,D,g", [
     (1, 1, 0, 32, 64, 128, 32), (2, 3, 64, 1920, 2048, 128, 32), (1, 2, 64, 320, 512, 128, 64), (1, 2, 0, 100, 256, 128, 32),
     (2, 2, 16, 48, 256, 128, 16), (1, 3, 32, 96, 256, 64, 32), (1, 2, 128, 256, 512, 256, 64), (1, 1, 0, 8, 256, 64, 8),
+    (1, 2, 128, 200, 512, 128, 128), (1, 1, 8, 88, 128, 256, 8),
 ])
 def test_round_trip_in_place_equals_the_two_round_trips(dtype, B, H, lo, n, cap, D, g):
     """Keys and values of a slice of two buffers in place: the bits of the two separate round trips, and no other row changes."""
