@@ -284,18 +284,6 @@ template <int SUB> __device__ __forceinline__ void pad_image(u32 *img) {
 
 // ---- sub-vectors -----------------------------------------------------------------------------
 
-// where the index of sub-vector sv goes: `rows_out` rows of a (sequence, head) in the output for the S of the input
-struct IndexDst {
-    int shift;          // log2(sub-vectors a token), or -1: densely, in order
-    u32 S;
-    int64_t rows_out;
-    __device__ __forceinline__ int64_t at(int64_t sv) const {
-        if (shift < 0) return sv;
-        const u32 token = (u32)(sv >> shift), bh = token / S;   // (dense otherwise: fewer than 2^32 tokens)
-        return (((int64_t)bh * rows_out + (token - bh * S)) << shift) + (sv & ((1 << shift) - 1));
-    }
-};
-
 // One lane's sub-vector and the operands of the wave's 64: column block b holds sub-vectors 32 b + (lane & 31).
 template <int SUB> struct SubVec {
     float xf[SUB];
@@ -442,8 +430,8 @@ __device__ __forceinline__ void scan_all(unsigned long long m, const float (&x)[
 
 template <int SUB, int LT>
 __device__ __forceinline__ void store_result(int64_t sv, int my_idx, const SubVec<SUB> &s, const void *cb, int ct, bool aligned, void *idx,
-                                             int it, const IndexDst &dst, const KeyXform &kx, int lane, bool live) {
-    if (live) st_idx(idx, it, dst.at(sv), my_idx);
+                                             int it, const KeyXform &kx, int lane, bool live) {
+    if (live) st_idx(idx, it, sv, my_idx);
     if constexpr (LT > 0) {
         if (kx.k_tilde != nullptr && live) {
 #pragma unroll
@@ -487,7 +475,6 @@ struct AssignJob {
     int ct, nc;
     void *idx;
     int it;
-    IndexDst dst;
     KeyXform kx;
 };
 
@@ -640,7 +627,7 @@ void vq_assign_image_kernel(AssignJob j) {
         if (__any(second)) { if (second) eval_cell(o1, 1 - h1); }
         const unsigned long long m = __ballot(all);
         if (m != 0) scan_all<SUB>(m, s.xf, j.cb, j.ct, aligned, j.nc, lane, my_idx);
-        store_result<SUB, LT>(sv, my_idx, s, j.cb, j.ct, aligned, j.idx, j.it, j.dst, j.kx, lane, live);
+        store_result<SUB, LT>(sv, my_idx, s, j.cb, j.ct, aligned, j.idx, j.it, j.kx, lane, live);
     }
 }
 
@@ -782,7 +769,7 @@ __device__ __forceinline__ void assign_split(const AssignJob &j, int64_t block, 
         if (l == 0) lds.idx[g] = i;
     }
     __syncthreads();
-    if (wave == 0) store_result<SUB, LT>(sv, lds.idx[lane], s, j.cb, j.ct, aligned, j.idx, j.it, j.dst, j.kx, lane, live);
+    if (wave == 0) store_result<SUB, LT>(sv, lds.idx[lane], s, j.cb, j.ct, aligned, j.idx, j.it, j.kx, lane, live);
 }
 
 template <int SUB, int LT, int WAVES, int TW>
@@ -825,7 +812,7 @@ bool launch_assign_mfma(const void *x, int xt, int64_t N, const void *cb, int ct
                         hipStream_t st) {
     if (!(sub == 4 || sub == 8)) return false;
     if (xt != VQ_F32 && ((uintptr_t)x & (sub == 8 ? 15u : 7u))) return false;
-    const AssignJob j = {x, xt, N, cb, ct, nc, idx, it, {-1, 1, 0}, {}};
+    const AssignJob j = {x, xt, N, cb, ct, nc, idx, it, {}};
     return sub == 8 ? launch_job<8, 0>(j, st) : launch_job<4, 0>(j, st);
 }
 
@@ -836,7 +823,7 @@ bool launch_encode_keys_mfma(const void *keys, int kt, int64_t B, int64_t heads,
     const int64_t lt = D / sub;
     if (!(lt == 8 || lt == 16 || lt == 32 || lt == 64)) return false;
     if (((uintptr_t)keys | (uintptr_t)k_hat | (uintptr_t)k_tilde | (uintptr_t)smooth) & 15u) return false;
-    const AssignJob j = {keys, kt, B * heads * S * lt, cb, ct, nc, idx, it, {-1, 1, 0}, {smooth, smooth_rows, heads, S, h, k_hat, kt, k_tilde}};
+    const AssignJob j = {keys, kt, B * heads * S * lt, cb, ct, nc, idx, it, {smooth, smooth_rows, heads, S, h, k_hat, kt, k_tilde}};
 #define VQ_ENC(SUB, LT) return launch_job<SUB, LT>(j, st)
     if (sub == 8) { if (lt == 8) VQ_ENC(8, 8); else if (lt == 16) VQ_ENC(8, 16); else if (lt == 32) VQ_ENC(8, 32); else VQ_ENC(8, 64); }
     else { if (lt == 8) VQ_ENC(4, 8); else if (lt == 16) VQ_ENC(4, 16); else if (lt == 32) VQ_ENC(4, 32); else VQ_ENC(4, 64); }
