@@ -556,3 +556,24 @@ def test_few_rows_over_small_codebooks_take_the_kernel_of_their_depth(monkeypatc
     other = c.fused_sdpa(q, 0.1 / D ** 0.5) if by_index else real(q, *c.state[:1], c._key_codebook, c.state[1], c._value_codebook, 0.1 / D ** 0.5, **kw)
     # both sum in float32 over at most 4097 tokens of unit variance; scores of a few units, D of them rounded
     assert other is None or float((out - other).abs().max()) < 2e-4
+
+
+def test_matrix_made_inside_a_graph_is_not_kept_for_eager_calls():
+    """A restored cache whose first call is captured: the matrix of that capture holds nothing until a replay, so a call outside
+    makes its own, and the graph replays to the same values."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    r = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    cfg = KVCacheConfig(method="vecinfer", head_dim=64, key_codebook_bits=4, key_sub_dim=16, key_codebook=r(16, 16), value_codebook=r(256, 8),
+                        smooth_factors=r(2, 64).exp(), fused_sdpa=True, fused_sdpa_memory_bound=True)
+    a, b, q = KVCacheFactory.create(cfg), KVCacheFactory.create(cfg), r(1, 4, 1, 64)
+    a.update_and_fetch(r(1, 2, 90, 64), r(1, 2, 90, 64))
+    want = a.fused_sdpa(q, 0.1)
+    b.state = a.state
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = b.fused_sdpa(q, 0.1)
+    assert torch.equal(b.fused_sdpa(q, 0.1), want)
+    for _ in range(3):
+        graph.replay()
+        assert torch.equal(out, want) and torch.equal(b.fused_sdpa(q, 0.1), want)

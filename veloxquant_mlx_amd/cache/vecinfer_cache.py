@@ -82,6 +82,7 @@ class VecInferKVCache(FP16KVCache):
         self._smooth = None if sm is None else torch.as_tensor(sm)
         self._validate_smooth()
         self._H: torch.Tensor | None = None   # made on the device of the first keys
+        self._H_in_graph = False
 
         n_kc, n_vc = 2 ** self._key_bits, 2 ** self._value_bits
         seed = opt["seed"]
@@ -163,7 +164,9 @@ class VecInferKVCache(FP16KVCache):
 
     def _to_device(self, ref: torch.Tensor) -> None:
         dev = ref.device
-        if self._H is None or self._H.device != dev:
+        if self._H is None or self._H.device != dev or self._H_in_graph:
+            # (one made while a graph is captured holds nothing until that graph is replayed: the next call makes its own)
+            self._H_in_graph = dev.type == "cuda" and torch.cuda.is_current_stream_capturing()
             self._H = walsh_hadamard_matrix(self._head_dim, device=dev)
             self._key_codebook = self._key_codebook.to(dev)
             self._value_codebook = self._value_codebook.to(dev)
