@@ -272,15 +272,27 @@ def test_channel_orders_match_the_stated_rule(dtype, B, H, r, D, bits, g):
         assert np.array_equal(host(inv[h])[got], np.arange(D))
 
 
-def test_channel_orders_put_ranges_that_are_not_numbers_last():
+def test_channel_orders_with_an_error_that_is_not_a_number():
+    """A head whose errors are not numbers keeps the stored order; another head of the same chunk, and the other tensor of the
+    same launches, take the order by range where that has the lower error."""
     require_gpu()
-    x = torch.randn((1, 2, 16, 64), device="cuda:0") * torch.linspace(3.0, 0.1, 64, device="cuda:0")
-    x[0, 0, 4, 10] = float("nan")
-    x[0, 0, 4, 20] = float("inf")
-    perm, inv = K.skvq_channel_orders(x, 4, 64, (1.0,))      # the error of that head is not a number: the stored order stays
-    assert np.array_equal(host(perm[0]), np.arange(64)) and np.array_equal(host(inv[0]), np.arange(64))
+    scales = _het_scales(64, seed=3).astype(np.float32)
+    x = np.random.default_rng(4).standard_normal((2, 3, 40, 64)).astype(np.float32) * scales
+    y = x[:, :, ::-1].copy()
+    x[0, 0, 4, 10], x[1, 0, 4, 20] = np.nan, np.inf
+    (perm, perm2), (inv, inv2) = K.skvq_channel_orders(to_dev(x), 2, 16, (1.0,), to_dev(y), 2)
+    for t, p, i, bad in ((x, host(perm), host(inv), 0), (y, host(perm2), host(inv2), None)):
+        for h in range(3):
+            xh = t[:, h:h + 1]
+            cand = np.argsort(xh.max(axis=(0, 1, 2)) - xh.min(axis=(0, 1, 2)), kind="stable").astype(np.int32)[None]
+            if h != bad:
+                err = [np.square((o.round_trip(xh, q, None if q is None else np.argsort(q, axis=-1).astype(np.int32), 2, 16, (1.0,)) - xh)
+                                 .astype(np.float64)).mean() for q in (None, cand)]
+                assert err[1] < 0.9 * err[0]        # the order by range wins by far
+            want = np.arange(64) if h == bad else cand[0]
+            assert np.array_equal(p[h], want) and np.array_equal(i[h][p[h]], np.arange(64))
     with pytest.raises(ValueError, match="non-empty"):
-        K.skvq_channel_orders(x[:, :, :0], 4, 64, (1.0,))
+        K.skvq_channel_orders(to_dev(x)[:, :, :0], 4, 64, (1.0,))
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])

@@ -408,6 +408,42 @@ def test_encode_keys_on_integer_keys_is_exact(D, sub):
     np.testing.assert_array_equal(host(idx8), idx_ref.astype(np.uint8))
 
 
+# the forms for more than 512 centroids: SPLIT up to 32768 sub-vectors against more than 1024 centroids (three heads: on both sides
+# of that), the image of the whole codebook otherwise; one lane group of a token each way
+@pytest.mark.parametrize("D,sub,nc,S", [
+    (128, 4, 4096, 1), (128, 4, 4096, 341), (128, 4, 4096, 342), (64, 4, 4096, 682), (64, 4, 4096, 683), (256, 4, 4096, 170), (256, 4, 4096, 171),
+    (128, 8, 2048, 682), (128, 8, 2048, 683), (512, 8, 2048, 20), (64, 8, 1500, 3), (32, 4, 1100, 77), (128, 4, 1000, 50), (256, 8, 600, 33),
+])
+@pytest.mark.parametrize("smooth_rows", [None, "vector", "heads"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, "integers"])
+def test_encode_keys_with_large_codebooks(dtype, smooth_rows, D, sub, nc, S):
+    """Indices exact on the kernel's own transformed keys; those exact on integer keys, and elsewhere no further from float64
+    than the float32 product that they replace; the way back from the kernel's own indices."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(D + nc + S)
+    r = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    whole = dtype == "integers"
+    keys = torch.randint(-8, 9, (1, 3, S, D), generator=gen, device="cuda").half() if whole else (r(1, 3, S, D) * r(D).exp()).to(dtype)
+    shape = {None: None, "vector": (D,), "heads": (3, D)}[smooth_rows]
+    smooth = None if shape is None else torch.exp2(torch.randint(-2, 3, shape, generator=gen, device="cuda").float()) if whole else r(*shape).exp()
+    Hm, cb = to_dev(ov.walsh_hadamard_matrix(D)), r(nc, sub) * D ** 0.25
+    k_hat, idx, k_tilde = K.vecinfer_encode_decode_metal(keys, cb, sub, Hm, smooth, want_k_tilde=True)
+    wide = lambda t: 1.0 if t is None else t[:, None, :] if t.ndim == 2 else t
+    exact = (keys.double() / wide(None if smooth is None else smooth.double())) @ Hm.double()
+    product = (keys.float() / wide(smooth)) @ Hm
+    err = lambda t: float((t.double() - exact).norm() / exact.norm())
+    if whole:   # every partial sum is a whole number of quarters below 2^24: only the last step, times the matrix' magnitude, rounds
+        h = float(Hm[0, 0])
+        assert torch.equal(k_tilde, ((keys.double() / wide(None if smooth is None else smooth.double())) @ (Hm.double() / h)).float() * h)
+    assert err(k_tilde) <= 1.05 * max(err(product), 2.0 ** -25)
+    np.testing.assert_array_equal(host(idx).reshape(-1), cref.vq_assign(host(k_tilde).reshape(-1, sub), host(cb), sub).reshape(-1))
+    back = (cb.double()[idx.long()].reshape(exact.shape) @ Hm.double()) * wide(None if smooth is None else smooth.double())
+    # log2(D) + 2 roundings of 2^-24 of the row's own size, and the output type's
+    tol = 2.0 ** -11 if keys.dtype == torch.float16 else 0.0
+    row = back.norm(dim=-1, keepdim=True) * (1 if smooth is None else float(smooth.max() / smooth.min()))
+    assert ((k_hat.double() - back).abs() <= back.abs() * tol + row * 2.0 ** -24 * (D.bit_length() + 2) + 6e-8).all()
+
+
 def test_encode_keys_at_any_storage_offset():
     """Keys and smoothing factors that are contiguous but start between 16-byte boundaries, at codebooks on both sides of 256
     centroids: the same values as from aligned memory."""
@@ -479,13 +515,13 @@ def test_encode_keys_random_keys(dtype, smooth_rows):
 
 
 def test_encode_keys_other_shapes_take_the_composition():
-    """sub_dim 16, a non-Hadamard matrix, more than 256 centroids: same contract through the
+    """sub_dim 16, a non-Hadamard matrix, a codebook past what a block holds: same contract through the
     matrix product and the assignment / gather kernels."""
     require_gpu()
     rng = np.random.default_rng(2)
     keys = rng.standard_normal((1, 2, 40, 64)).astype(np.float16)
     Hm = ov.walsh_hadamard_matrix(64)
-    for sub, C, Hmat in ((16, 64, Hm), (8, 300, Hm), (8, 64, np.linalg.qr(rng.standard_normal((64, 64)))[0].astype(np.float32))):
+    for sub, C, Hmat in ((16, 64, Hm), (8, 2100, Hm), (8, 64, np.linalg.qr(rng.standard_normal((64, 64)))[0].astype(np.float32))):
         cb = rng.standard_normal((C, sub)).astype(np.float32)
         k_hat, idx, k_tilde = K.vecinfer_encode_decode_metal(to_dev(keys), to_dev(cb), sub, to_dev(Hmat), want_k_tilde=True)
         np.testing.assert_array_equal(host(idx), ov.quantize_vq(host(k_tilde), cb, sub))
