@@ -378,13 +378,14 @@ class VecInferKVCache(FP16KVCache):
         # 54 / 41, 8192 162 / 93; 64 channels 4096 49 / 62, 6000 69 / 61, 8192 93 / 72; 256 channels 1504 61 / 115, 1664 69 / 79 and
         # 62 / 62, 2000 80 / 67, 6000 205 / 123.  (Key sub-vectors of four: 119 / 328 at the deepest measured.)
         H_kv = self._stored_k_indices.shape[1]
-        rows = (q.shape[1] // H_kv) * q.shape[2] if q.shape[1] % H_kv == 0 else 256
+        B, H_q, S_q = q.shape[:3]
+        rows = (H_q // H_kv) * S_q if H_q % H_kv == 0 else 256
         if rows <= (8 if table_kernel else 255) and not (
-                table_kernel and kcb.shape[1] == 8 and q.shape[2] > 0
-                and K.index_attend_depth(q.shape[0] * H_kv, rows // q.shape[2], q.shape[2], n) > min(4096, 3072 * 128 // self._head_dim)):
+                table_kernel and kcb.shape[1] == 8 and S_q > 0
+                and K.index_attend_depth(B * H_kv, H_q // H_kv, S_q, n) > min(4096, 3072 * 128 // self._head_dim)):
             out = K.vecinfer_attend_indices(q, self._stored_k_indices, kcb, self._stored_v_indices, vcb, float(scale), n_tokens=n,
                                             smooth=None if self._smooth is None else self._smooth.float(), H_mat=self._H,
-                                            causal=bool(causal) and q.shape[2] > 1, sliding_window=int(sliding_window or 0))
+                                            causal=bool(causal) and S_q > 1, sliding_window=int(sliding_window or 0))
             if out is not None:
                 return out
         smooth = self._smooth.float() if self._smooth is not None else torch.ones(

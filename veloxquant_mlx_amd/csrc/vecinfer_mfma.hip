@@ -8,9 +8,12 @@
 //   d2[c, v] = |c|^2 - 2 c.v + |v|^2   v_mfma_f32_32x32x16_f16, 32 centroids x 32 sub-vectors a product.  c and v
 //       travel as fp16 high part + fp16 remainder, |c|^2 and |v|^2 as two fp16 parts in k-slots of their own, so the
 //       accumulator input is the constant zero.  Codebook and sub-vectors are first multiplied by one power of two that
-//       puts max|c|^2 in [256, 1024) (remainders stay out of the subnormals); d2 is then good to 2^-19 (|c|^2 + |v|^2):
-//       3 2^-22 from the parts of c and v and the product of remainders that is left out, 2^-22 from those of |c|^2, 2^-21
-//       from the accumulation (16 terms: 5e-7 of the largest measured).
+//       puts max|c|^2 in [256, 1024) (remainders stay out of the subnormals); d2 is then good to 2^-19 (|c|^2 + |v|^2), apart from
+//       an error of |v|^2 that all scores of a sub-vector share: 3 2^-22 from the parts of c and v and the product of remainders
+//       that is left out, 2^-22 from those of |c|^2, 2^-21 from the accumulation, whose rounding the unit does not
+//       document.  That last part is measured: over 5 x 10^5 scores each of normal, equal, near, very long, all-mantissa-bits, fp16
+//       half-way, wide-exponent and one-large-channel vectors the accumulation is off by 2^-21.5 at most (beyond the constant
+//       margin's reach), and twice the largest error of a score is 13 % of the margin below without its tag bits.
 //   A *cell* is the 16 scores one lane holds of a product: 16 centroids, one sub-vector.  |v|^2 carries a small surplus
 //       that keeps every score positive, so float bits order as integers: the smallest of a cell costs eight min3, the
 //       tile number goes into its seven low bits (one and-or), and the two smallest cells of the lane are kept in two
@@ -511,22 +514,26 @@ void vq_assign_image_kernel(AssignJob j) {
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) cmax2 = fmaxf(cmax2, s_red[w]);
     const float cs = codebook_scale(cmax2);
-    for (int c = tid; c < ntiles * 32; c += 64 * WAVES) {
-        u32 img[IW];
-        if (c < j.nc) {
-            float row[SUB];
-            if constexpr (FINE) {
-#pragma unroll
-                for (int e = 0; e < SUB; ++e) row[e] = kept[e];
-            } else {
-                load_centroid<SUB>(j.cb, j.ct, aligned, c, row);
-            }
-            centroid_image<SUB>(row, cs, img);
-        } else {
-            pad_image<SUB>(img);
-        }
+    auto put = [&](int c, const u32 *img) {
 #pragma unroll
         for (int e = 0; e < IW; e += 2) *reinterpret_cast<uint2 *>(&s_img[c * IW + e]) = make_uint2(img[e], img[e + 1]);
+    };
+    u32 img[IW];
+    if constexpr (FINE) {
+        if (tid < ntiles * 32) {
+            if (tid < j.nc) centroid_image<SUB>(kept, cs, img);
+            else pad_image<SUB>(img);
+            put(tid, img);
+        }
+    } else {
+        for (int c = tid; c < j.nc; c += 64 * WAVES) {
+            float row[SUB];
+            load_centroid<SUB>(j.cb, j.ct, aligned, c, row);
+            centroid_image<SUB>(row, cs, img);
+            put(c, img);
+        }
+        pad_image<SUB>(img);
+        for (int c = j.nc + tid; c < ntiles * 32; c += 64 * WAVES) put(c, img);
     }
     __syncthreads();
 

@@ -13,6 +13,7 @@ import ctypes as C
 import math
 
 import torch
+from torch.autograd import forward_ad as _forward_ad
 
 from . import _lib
 from ._lib import (VQ_AXIS_CHANNEL, VQ_AXIS_TOKEN, VQ_BF16, VQ_F16, VQ_F32, VQ_I32, VQ_U8,
@@ -530,7 +531,7 @@ def _plain_eager() -> bool:
     """Outside tracing, function transforms, forward-mode levels and dispatch modes: a call that hands raw pointers
     to a kernel sees what the torch operation in its place would."""
     return not (torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None
-                or torch._C._len_torch_dispatch_stack() > 0 or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._len_torch_dispatch_stack() > 0 or _forward_ad._current_level >= 0
                 or torch.compiler.is_compiling())
 
 
@@ -796,9 +797,9 @@ def _sylvester_scale(H_mat: torch.Tensor) -> float:
     (every entry ``(-1)^popcount(a & b)`` times one magnitude), else 0.  Checked once per tensor
     object and version (the verdict rides on the tensor itself), on every call where there is no version (a tensor made
     under ``torch.inference_mode``)."""
-    version = None if H_mat.is_inference() else H_mat._version
-    memo = getattr(H_mat, "_vq_sylvester", None)
-    if memo is None or version is None or memo[0] != version:
+    memo = getattr(H_mat, "_vq_sylvester", None)   # (never on a tensor without a version)
+    if memo is None or memo[0] != H_mat._version:
+        version = None if H_mat.is_inference() else H_mat._version
         D = H_mat.shape[0]
         ok = H_mat.ndim == 2 and H_mat.shape[1] == D and D >= 1 and (D & (D - 1)) == 0
         h = 0.0
@@ -856,10 +857,13 @@ def vecinfer_encode_decode_metal(keys: torch.Tensor, k_codebook: torch.Tensor, s
     h = _sylvester_scale(H_mat)
     fused = h > 0 and sub_dim in (4, 8) and n_sub in (8, 16, 32, 64) and cb.shape[0] * sub_dim <= 16384
     if fused and cb.shape[0] > 256:   # the composition's products carry gradients and tangents: a caller who asks for them keeps them
-        fused = torch.autograd.forward_ad._current_level < 0 and not (torch.is_grad_enabled() and (
-            H_mat.requires_grad or (sm is not None and sm.requires_grad) or (want_k_tilde and keys.requires_grad)))
+        fused = _forward_ad._current_level < 0 and not (
+            (H_mat.requires_grad or (sm is not None and sm.requires_grad) or (want_k_tilde and keys.requires_grad)) and torch.is_grad_enabled())
     if fused:
-        kk, sm = (t if t is None or t.data_ptr() % 16 == 0 else t.clone() for t in (kk, sm))   # contiguous, but off the boundary
+        if kk.data_ptr() & 15:   # contiguous, but off the boundary
+            kk = kk.clone()
+        if sm is not None and sm.data_ptr() & 15:
+            sm = sm.clone()
         idx = torch.empty((B, Hh, S, n_sub), dtype=index_dtype, device=keys.device)
         k_hat = torch.empty_like(kk) if want_k_hat else None
         k_tilde = torch.empty((B, Hh, S, D), dtype=torch.float32, device=keys.device) if want_k_tilde else None
