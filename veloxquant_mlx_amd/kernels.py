@@ -784,7 +784,10 @@ vecinfer_dequant_hip = vecinfer_dequant_metal
 def hadamard_matrix(D: int, magnitude: float, device: torch.device) -> torch.Tensor:
     """The Sylvester-Hadamard matrix of entries +-``magnitude`` (a float32 value) made on the GPU, known to be one.  An ordinary
     tensor under ``torch.inference_mode`` too: it outlives the call, and the verdict is held against its version."""
-    with torch.inference_mode(False):
+    if torch.is_inference_mode_enabled():
+        with torch.inference_mode(False):
+            H = torch.empty((D, D), dtype=torch.float32, device=device)
+    else:
         H = torch.empty((D, D), dtype=torch.float32, device=device)
     with torch.cuda.device(H.device):
         _lib.check(_lib.load().vq_hadamard(H.data_ptr(), D, magnitude, _stream(H)))
