@@ -269,13 +269,13 @@ int vq_vecinfer_encode_keys(const void *keys, int k_dtype, int64_t B, int64_t H,
                             int cb_dtype, int n_centroids, int sub_dim, void *idx, int idx_dtype, void *k_hat,
                             float *k_tilde, void *stream);
 
-/* Centroid gather, out [N, sub_dim] = codebook[min(idx, n_centroids-1)].
- * Replaces dequantize_vq (allocators/vecinfer.py:321-335) and
- * vecinfer_dequant_metal (metal/_vecinfer.py:144-178). */
 /* The D x D Sylvester-Hadamard matrix in natural order, entries (-1)^popcount(i & j) * magnitude, D a power of two
  * (walsh_hadamard_matrix, veloxquant_mlx/allocators/vecinfer.py:60-87). */
 int vq_hadamard(float *out, int64_t D, float magnitude, void *stream);
 
+/* Centroid gather, out [N, sub_dim] = codebook[min(idx, n_centroids-1)].
+ * Replaces dequantize_vq (allocators/vecinfer.py:321-335) and
+ * vecinfer_dequant_metal (metal/_vecinfer.py:144-178). */
 int vq_vecinfer_dequant(const void *idx, int idx_dtype, int64_t N, const void *codebook,
                         int cb_dtype, int n_centroids, int sub_dim, void *out, int out_dtype,
                         void *stream);

@@ -105,8 +105,8 @@ template <typename T> struct Vec8 {
 // The clip factors whose error can be the smallest, as bits.  The stated error of a factor -- codes by division, every step
 // rounded, squares added left to right -- costs ten operations a value and a division where a code is near a tie; five give r = sc * sqrt(sum((t - q)^2)) with
 // t = (x - lo) / sc in one fma and q = clamp(rint(t)), which is close enough to rule out
-// all factors but one in 99.6 % of the groups at 4 bits (a 4100-token prompt of 8 x 8 heads, both tensors: 243 -> 230 us; what
-// is left is the exchange of rows with LDS in the head's order and the latency of a wave's one batch of rows).
+// all factors but one in 99.6 % of the groups at 4 bits (a 4100-token prompt of 8 x 8 heads, both tensors with their orders: 243 ->
+// 230 us, 222 now; what is left is vector issue, 93 % of the SIMD-busy cycles).
 // How close (u = 2^-24, W = levels * sc, M the largest |x|, so |lo| <= M and |x - lo| <= rng to within a few u * M):
 //   * the stated difference d = q * sc + lo - x of a code has an error of u (3 W + 3 M);
 //   * t has an error of u (2 rng + M) / sc (1 / sc is good to u after the Newton step), the stated quotient one of 2 u rng / sc;
