@@ -426,6 +426,21 @@ int vq_kivi_attend_plan(const vq_attend_args *a, int *path, int *nparts);
  * flash_prefill_attend (veloxquant_mlx/metal/_flash_prefill.py:171-237). */
 int vq_kivi_attend(const vq_attend_args *a);
 
+/* What a call may add to its argument block. */
+typedef struct vq_attend_ext {
+    /* > 0: the cache holds kv heads of 64 channels in pairs -- heads 2m and 2m + 1 side by side as head m of 128
+     * channels, an odd number's last one beside zeros -- and this is their number; a->D = 128,
+     * a->Hkv = (pair_heads + 1) / 2, a->Hq = 2 * a->Hkv times the query heads of a kv head (the workspace
+     * is sized by these).  q and out are the caller's own [B, pair_heads * R, 1, 64], k_new / v_new
+     * [B, pair_heads, 64].  Single-query decode path with sync_counters only, VQ_ERR_UNSUPPORTED otherwise. */
+    int64_t pair_heads;
+    /* Live slots of every sequence, prefix and tail together: int64 [B] on the device, in place of packed_lens /
+     * tail_lens (sequence b sees its first min(seq_lens[b], n_packed + n_tail) slots, its queries align to the
+     * end of those).  k_new / v_new go to row n_tail - 1 of every sequence's tail, live or not. */
+    const int64_t *seq_lens;
+} vq_attend_ext;
+int vq_kivi_attend_ext(const vq_attend_args *a, const vq_attend_ext *x);
+
 /* vq_kivi_attend for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The
  * split partials and the sync counters come from a device array built into the library (8 MiB +

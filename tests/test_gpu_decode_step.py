@@ -1,0 +1,108 @@
+"""Decode steps in one launch: kv heads of 64 channels kept in pairs, and batches whose sequences differ in length,
+each against the form with its arguments prepared by torch operations, bit for bit."""
+
+import math
+
+import pytest
+import torch
+
+from tests._gpu import gpu, require_gpu
+from veloxquant_mlx_amd import kernels as K
+from veloxquant_mlx_amd.cache import KVCacheConfig, KVCacheFactory
+from veloxquant_mlx_amd.cache.kivi_cache import own_half_of_paired_output, pad_queries_for_paired_heads
+
+pytestmark = gpu
+
+
+def _cache(D, bits, g, B, H, ctx, dtype, seed, meta="float16", R=128):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    rand = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    c = KVCacheFactory.create(KVCacheConfig(method="kivi", head_dim=D, bit_width_inlier=bits, kivi_group_size=g, residual_length=R,
+                                            fused_sdpa=True, fused_sdpa_memory_bound=True, kivi_meta_dtype=meta))
+    f = torch.exp(rand(D))
+    c.update_and_fetch((rand(B, H, ctx, D) * f).to(dtype), rand(B, H, ctx, D).to(dtype))
+    return c, lambda: ((rand(B, H, 1, D) * f).to(dtype), rand(B, H, 1, D).to(dtype)), rand
+
+
+@pytest.mark.parametrize("Hq,H,bits,g,B,ctx,dtype,meta", [
+    (32, 8, 2, 32, 1, 700, torch.float16, "float16"), (32, 8, 4, 64, 3, 192, torch.bfloat16, "float16"),
+    (14, 2, 4, 32, 2, 1000, torch.float16, "float16"), (9, 3, 3, 32, 2, 161, torch.bfloat16, "float16"),
+    (5, 5, 2, 32, 1, 4099, torch.float16, "float32"), (40, 2, 4, 32, 1, 333, torch.float16, "float16"),
+    (8, 8, 4, 32, 40, 200, torch.float16, "float16")])
+def test_paired_heads_step_is_the_padded_one(Hq, H, bits, g, B, ctx, dtype, meta):
+    """Queries read and outputs written by halves against queries padded with zeros and halves taken afterwards: the same
+    bits under a fixed order, token after token across a flush, with the newest token brought along by the launch."""
+    require_gpu()
+    scale = 0.125
+    a, new, rand = _cache(64, bits, g, B, H, ctx, dtype, Hq + ctx, meta)
+    b, _, _ = _cache(64, bits, g, B, H, ctx, dtype, Hq + ctx, meta)
+    deferred = 0
+    for step in range(g + 2):
+        k, v = new()
+        for c in (a, b):
+            c.update_and_fetch(k, v)
+        q = rand(B, Hq, 1, 64).to(dtype)
+        deferred += a._pending is not None
+        got = a.fused_sdpa(q, scale, fixed_order=True)
+        b._store_pending()
+        kw = dict(causal=True, sliding_window=0, fixed_order=True, lengths=None, num_splits=0)
+        want = own_half_of_paired_output(b._attend(pad_queries_for_paired_heads(q, H), scale, **kw), H)
+        assert got.shape == q.shape and got.dtype == q.dtype and a._pending is None
+        assert torch.equal(got, want), step
+        n = a.offset - a._n_quantized
+        assert torch.equal(a._tail_k[:, :, :n], b._tail_k[:, :, :n]) and torch.equal(a._tail_v[:, :, :n], b._tail_v[:, :, :n])
+    assert deferred >= g - 1
+    assert int(K._counters(q.device).abs().sum()) == 0
+
+
+@pytest.mark.parametrize("D,Hq,H,bits,dtype", [(128, 32, 8, 4, torch.float16), (64, 9, 3, 2, torch.bfloat16), (64, 8, 4, 4, torch.float16),
+                                               (256, 12, 4, 2, torch.bfloat16), (128, 6, 2, 8, torch.float16)])
+def test_lengths_of_a_batch_in_the_launch(D, Hq, H, bits, dtype):
+    """One length a sequence, clamped to prefix and tail inside the kernels, against the two clamped lists: the same bits, for
+    lengths at every edge; the newest token is stored whether its sequence sees it or not."""
+    require_gpu()
+    B, g, ctx, scale = 9, 32, 700, 1 / math.sqrt(D)
+    c, new, rand = _cache(D, bits, g, B, H, ctx, dtype, D + Hq)
+    k, v = new()
+    c.update_and_fetch(k, v)
+    nq, total = c._n_quantized, c.offset
+    lens = torch.tensor([0, 1, nq - 1, nq, nq + 1, total - 1, total, total + 5, 33], device="cuda")
+    q = rand(B, Hq, 1, D).to(dtype)
+    got = c.fused_sdpa(q, scale, lengths=lens, fixed_order=True)
+    n_tail = total - nq
+    pairs = k.shape[-1] == 64
+    rows = c._tail_k[:, :, n_tail - 1]
+    rows = rows.reshape(B, -1, 2, 64).reshape(B, -1, 64)[:, :H] if pairs else rows
+    assert torch.equal(rows, k[:, :, 0])
+    wide = pad_queries_for_paired_heads(q, H) if pairs else q
+    want = K.kivi_packed_attend(wide, k_packed=c._kp, k_scale=c._ks, k_zero=c._kz, v_packed=c._vp, v_scale=c._vs, v_zero=c._vz,
+                                n_packed=nq, bits=c._field, group_size=g, v_layout=c._v_layout, k_tail=c._tail_k,
+                                v_tail=c._tail_v, n_tail=n_tail, scale=scale, out_dtype=dtype, fixed_order=True,
+                                packed_lens=torch.clamp(lens, max=nq), tail_lens=torch.clamp(lens - nq, min=0, max=n_tail))
+    want = own_half_of_paired_output(want, H) if pairs else want
+    assert torch.equal(got, want)
+    assert torch.equal(c.fused_sdpa(q, scale, lengths=lens.tolist(), fixed_order=True), want)                # host lengths
+    assert torch.equal(c.fused_sdpa(q, scale, lengths=torch.stack([lens, lens], 1)[:, 0], fixed_order=True), want)   # strided ones
+    # several query positions of such a batch (rows kernel, decode tiles or prefill blocks: whatever takes it)
+    q = rand(B, Hq, 3, D).to(dtype)
+    some = torch.clamp(lens, min=3)
+    got = c.fused_sdpa(q, scale, lengths=some, fixed_order=True)
+    alone = [c.fused_sdpa(q, scale, lengths=torch.full((B,), int(n), device="cuda"), fixed_order=True)[i] for i, n in enumerate(some)]
+    assert torch.equal(got, torch.stack(alone))
+
+
+def test_pair_heads_refusals():
+    """What the launch for pairs does not take is refused before anything is written."""
+    require_gpu()
+    c, new, rand = _cache(64, 4, 32, 1, 4, 300, torch.float16, 3)
+    nq = c._n_quantized
+    kw = dict(k_packed=c._kp, k_scale=c._ks, k_zero=c._kz, v_packed=c._vp, v_scale=c._vs, v_zero=c._vz, n_packed=nq, bits=4,
+              group_size=32, v_layout="token", k_tail=c._tail_k, v_tail=c._tail_v, n_tail=c.offset - nq, scale=0.1)
+    ok = rand(1, 8, 1, 64).half()
+    for q, extra in ((rand(1, 8, 2, 64).half(), {}), (rand(1, 6, 1, 64).half(), {}), (rand(1, 8, 1, 128).half(), {}),
+                     (ok, dict(static_scratch=True)), (ok, dict(_single_launch=False)), (ok, dict(num_splits=-1)),
+                     (ok, dict(seq_lens=torch.tensor([5], dtype=torch.int32, device="cuda")))):
+        with pytest.raises(ValueError):
+            K.kivi_packed_attend(q, pair_heads=4, **{**kw, **extra})
+    with pytest.raises(ValueError):
+        K.kivi_packed_attend(ok, pair_heads=8, **kw)

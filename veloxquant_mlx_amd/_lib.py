@@ -46,6 +46,12 @@ class AttendArgs(C.Structure):
     ]
 
 
+class AttendExt(C.Structure):
+    """Mirror of ``vq_attend_ext``."""
+
+    _fields_ = [("pair_heads", i64), ("seq_lens", vp)]
+
+
 class LutAttendArgs(C.Structure):
     """Mirror of ``vq_lut_attend_args``."""
 
@@ -129,6 +135,7 @@ _SIGNATURES = {
     "vq_kivi_attend_workspace": (sz, [C.POINTER(AttendArgs)]),
     "vq_kivi_attend_plan": (i32, [C.POINTER(AttendArgs), C.POINTER(i32), C.POINTER(i32)]),
     "vq_kivi_attend": (i32, [C.POINTER(AttendArgs)]),
+    "vq_kivi_attend_ext": (i32, [C.POINTER(AttendArgs), C.POINTER(AttendExt)]),
     "vq_kivi_attend_static": (i32, [C.POINTER(AttendArgs)]),
     "vq_kivi_prefill_tiles": (i32, [C.POINTER(AttendArgs), i64, i64]),
     "vq_vecinfer_attend_workspace": (sz, [C.POINTER(LutAttendArgs)]),

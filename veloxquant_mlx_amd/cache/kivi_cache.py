@@ -270,7 +270,8 @@ class KIVIKVCache(FP16KVCache):
                                      f"got {tuple(keys.shape)}")
                 self._kv_heads = H
                 self._shape_bhd = (B, (H + 1) // 2, 2 * D)
-                self._update_memory_bound(pair_heads(keys), pair_heads(values))
+                if not self._defer_token(keys, values):
+                    self._update_memory_bound(pair_heads(keys), pair_heads(values))
                 z = self._zero_scalar
                 return z.expand(B, H, self.offset, D), z.expand(B, H, self.offset, D)
             self._shape_bhd = (B, H, D)
@@ -298,31 +299,44 @@ class KIVIKVCache(FP16KVCache):
         if self._pending is not None:
             k, v = self._pending
             self._pending = None
+            if self._pair:
+                k, v = pair_heads(k), pair_heads(v)
             K.kv_tail_append(k, v, self._tail_k, self._tail_v, self.offset - self._n_quantized - 1)
+
+    def _defer_token(self, keys: torch.Tensor, values: torch.Tensor) -> bool:
+        """A plain decode step with no flush due: the attention launch of this step stores the token (kv heads kept in pairs: the
+        caller's own rows of 64 channels).  Until then the cache holds the caller's tensors, not a copy: a caller that
+        reuses its key / value buffers between update_and_fetch and fused_sdpa must pass clones."""
+        if keys.shape[2] != 1 or self._n_quantized == 0 or self._tail_k is None:
+            return False
+        self._store_pending()
+        n_tail = self.offset - self._n_quantized
+        if not (n_tail < self._tail_k.shape[2] and keys.shape == values.shape and keys.dtype == self._tail_k.dtype
+                and values.dtype == keys.dtype and (keys.shape[3] == 128 or self._pair)
+                and keys.is_contiguous() and values.is_contiguous() and keys.data_ptr() % 16 == 0
+                and values.data_ptr() % 16 == 0
+                and (max(0, self.offset + 1 - self._residual_length) // self._group_size) * self._group_size
+                == self._n_quantized):
+            return False
+        self._drop_tiles()   # decoding has begun: the prefill scratch goes back
+        self._pending = (keys, values)
+        self.offset += 1
+        self._account_bytes(*self._shape_bhd[:2], 1, self._shape_bhd[2], 0)
+        z = self._zero_scalar
+        if z is None or z.dtype != keys.dtype or z.device != keys.device:
+            self._zero_scalar = torch.zeros((), dtype=keys.dtype, device=keys.device)
+        return True
 
     def _update_memory_bound(self, keys: torch.Tensor, values: torch.Tensor):
         B, H, S, D = keys.shape
+        if not self._pair and self._defer_token(keys, values):
+            z = self._zero_scalar
+            return z.expand(B, H, self.offset, D), z.expand(B, H, self.offset, D)
         self._store_pending()
         if S == 1:
             self._drop_tiles()   # decoding has begun: the prefill scratch goes back
         n_tail = self.offset - self._n_quantized
         need = n_tail + S
-        if (S == 1 and self._n_quantized > 0 and self._tail_k is not None and need <= self._tail_k.shape[2]
-                and keys.dtype == self._tail_k.dtype and values.dtype == keys.dtype and D == 128
-                and keys.is_contiguous() and values.is_contiguous() and keys.data_ptr() % 16 == 0
-                and values.data_ptr() % 16 == 0
-                and (max(0, self.offset + 1 - self._residual_length) // self._group_size) * self._group_size
-                == self._n_quantized):
-            # a plain decode step with no flush due: the attention launch of this step stores the token.
-            # Until then the cache holds the caller's tensors, not a copy: a caller that reuses its key /
-            # value buffers between update_and_fetch and fused_sdpa must pass clones.
-            self._pending = (keys, values)
-            self.offset += 1
-            self._account_bytes(B, H, S, D, 0)
-            z = self._zero_scalar
-            if z is None or z.dtype != keys.dtype or z.device != keys.device:
-                z = self._zero_scalar = torch.zeros((), dtype=keys.dtype, device=keys.device)
-            return z.expand(B, H, self.offset, D), z.expand(B, H, self.offset, D)
         # a flush that would pass fused_sdpa_max_ctx is refused here, before offset or rows change
         new_boundary = (max(0, self.offset + S - self._residual_length) // self._group_size) * self._group_size
         n_quant_now = new_boundary - self._n_quantized
@@ -408,13 +422,29 @@ class KIVIKVCache(FP16KVCache):
                 H -= 1   # a state restored without its meta_state: the query heads do not divide over an even count
             if q.shape[1] % H:
                 raise ValueError(f"KIVIKVCache.fused_sdpa: {q.shape[1]} query heads over {H} kv heads")
+            opts = dict(causal=causal, sliding_window=sliding_window, fixed_order=fixed_order, lengths=lengths, num_splits=num_splits)
+            if q.shape[2] == 1 and self._pairs_attend_direct():
+                try:   # a launch that reads queries and writes outputs by halves
+                    return self._attend(q, scale, pair_heads=H, **opts)
+                except ValueError:   # a shape it does not take
+                    pass
+            self._store_pending()
             key = (tuple(q.shape), q.dtype, q.device, K._stream_of(q.device))
             if self._q_pad is None or self._q_pad[0] != key:   # the zero halves are written once
                 wide_heads = 2 * self._shape_bhd[1] * (q.shape[1] // H)
                 self._q_pad = (key, q.new_zeros((q.shape[0], wide_heads, q.shape[2], 128)))
-            wide = self.fused_sdpa(pad_queries_for_paired_heads(q, H, self._q_pad[1]), scale, causal=causal,
-                                   sliding_window=sliding_window, fixed_order=fixed_order, lengths=lengths, num_splits=num_splits)
+            wide = self._attend(pad_queries_for_paired_heads(q, H, self._q_pad[1]), scale, **opts)
             return own_half_of_paired_output(wide, H)
+        return self._attend(q, scale, causal=causal, sliding_window=sliding_window, fixed_order=fixed_order, lengths=lengths,
+                            num_splits=num_splits)
+
+    def _pairs_attend_direct(self) -> bool:
+        """Whether a decode step over kv heads kept in pairs takes the matrix-unit decode launch (its gate on the cache's side)."""
+        return (self._n_quantized > 0 and self._field in (2, 4) and self._group_size >= 32 and self._v_layout == "token"
+                and (self._tail_k is None or self._tail_k.dtype in (torch.float16, torch.bfloat16)))
+
+    def _attend(self, q: torch.Tensor, scale: float, *, causal: bool, sliding_window: int, fixed_order: bool | None, lengths,
+                num_splits: int, pair_heads: int = 0):
         nq = self._n_quantized
         n_tail = self.offset - nq
         if q.shape[2] == 1:
@@ -435,11 +465,12 @@ class KIVIKVCache(FP16KVCache):
         if lengths is None and self._offer_tiles(q, kw):
             plan = kw["_plan_out"] = {}
         if lengths is not None:
-            self._store_pending()
-            n = torch.as_tensor(lengths, device=q.device).to(torch.int64).reshape(-1)
+            n = torch.as_tensor(lengths, device=q.device).to(torch.int64).reshape(-1).contiguous()
             if n.numel() != q.shape[0]:
                 raise ValueError(f"KIVIKVCache.fused_sdpa: lengths has {n.numel()} entries for a batch of {q.shape[0]}")
-            kw.update(packed_lens=torch.clamp(n, max=nq), tail_lens=torch.clamp(n - nq, min=0, max=n_tail))
+            kw["seq_lens"] = n
+        if pair_heads:
+            kw["pair_heads"] = pair_heads
         if self._pending is not None:
             try:   # append and attend in one launch (single-query MFMA decode path)
                 out = K.kivi_packed_attend(q, k_new=self._pending[0], v_new=self._pending[1], **kw)

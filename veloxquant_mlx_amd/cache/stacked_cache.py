@@ -193,13 +193,25 @@ class LayerStackedKIVICache:
             H = abs(self.layers[0]._kv_heads)
             if q.shape[2] % H:
                 raise ValueError(f"LayerStackedKIVICache.fused_sdpa_all: {q.shape[2]} query heads over {H} kv heads")
+            opts = dict(causal=causal, sliding_window=sliding_window, fixed_order=fixed_order, num_splits=num_splits)
+            if q.shape[3] == 1 and all(c._pairs_attend_direct() for c in self.layers):
+                try:   # a launch that reads queries and writes outputs by halves
+                    return self._attend_all(q, scale, pair_heads=H, **opts)
+                except ValueError:   # a shape it does not take
+                    pass
+            for c in self.layers:
+                c._store_pending()
             key = (tuple(q.shape), q.dtype, q.device, K._stream_of(q.device))
             if self._q_pad is None or self._q_pad[0] != key:
                 wide_heads = 2 * self.layers[0]._shape_bhd[1] * (q.shape[2] // H)
                 self._q_pad = (key, q.new_zeros((q.shape[0], q.shape[1], wide_heads, q.shape[3], 128)))
-            wide = self.fused_sdpa_all(pad_queries_for_paired_heads(q, H, self._q_pad[1]), scale, causal=causal,
-                                       sliding_window=sliding_window, fixed_order=fixed_order, num_splits=num_splits)
+            wide = self._attend_all(pad_queries_for_paired_heads(q, H, self._q_pad[1]), scale, **opts)
             return own_half_of_paired_output(wide, H)
+        return self._attend_all(q, scale, causal=causal, sliding_window=sliding_window, fixed_order=fixed_order, num_splits=num_splits)
+
+    def _attend_all(self, q: torch.Tensor, scale: float, *, causal: bool, sliding_window: int, fixed_order: bool | None,
+                    num_splits: int, pair_heads: int = 0) -> torch.Tensor:
+        NL, B = len(self.layers), q.shape[1]
         for l, c in enumerate(self.layers):
             if c.offset == 0 or c._n_quantized == 0:
                 raise RuntimeError(f"LayerStackedKIVICache.fused_sdpa_all: layer {l} has no packed tokens yet")
@@ -220,8 +232,8 @@ class LayerStackedKIVICache:
         k_new = v_new = None
         if all(p is not None for p in pending) and q.shape[3] == 1 and not ragged:
             # a decode step of all layers: the launch stores every layer's newest token and attends over it
-            k_new = torch.stack([p[0] for p in pending]).reshape(NL * B, tk.shape[1], tk.shape[3])
-            v_new = torch.stack([p[1] for p in pending]).reshape(NL * B, tk.shape[1], tk.shape[3])
+            k_new = torch.stack([p[0] for p in pending])
+            v_new = torch.stack([p[1] for p in pending])
         else:
             for c in self.layers:
                 c._store_pending()
@@ -239,6 +251,8 @@ class LayerStackedKIVICache:
                   causal=bool(causal) and q.shape[3] > 1, out_dtype=q.dtype, fixed_order=fixed_order,
                   sliding_window=int(sliding_window or 0), num_splits=max(0, int(num_splits)), **lens,
                   **self._stacked_sinks(B))
+        if pair_heads:
+            kw["pair_heads"] = pair_heads
         qf = q.reshape((NL * B,) + tuple(q.shape[2:]))
         if k_new is not None:
             try:

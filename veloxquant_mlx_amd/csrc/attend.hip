@@ -12,7 +12,7 @@ static std::atomic<int> g_fixed_order{0};
 // what a tail token costs the block of split 0, in packed tokens, when the plan balances the splits
 constexpr int64_t TAIL_EQUIV = 4;
 
-AttendPlan plan_attend(const vq_attend_args &a) {
+AttendPlan plan_attend(const AttendCall &a) {
     AttendPlan p;
     // bit 0: fixed chunk order; bit 1 (fixed_order == 3): the decode kernel also waits for every copy in flight
     p.fixed_order = a.fixed_order == 1 ? 1 : a.fixed_order == 3 ? 3 : a.fixed_order == 2 ? 0 : g_fixed_order.load(std::memory_order_relaxed);
@@ -107,8 +107,8 @@ static int64_t gcd64(int64_t x, int64_t y) { while (y) { const int64_t t = x % y
 // codes of a word) are dropped by moving the buffer bases forward; the strides between sequences
 // and heads stay those of cap_tokens, so the kernels address the rest as before.  What is left
 // below the window inside the first stretch is masked in the kernels.
-static vq_attend_args skip_below_window(const vq_attend_args &a) {
-    if (a.sliding_window <= 0 || a.packed_lens != nullptr || a.n_packed <= 0) return a;
+static AttendCall skip_below_window(const AttendCall &a) {
+    if (a.sliding_window <= 0 || a.own_lengths() || a.n_packed <= 0) return a;
     int64_t first = a.n_packed + a.n_tail - a.Sq + 1 - a.sliding_window;   // first slot of the first query
     if (first > a.n_packed) first = a.n_packed;
     const int64_t per = 32 / a.pack_bits;
@@ -116,7 +116,7 @@ static vq_attend_args skip_below_window(const vq_attend_args &a) {
     unit = unit / gcd64(unit, per) * per;
     const int64_t skip = first > 0 ? first / unit * unit : 0;
     if (skip <= 0) return a;
-    vq_attend_args b = a;
+    AttendCall b = a;
     const int64_t W = cdiv(a.D, per), GV = cdiv(a.D, a.group), es = a.meta_dtype == VQ_F16 ? 2 : 4;
     auto fwd = [](const void *p, int64_t bytes) { return (const void *)((const char *)p + bytes); };
     b.k_packed = fwd(a.k_packed, skip * W * 4);
@@ -185,14 +185,14 @@ static int validate(const vq_attend_args *a, const char *fn) {
 // does not.  A prefill-sized call with more than eight heads a group runs eight of them at a time through the prefill
 // blocks (one pass per eight heads, the last filled up) instead of one position a tile through the decode kernel.
 // Returns the group size of the calls that run, 0 when the call runs as it is.
-static int64_t padded_group(const vq_attend_args &a) {
+static int64_t padded_group(const AttendCall &a) {
     if (a.Sq < 2 || a.Hkv < 1 || a.Hq % a.Hkv != 0 || a.k_new != nullptr || a.num_splits < 0) return 0;
     const int64_t R = a.Hq / a.Hkv;
     if (R == 1 || R == 2 || R == 4 || R == 8) return 0;
     if ((a.Sq * a.D * (a.q_dtype == VQ_F32 ? 4 : 2)) % 16 != 0 || (a.Sq * a.D * (a.out_dtype == VQ_F32 ? 4 : 2)) % 16 != 0) return 0;
     if ((((uintptr_t)a.q | (uintptr_t)a.out) & 15u) != 0) return 0;
     const int path = plan_attend(a).path;
-    vq_attend_args b = a;
+    AttendCall b = a;
     b.q = nullptr;   // stands for a 256-byte aligned buffer
     if (R > 8) {
         if (a.Sq < 16 || path == 2) return 0;
@@ -236,24 +236,30 @@ extern "C" int vq_kivi_attend_fixed_order(int enable) {
     return g_fixed_order.exchange(enable ? 1 : 0, std::memory_order_relaxed);
 }
 
-extern "C" size_t vq_kivi_attend_workspace(const vq_attend_args *a) {
+static size_t attend_workspace(const AttendCall *a) {
     // the plan divides by the shapes: arguments that would not pass vq_kivi_attend need no workspace
     if (!a || a->B < 1 || a->Hq < 1 || a->Hkv < 1 || a->Sq < 1 || a->D < 1 || a->Hq % a->Hkv != 0 ||
         a->n_packed < 0 || a->n_tail < 0 || (a->n_packed > 0 && (a->pack_bits < 1 || a->pack_bits > 8 || a->group < 1)))
         return 0;
-    const vq_attend_args w = skip_below_window(*a);
+    const AttendCall w = skip_below_window(*a);
     if (const int64_t Rp = padded_group(w)) {
         // the padded call's own workspace, then its queries and its outputs
-        vq_attend_args b = *a;
+        AttendCall b = *a;
         b.Hq = a->Hkv * Rp;
         b.q = nullptr;
         const size_t rows = (size_t)(b.B * b.Hq * b.Sq) * (size_t)b.D;
-        return round256(vq_kivi_attend_workspace(&b)) + round256(rows * (a->q_dtype == VQ_F32 ? 4 : 2)) +
+        return round256(attend_workspace(&b)) + round256(rows * (a->q_dtype == VQ_F32 ? 4 : 2)) +
                round256(rows * (a->out_dtype == VQ_F32 ? 4 : 2));
     }
     AttendPlan p = plan_attend(w);
     if (p.path == 2 && mfma_prefill_direct_output(w, p.nparts)) return 0;   // the kernel writes `out` itself
     return (size_t)(a->B * a->Hq * a->Sq) * (size_t)p.nparts * (size_t)(a->D + 2) * sizeof(float);
+}
+
+extern "C" size_t vq_kivi_attend_workspace(const vq_attend_args *a) {
+    if (a == nullptr) return 0;
+    const AttendCall call(*a);
+    return attend_workspace(&call);
 }
 
 extern "C" int vq_kivi_prefill_tiles(const vq_attend_args *a, int64_t first_unit, int64_t n_units) {
@@ -270,13 +276,13 @@ extern "C" int vq_kivi_prefill_tiles(const vq_attend_args *a, int64_t first_unit
                    "%s: null packed-cache pointer", fn);
     if (a->n_tail > 0) VQ_REQUIRE(a->k_tail && a->v_tail, VQ_ERR_INVALID, "%s: null tail pointer", fn);
     if (n_units == 0) return VQ_OK;
-    return launch_prefill_tiles(*a, first_unit, n_units);
+    return launch_prefill_tiles(AttendCall(*a), first_unit, n_units);
 }
 
 extern "C" int vq_kivi_attend_plan(const vq_attend_args *a, int *path, int *nparts) {
     int rc = validate(a, "vq_kivi_attend_plan");
     if (rc != VQ_OK) return rc;
-    vq_attend_args w = skip_below_window(*a);
+    AttendCall w = skip_below_window(AttendCall(*a));
     if (const int64_t Rp = padded_group(w)) {   // the plan of the call that runs
         w.Hq = w.Hkv * Rp;
         w.q = nullptr;
@@ -287,12 +293,12 @@ extern "C" int vq_kivi_attend_plan(const vq_attend_args *a, int *path, int *npar
     return VQ_OK;
 }
 
-extern "C" int vq_kivi_attend(const vq_attend_args *a_in) {
+static int attend(const AttendCall *a_in) {
     const char *fn = "vq_kivi_attend";
     int rc = validate(a_in, fn);
     if (rc != VQ_OK) return rc;
-    const vq_attend_args windowed = skip_below_window(*a_in);
-    const vq_attend_args *a = &windowed;
+    const AttendCall windowed = skip_below_window(*a_in);
+    const AttendCall *a = &windowed;
     VQ_REQUIRE(a->q && a->out, VQ_ERR_INVALID, "%s: null q/out", fn);
     if (a->n_packed > 0)
         VQ_REQUIRE(a->k_packed && a->v_packed && a->k_scale && a->k_zero && a->v_scale && a->v_zero, VQ_ERR_INVALID,
@@ -307,15 +313,15 @@ extern "C" int vq_kivi_attend(const vq_attend_args *a_in) {
                    "%s: k_new / v_new must be 16-byte aligned", fn);
     }
     if (const int64_t Rp = padded_group(*a)) {
-        const size_t need = vq_kivi_attend_workspace(a_in);
+        const size_t need = attend_workspace(a_in);
         VQ_REQUIRE(a_in->workspace != nullptr && a_in->workspace_bytes >= need, VQ_ERR_WORKSPACE,
                    "%s: workspace of %zu bytes required, %zu given", fn, need, a_in->workspace_bytes);
         VQ_REQUIRE(((uintptr_t)a_in->workspace & 255u) == 0, VQ_ERR_INVALID, "%s: the workspace must be 256-byte aligned", fn);
         const int64_t R = a_in->Hq / a_in->Hkv;
-        vq_attend_args b = *a_in;   // the arguments as given: the inner call cuts the window itself
+        AttendCall b = *a_in;   // the arguments as given: the inner call cuts the window itself
         b.Hq = a_in->Hkv * Rp;
         b.q = nullptr;
-        const size_t inner = round256(vq_kivi_attend_workspace(&b));
+        const size_t inner = round256(attend_workspace(&b));
         const size_t rows = (size_t)(b.B * b.Hq * b.Sq) * (size_t)b.D;
         char *base = static_cast<char *>(a_in->workspace);
         void *q_wide = base + inner;
@@ -331,7 +337,7 @@ extern "C" int vq_kivi_attend(const vq_attend_args *a_in) {
             const int64_t n_valid = R - first < Rp ? R - first : Rp;
             launch_regroup(a_in->q, q_wide, groups, R, first, Rp, 0, Rp, n_valid, q_row, st);
             VQ_HIP_CHECK_LAUNCH(fn);
-            rc = vq_kivi_attend(&b);
+            rc = attend(&b);
             if (rc != VQ_OK) return rc;
             launch_regroup(out_wide, a_in->out, groups, Rp, 0, R, first, n_valid, n_valid, out_row, st);
             VQ_HIP_CHECK_LAUNCH(fn);
@@ -343,13 +349,23 @@ extern "C" int vq_kivi_attend(const vq_attend_args *a_in) {
     if (a->k_new != nullptr)
         VQ_REQUIRE(p.path == 1 && a->Sq == 1, VQ_ERR_UNSUPPORTED,
                    "%s: k_new / v_new need the single-query MFMA decode path; append with vq_kv_tail_append first", fn);
-    size_t need = vq_kivi_attend_workspace(a);
+    if (a->pair_heads != 0) {
+        const int64_t H = a->pair_heads;
+        VQ_REQUIRE(H >= 2 && a->Hkv == (H + 1) / 2 && a->D == 128 && a->Hq % (2 * a->Hkv) == 0 && a->Sq == 1, VQ_ERR_INVALID,
+                   "%s: pair_heads = %lld goes with %lld kv heads of 128 channels, query heads in multiples of twice that and one "
+                   "query position", fn, (long long)H, (long long)((H + 1) / 2));
+        // the launch that merges inside the kernel is the one that reads queries and writes outputs by halves
+        VQ_REQUIRE(p.path == 1 && a->sync_counters != nullptr && a->sink_k == nullptr &&
+                       (a->q_dtype == VQ_F32 || ((uintptr_t)a->q & 15u) == 0),
+                   VQ_ERR_UNSUPPORTED, "%s: pair_heads needs the single-launch decode path and 16-byte aligned queries", fn);
+    }
+    size_t need = attend_workspace(a);
     VQ_REQUIRE(need == 0 || (a->workspace != nullptr && a->workspace_bytes >= need), VQ_ERR_WORKSPACE,
                "%s: workspace of %zu bytes required, %zu given", fn, need, a->workspace_bytes);
     // protected rows: the patch pass reads the partials and the original (unshifted) packed store
     auto finish = [&]() -> int {
         if (a_in->sink_k == nullptr) return VQ_OK;
-        vq_attend_args full = *a_in;
+        AttendCall full = *a_in;
         full.workspace = a->workspace;
         launch_sink_patch(full, p.nparts);
         VQ_HIP_CHECK_LAUNCH(fn);
@@ -399,6 +415,20 @@ extern "C" int vq_kivi_attend(const vq_attend_args *a_in) {
     return rc;
 }
 
+extern "C" int vq_kivi_attend(const vq_attend_args *a) {
+    VQ_REQUIRE(a != nullptr, VQ_ERR_INVALID, "%s: null argument block", "vq_kivi_attend");
+    const AttendCall call(*a);
+    return attend(&call);
+}
+
+extern "C" int vq_kivi_attend_ext(const vq_attend_args *a, const vq_attend_ext *x) {
+    VQ_REQUIRE(a != nullptr, VQ_ERR_INVALID, "%s: null argument block", "vq_kivi_attend_ext");
+    VQ_REQUIRE(x == nullptr || x->seq_lens == nullptr || a->packed_lens == nullptr, VQ_ERR_INVALID,
+               "%s: seq_lens and packed_lens exclude each other", "vq_kivi_attend_ext");
+    const AttendCall call(*a, x);
+    return attend(&call);
+}
+
 // ---------------------------------------------------------------------------
 // vq_kivi_attend for callers that cannot allocate: the split partials and the sync counters
 // live in a file-scope device array instead of a caller-provided workspace.
@@ -427,7 +457,7 @@ extern "C" int vq_kivi_attend_static(const vq_attend_args *a) {
     VQ_REQUIRE(need <= STATIC_WS_BYTES, VQ_ERR_WORKSPACE,
                "%s: these shapes need %zu bytes of split partials, the built-in scratch holds %zu; use vq_kivi_attend "
                "with a workspace of its own", fn, need, STATIC_WS_BYTES);
-    vq_attend_args w = skip_below_window(*a);
+    AttendCall w = skip_below_window(AttendCall(*a));
     if (const int64_t Rp = padded_group(w)) {   // the call that runs: its GQA groups filled up
         w.Hq = w.Hkv * Rp;
         w.q = nullptr;

@@ -4,18 +4,32 @@
 
 namespace vq {
 
+// A call as the kernels take it: the caller's argument block and what vq_attend_ext adds to it.
+struct AttendCall : vq_attend_args {
+    int64_t pair_heads;          // > 0: kv heads of 64 channels, kept in pairs; the caller's kv head count
+    const int64_t *seq_lens;     // live slots of every sequence, prefix and tail together
+    AttendCall() = default;
+    explicit AttendCall(const vq_attend_args &a, const vq_attend_ext *x = nullptr)
+        : vq_attend_args(a), pair_heads(x ? x->pair_heads : 0), seq_lens(x ? x->seq_lens : nullptr) {}
+    __host__ __device__ bool own_lengths() const { return packed_lens != nullptr || seq_lens != nullptr; }
+};
+
 // a batch whose sequences differ in length: the block's copy of the arguments takes the lengths
 // of its own sequence
-__device__ __forceinline__ void take_sequence_lengths(vq_attend_args &a, int64_t b) {
+__device__ __forceinline__ void take_sequence_lengths(AttendCall &a, int64_t b) {
     if (a.packed_lens != nullptr) {
         a.n_packed = a.packed_lens[b];
         a.n_tail = a.tail_lens[b];
+    } else if (a.seq_lens != nullptr) {
+        const int64_t n = a.seq_lens[b], tail = n - a.n_packed;
+        if (tail < a.n_tail) a.n_tail = tail < 0 ? 0 : tail;
+        if (n < a.n_packed) a.n_packed = n;
     }
 }
 
 // first slot a query at position `pos` (of Sq, aligned to the end of n_total slots) sees under a
 // sliding window; 0 without one
-__device__ __host__ __forceinline__ int64_t window_first(const vq_attend_args &a, int64_t n_total, int64_t pos) {
+__device__ __host__ __forceinline__ int64_t window_first(const AttendCall &a, int64_t n_total, int64_t pos) {
     const int64_t lo = n_total - a.Sq + pos + 1 - a.sliding_window;
     return a.sliding_window > 0 && lo > 0 ? lo : 0;
 }
@@ -97,24 +111,24 @@ __device__ __forceinline__ float merge_records(const float *p, int nparts, int64
 
 // Decides kernel and split count from shapes only, so that the workspace query
 // and the launch agree.
-AttendPlan plan_attend(const vq_attend_args &a);
+AttendPlan plan_attend(const AttendCall &a);
 
-int launch_attend_generic(const vq_attend_args &a, int nsplit, int64_t split_len);
+int launch_attend_generic(const AttendCall &a, int nsplit, int64_t split_len);
 // vector-unit kernel with the kv head's bytes shared by its query heads (attend_rows.hip): whether it takes the
 // shapes, its row tiling (positions per tile, tiles per (sequence, kv head)), the launch
-bool rows_kernel_supported(const vq_attend_args &a);
-void rows_tiling(const vq_attend_args &a, int &pq, int &tiles);
-int launch_attend_rows(const vq_attend_args &a, const AttendPlan &p);
+bool rows_kernel_supported(const AttendCall &a);
+void rows_tiling(const AttendCall &a, int &pq, int &tiles);
+int launch_attend_rows(const AttendCall &a, const AttendPlan &p);
 // the same kernel over the tail tokens only, into partial `part0` of `nparts` per query row
-int launch_attend_rows_tail(const vq_attend_args &a, int part0, int nparts);
+int launch_attend_rows_tail(const AttendCall &a, int part0, int nparts);
 // byte codes, sixteen channels a lane (attend_wide.hip): whether it takes the shapes, its splits, the launch
-bool wide_kernel_supported(const vq_attend_args &a);
-void plan_attend_wide(const vq_attend_args &a, AttendPlan &p);
-void launch_attend_wide(const vq_attend_args &a, const AttendPlan &p);
-int launch_attend_merge(const vq_attend_args &a, int nparts);
-// protected rows (vq_attend_args.sink_k): rewrites every output row from the partials in the
+bool wide_kernel_supported(const AttendCall &a);
+void plan_attend_wide(const AttendCall &a, AttendPlan &p);
+void launch_attend_wide(const AttendCall &a, const AttendPlan &p);
+int launch_attend_merge(const AttendCall &a, int nparts);
+// protected rows (AttendCall.sink_k): rewrites every output row from the partials in the
 // workspace, with the stand-ins' weights taken out and the exact rows put in
-void launch_sink_patch(const vq_attend_args &a, int nparts);
+void launch_sink_patch(const AttendCall &a, int nparts);
 // merges partials [rows][nparts][D + 2] of (max, sum, accumulator) into out [rows][D]
 void launch_merge_rows(const float *ws, int64_t rows, int nparts, int64_t D, void *out, int out_dtype, hipStream_t st);
 // the same with a block a row where partials are many (sums in another order: not for launches whose other form merges
@@ -122,22 +136,22 @@ void launch_merge_rows(const float *ws, int64_t rows, int nparts, int64_t D, voi
 void launch_merge_splits(const float *ws, int64_t rows, int nparts, int64_t D, void *out, int out_dtype, hipStream_t st);
 
 // MFMA decode path (attend_mfma.hip)
-bool mfma_decode_supported(const vq_attend_args &a);
-int mfma_row_tiles(const vq_attend_args &a);
-int mfma_positions_per_tile(const vq_attend_args &a);
+bool mfma_decode_supported(const AttendCall &a);
+int mfma_row_tiles(const AttendCall &a);
+int mfma_positions_per_tile(const AttendCall &a);
 
 // MFMA prefill path (attend_prefill.hip): packed prefix into partial slot 0, tail into slot 1
-bool mfma_prefill_supported(const vq_attend_args &a);
-int mfma_prefill_block_rows(const vq_attend_args &a);   // 64, or 256 when a kv head has that many query rows
+bool mfma_prefill_supported(const AttendCall &a);
+int mfma_prefill_block_rows(const AttendCall &a);   // 64, or 256 when a kv head has that many query rows
 // returns true when the kernel wrote the output itself (one run per row: nothing to merge)
-bool launch_attend_mfma_prefill(const vq_attend_args &a, const AttendPlan &p);
+bool launch_attend_mfma_prefill(const AttendCall &a, const AttendPlan &p);
 // that case, from the shapes alone: such a launch writes no partials and needs no workspace
-bool mfma_prefill_direct_output(const vq_attend_args &a, int nparts);
+bool mfma_prefill_direct_output(const AttendCall &a, int nparts);
 // whether a launch of the 256-row blocks takes its units from a.kv_tiles
-bool mfma_prefill_uses_tiles(const vq_attend_args &a);
+bool mfma_prefill_uses_tiles(const AttendCall &a);
 // writes tiles [first_unit, first_unit + n_units) of every (sequence, kv head); VQ_OK or an error code
-int launch_prefill_tiles(const vq_attend_args &a, int64_t first_unit, int64_t n_units);
+int launch_prefill_tiles(const AttendCall &a, int64_t first_unit, int64_t n_units);
 // returns true when the kernel also merged the partials (sync counters were given)
-bool launch_attend_mfma_decode(const vq_attend_args &a, const AttendPlan &p);
+bool launch_attend_mfma_decode(const AttendCall &a, const AttendPlan &p);
 
 }  // namespace vq

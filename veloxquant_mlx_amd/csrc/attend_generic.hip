@@ -31,7 +31,7 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-__global__ __launch_bounds__(256) void attend_generic_kernel(vq_attend_args a, int nsplit, int64_t split_len,
+__global__ __launch_bounds__(256) void attend_generic_kernel(AttendCall a, int nsplit, int64_t split_len,
                                                              float *__restrict__ ws) {
     const int lane = threadIdx.x & 63;
     const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(MS_THREADS) void attend_merge_splits_kernel(const f
 // apart, takes the weight of every visible stand-in out of the softmax sum (its values are stored
 // as zeros, so the numerators never saw it; its key is rebuilt from the packed store as
 // code * scale + zero), then folds the exact rows in with a running maximum and writes the row.
-__global__ __launch_bounds__(256) void attend_sink_patch_kernel(vq_attend_args a, int nparts, const float *__restrict__ ws) {
+__global__ __launch_bounds__(256) void attend_sink_patch_kernel(AttendCall a, int nparts, const float *__restrict__ ws) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int64_t rows = a.B * a.Hq * a.Sq;
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(256) void attend_sink_patch_kernel(vq_attend_args a
     }
 }
 
-void launch_sink_patch(const vq_attend_args &a, int nparts) {
+void launch_sink_patch(const AttendCall &a, int nparts) {
     const int64_t rows = a.B * a.Hq * a.Sq;
     hipLaunchKernelGGL(attend_sink_patch_kernel, dim3((unsigned)cdiv(rows, 4)), dim3(256), 0, (hipStream_t)a.stream, a, nparts,
                        (const float *)a.workspace);
@@ -310,7 +310,7 @@ static void launch_merge(const float *ws, int64_t rows, int nparts, int64_t D, v
     else hipLaunchKernelGGL(attend_merge_kernel, dim3((unsigned)g), dim3(256), 0, st, ws, rows, nparts, D, out, out_dtype);
 }
 
-int launch_attend_generic(const vq_attend_args &a, int nsplit, int64_t split_len) {
+int launch_attend_generic(const AttendCall &a, int nsplit, int64_t split_len) {
     hipStream_t st = (hipStream_t)a.stream;
     const int64_t rows = a.B * a.Hq * a.Sq;
     const int64_t waves = rows * nsplit;
@@ -334,7 +334,7 @@ void launch_merge_rows(const float *ws, int64_t rows, int nparts, int64_t D, voi
     launch_merge(ws, rows, nparts, D, out, out_dtype, st);
 }
 
-int launch_attend_merge(const vq_attend_args &a, int nparts) {
+int launch_attend_merge(const AttendCall &a, int nparts) {
     launch_merge((const float *)a.workspace, a.B * a.Hq * a.Sq, nparts, a.D, a.out, a.out_dtype, (hipStream_t)a.stream);
     return VQ_OK;
 }

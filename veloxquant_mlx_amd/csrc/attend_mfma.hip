@@ -6,7 +6,7 @@ namespace vq {
 
 // Query positions one block takes: rows = (heads of the GQA group) x positions, at most eight
 // (a high and a remainder column each in the 16-wide tile).
-int mfma_positions_per_tile(const vq_attend_args &a) {
+int mfma_positions_per_tile(const AttendCall &a) {
     const int64_t R = a.Hq / a.Hkv;
     if (a.Sq == 1 || R > 8) return 1;
     return (int)(8 / R);
@@ -14,12 +14,12 @@ int mfma_positions_per_tile(const vq_attend_args &a) {
 
 // Row tiles per (sequence, kv head): positions in steps of mfma_positions_per_tile, times the tiles of
 // eight heads a GQA group of more than eight falls into.
-int mfma_row_tiles(const vq_attend_args &a) {
+int mfma_row_tiles(const AttendCall &a) {
     const int64_t R = a.Hq / a.Hkv;
     return (int)(cdiv(a.Sq, mfma_positions_per_tile(a)) * (R > 8 ? cdiv(R, 8) : 1));
 }
 
-bool mfma_decode_supported(const vq_attend_args &a) {
+bool mfma_decode_supported(const AttendCall &a) {
     if ((a.D != MF_D && a.D != 2 * MF_D) || a.n_packed <= 0) return false;
     // a head of 256 channels: packed prefix only (its tail goes through the vector kernel, one more launch), no
     // token brought along by the call
@@ -45,7 +45,7 @@ bool mfma_decode_supported(const vq_attend_args &a) {
     return true;
 }
 
-bool launch_attend_mfma_decode(const vq_attend_args &a, const AttendPlan &p) {
+bool launch_attend_mfma_decode(const AttendCall &a, const AttendPlan &p) {
     hipStream_t st = (hipStream_t)a.stream;
     float *ws = (float *)a.workspace;
     // rows a block carries: the GQA group at p.pq positions, padded to 4 or 8

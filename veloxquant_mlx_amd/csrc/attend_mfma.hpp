@@ -250,7 +250,16 @@ struct RowTile {
     // of eight heads at one position), RT = R * positions rows in all
     int R, RT, pos0, causal, h0;
     int64_t window;     // sliding window (0: none)
-    __device__ __forceinline__ bool valid(int j) const { return j < RT && pos0 + j / R < Sq; }
+    // kv heads of 64 channels kept in pairs (one query position): pair_R query heads a kv head (0: not pairs), pair_rows of
+    // them in this pair of kv heads (pair_R where the last kv head has no partner), io_base the first one's row of q and out
+    int pair_R = 0, pair_rows = 0;
+    int64_t io_base = 0;
+    __device__ __forceinline__ bool valid(int j) const {
+        return j < RT && pos0 + j / R < Sq && (pair_R == 0 || h0 + j % R < pair_rows);
+    }
+    // which half of the 128 channels tile row j's own kv head has, its row of q and out
+    __device__ __forceinline__ int pair_half(int j) const { return h0 + j % R >= pair_R; }
+    __device__ __forceinline__ int64_t io_row(int j) const { return io_base + h0 + j % R; }
     // first visible slot of tile row j
     __device__ __forceinline__ int64_t first(int j) const {
         int64_t pos = pos0 + j / R;
@@ -342,14 +351,25 @@ __device__ __forceinline__ f16x8 ld_tail8(const void *base, int64_t elem, bool b
     return tail8_from_raw(*reinterpret_cast<const uint4 *>((const u16 *)base + elem), bf16);
 }
 
+// The newest token's row of (sequence, kv head) bh where the caller holds it: first element, and how many of the 128
+// channels there are (kv heads of 64 channels kept in pairs: the last one of an odd number has no partner, whose channels
+// are zeros).
+__device__ __forceinline__ int64_t new_row_base(const AttendCall &a, int64_t bh) {
+    if (a.pair_heads == 0) return bh * MF_D;
+    return ((bh / a.Hkv) * a.pair_heads + 2 * (bh % a.Hkv)) * (MF_D / 2);
+}
+__device__ __forceinline__ int new_row_cols(const AttendCall &a, int64_t bh) {
+    return a.pair_heads != 0 && 2 * (bh % a.Hkv) + 1 >= a.pair_heads ? MF_D / 2 : MF_D;
+}
+
 // One wave's share of the tail: units w, w + T, ... of 32 tokens (w = which of the T tail waves this
 // is), written as a partial of its own into slot `slot` straight from the accumulators -- no
 // block-shared memory and no barrier, so the other waves of the block stream the packed prefix
 // meanwhile.  s_qraw: the query rows of this kv head as fp16, q_stride halves apart.  A wave
 // without units (a sequence with a shorter tail) writes an empty partial (max -inf, sum 0).
-__device__ __forceinline__ void tail_wave(const vq_attend_args &a, int64_t bh, const RowTile &tile, float c, int slot,
+__device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const RowTile &tile, float c, int slot,
                                           int nparts, float *__restrict__ ws, const f16 *s_qraw, int q_stride, int lane,
-                                          int w, int T, bool device_scope) {
+                                          int w, int T, bool device_scope, int64_t newest) {
     const int i = lane & 15, blk = lane >> 4;
     const int R = tile.RT;
     // tail tokens this lane's query row sees
@@ -369,15 +389,19 @@ __device__ __forceinline__ void tail_wave(const vq_attend_args &a, int64_t bh, c
 
     struct TUnit { f16x8 kr[2][4], vr[8]; };
     // the newest token's rows, when the call brings them, are read from where the caller holds
-    // them (row n_tail - 1 of the tail is being written by this block at the same time)
-    const int64_t newest = a.k_new != nullptr ? a.n_tail - 1 : -1;
+    // them (row `newest` of the tail is being written by this block at the same time)
+    const int64_t new_base = new_row_base(a, bh);
+    const int new_cols = new_row_cols(a, bh);
+    auto new_piece = [&](const void *p, int64_t col) {
+        return col < new_cols ? ld_tail8(p, new_base + col, bf16) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    };
     auto key_row = [&](int64_t tok, int64_t col) {
         if (tok >= a.n_tail) tok = 0;
-        return tok == newest ? ld_tail8(a.k_new, bh * MF_D + col, bf16) : ld_tail8(a.k_tail, tbase + tok * MF_D + col, bf16);
+        return tok == newest ? new_piece(a.k_new, col) : ld_tail8(a.k_tail, tbase + tok * MF_D + col, bf16);
     };
     auto value_row = [&](int64_t tok, int64_t col) {
         if (tok >= a.n_tail) tok = 0;
-        return tok == newest ? ld_tail8(a.v_new, bh * MF_D + col, bf16) : ld_tail8(a.v_tail, tbase + tok * MF_D + col, bf16);
+        return tok == newest ? new_piece(a.v_new, col) : ld_tail8(a.v_tail, tbase + tok * MF_D + col, bf16);
     };
     // every load of a unit is issued before its first product; clamped rows are masked below
     auto load = [&](int u, TUnit &d) {
@@ -438,8 +462,9 @@ __device__ __forceinline__ void tail_wave(const vq_attend_args &a, int64_t bh, c
         const int row = 4 * blk + r;
         if (!tile.valid(row)) continue;
         float *o = ws + (tile.row(row) * nparts + slot) * MF_PART;
+        if (tile.pair_R == 0 || tile.pair_half(row) == (i >> 3))   // (of a pair's channels only the row's own half is asked for)
 #pragma unroll
-        for (int nt = 0; nt < 8; ++nt) st_partial(o + 2 + 8 * i + nt, acc.O[nt][r], device_scope);
+            for (int nt = 0; nt < 8; ++nt) st_partial(o + 2 + 8 * i + nt, acc.O[nt][r], device_scope);
         if (i == 0) st_partial(o + 1, acc.O[8][r], device_scope);
     }
     if (blk == 0 && tile.valid(i)) st_partial(ws + (tile.row(i) * nparts + slot) * MF_PART, acc.m_run * LN2, device_scope);
@@ -449,16 +474,20 @@ __device__ __forceinline__ void tail_wave(const vq_attend_args &a, int64_t bh, c
 // arithmetic of attend_merge_kernel, which shares merge_partials).  Partials written by
 // other blocks of this launch are read with device-scope loads.
 template <int DH = 1>
-__device__ __forceinline__ void merge_rows(const vq_attend_args &a, const RowTile &tile, int nparts, const float *ws,
+__device__ __forceinline__ void merge_rows(const AttendCall &a, const RowTile &tile, int nparts, const float *ws,
                                            int tid, int nthreads) {
     constexpr int DD = MF_D * DH, PART = DD + 2;
-    for (int e = tid; e < tile.RT * DD; e += nthreads) {
-        const int j = e / DD, d = e % DD;
+    // (kv heads kept in pairs: a query head's own half of the pair's channels)
+    const bool pairs = DH == 1 && tile.pair_R != 0;
+    const int W = pairs ? DD / 2 : DD;
+    for (int e = tid; e < tile.RT * W; e += nthreads) {
+        const int j = pairs ? e / (DD / 2) : e / DD;
         if (!tile.valid(j)) continue;
         const int64_t row = tile.row(j);
+        const int c = e - j * W, d = pairs ? c + (DD / 2) * tile.pair_half(j) : c;
         // partials of other blocks come from beyond this XCD's L2: as few rounds of loads as possible
         const float v = merge_records<true>(ws + row * nparts * PART, nparts, PART, d);
-        const int64_t oi = row * DD + d;
+        const int64_t oi = (pairs ? tile.io_row(j) : row) * W + c;
         if (a.out_dtype == VQ_F16) ((f16 *)a.out)[oi] = (f16)v;
         else if (a.out_dtype == VQ_BF16) ((u16 *)a.out)[oi] = f32_to_bf16(v);
         else ((float *)a.out)[oi] = v;
@@ -468,14 +497,14 @@ __device__ __forceinline__ void merge_rows(const vq_attend_args &a, const RowTil
 // launchers of the packed-prefix kernel (it also runs the fp16 tail and, given sync counters,
 // the final merge); partials are [rows][nparts][MF_PART] floats of (max, sum, accumulator)
 // (one translation unit per scale / zero type and per number of query rows a block carries: 4 or 8)
-void launch_mfma_packed_f16meta_r4(const vq_attend_args &a, const AttendPlan &p, float *ws, hipStream_t st);
-void launch_mfma_packed_f16meta_r8(const vq_attend_args &a, const AttendPlan &p, float *ws, hipStream_t st);
-void launch_mfma_packed_f32meta_r4(const vq_attend_args &a, const AttendPlan &p, float *ws, hipStream_t st);
-void launch_mfma_packed_f32meta_r8(const vq_attend_args &a, const AttendPlan &p, float *ws, hipStream_t st);
+void launch_mfma_packed_f16meta_r4(const AttendCall &a, const AttendPlan &p, float *ws, hipStream_t st);
+void launch_mfma_packed_f16meta_r8(const AttendCall &a, const AttendPlan &p, float *ws, hipStream_t st);
+void launch_mfma_packed_f32meta_r4(const AttendCall &a, const AttendPlan &p, float *ws, hipStream_t st);
+void launch_mfma_packed_f32meta_r8(const AttendCall &a, const AttendPlan &p, float *ws, hipStream_t st);
 // the same for a head of 256 channels (packed prefix only)
-void launch_mfma_packed_d256_f16meta_r4(const vq_attend_args &a, const AttendPlan &p, float *ws, hipStream_t st);
-void launch_mfma_packed_d256_f16meta_r8(const vq_attend_args &a, const AttendPlan &p, float *ws, hipStream_t st);
-void launch_mfma_packed_d256_f32meta_r4(const vq_attend_args &a, const AttendPlan &p, float *ws, hipStream_t st);
-void launch_mfma_packed_d256_f32meta_r8(const vq_attend_args &a, const AttendPlan &p, float *ws, hipStream_t st);
+void launch_mfma_packed_d256_f16meta_r4(const AttendCall &a, const AttendPlan &p, float *ws, hipStream_t st);
+void launch_mfma_packed_d256_f16meta_r8(const AttendCall &a, const AttendPlan &p, float *ws, hipStream_t st);
+void launch_mfma_packed_d256_f32meta_r4(const AttendCall &a, const AttendPlan &p, float *ws, hipStream_t st);
+void launch_mfma_packed_d256_f32meta_r8(const AttendCall &a, const AttendPlan &p, float *ws, hipStream_t st);
 
 }  // namespace vq

@@ -177,13 +177,14 @@ template <int BITS, typename M, int GV, int RTP, int DH = 1> struct Ring {
 
 // The query rows of the block as fp16 in LDS, PK_QROW halves apart; rows the tile does not have are zero.
 template <int RTP, int THREADS, int DH = 1>
-__device__ __forceinline__ void stage_query(const vq_attend_args &a, const RowTile &tile, int tid, f16 *s_qraw) {
+__device__ __forceinline__ void stage_query(const AttendCall &a, const RowTile &tile, int tid, f16 *s_qraw) {
     constexpr int DD = MF_D * DH, PK_QROW = DD + 8;
     for (int e = tid; e < RTP * DD / 8; e += THREADS) {
         const int row = e / (DD / 8), d = 8 * (e % (DD / 8));
         f16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (tile.valid(row)) {
-            const int64_t i = tile.row(row) * DD + d;
+        const bool pairs = DH == 1 && tile.pair_R != 0;   // a query head's channels in its kv head's half, zeros in the other
+        if (tile.valid(row) && (!pairs || tile.pair_half(row) == d / (DD / 2))) {
+            const int64_t i = pairs ? tile.io_row(row) * (DD / 2) + d % (DD / 2) : tile.row(row) * DD + d;
             if (a.q_dtype == VQ_F16) v = *reinterpret_cast<const f16x8 *>((const f16 *)a.q + i);
             else {
 #pragma unroll
@@ -202,7 +203,7 @@ template <int N> __device__ __forceinline__ float row_ror(float x) {
 // order: bit 0 = deal the chunks round robin, bit 1 = wait for every copy in flight instead of the
 // counted ones (a slower, count-free cross-check of the ring's accounting)
 template <int BITS, typename M, int GV, int RTP, int DH = 1>
-__device__ __forceinline__ void packed_units(const vq_attend_args &a, int64_t bh, float c, int64_t t_begin,
+__device__ __forceinline__ void packed_units(const AttendCall &a, int64_t bh, float c, int64_t t_begin,
                                              int n_units, int lane_vis, int full_vis, int lane_lo, int lo_edge, int lane, int wave,
                                              PackedAcc<8 * DH> &acc, const f16 *s_qraw,
                                              const char *s_const, char *ring, int *s_next, int order) {
@@ -693,7 +694,7 @@ __device__ __forceinline__ void packed_units(const vq_attend_args &a, int64_t bh
 // tail waves (the fp16 tail comes as a partial of its own from the vector kernel) and takes no k_new / v_new.
 template <int BITS, typename M, int GV, int RTP, int DH = 1, int WAVES = Ring<BITS, M, GV, RTP, DH>::WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES / 4, WAVES / 4)))
-void attend_mfma_packed_kernel(vq_attend_args a, int64_t split_len, int64_t tail_equiv, int nparts, int pq, int tiles,
+void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equiv, int nparts, int pq, int tiles,
                                int order, float *__restrict__ ws) {
     using CL = Cols<GV, RTP, DH>;
     using RG = Ring<BITS, M, GV, RTP, DH>;
@@ -723,7 +724,11 @@ void attend_mfma_packed_kernel(vq_attend_args a, int64_t split_len, int64_t tail
     const int sp = (int)blockIdx.x, nsplit = (int)gridDim.x;
     const int64_t bh = by / tiles;
     const int64_t hkv = bh % a.Hkv, b = bh / a.Hkv;
+    const int64_t n_tail_all = a.n_tail;
     take_sequence_lengths(a, b);
+    // the newest token of the call (k_new) is the last row of the tail: of the whole batch's under seq_lens, of the sequence's
+    // own under tail_lens
+    const int64_t newest = a.k_new == nullptr ? -1 : (a.seq_lens != nullptr ? n_tail_all : a.n_tail) - 1;
     const float c = a.scale * LOG2E;
 
     RowTile tile;
@@ -739,18 +744,21 @@ void attend_mfma_packed_kernel(vq_attend_args a, int64_t split_len, int64_t tail
     tile.causal = a.causal;
     tile.window = a.sliding_window;
     tile.base_row = (b * a.Hq + hkv * group) * a.Sq;
+    tile.pair_R = a.pair_heads != 0 ? group / 2 : 0;
+    tile.pair_rows = 2 * hkv + 1 < a.pair_heads ? group : group / 2;
+    tile.io_base = (b * a.pair_heads + 2 * hkv) * tile.pair_R;
     const int RT = tile.RT;
 
     const bool single_launch = a.sync_counters != nullptr;
     stage_query<RTP, PK_THREADS, DH>(a, tile, tid, s_qraw);
-    if (DH == 1 && sp == 0 && a.k_new != nullptr && a.n_tail >= 1 && tid < 32) {
+    if (DH == 1 && sp == 0 && newest >= 0 && tid < 32) {
         // the newest token's key and value rows become the last tail row: 16 pieces of 16 bytes each
         const int piece = tid & 15;
         const bool val = tid >= 16;
-        const uint4 *src = reinterpret_cast<const uint4 *>(val ? a.v_new : a.k_new) + bh * (MF_D / 8) + piece;
+        const uint4 *src = reinterpret_cast<const uint4 *>(val ? a.v_new : a.k_new) + new_row_base(a, bh) / 8 + piece;
         uint4 *dst = reinterpret_cast<uint4 *>(const_cast<void *>(val ? a.v_tail : a.k_tail)) +
-                     (bh * a.tail_cap + a.n_tail - 1) * (MF_D / 8) + piece;
-        *dst = *src;
+                     (bh * a.tail_cap + newest) * (MF_D / 8) + piece;
+        *dst = 8 * piece < new_row_cols(a, bh) ? *src : make_uint4(0u, 0u, 0u, 0u);
     }
     __syncthreads();
     // the launch has nparts - nsplit tail slots (filled even when this sequence's tail is empty): the
@@ -759,7 +767,7 @@ void attend_mfma_packed_kernel(vq_attend_args a, int64_t split_len, int64_t tail
         const int tail_waves = nparts - nsplit;
         if (sp == 0 && wave >= PK_WAVES - tail_waves)
             tail_wave(a, bh, tile, c, nsplit + wave - (PK_WAVES - tail_waves), nparts, ws, s_qraw, PK_QROW, lane,
-                      wave - (PK_WAVES - tail_waves), tail_waves, single_launch);
+                      wave - (PK_WAVES - tail_waves), tail_waves, single_launch, newest);
     }
     // what the unit loop derives from the lane number is formed from here on, not ahead of the tail: the tail
     // needs its 168 registers to itself
@@ -840,7 +848,7 @@ void attend_mfma_packed_kernel(vq_attend_args a, int64_t split_len, int64_t tail
             den += s_l[w][row] * f;
         }
         float *o = ws + (tile.row(row) * nparts + sp) * PART;
-        st_partial(o + 2 + d, num, single_launch);
+        if (DH != 1 || tile.pair_R == 0 || tile.pair_half(row) == d / (DD / 2)) st_partial(o + 2 + d, num, single_launch);
         if (d == 0) { st_partial(o, gm * LN2, single_launch); st_partial(o + 1, den, single_launch); }
     }
 
@@ -868,7 +876,7 @@ void attend_mfma_packed_kernel(vq_attend_args a, int64_t split_len, int64_t tail
 }
 
 template <typename M, int RTP, int DH = 1>
-static void launch_mfma_packed(const vq_attend_args &a, const AttendPlan &p, float *ws, hipStream_t st) {
+static void launch_mfma_packed(const AttendCall &a, const AttendPlan &p, float *ws, hipStream_t st) {
     const dim3 grid((unsigned)p.nsplit, (unsigned)(a.B * a.Hkv * p.tiles));
     const int gv = (int)(MF_D * DH / a.group);   // groups of the whole head
     // more than 64 KB of block-shared memory has to be allowed per kernel and device, once

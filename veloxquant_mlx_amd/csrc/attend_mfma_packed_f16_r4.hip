@@ -3,7 +3,7 @@
 
 namespace vq {
 
-void launch_mfma_packed_f16meta_r4(const vq_attend_args &a, const AttendPlan &p, float *ws, hipStream_t st) {
+void launch_mfma_packed_f16meta_r4(const AttendCall &a, const AttendPlan &p, float *ws, hipStream_t st) {
     launch_mfma_packed<f16, 4>(a, p, ws, st);
 }
 

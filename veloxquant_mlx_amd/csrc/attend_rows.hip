@@ -45,14 +45,14 @@ __device__ __forceinline__ void ar_piece8(const uint4 &v, int tag, float (&o)[8]
 }  // namespace
 
 // Rows of a tile: heads h0 .. h0 + R - 1 of the kv head's group at pq consecutive positions.
-void rows_tiling(const vq_attend_args &a, int &pq, int &tiles) {
+void rows_tiling(const AttendCall &a, int &pq, int &tiles) {
     const int64_t R = a.Hq / a.Hkv;
     pq = (a.Sq > 1 && R <= AR_NR && AR_NR % R == 0) ? (int)(AR_NR / R) : 1;
     const int64_t htiles = R > AR_NR ? cdiv(R, AR_NR) : 1;
     tiles = (int)(cdiv(a.Sq, pq) * htiles);
 }
 
-bool rows_kernel_supported(const vq_attend_args &a) {
+bool rows_kernel_supported(const AttendCall &a) {
     if (a.D < 8 || a.D > 256 || a.Hq % a.Hkv != 0) return false;
     if (!(a.scale > 0.f)) return false;
     int bits = 4;
@@ -73,7 +73,7 @@ bool rows_kernel_supported(const vq_attend_args &a) {
 
 // NR: the rows a tile can hold (1 .. AR_NR): the per-row loops of a launch whose tiles are smaller shrink with it
 template <int BITS, int NR>
-__global__ __launch_bounds__(256) void attend_rows_kernel(vq_attend_args a, int64_t split_len, int pq, int tiles,
+__global__ __launch_bounds__(256) void attend_rows_kernel(AttendCall a, int64_t split_len, int pq, int tiles,
                                                           float *__restrict__ ws, int part0, int nparts) {
     constexpr int PER = 32 / BITS, CPL = ar_cpl(PER), SUBW = PER / CPL;   // SUBW lanes share a word
     constexpr uint32_t MASK = (1u << BITS) - 1u;
@@ -375,7 +375,7 @@ __global__ __launch_bounds__(256) void attend_rows_kernel(vq_attend_args a, int6
 }
 
 template <int BITS>
-static void launch_rows_bits(const vq_attend_args &a, const AttendPlan &p, dim3 grid, hipStream_t st, float *ws) {
+static void launch_rows_bits(const AttendCall &a, const AttendPlan &p, dim3 grid, hipStream_t st, float *ws) {
     const int64_t R = a.Hq / a.Hkv;
     const int rows = (int)((R > AR_NR ? AR_NR : R) * p.pq);   // rows of the largest tile
     switch (rows) {
@@ -386,7 +386,7 @@ static void launch_rows_bits(const vq_attend_args &a, const AttendPlan &p, dim3 
     }
 }
 
-int launch_attend_rows_tail(const vq_attend_args &a, int part0, int nparts) {
+int launch_attend_rows_tail(const AttendCall &a, int part0, int nparts) {
     AttendPlan p = {};
     p.path = 3;
     rows_tiling(a, p.pq, p.tiles);
@@ -397,7 +397,7 @@ int launch_attend_rows_tail(const vq_attend_args &a, int part0, int nparts) {
     return launch_attend_rows(a, p);
 }
 
-int launch_attend_rows(const vq_attend_args &a, const AttendPlan &p) {
+int launch_attend_rows(const AttendCall &a, const AttendPlan &p) {
     const dim3 grid((unsigned)p.nsplit, (unsigned)(a.B * a.Hkv * p.tiles));
     hipStream_t st = (hipStream_t)a.stream;
     float *ws = (float *)a.workspace;

@@ -384,7 +384,7 @@ void wide_splits(int64_t units, int64_t n, int want, int64_t &split_len, int &ns
 }
 
 void wide_tiling(int64_t Hq, int64_t Hkv, int64_t Sq, int &pq, int &tiles) {
-    vq_attend_args a = {};
+    AttendCall a = {};
     a.Hq = Hq;
     a.Hkv = Hkv;
     a.Sq = Sq;
@@ -435,7 +435,7 @@ constexpr int64_t WD_MAX_ROWS = 16, WD_MAX_INDEX_ROWS = 255;
 // group and every unit of tokens in one key group, and all pieces are 16-byte aligned.  The batch counts only where the grid ends
 // (grid y, as in rows_kernel_supported): layers stacked into one call take the kernel that a call a layer takes (600 sequences
 // of 32 / 8 heads of 128 channels, 4096 tokens: 5970 us in attend_rows.hip, 1403 here; 4607 x 8 / 8 of 64, 512 tokens 1602 and 614).
-bool wide_kernel_supported(const vq_attend_args &a) {
+bool wide_kernel_supported(const AttendCall &a) {
     if (a.Hkv < 1 || a.Hq % a.Hkv != 0 || (a.Hq / a.Hkv) * a.Sq > WD_MAX_ROWS) return false;
     int pq, tiles;
     rows_tiling(a, pq, tiles);
@@ -448,18 +448,18 @@ bool wide_kernel_supported(const vq_attend_args &a) {
     const int64_t blocks = a.B * a.Hkv * (int64_t)tiles;
     if (a.num_splits == 0 && blocks > 256 && a.n_packed * a.D <= (blocks > 1536 ? 8192 : 4608)) return false;
     return a.num_splits >= 0 && a.n_packed > 0 && a.n_tail == 0 && a.pack_bits == 8 && a.v_layout == VQ_V_CHANNEL_PACKED &&
-           a.meta_dtype == VQ_F32 && wide_head(a.D) && a.group % 32 == 0 && a.packed_lens == nullptr && a.k_new == nullptr &&
+           a.meta_dtype == VQ_F32 && wide_head(a.D) && a.group % 32 == 0 && !a.own_lengths() && a.k_new == nullptr &&
            a.sink_k == nullptr && a.scale > 0.f && blocks <= 65535 &&
            (((uintptr_t)a.k_packed | (uintptr_t)a.v_packed | (uintptr_t)a.k_scale | (uintptr_t)a.k_zero) & 15u) == 0;
 }
 
-void plan_attend_wide(const vq_attend_args &a, AttendPlan &p) {
+void plan_attend_wide(const AttendCall &a, AttendPlan &p) {
     rows_tiling(a, p.pq, p.tiles);
     wide_splits(a.B * a.Hkv * p.tiles, a.n_packed, a.num_splits, p.split_len, p.nsplit);
     p.nparts = p.nsplit;
 }
 
-void launch_attend_wide(const vq_attend_args &a, const AttendPlan &p) {
+void launch_attend_wide(const AttendCall &a, const AttendPlan &p) {
     const WideArgs w = {a.q, a.q_dtype, a.Hq, a.Hkv, a.Sq, a.n_packed, a.cap_tokens, a.scale, a.causal, a.sliding_window,
                         nullptr, 1, 0.f, p.split_len, p.pq, p.tiles, (float *)a.workspace};
     const ByteRows rows = {(const uint8_t *)a.k_packed, (const uint8_t *)a.v_packed, (const float *)a.k_scale, (const float *)a.k_zero,

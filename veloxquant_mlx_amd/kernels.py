@@ -1078,7 +1078,8 @@ def kivi_packed_attend(q: torch.Tensor, *, k_packed=None, k_scale=None, k_zero=N
                        v_new: torch.Tensor | None = None, fixed_order: bool | None = None,
                        out: torch.Tensor | None = None, static_scratch: bool = False, sliding_window: int = 0,
                        sinks: tuple | None = None, tiles: torch.Tensor | None = None, tiles_stale_from: int | None = None,
-                       _plan_out: dict | None = None, _single_launch: bool = True) -> torch.Tensor:
+                       _plan_out: dict | None = None, _single_launch: bool = True, pair_heads: int = 0,
+                       seq_lens: torch.Tensor | None = None) -> torch.Tensor:
     """softmax(q k^T * scale) v over ``[quantised prefix | fp16 tail]``.
 
     q ``[B,Hq,Sq,D]``; packed buffers as :func:`kivi_quant_pack` lays them out
@@ -1099,7 +1100,12 @@ def kivi_packed_attend(q: torch.Tensor, *, k_packed=None, k_scale=None, k_zero=N
     them instead of reconstructing the prefix in every block (same bits), other calls ignore them.  With
     ``tiles_stale_from`` a call that reads the tiles first rewrites them from that unit on (None: they are up to
     date).  A causal call over plain keys and values with two dozen row tiles or more per kv head makes such tiles
-    itself, in a scratch kept per device and stream (``tiles=False``: not even then)."""
+    itself, in a scratch kept per device and stream (``tiles=False``: not even then).
+    ``pair_heads``: the kv heads of a cache that keeps heads of 64 channels in pairs (its arrays have half as many heads
+    of 128 channels); ``q``, ``out``, ``k_new`` and ``v_new`` are the caller's own heads of 64 channels.  One query
+    position, the single-launch decode path only (``ValueError`` otherwise).
+    ``seq_lens`` (int64 ``[B]`` on the device): the live slots of every sequence, prefix and tail together, in place of
+    ``packed_lens`` / ``tail_lens``; ``k_new`` / ``v_new`` still go to tail row ``n_tail - 1``."""
     name = "kivi_packed_attend"
     if q.ndim != 4:
         raise ValueError(f"{name}: q must be 4D, got {tuple(q.shape)}")
@@ -1120,6 +1126,11 @@ def kivi_packed_attend(q: torch.Tensor, *, k_packed=None, k_scale=None, k_zero=N
     keep = [q, out]
     Hkv, k_tail = _cache_side(name, a, keep, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero, n_packed, bits,
                               group_size, v_layout, k_tail, v_tail, n_tail)
+    new_row = Hkv * D
+    if pair_heads:
+        if D != 64 or Sq != 1 or Hq % pair_heads or static_scratch or not _single_launch or sinks is not None:
+            raise ValueError(f"{name}: pair_heads takes single queries of 64 channels, heads a multiple of {pair_heads}, got {tuple(q.shape)}")
+        Hq, D, new_row = 2 * Hkv * (Hq // pair_heads), 128, pair_heads * 64
     a.B, a.Hq, a.Hkv, a.Sq, a.D = B, Hq, Hkv, Sq, D
     a.scale, a.causal, a.num_splits = float(scale), int(bool(causal)), int(num_splits)
     a.sliding_window = int(sliding_window or 0)
@@ -1135,7 +1146,7 @@ def kivi_packed_attend(q: torch.Tensor, *, k_packed=None, k_scale=None, k_zero=N
         keep += [sk, sv, sp]
     if (tiles is None and n_packed == 0 and causal and D == 128 and Hq % Hkv == 0 and 1 <= Hq // Hkv <= 8
             and (Hq // Hkv) * Sq >= 24 * 256 and k_tail.dtype in (torch.float16, torch.bfloat16)
-            and packed_lens is None and sinks is None and k_new is None and not static_scratch
+            and packed_lens is None and seq_lens is None and sinks is None and k_new is None and not static_scratch
             and B * Hkv * -(-int(n_tail) // 32) * PREFILL_TILE_BYTES <= _TILE_SCRATCH_MAX):
         # Plain keys and values under so many row tiles that every unit is read two dozen times or more: written
         # once as tiles (a scratch kept per device and stream, 608 B per slot and kv head) they are copied into
@@ -1159,12 +1170,15 @@ def kivi_packed_attend(q: torch.Tensor, *, k_packed=None, k_scale=None, k_zero=N
                 raise ValueError(f"{name}: {nm} must be a device tensor of shape [{B}]")
             lens.append(t.to(torch.int32).contiguous())
         a.packed_lens, a.tail_lens = lens[0].data_ptr(), lens[1].data_ptr()
+    if seq_lens is not None and (packed_lens is not None or seq_lens.shape != (B,) or seq_lens.dtype != torch.int64
+                                 or seq_lens.device != q.device or not seq_lens.is_contiguous() or static_scratch):
+        raise ValueError(f"{name}: seq_lens must be a contiguous int64 [{B}] tensor on the device, without packed_lens")
     if (k_new is None) != (v_new is None):
         raise ValueError(f"{name}: k_new and v_new go together")
     if k_new is not None:
         # the newest token's rows [B, Hkv, 1, D]: stored as the last tail row and attended in the same launch
         for nm, t in (("k_new", k_new), ("v_new", v_new)):
-            if k_tail is None or t.dtype != k_tail.dtype or t.numel() != B * Hkv * D or not t.is_contiguous() or not t.is_cuda:
+            if k_tail is None or t.dtype != k_tail.dtype or t.numel() != B * new_row or not t.is_contiguous() or not t.is_cuda:
                 raise ValueError(f"{name}: {nm} must be a contiguous [{B}, {Hkv}, 1, {D}] device tensor in the dtype of the tail")
         a.k_new, a.v_new = k_new.data_ptr(), v_new.data_ptr()
     lib = _lib.load()
@@ -1181,7 +1195,10 @@ def kivi_packed_attend(q: torch.Tensor, *, k_packed=None, k_scale=None, k_zero=N
     ws = _workspace(q.device, need)
     a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
     a.sync_counters = _counters(q.device).data_ptr() if _single_launch else None
-    _lib.check(lib.vq_kivi_attend(a))
+    if pair_heads or seq_lens is not None:
+        _lib.check(lib.vq_kivi_attend_ext(a, _lib.AttendExt(pair_heads, None if seq_lens is None else seq_lens.data_ptr())))
+    else:
+        _lib.check(lib.vq_kivi_attend(a))
     return out
 
 
