@@ -7,6 +7,8 @@
 // MFMA sums over k, so any assignment of channels (tokens) to k-slots is valid as
 // long as A and B agree.
 #pragma once
+#include <limits.h>
+
 #include "attend.hpp"
 
 namespace vq {
@@ -254,23 +256,26 @@ struct RowTile {
     // them in this pair of kv heads (pair_R where the last kv head has no partner), io_base the first one's row of q and out
     int pair_R = 0, pair_rows = 0;
     int64_t io_base = 0;
+    // head and position of tile row j, counted from the tile's first (a tile of one position takes no division)
+    __device__ __forceinline__ int head_of(int j) const { return RT == R ? j : j % R; }
+    __device__ __forceinline__ int pos_of(int j) const { return RT == R ? 0 : j / R; }
     __device__ __forceinline__ bool valid(int j) const {
-        return j < RT && pos0 + j / R < Sq && (pair_R == 0 || h0 + j % R < pair_rows);
+        return j < RT && pos0 + pos_of(j) < Sq && (pair_R == 0 || h0 + head_of(j) < pair_rows);
     }
     // which half of the 128 channels tile row j's own kv head has, its row of q and out
-    __device__ __forceinline__ int pair_half(int j) const { return h0 + j % R >= pair_R; }
-    __device__ __forceinline__ int64_t io_row(int j) const { return io_base + h0 + j % R; }
+    __device__ __forceinline__ int pair_half(int j) const { return h0 + head_of(j) >= pair_R; }
+    __device__ __forceinline__ int64_t io_row(int j) const { return io_base + h0 + head_of(j); }
     // first visible slot of tile row j
     __device__ __forceinline__ int64_t first(int j) const {
-        int64_t pos = pos0 + j / R;
+        int64_t pos = pos0 + pos_of(j);
         if (pos > Sq - 1) pos = Sq - 1;
         const int64_t lo = n_total - Sq + pos + 1 - window;
         return window > 0 && lo > 0 ? lo : 0;
     }
-    __device__ __forceinline__ int64_t row(int j) const { return base_row + (int64_t)(h0 + j % R) * Sq + pos0 + j / R; }
+    __device__ __forceinline__ int64_t row(int j) const { return base_row + (int64_t)(h0 + head_of(j)) * Sq + pos0 + pos_of(j); }
     // number of visible slots of tile row j (queries align to the end of the slots)
     __device__ __forceinline__ int64_t visible(int j) const {
-        int64_t pos = pos0 + j / R;
+        int64_t pos = pos0 + pos_of(j);
         if (pos > Sq - 1) pos = Sq - 1;
         return causal ? n_total - Sq + pos + 1 : n_total;
     }
@@ -294,13 +299,14 @@ struct TailAcc {
 // so that accumulator register r of tile T is k-slot pair r of the P.V product
 __device__ __forceinline__ int tail_tok(int blk, int r, int T) { return 8 * blk + r + 4 * T; }
 
-__device__ __forceinline__ f16x8 tail_softmax_unit(const f32x4 (&S)[2], float c, TailAcc &acc, int blk) {
+__device__ __forceinline__ f16x8 tail_softmax_unit(const f32x4 (&S)[2], float c, TailAcc &acc, int blk, bool first) {
     float mx = fmaxf(fmaxf(fmaxf(S[0][0], S[0][1]), fmaxf(S[0][2], S[0][3])),
                      fmaxf(fmaxf(S[1][0], S[1][1]), fmaxf(S[1][2], S[1][3])));
     mx = fmaxf(mx, __shfl_xor(mx, 16));
     mx = fmaxf(mx, __shfl_xor(mx, 32));
     const float m_seen = mx * c;
-    if (__any(m_seen > acc.m_run + RESCALE_SLACK)) {
+    if (first) acc.m_run = m_seen;   // nothing accumulated yet
+    else if (__any(m_seen > acc.m_run + RESCALE_SLACK)) {
         const float m_new = fmaxf(acc.m_run, m_seen);
         const float alpha = m_new == -INFINITY ? 1.f : exp2f(acc.m_run - m_new);   // 0 on the first unit
         float al[4];
@@ -327,6 +333,13 @@ __device__ __forceinline__ f16x8 tail_softmax_unit(const f32x4 (&S)[2], float c,
 __device__ __forceinline__ void st_partial(float *p, float v, bool device_scope) {
     if (device_scope) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else *p = v;
+}
+
+// two neighbouring floats at an even offset of a record (records start on 8 bytes)
+__device__ __forceinline__ void st_partial2(float *p, float v0, float v1, bool device_scope) {
+    const uint64_t u = (uint64_t)__float_as_uint(v0) | ((uint64_t)__float_as_uint(v1) << 32);
+    if (device_scope) __hip_atomic_store(reinterpret_cast<uint64_t *>(p), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *reinterpret_cast<uint64_t *>(p) = u;
 }
 
 // Eight consecutive tail elements as fp16.  A bf16 tail is converted: exact for magnitudes in
@@ -372,54 +385,70 @@ __device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const
                                           int w, int T, bool device_scope, int64_t newest) {
     const int i = lane & 15, blk = lane >> 4;
     const int R = tile.RT;
-    // tail tokens this lane's query row sees
-    int64_t n_vis = tile.visible(i < R ? i : 0) - a.n_packed;
-    if (n_vis > a.n_tail) n_vis = a.n_tail;
-    int64_t n_lo = tile.first(i < R ? i : 0) - a.n_packed;   // first tail token the row sees
-    if (n_lo < 0) n_lo = 0;
+    // tail tokens this lane's query row sees; lanes without a row see all of them
+    int n_vis = INT_MAX, n_lo = 0;
+    const int n_tail = (int)a.n_tail, newest_row = (int)newest;
+    if (i < R) {
+        const int64_t vis = tile.visible(i) - a.n_packed, lo = tile.first(i) - a.n_packed;
+        n_vis = vis > n_tail ? n_tail : (int)vis;
+        n_lo = lo < 0 ? 0 : lo > n_tail ? n_tail : (int)lo;   // first tail token the row sees
+    }
     TailAcc acc;
 #pragma unroll
     for (int n = 0; n < 9; ++n) acc.O[n] = f32x4{0.f, 0.f, 0.f, 0.f};
     acc.m_run = -INFINITY;
 
     const bool bf16 = a.tail_dtype == VQ_BF16;
-    const int64_t tbase = bh * a.tail_cap * MF_D;
+    const u16 *kt = (const u16 *)a.k_tail + bh * a.tail_cap * MF_D, *vt = (const u16 *)a.v_tail + bh * a.tail_cap * MF_D;
     const f16x8 ones = ones8();
-    const int n_tu = (int)((a.n_tail + 31) / 32);
+    const int n_tu = (n_tail + 31) / 32;
 
-    struct TUnit { f16x8 kr[2][4], vr[8]; };
-    // the newest token's rows, when the call brings them, are read from where the caller holds
-    // them (row `newest` of the tail is being written by this block at the same time)
+    // A unit's rows as they lie in memory, 16 pieces of 16 bytes a lane.  One wave runs a unit of a short context while the
+    // rest of the block waits for it, so that what counts is the number of instructions on the way and one round of
+    // memory latency: a row's ADDRESS is chosen (the newest token's rows, when the call brings them, are read from where the
+    // caller holds them: row `newest` of the tail is being written by this block at the same time), never a
+    // loaded value, and a conversion of the whole unit follows the last load (a unit from loads to stored partial: 7.0 us
+    // with a choice between two loads and 64-bit comparisons, 5.0 us now).
+    struct TUnit { uint4 kr[2][4], vr[8]; };
     const int64_t new_base = new_row_base(a, bh);
     const int new_cols = new_row_cols(a, bh);
-    auto new_piece = [&](const void *p, int64_t col) {
-        return col < new_cols ? ld_tail8(p, new_base + col, bf16) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    // first of the lane's pieces (at channel `col`) of a token's row: a lane's channels lie in one half of the row, all of them
+    // there or none (then the row's first channels stand in, dropped below)
+    auto row_at = [&](const u16 *rows, const void *row_new, int tok, int col) {
+        if (tok >= n_tail) tok = 0;   // masked below
+        const u16 *p = rows + (int64_t)tok * MF_D + col;
+        return tok == newest_row ? (const u16 *)row_new + new_base + (col < new_cols ? col : 0) : p;
     };
-    auto key_row = [&](int64_t tok, int64_t col) {
-        if (tok >= a.n_tail) tok = 0;
-        return tok == newest ? new_piece(a.k_new, col) : ld_tail8(a.k_tail, tbase + tok * MF_D + col, bf16);
-    };
-    auto value_row = [&](int64_t tok, int64_t col) {
-        if (tok >= a.n_tail) tok = 0;
-        return tok == newest ? new_piece(a.v_new, col) : ld_tail8(a.v_tail, tbase + tok * MF_D + col, bf16);
-    };
-    // every load of a unit is issued before its first product; clamped rows are masked below
+    auto dropped = [&](int tok, int col) { return (tok >= n_tail ? 0 : tok) == newest_row && col >= new_cols; };
     auto load = [&](int u, TUnit &d) {
-        const int64_t base = (int64_t)u * 32;
 #pragma unroll
         for (int Tt = 0; Tt < 2; ++Tt) {
-            const int64_t tok = base + tail_tok(i >> 2, i & 3, Tt);
+            const u16 *p = row_at(kt, a.k_new, u * 32 + tail_tok(i >> 2, i & 3, Tt), 32 * blk);
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) d.kr[Tt][ks] = key_row(tok, 32 * blk + 8 * ks);
+            for (int ks = 0; ks < 4; ++ks) d.kr[Tt][ks] = *reinterpret_cast<const uint4 *>(p + 8 * ks);
         }
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            d.vr[2 * p] = value_row(base + tail_tok(blk, p, 0), 8 * i);
-            d.vr[2 * p + 1] = value_row(base + tail_tok(blk, p, 1), 8 * i);
+        for (int p = 0; p < 8; ++p)
+            d.vr[p] = *reinterpret_cast<const uint4 *>(row_at(vt, a.v_new, u * 32 + tail_tok(blk, p >> 1, p & 1), 8 * i));
+        __builtin_amdgcn_sched_barrier(0);
+        if (bf16) {
+#pragma unroll
+            for (int p = 0; p < 8; ++p) {
+                d.kr[p >> 2][p & 3] = __builtin_bit_cast(uint4, tail8_from_raw(d.kr[p >> 2][p & 3], true));
+                d.vr[p] = __builtin_bit_cast(uint4, tail8_from_raw(d.vr[p], true));
+            }
+        }
+        if (new_cols < MF_D) {
+            const uint4 none = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+            for (int p = 0; p < 8; ++p) {
+                if (dropped(u * 32 + tail_tok(i >> 2, i & 3, p >> 2), 32 * blk)) d.kr[p >> 2][p & 3] = none;
+                if (dropped(u * 32 + tail_tok(blk, p >> 1, p & 1), 8 * i)) d.vr[p] = none;
+            }
         }
     };
     auto compute = [&](int u, const TUnit &d) {
-        const int64_t base = (int64_t)u * 32;
+        const int base = u * 32;
         // the query operand is read again for every unit: sixteen registers that need not live across the loads
         f16x8 qT[4];
 #pragma unroll
@@ -432,19 +461,22 @@ __device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const
         for (int Tt = 0; Tt < 2; ++Tt) {
             S[Tt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) S[Tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(d.kr[Tt][ks], qT[ks], S[Tt], 0, 0, 0);
+            for (int ks = 0; ks < 4; ++ks)
+                S[Tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(d.kr[Tt][ks]), qT[ks], S[Tt], 0, 0, 0);
         }
 #pragma unroll
         for (int Tt = 0; Tt < 2; ++Tt)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (i < R && (base + tail_tok(blk, r, Tt) >= n_vis || base + tail_tok(blk, r, Tt) < n_lo)) S[Tt][r] = -INFINITY;
-        const f16x8 P = tail_softmax_unit(S, c, acc, blk);
+            for (int r = 0; r < 4; ++r) {
+                const int t = base + tail_tok(blk, r, Tt);
+                if ((t >= n_vis) | (t < n_lo)) S[Tt][r] = -INFINITY;
+            }
+        const f16x8 P = tail_softmax_unit(S, c, acc, blk, u == w);
 #pragma unroll
         for (int nt = 0; nt < 8; ++nt) {   // lane column i is channel 8*i + nt
             f16x8 Bv;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) Bv[j] = d.vr[j][nt];
+            for (int j = 0; j < 8; ++j) Bv[j] = as_h8(d.vr[j])[nt];
             acc.O[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(P, Bv, acc.O[nt], 0, 0, 0);
         }
         acc.O[8] = __builtin_amdgcn_mfma_f32_16x16x32_f16(P, ones, acc.O[8], 0, 0, 0);
@@ -464,34 +496,125 @@ __device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const
         float *o = ws + (tile.row(row) * nparts + slot) * MF_PART;
         if (tile.pair_R == 0 || tile.pair_half(row) == (i >> 3))   // (of a pair's channels only the row's own half is asked for)
 #pragma unroll
-            for (int nt = 0; nt < 8; ++nt) st_partial(o + 2 + 8 * i + nt, acc.O[nt][r], device_scope);
+            for (int nt = 0; nt < 8; nt += 2) st_partial2(o + 2 + 8 * i + nt, acc.O[nt][r], acc.O[nt + 1][r], device_scope);
         if (i == 0) st_partial(o + 1, acc.O[8][r], device_scope);
     }
     if (blk == 0 && tile.valid(i)) st_partial(ws + (tile.row(i) * nparts + slot) * MF_PART, acc.m_run * LN2, device_scope);
 }
 
-// Combine the nparts partials of the tile's query rows into the output (the
-// arithmetic of attend_merge_kernel, which shares merge_partials).  Partials written by
-// other blocks of this launch are read with device-scope loads.
-template <int DH = 1>
-__device__ __forceinline__ void merge_rows(const AttendCall &a, const RowTile &tile, int nparts, const float *ws,
-                                           int tid, int nthreads) {
+// Combine the nparts partials of the tile's query rows into the output, in the order in which attend_merge_kernel
+// adds them (merge_partials: rounds of CH records).  Partials written by other blocks of this launch are read with
+// device-scope loads, which come from beyond this XCD's L2: a round's records are fetched by the whole block at
+// once, a wave a record, into `lds`, and summed from there, a thread two neighbouring channels of a row.  The
+// wave that has a row's maxima and sums turns them into factors while the accumulators are on their way (28 records of
+// four rows: 3.7 us where every thread fetched its channel of every record, 4.6; eight records of eight rows 4.3 of 5.5).
+// The whole launch, 32 / 8 heads at 2 bits: 8320 tokens of 128 channels 17.1 -> 15.1 us, 700 of 64 channels 16.4 -> 13.7.
+// RTP: rows of a tile at most.  lds: LDS_BYTES, the block's alone by now.
+constexpr int MERGE_MAX_CH = 36;
+template <int DH, int RTP, int WAVES, int LDS_BYTES, int CH>
+__device__ __forceinline__ void merge_rows_ch(const AttendCall &a, const RowTile &tile, int nparts, const float *ws,
+                                              int tid, int wave, uint64_t *lds) {
     constexpr int DD = MF_D * DH, PART = DD + 2;
+    constexpr int VAL = DD / 2;                                     // channel pairs of a record
+    // rows at a time: what the threads cover at two channels each and the records' places hold, a power of two
+    constexpr int ROOM = LDS_BYTES / (MERGE_MAX_CH * 8 * (VAL + 1)), COVER = WAVES / DH;
+    constexpr int FIT = ROOM < COVER ? ROOM : COVER, POW = FIT >= 8 ? 8 : FIT >= 4 ? 4 : FIT >= 2 ? 2 : 1;
+    constexpr int ROWS = RTP < POW ? RTP : POW, PER_ROW = WAVES / ROWS;   // waves that fetch a row's records
+    static_assert(ROOM >= 1 && ROWS * VAL <= 64 * WAVES, "a row's records fit the rings, a thread a channel pair");
+    // [ROWS][CH][VAL] channel pairs, [ROWS][CH + 1] (factor, factor * sum) of a record, the last the factor of what came before
+    uint64_t *s_val = lds, *s_fac = lds + ROWS * CH * VAL;
+    static_assert(8 * (ROWS * CH * VAL + ROWS * (CH + 1)) <= LDS_BYTES, "");
+    const int lane = tid & 63;
     // (kv heads kept in pairs: a query head's own half of the pair's channels)
     const bool pairs = DH == 1 && tile.pair_R != 0;
-    const int W = pairs ? DD / 2 : DD;
-    for (int e = tid; e < tile.RT * W; e += nthreads) {
-        const int j = pairs ? e / (DD / 2) : e / DD;
-        if (!tile.valid(j)) continue;
-        const int64_t row = tile.row(j);
-        const int c = e - j * W, d = pairs ? c + (DD / 2) * tile.pair_half(j) : c;
-        // partials of other blocks come from beyond this XCD's L2: as few rounds of loads as possible
-        const float v = merge_records<true>(ws + row * nparts * PART, nparts, PART, d);
-        const int64_t oi = (pairs ? tile.io_row(j) : row) * W + c;
-        if (a.out_dtype == VQ_F16) ((f16 *)a.out)[oi] = (f16)v;
-        else if (a.out_dtype == VQ_BF16) ((u16 *)a.out)[oi] = f32_to_bf16(v);
-        else ((float *)a.out)[oi] = v;
+    const int my_row = pairs ? tid / (VAL / 2) : tid / VAL, c2 = pairs ? tid % (VAL / 2) : tid % VAL;
+    const int fr = wave % ROWS, fp = wave / ROWS;   // the row whose records the wave fetches, the first of them
+    auto pack = [](float x, float y) { return (uint64_t)__float_as_uint(x) | ((uint64_t)__float_as_uint(y) << 32); };
+    auto lo = [](uint64_t u) { return __uint_as_float((uint32_t)u); };
+    auto hi = [](uint64_t u) { return __uint_as_float((uint32_t)(u >> 32)); };
+#pragma unroll 1
+    for (int r0 = 0; r0 < tile.RT; r0 += ROWS) {
+        float num0 = 0.f, num1 = 0.f, den = 0.f;
+        float gm = -INFINITY;   // of the row the wave fetches
+        const int j = r0 + my_row;
+        const bool mine = my_row < ROWS && tile.valid(j);
+        const int half = pairs && mine ? tile.pair_half(j) : 0;
+        const bool fetch = fp < PER_ROW && tile.valid(r0 + fr);
+        const uint64_t *row = reinterpret_cast<const uint64_t *>(ws + (fetch ? tile.row(r0 + fr) * nparts * PART : 0));
+#pragma unroll 1
+        for (int s0 = 0; s0 < nparts; s0 += CH) {
+            const int cnt = nparts - s0 < CH ? nparts - s0 : CH;
+            if (fetch) {
+                const uint64_t *rec = row + (int64_t)s0 * (PART / 2);
+                uint64_t hdr = 0;
+                if (fp == 0) hdr = __hip_atomic_load(rec + (lane < cnt ? lane : cnt - 1) * (PART / 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                constexpr int UN = ((CH + PER_ROW - 1) / PER_ROW < 12 ? (CH + PER_ROW - 1) / PER_ROW : 12) / DH;
+#pragma unroll 1
+                for (int p0 = fp; p0 < cnt; p0 += UN * PER_ROW) {
+                    uint64_t v[UN][DH];
+#pragma unroll
+                    for (int k = 0; k < UN; ++k)   // every load of the round before the first use
+                        if (p0 + k * PER_ROW < cnt)
+#pragma unroll
+                            for (int h = 0; h < DH; ++h)
+                                v[k][h] = __hip_atomic_load(rec + (p0 + k * PER_ROW) * (PART / 2) + 1 + 64 * h + lane,
+                                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (fp == 0 && p0 == fp) {
+                        const float m = lane < cnt ? lo(hdr) : -INFINITY;
+                        float cm = m;
+#pragma unroll
+                        for (int x = 32; x > 0; x >>= 1) cm = fmaxf(cm, __shfl_xor(cm, x));
+                        cm = fmaxf(cm, gm);
+                        // a record that saw nothing counts for nothing, whatever it holds: the factor -0 says so
+                        const float f = m == -INFINITY ? -0.f : __expf(m - cm);
+                        if (lane < cnt) s_fac[fr * (CH + 1) + lane] = pack(f, m == -INFINITY ? 0.f : hi(hdr) * f);
+                        if (lane == 0) s_fac[fr * (CH + 1) + CH] = pack(cm == -INFINITY ? 1.f : __expf(gm - cm), 0.f);   // 0 in the first round
+                        gm = cm;
+                    }
+#pragma unroll
+                    for (int k = 0; k < UN; ++k)
+                        if (p0 + k * PER_ROW < cnt)
+#pragma unroll
+                            for (int h = 0; h < DH; ++h) s_val[(fr * CH + p0 + k * PER_ROW) * VAL + 64 * h + lane] = v[k][h];
+                }
+            }
+            __syncthreads();
+            if (mine) {
+                const uint64_t *fac = s_fac + my_row * (CH + 1);
+                const uint64_t *val = s_val + my_row * CH * VAL + c2 + (half ? VAL / 2 : 0);
+                const float f0 = lo(fac[CH]);
+                num0 *= f0;
+                num1 *= f0;
+                den *= f0;
+#pragma unroll 8
+                for (int k = 0; k < cnt; ++k) {
+                    const uint64_t fk = fac[k], vk = val[k * VAL];
+                    const bool seen = (int)(uint32_t)fk >= 0;
+                    den += hi(fk);
+                    num0 += seen ? lo(vk) * lo(fk) : 0.f;
+                    num1 += seen ? hi(vk) * lo(fk) : 0.f;
+                }
+            }
+            if (s0 + CH < nparts || r0 + ROWS < tile.RT) __syncthreads();   // the records' places are filled again
+        }
+        if (mine) {
+            const float v0 = den > 0.f ? num0 / den : 0.f, v1 = den > 0.f ? num1 / den : 0.f;
+            const int64_t oi = pairs ? tile.io_row(j) * VAL + 2 * c2 : tile.row(j) * DD + 2 * c2;
+            if (a.out_dtype == VQ_F16) { ((f16 *)a.out)[oi] = (f16)v0; ((f16 *)a.out)[oi + 1] = (f16)v1; }
+            else if (a.out_dtype == VQ_BF16) { ((u16 *)a.out)[oi] = f32_to_bf16(v0); ((u16 *)a.out)[oi + 1] = f32_to_bf16(v1); }
+            else { ((float *)a.out)[oi] = v0; ((float *)a.out)[oi + 1] = v1; }
+        }
     }
+}
+template <int DH, int RTP, int WAVES, int LDS_BYTES>
+__device__ __forceinline__ void merge_rows(const AttendCall &a, const RowTile &tile, int nparts, const float *ws,
+                                           int tid, int wave, void *lds) {
+    uint64_t *l = reinterpret_cast<uint64_t *>(lds);
+    // (the round sizes of merge_records)
+    if (nparts <= 8) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, 8>(a, tile, nparts, ws, tid, wave, l);
+    else if (nparts <= 16) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, 16>(a, tile, nparts, ws, tid, wave, l);
+    else merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_MAX_CH>(a, tile, nparts, ws, tid, wave, l);
 }
 
 // launchers of the packed-prefix kernel (it also runs the fp16 tail and, given sync counters,
