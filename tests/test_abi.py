@@ -70,3 +70,10 @@ def test_argument_errors_surface_without_a_gpu():
     assert lib.vq_kivi_attend(t) == _lib.VQ_ERR_INVALID
     assert "room for all 64 slots" in _lib.last_error()
 
+
+
+def test_packed_argument_block_is_the_structure():
+    """The decode step's argument block, packed by ``struct``, lands in the fields of the ctypes mirror."""
+    values = [0.5 if t is _lib.f32 else i + 1 for i, (_, t) in enumerate(_lib.AttendArgs._fields_)]
+    a = _lib.AttendArgs.from_buffer_copy(_lib.ATTEND_PACK.pack(*values))
+    assert [getattr(a, n) for n, _ in _lib.AttendArgs._fields_] == values

@@ -106,3 +106,29 @@ def test_pair_heads_refusals():
             K.kivi_packed_attend(q, pair_heads=4, **{**kw, **extra})
     with pytest.raises(ValueError):
         K.kivi_packed_attend(ok, pair_heads=8, **kw)
+
+
+@pytest.mark.parametrize("D,Hq,H,bits,g,meta,dtype", [(128, 8, 2, 2, 32, "float16", torch.bfloat16), (128, 3, 3, 4, 128, "float16", torch.float16),
+                                                      (64, 16, 4, 2, 64, "float32", torch.float16), (256, 12, 4, 4, 32, "float16", torch.float16)])
+@pytest.mark.parametrize("units", [1, 2, 11, 12, 13, 24, 47, 48, 49, 59, 60, 61, 73])
+def test_units_dealt_over_the_waves_of_one_block(D, Hq, H, bits, g, meta, dtype, units):
+    """One block a kv head (num_splits=1) over numbers of 32-token units around one chunk a wave, where they are dealt out
+    evenly, and beyond, where waves draw chunks: against the general kernel, which sums token by token in float32.  Output
+    rounding is 2^-11 (fp16) or 2^-8 (bf16) of values of order one, the products' remainder terms 2^-21; the
+    three-step call of a cache is the same bits as the general wrapper's."""
+    require_gpu()
+    ctx = 128 + -(-32 * units // g) * g
+    c, new, rand = _cache(D, bits, g, 2, H, ctx, dtype, units, meta)
+    q = rand(2, Hq, 1, D).to(dtype)
+    got = c.fused_sdpa(q, D ** -0.5, fixed_order=True, num_splits=1)
+    kw = dict(k_packed=c._kp, k_scale=c._ks, k_zero=c._kz, v_packed=c._vp, v_scale=c._vs, v_zero=c._vz, n_packed=c._n_quantized,
+              bits=c._field, group_size=g, v_layout=c._v_layout, k_tail=c._tail_k, v_tail=c._tail_v, n_tail=c.offset - c._n_quantized,
+              scale=D ** -0.5)
+    wide = q if D > 64 else pad_queries_for_paired_heads(q, H)
+    half = (lambda o: o) if D > 64 else (lambda o: own_half_of_paired_output(o, H))
+    assert torch.equal(got, half(K.kivi_packed_attend(wide, fixed_order=True, num_splits=1, **kw)))
+    want = half(K.kivi_packed_attend(wide.float(), num_splits=-1, out_dtype=torch.float32, **kw))
+    eps = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    assert float((got.float() - want).abs().max()) <= eps * float(want.abs().max()) + 1e-3
+    free = c.fused_sdpa(q, D ** -0.5)
+    assert float((free.float() - want).abs().max()) <= eps * float(want.abs().max()) + 1e-3

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("VELOXQUANT_HIP_LIB", os.path.join(_HERE, "libveloxquant_hip.so"))
@@ -50,6 +51,13 @@ class AttendExt(C.Structure):
     """Mirror of ``vq_attend_ext``."""
 
     _fields_ = [("pair_heads", i64), ("seq_lens", vp)]
+
+
+# The same block packed by ``struct`` in one go: filling a ctypes structure field by field costs a decode step ~4 us.
+ATTEND_PACK = struct.Struct("@" + "".join({vp: "P", i64: "q", i32: "i", C.c_int32: "i", f32: "f", sz: "N"}[t]
+                                          for _, t in AttendArgs._fields_) + "0q")
+ATTEND_EXT_PACK = struct.Struct("@qP")
+assert ATTEND_PACK.size == C.sizeof(AttendArgs) and ATTEND_EXT_PACK.size == C.sizeof(AttendExt)
 
 
 class LutAttendArgs(C.Structure):
@@ -162,6 +170,8 @@ def load():
                 fn = getattr(lib, name)
                 fn.restype = res
                 fn.argtypes = args
+            # the same entry point over a packed argument block (ATTEND_PACK), and its extension or None
+            lib.attend_packed = C.CFUNCTYPE(i32, C.c_char_p, C.c_char_p)(("vq_kivi_attend_ext", lib))
             _lib = lib
             return _lib
         except (OSError, AttributeError) as e:  # missing file or symbol

@@ -272,8 +272,8 @@ class KIVIKVCache(FP16KVCache):
                 self._shape_bhd = (B, (H + 1) // 2, 2 * D)
                 if not self._defer_token(keys, values):
                     self._update_memory_bound(pair_heads(keys), pair_heads(values))
-                z = self._zero_scalar
-                return z.expand(B, H, self.offset, D), z.expand(B, H, self.offset, D)
+                z = self._zero_scalar.expand(B, H, self.offset, D)
+                return z, z
             self._shape_bhd = (B, H, D)
             return self._update_memory_bound(keys, values)
         self._shape_bhd = (B, H, D)
@@ -310,9 +310,9 @@ class KIVIKVCache(FP16KVCache):
         if keys.shape[2] != 1 or self._n_quantized == 0 or self._tail_k is None:
             return False
         self._store_pending()
-        n_tail = self.offset - self._n_quantized
-        if not (n_tail < self._tail_k.shape[2] and keys.shape == values.shape and keys.dtype == self._tail_k.dtype
-                and values.dtype == keys.dtype and (keys.shape[3] == 128 or self._pair)
+        n_tail, dtype = self.offset - self._n_quantized, keys.dtype
+        if not (n_tail < self._tail_k.shape[2] and keys.shape == values.shape and dtype == self._tail_k.dtype
+                and values.dtype == dtype and (keys.shape[3] == 128 or self._pair)
                 and keys.is_contiguous() and values.is_contiguous() and keys.data_ptr() % 16 == 0
                 and values.data_ptr() % 16 == 0
                 and (max(0, self.offset + 1 - self._residual_length) // self._group_size) * self._group_size
@@ -321,17 +321,18 @@ class KIVIKVCache(FP16KVCache):
         self._drop_tiles()   # decoding has begun: the prefill scratch goes back
         self._pending = (keys, values)
         self.offset += 1
-        self._account_bytes(*self._shape_bhd[:2], 1, self._shape_bhd[2], 0)
+        B, H, D = self._shape_bhd
+        self._account_bytes(B, H, 1, D, 0)
         z = self._zero_scalar
-        if z is None or z.dtype != keys.dtype or z.device != keys.device:
-            self._zero_scalar = torch.zeros((), dtype=keys.dtype, device=keys.device)
+        if z is None or z.dtype != dtype or z.device != keys.device:
+            self._zero_scalar = torch.zeros((), dtype=dtype, device=keys.device)
         return True
 
     def _update_memory_bound(self, keys: torch.Tensor, values: torch.Tensor):
         B, H, S, D = keys.shape
         if not self._pair and self._defer_token(keys, values):
-            z = self._zero_scalar
-            return z.expand(B, H, self.offset, D), z.expand(B, H, self.offset, D)
+            z = self._zero_scalar.expand(B, H, self.offset, D)
+            return z, z
         self._store_pending()
         if S == 1:
             self._drop_tiles()   # decoding has begun: the prefill scratch goes back
@@ -451,6 +452,22 @@ class KIVIKVCache(FP16KVCache):
             self._drop_tiles()   # a decode step, with or without per-sequence lengths
         if self._pending is not None and q.shape[2] != 1:
             self._store_pending()
+        extra = self._extra_attend_args()
+        if lengths is not None:
+            n = lengths
+            if not (isinstance(n, torch.Tensor) and n.dtype == torch.int64 and n.ndim == 1 and n.device == q.device and n.is_contiguous()):
+                n = torch.as_tensor(lengths, device=q.device).to(torch.int64).reshape(-1).contiguous()
+            if n.numel() != q.shape[0]:
+                raise ValueError(f"KIVIKVCache.fused_sdpa: lengths has {n.numel()} entries for a batch of {q.shape[0]}")
+            lengths = n
+        if q.ndim == 4 and q.shape[2] == 1 and self._memory_bound and nq > 0 and n_tail > 0 and not extra:
+            k_new, v_new = self._pending if self._pending is not None else (None, None)
+            out = K.kivi_decode_attend(q, self._kp, self._ks, self._kz, self._vp, self._vs, self._vz, nq, self._field, self._group_size,
+                                       self._v_layout, self._tail_k, self._tail_v, n_tail, float(scale), max(0, int(num_splits)),
+                                       fixed_order, int(sliding_window or 0), k_new, v_new, pair_heads, lengths)
+            if out is not None:
+                self._pending = None
+                return out
         if self._memory_bound:
             tk, tv = self._tail_k, self._tail_v
         else:
@@ -460,15 +477,12 @@ class KIVIKVCache(FP16KVCache):
                   k_tail=tk if n_tail else None, v_tail=tv if n_tail else None, n_tail=n_tail, scale=float(scale),
                   causal=bool(causal) and q.shape[2] > 1, out_dtype=q.dtype, fixed_order=fixed_order,
                   sliding_window=int(sliding_window or 0), num_splits=max(0, int(num_splits)))
-        kw.update(self._extra_attend_args())
+        kw.update(extra)
         plan = None
         if lengths is None and self._offer_tiles(q, kw):
             plan = kw["_plan_out"] = {}
         if lengths is not None:
-            n = torch.as_tensor(lengths, device=q.device).to(torch.int64).reshape(-1).contiguous()
-            if n.numel() != q.shape[0]:
-                raise ValueError(f"KIVIKVCache.fused_sdpa: lengths has {n.numel()} entries for a batch of {q.shape[0]}")
-            kw["seq_lens"] = n
+            kw["seq_lens"] = lengths
         if pair_heads:
             kw["pair_heads"] = pair_heads
         if self._pending is not None:
@@ -761,9 +775,10 @@ class KIVIKVCache(FP16KVCache):
             self._key_bytes_compressed += k
             self._value_bytes_compressed += v
         n_res = self.offset - self._n_quantized
-        self._residual_fp16_bytes = n_res * D * 2 * 2 * H * B
-        self._key_bytes_fp16 += H * B * S * D * 2
-        self._value_bytes_fp16 += H * B * S * D * 2
+        row16 = H * B * D * 2
+        self._residual_fp16_bytes = n_res * row16 * 2
+        self._key_bytes_fp16 += S * row16
+        self._value_bytes_fp16 += S * row16
         self._tokens_seen += S
 
     @property

@@ -922,8 +922,8 @@ def vecinfer_encode_decode_simple_metal(values: torch.Tensor, v_codebook: torch.
 _workspaces: dict[tuple, torch.Tensor] = {}
 
 
-def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
-    key = (device.type, device.index, _stream_of(device))
+def _workspace(device: torch.device, nbytes: int, stream: int | None = None) -> torch.Tensor:
+    key = (device.type, device.index, _stream_of(device) if stream is None else stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
@@ -955,10 +955,10 @@ def release_tile_scratch() -> int:
 _sync_counters: dict[tuple, torch.Tensor] = {}
 
 
-def _counters(device: torch.device) -> torch.Tensor:
+def _counters(device: torch.device, stream: int | None = None) -> torch.Tensor:
     """Per-(device, stream) int32 counters the single-launch decode path needs: zero when a
     call is enqueued, left zero by it (65536 = the largest B*H_kv the MFMA path takes)."""
-    key = (device.type, device.index, _stream_of(device))
+    key = (device.type, device.index, _stream_of(device) if stream is None else stream)
     c = _sync_counters.get(key)
     if c is None:
         c = torch.zeros(65536, dtype=torch.int32, device=device)
@@ -1200,6 +1200,72 @@ def kivi_packed_attend(q: torch.Tensor, *, k_packed=None, k_scale=None, k_zero=N
     else:
         _lib.check(lib.vq_kivi_attend(a))
     return out
+
+
+def kivi_decode_attend(q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero, n_packed, bits, group_size, v_layout,
+                       k_tail, v_tail, n_tail, scale, num_splits, fixed_order, sliding_window, k_new, v_new, pair_heads,
+                       seq_lens):
+    """One decode step of :func:`kivi_packed_attend` at a fraction of its host time (a step of one layer is shorter on
+    the GPU than the general wrapper takes to issue it): ``q [B,Hq,1,D]``, a live prefix and tail, arguments as there.
+    Checks what the library does not check for itself and returns ``None``, with nothing launched, for whatever it or the
+    library does not take; the general function then runs the call or raises."""
+    B, Hq, _, D = q.shape
+    dt, tail_dt, meta = q.dtype, k_tail.dtype, k_scale.dtype
+    tag, tail_tag = _FLOAT_TAG.get(dt), _FLOAT_TAG.get(tail_dt)
+    Hkv, cap = k_packed.shape[1], k_packed.shape[2]
+    if not (tag is not None and tail_tag is not None and q.is_cuda and k_packed.is_cuda and k_scale.is_cuda and k_zero.is_cuda
+            and v_packed.is_cuda and v_scale.is_cuda and v_zero.is_cuda and k_tail.is_cuda and v_tail.is_cuda
+            and k_packed.is_contiguous() and k_scale.is_contiguous() and k_zero.is_contiguous() and v_packed.is_contiguous()
+            and v_scale.is_contiguous() and v_zero.is_contiguous() and k_tail.is_contiguous() and v_tail.is_contiguous()
+            and (meta == torch.float16 or meta == torch.float32) and k_zero.dtype == meta and v_scale.dtype == meta
+            and v_zero.dtype == meta and v_tail.dtype == tail_dt and k_tail.shape == v_tail.shape and k_tail.shape[1] == Hkv and k_packed.shape[0] == B
+            and cap == (v_packed.shape[2] * (32 // bits) if v_layout == "token" else v_packed.shape[2])):
+        return None
+    new_k = new_v = 0
+    if pair_heads:
+        if D != 64 or Hq % pair_heads:
+            return None
+        Hq, D, new_row = 2 * Hkv * (Hq // pair_heads), 128, pair_heads * 64
+    else:
+        new_row = Hkv * D
+    if k_new is not None:
+        if not (k_new.dtype == tail_dt and v_new.dtype == tail_dt and k_new.numel() == B * new_row and v_new.numel() == B * new_row
+                and k_new.is_contiguous() and v_new.is_contiguous() and k_new.is_cuda and v_new.is_cuda):
+            return None
+        new_k, new_v = k_new.data_ptr(), v_new.data_ptr()
+    ext = None
+    if seq_lens is not None:
+        if seq_lens.shape != (B,) or seq_lens.dtype != torch.int64 or seq_lens.device != q.device or not seq_lens.is_contiguous():
+            return None
+        ext = _lib.ATTEND_EXT_PACK.pack(pair_heads, seq_lens.data_ptr())
+    elif pair_heads:
+        ext = _lib.ATTEND_EXT_PACK.pack(pair_heads, 0)
+    q = q.contiguous()
+    out = torch.empty_like(q)
+    lib = _lib.load()
+    device = q.device
+    stream = _stream_of(device)
+    ws = _workspace(device, 0, stream)
+    order = 0 if fixed_order is None else 1 if fixed_order is True else 2 if fixed_order is False else None
+    if order is None:
+        return None
+    for _ in range(2):
+        args = _lib.ATTEND_PACK.pack(
+            q.data_ptr(), out.data_ptr(), tag, tag, B, Hq, Hkv, 1, D,
+            k_packed.data_ptr(), k_scale.data_ptr(), k_zero.data_ptr(), v_packed.data_ptr(), v_scale.data_ptr(), v_zero.data_ptr(),
+            bits, group_size, VQ_F16 if meta == torch.float16 else VQ_F32, _V_LAYOUT[v_layout], n_packed, cap,
+            k_tail.data_ptr(), v_tail.data_ptr(), tail_tag, n_tail, k_tail.shape[2], scale, 0, num_splits,
+            ws.data_ptr(), ws.numel(), stream, _counters(device, stream).data_ptr(), 0, 0, new_k, new_v, order, sliding_window,
+            0, 0, 0, 0, 0, 0, 0, 0)
+        rc = lib.attend_packed(args, ext)
+        if rc == 0:
+            return out
+        if rc != _lib.VQ_ERR_WORKSPACE:
+            break
+        ws = _workspace(device, lib.vq_kivi_attend_workspace(AttendArgs.from_buffer_copy(args)), stream)
+    if rc != _lib.VQ_ERR_INVALID and rc != _lib.VQ_ERR_UNSUPPORTED:
+        _lib.check(rc)
+    return None
 
 
 def _check_fused_args(name, q, k_codes, v_codes, ndim):
