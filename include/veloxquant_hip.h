@@ -269,6 +269,16 @@ int vq_vecinfer_encode_keys(const void *keys, int k_dtype, int64_t B, int64_t H,
                             int cb_dtype, int n_centroids, int sub_dim, void *idx, int idx_dtype, void *k_hat,
                             float *k_tilde, void *stream);
 
+/* A decode step's key and value indices in one launch, written into index stores [B, H, cap_tokens, D / sub_dim] from token
+ * token0 on: keys by the rule of vq_vecinfer_encode_keys, values by that of vq_vecinfer_assign (one index rule, the same
+ * bits).  VQ_ERR_UNSUPPORTED, with nothing launched, beyond what one round of blocks takes (B * H * S * (D / k_sub_dim +
+ * D / v_sub_dim) / 64 <= 256) and for shapes that vq_vecinfer_encode_keys does not cover, on either side. */
+int vq_vecinfer_encode_step(const void *keys, int k_dtype, const void *values, int v_dtype, int64_t B, int64_t H, int64_t S,
+                            int64_t D, const float *smooth, int smooth_rows, float hadamard_scale, const void *k_codebook,
+                            int k_cb_dtype, int k_centroids, int k_sub_dim, const void *v_codebook, int v_cb_dtype,
+                            int v_centroids, int v_sub_dim, void *k_idx, int k_idx_dtype, void *v_idx, int v_idx_dtype,
+                            int64_t cap_tokens, int64_t token0, void *stream);
+
 /* The D x D Sylvester-Hadamard matrix in natural order, entries (-1)^popcount(i & j) * magnitude, D a power of two
  * (walsh_hadamard_matrix, veloxquant_mlx/allocators/vecinfer.py:60-87). */
 int vq_hadamard(float *out, int64_t D, float magnitude, void *stream);

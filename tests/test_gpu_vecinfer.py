@@ -10,6 +10,7 @@ import torch
 from oracle import cref, vecinfer as ov
 from tests._gpu import gpu, host, require_gpu, to_dev
 from veloxquant_mlx_amd import kernels as K
+from veloxquant_mlx_amd.allocators.vecinfer import walsh_hadamard_matrix
 from veloxquant_mlx_amd.cache import KVCacheConfig, KVCacheFactory
 
 pytestmark = gpu
@@ -613,3 +614,35 @@ def test_matrix_made_inside_a_graph_is_not_kept_for_eager_calls():
     for _ in range(3):
         graph.replay()
         assert torch.equal(out, want) and torch.equal(b.fused_sdpa(q, 0.1), want)
+
+
+@pytest.mark.parametrize("B,H,S,D,kn,ks,vn,vs,dtype,rows", [
+    (2, 8, 1, 128, 4096, 4, 256, 8, torch.float16, 8), (1, 3, 5, 64, 256, 8, 256, 8, torch.bfloat16, 1), (1, 4, 1, 256, 4096, 4, 2048, 8, torch.float32, 0),
+    (4, 8, 3, 128, 33, 4, 4096, 4, torch.float16, 1), (1, 1, 1, 512, 2048, 8, 7, 8, torch.bfloat16, 0), (8, 8, 5, 128, 300, 4, 31, 8, torch.float16, 8),
+    (1, 16, 21, 128, 256, 8, 256, 8, torch.float16, 1), (5, 2, 1, 32, 1, 4, 1, 8, torch.float32, 2), (8, 8, 6, 128, 256, 4, 256, 8, torch.float16, 1)])
+def test_step_indices_go_into_the_store(B, H, S, D, kn, ks, vn, vs, dtype, rows):
+    """A few tokens in one launch, into the store at a token of its own, against the two launches with the same rule: the
+    same whole numbers, and nothing else of the store touched.  The last row is more than one round of blocks takes
+    and must be refused."""
+    require_gpu()
+    g = torch.Generator(device="cuda").manual_seed(B * D + S + kn)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda")
+    keys, values = (rand(B, H, S, D) * torch.exp(rand(D))).to(dtype), rand(B, H, S, D).to(dtype)
+    keys[0, 0, 0, :ks] = 300.0 if S > 1 else 0.0
+    kcb, vcb = rand(kn, ks), rand(vn, vs)
+    smooth = None if rows == 0 else torch.exp(0.3 * rand(rows, D))
+    Hm = walsh_hadamard_matrix(D, device="cuda")
+    it = lambda n: torch.uint8 if n <= 256 else torch.int32
+    cap, at = S + 9, 5
+    ks_store = torch.full((B, H, cap, D // ks), 77, dtype=it(kn), device="cuda")
+    vs_store = torch.full((B, H, cap, D // vs), 77, dtype=it(vn), device="cuda")
+    want_k, want_v = ks_store.clone(), vs_store.clone()
+    took = K.vecinfer_encode_step(keys, values, kcb, ks, vcb, vs, Hm, smooth, ks_store, vs_store, at)
+    assert took == (-(-B * H * S * D // ks // 64) + -(-B * H * S * D // vs // 64) <= 256)
+    if took:
+        want_k[:, :, at:at + S] = K.vecinfer_encode_decode_metal(keys, kcb, ks, Hm, smooth, index_dtype=it(kn), want_k_hat=False)[1]
+        want_v[:, :, at:at + S] = K.vecinfer_quantize_metal(values, vcb, vs, index_dtype=it(vn))
+    assert torch.equal(ks_store, want_k) and torch.equal(vs_store, want_v)
+    # what does not fit the store is refused by the library before any launch
+    assert not K.vecinfer_encode_step(keys, values, kcb, ks, vcb, vs, Hm, smooth, ks_store, vs_store, cap - S + 1)
+    assert torch.equal(ks_store, want_k) and torch.equal(vs_store, want_v)

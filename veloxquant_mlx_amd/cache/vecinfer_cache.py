@@ -130,6 +130,7 @@ class VecInferKVCache(FP16KVCache):
         self._stored_v_indices: torch.Tensor | None = None
         self._stored_S_kv = 0
         self._smooth_kv_heads: int | None = None
+        self._zero: torch.Tensor | None = None   # what the zero-stride placeholders expand
 
     # ------------------------------------------------------------------ smooth factors
     def _validate_smooth(self) -> None:
@@ -266,16 +267,33 @@ class VecInferKVCache(FP16KVCache):
     def _update_and_fetch_fused(self, keys, values):
         """Indices only; returns zero-stride placeholders (vecinfer_cache.py:491-532)."""
         B, H, S, D = keys.shape
-        _, k_idx = K.vecinfer_encode_decode_metal(keys, self._key_codebook, self._key_sub_dim, self._H, self._smooth,
-                                                  index_dtype=self._k_idx_dtype, want_k_hat=False)
-        v_idx = K.vecinfer_quantize_metal(values, self._value_codebook, self._value_sub_dim,
-                                          index_dtype=self._v_idx_dtype)
-        self._stash(k_idx, v_idx)
+        if keys.shape == values.shape and 0 < B * H * S * (self._n_sub_k + self._n_sub_v) <= 256 * 64:   # a few tokens: one launch
+            self._ensure_index_capacity(B, H, S, keys.device)
+        if self._stored_k_indices is not None and S > 0 and self._stored_S_kv + S <= self._stored_k_indices.shape[2] and K.vecinfer_encode_step(
+                keys, values, self._key_codebook, self._key_sub_dim, self._value_codebook, self._value_sub_dim, self._H, self._smooth,
+                self._stored_k_indices, self._stored_v_indices, self._stored_S_kv):
+            self._stored_S_kv += S
+        else:
+            _, k_idx = K.vecinfer_encode_decode_metal(keys, self._key_codebook, self._key_sub_dim, self._H, self._smooth,
+                                                      index_dtype=self._k_idx_dtype, want_k_hat=False)
+            v_idx = K.vecinfer_quantize_metal(values, self._value_codebook, self._value_sub_dim,
+                                              index_dtype=self._v_idx_dtype)
+            self._stash(k_idx, v_idx)
         self.offset += S
         self._account_bytes(B, H, S, D)
-        zk = torch.zeros((), dtype=keys.dtype, device=keys.device)
-        zv = torch.zeros((), dtype=values.dtype, device=values.device)
-        return zk.expand(B, H, self._stored_S_kv, D), zv.expand(B, H, self._stored_S_kv, D)
+        zk = self._placeholder(keys).expand(B, H, self._stored_S_kv, D)
+        return zk, zk if values.dtype == keys.dtype and values.device == keys.device else self._placeholder(values).expand(
+            B, H, self._stored_S_kv, D)
+
+    def _placeholder(self, like: torch.Tensor) -> torch.Tensor:
+        """A zero of the dtype and device of ``like`` (kept from call to call, unless it was made while a graph is captured or
+        under ``torch.inference_mode``)."""
+        z = self._zero
+        if z is None or z.dtype != like.dtype or z.device != like.device:
+            z = torch.zeros((), dtype=like.dtype, device=like.device)
+            if not (z.is_inference() or (like.is_cuda and torch.cuda.is_current_stream_capturing())):
+                self._zero = z
+        return z
 
     # ------------------------------------------------------------------ state / trim
     @property

@@ -163,6 +163,34 @@ extern "C" int vq_vecinfer_encode_keys(const void *keys, int k_dtype, int64_t B,
     return VQ_OK;
 }
 
+extern "C" int vq_vecinfer_encode_step(const void *keys, int k_dtype, const void *values, int v_dtype, int64_t B, int64_t H, int64_t S,
+                                       int64_t D, const float *smooth, int smooth_rows, float hadamard_scale, const void *k_codebook,
+                                       int k_cb_dtype, int k_centroids, int k_sub_dim, const void *v_codebook, int v_cb_dtype,
+                                       int v_centroids, int v_sub_dim, void *k_idx, int k_idx_dtype, void *v_idx, int v_idx_dtype,
+                                       int64_t cap_tokens, int64_t token0, void *stream) {
+    const char *fn = "vq_vecinfer_encode_step";
+    VQ_REQUIRE(is_float_tag(k_dtype) && is_float_tag(v_dtype) && is_float_tag(k_cb_dtype) && is_float_tag(v_cb_dtype), VQ_ERR_INVALID,
+               "%s: unsupported float dtype", fn);
+    VQ_REQUIRE(B >= 1 && H >= 1 && S >= 1 && D >= 1 && (D & (D - 1)) == 0, VQ_ERR_INVALID, "%s: keys must be 4D [B, H, S, D], D a power of 2", fn);
+    VQ_REQUIRE(k_centroids >= 1 && v_centroids >= 1 && k_sub_dim >= 1 && v_sub_dim >= 1 && D % k_sub_dim == 0 && D % v_sub_dim == 0,
+               VQ_ERR_INVALID, "%s: D=%lld not divisible by sub_dim", fn, (long long)D);
+    VQ_REQUIRE((k_idx_dtype == VQ_I32 || (k_idx_dtype == VQ_U8 && k_centroids <= 256)) &&
+                   (v_idx_dtype == VQ_I32 || (v_idx_dtype == VQ_U8 && v_centroids <= 256)),
+               VQ_ERR_INVALID, "%s: indices must be int32, or uint8 for at most 256 centroids", fn);
+    VQ_REQUIRE(smooth == nullptr || smooth_rows == 1 || smooth_rows == H, VQ_ERR_INVALID, "%s: smooth must have 1 or H=%lld rows, got %d", fn,
+               (long long)H, smooth_rows);
+    VQ_REQUIRE(token0 >= 0 && token0 + S <= cap_tokens, VQ_ERR_INVALID, "%s: tokens [%lld, %lld) do not fit the store of %lld", fn,
+               (long long)token0, (long long)(token0 + S), (long long)cap_tokens);
+    VQ_REQUIRE(keys && values && k_codebook && v_codebook && k_idx && v_idx, VQ_ERR_INVALID, "%s: null pointer", fn);
+    auto at = [&](void *p, int tag, int64_t per) { return (void *)((char *)p + token0 * per * (tag == VQ_U8 ? 1 : 4)); };
+    const EncodeSide k = {keys, k_dtype, k_codebook, k_cb_dtype, k_centroids, k_sub_dim, at(k_idx, k_idx_dtype, D / k_sub_dim), k_idx_dtype};
+    const EncodeSide v = {values, v_dtype, v_codebook, v_cb_dtype, v_centroids, v_sub_dim, at(v_idx, v_idx_dtype, D / v_sub_dim), v_idx_dtype};
+    VQ_REQUIRE(launch_encode_step_mfma(k, v, B, H, S, D, smooth, smooth_rows, hadamard_scale, cap_tokens, (hipStream_t)stream),
+               VQ_ERR_UNSUPPORTED, "%s: more tokens or other shapes than one launch takes", fn);
+    VQ_HIP_CHECK_LAUNCH(fn);
+    return VQ_OK;
+}
+
 namespace vq {
 // 64 KB at D = 128: the launch is all it costs (built on the host and copied: 300 us and a synchronisation)
 __global__ void hadamard_kernel(float *__restrict__ out, int64_t D, float magnitude) {

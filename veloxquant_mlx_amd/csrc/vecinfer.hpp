@@ -38,4 +38,18 @@ bool launch_encode_keys_mfma(const void *keys, int kt, int64_t B, int64_t heads,
                              int smooth_rows, float h, const void *cb, int ct, int nc, int sub, void *idx, int it, void *k_hat,
                              float *k_tilde, hipStream_t st);
 
+// Keys and values of a few tokens in one launch, indices straight into stores of `cap` tokens a (sequence, head); idx: the
+// first of the S tokens.  Returns false, launching nothing, for what it does not cover (shapes as above, values of
+// sub_dim 4 or 8, more sub-vectors than one round of blocks).
+struct EncodeSide {
+    const void *x;
+    int xt;
+    const void *cb;
+    int ct, nc, sub;
+    void *idx;
+    int it;
+};
+bool launch_encode_step_mfma(const EncodeSide &k, const EncodeSide &v, int64_t B, int64_t heads, int64_t S, int64_t D, const float *smooth,
+                             int smooth_rows, float h, int64_t cap, hipStream_t st);
+
 }  // namespace vq

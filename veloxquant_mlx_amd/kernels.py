@@ -895,6 +895,42 @@ def vecinfer_encode_decode_metal(keys: torch.Tensor, k_codebook: torch.Tensor, s
     return (k_hat, idx, k_tilde) if want_k_tilde else (k_hat, idx)
 
 
+def vecinfer_encode_step(keys, values, k_codebook, k_sub_dim, v_codebook, v_sub_dim, H_mat, smooth, k_store, v_store, token0: int) -> bool:
+    """Key and value indices of a few tokens, in one launch, into stores ``[B,H,capacity,n_sub]`` from token ``token0`` on:
+    the indices of :func:`vecinfer_encode_decode_metal` and :func:`vecinfer_quantize_metal`.  Returns ``False``, with
+    nothing launched, for what that launch does not take; the two functions then do it."""
+    B, Hh, S, D = keys.shape
+    if not (keys.shape == values.shape and keys.is_cuda and values.is_cuda and keys.dtype in _FLOAT_TAG and values.dtype in _FLOAT_TAG
+            and k_codebook.dtype in _FLOAT_TAG and v_codebook.dtype in _FLOAT_TAG and k_codebook.is_contiguous() and v_codebook.is_contiguous()
+            and k_codebook.shape[1] == k_sub_dim and v_codebook.shape[1] == v_sub_dim and k_codebook.is_cuda and v_codebook.is_cuda
+            and B * Hh * S * (D // k_sub_dim + D // v_sub_dim) <= 256 * 64 and k_store.is_contiguous() and v_store.is_contiguous()
+            and k_store.is_cuda and v_store.is_cuda and k_store.shape[:2] == (B, Hh) and v_store.shape[:3] == k_store.shape[:3]
+            and k_store.shape[3] * k_sub_dim == D and v_store.shape[3] * v_sub_dim == D
+            and k_store.dtype in (torch.uint8, torch.int32) and v_store.dtype in (torch.uint8, torch.int32) and H_mat.shape[0] == D):
+        return False
+    if k_codebook.shape[0] > 256 and (_forward_ad._current_level >= 0 or (
+            torch.is_grad_enabled() and (H_mat.requires_grad or (smooth is not None and smooth.requires_grad)))):
+        return False   # the composition's transform, as in vecinfer_encode_decode_metal
+    sm = smooth
+    if sm is not None:
+        if sm.dtype != torch.float32 or not sm.is_cuda or not sm.is_contiguous() or (sm.ndim == 2 and sm.shape[0] not in (1, Hh)):
+            return False
+    h = _sylvester_scale(H_mat)
+    if not h > 0:
+        return False
+    k, v = keys.contiguous(), values.contiguous()
+    rc = _lib.load().vq_vecinfer_encode_step(
+        k.data_ptr(), _FLOAT_TAG[k.dtype], v.data_ptr(), _FLOAT_TAG[v.dtype], B, Hh, S, D, None if sm is None else sm.data_ptr(),
+        1 if sm is None or sm.ndim == 1 else sm.shape[0], h, k_codebook.data_ptr(), _FLOAT_TAG[k_codebook.dtype], k_codebook.shape[0],
+        k_sub_dim, v_codebook.data_ptr(), _FLOAT_TAG[v_codebook.dtype], v_codebook.shape[0], v_sub_dim, k_store.data_ptr(),
+        VQ_U8 if k_store.dtype == torch.uint8 else VQ_I32, v_store.data_ptr(), VQ_U8 if v_store.dtype == torch.uint8 else VQ_I32,
+        k_store.shape[2], token0, _stream(keys))
+    if rc == _lib.VQ_ERR_INVALID or rc == _lib.VQ_ERR_UNSUPPORTED:
+        return False
+    _lib.check(rc)
+    return True
+
+
 def vecinfer_encode_decode_simple_metal(values: torch.Tensor, v_codebook: torch.Tensor, sub_dim: int, *,
                                         index_dtype: torch.dtype = torch.int32):
     """Value encode+decode: nearest centroid and its gather; drop-in for
