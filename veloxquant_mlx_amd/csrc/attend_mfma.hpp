@@ -281,6 +281,24 @@ struct RowTile {
     }
 };
 
+// What the rest of a block asks of its tile's rows, worked out once by sixteen threads: in a short context's launch every
+// further copy of the divisions and comparisons behind these numbers is fetched for the first time by waves that others wait for.
+struct RowTable {
+    int off[MF_ROWS];        // row of q, out and partials, counted from base_row; -1: not a row of the tile
+    int io[MF_ROWS];         // pairs: row of q and out, counted from io_base
+    int half[MF_ROWS];       // pairs: the half of the channels that is the row's own
+    int64_t vis[MF_ROWS], first[MF_ROWS];   // visible slots, first of them (of row 0 where there is none)
+    __device__ __forceinline__ void fill(const RowTile &t, int j) {
+        const bool there = t.valid(j);
+        off[j] = there ? (int)(t.row(j) - t.base_row) : -1;
+        io[j] = t.h0 + t.head_of(j);
+        half[j] = t.pair_R != 0 && t.pair_half(j);
+        const int k = j < t.RT ? j : 0;
+        vis[j] = t.visible(k);
+        first[j] = t.first(k);
+    }
+};
+
 // ---------------------------------------------------------------------------
 // Un-quantised fp16 / bf16 tail, run by the four waves of one block in units of 32 tokens:
 //   S^T[token, row] = K[token, :] . q[row, :]          A = K as stored, B = q
@@ -329,17 +347,12 @@ __device__ __forceinline__ f16x8 tail_softmax_unit(const f32x4 (&S)[2], float c,
 }
 
 // Partials another block will read in this launch go out as device-scope stores (written
-// through to where every compute die sees them); otherwise plain stores.
-__device__ __forceinline__ void st_partial(float *p, float v, bool device_scope) {
-    if (device_scope) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else *p = v;
-}
-
+// through to where every compute die sees them); where a launch of their own merges them, plain ones would do as well.
+__device__ __forceinline__ void st_partial(float *p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 // two neighbouring floats at an even offset of a record (records start on 8 bytes)
-__device__ __forceinline__ void st_partial2(float *p, float v0, float v1, bool device_scope) {
+__device__ __forceinline__ void st_partial2(float *p, float v0, float v1) {
     const uint64_t u = (uint64_t)__float_as_uint(v0) | ((uint64_t)__float_as_uint(v1) << 32);
-    if (device_scope) __hip_atomic_store(reinterpret_cast<uint64_t *>(p), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else *reinterpret_cast<uint64_t *>(p) = u;
+    __hip_atomic_store(reinterpret_cast<uint64_t *>(p), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Eight consecutive tail elements as fp16.  A bf16 tail is converted: exact for magnitudes in
@@ -380,16 +393,16 @@ __device__ __forceinline__ int new_row_cols(const AttendCall &a, int64_t bh) {
 // block-shared memory and no barrier, so the other waves of the block stream the packed prefix
 // meanwhile.  s_qraw: the query rows of this kv head as fp16, q_stride halves apart.  A wave
 // without units (a sequence with a shorter tail) writes an empty partial (max -inf, sum 0).
-__device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const RowTile &tile, float c, int slot,
+__device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const RowTile &tile, const RowTable &tab, float c, int slot,
                                           int nparts, float *__restrict__ ws, const f16 *s_qraw, int q_stride, int lane,
-                                          int w, int T, bool device_scope, int64_t newest) {
+                                          int w, int T, int64_t newest) {
     const int i = lane & 15, blk = lane >> 4;
     const int R = tile.RT;
     // tail tokens this lane's query row sees; lanes without a row see all of them
     int n_vis = INT_MAX, n_lo = 0;
     const int n_tail = (int)a.n_tail, newest_row = (int)newest;
     if (i < R) {
-        const int64_t vis = tile.visible(i) - a.n_packed, lo = tile.first(i) - a.n_packed;
+        const int64_t vis = tab.vis[i] - a.n_packed, lo = tab.first[i] - a.n_packed;
         n_vis = vis > n_tail ? n_tail : (int)vis;
         n_lo = lo < 0 ? 0 : lo > n_tail ? n_tail : (int)lo;   // first tail token the row sees
     }
@@ -489,17 +502,20 @@ __device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const
     }
     // the partial: accumulator register r of lane (i, blk) is row 4*blk + r, channels 8*i .. 8*i + 7;
     // the maximum of row i sits in lane i of every lane group
+    float *base = ws + (tile.base_row * nparts + slot) * MF_PART;
+    const int64_t step = (int64_t)nparts * MF_PART;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        const int row = 4 * blk + r;
-        if (!tile.valid(row)) continue;
-        float *o = ws + (tile.row(row) * nparts + slot) * MF_PART;
-        if (tile.pair_R == 0 || tile.pair_half(row) == (i >> 3))   // (of a pair's channels only the row's own half is asked for)
+        const int off = tab.off[4 * blk + r];
+        if (off >= 0) {
+            float *o = base + off * step;
+            if (tile.pair_R == 0 || tab.half[4 * blk + r] == (i >> 3))   // (of a pair's channels only the row's own half is asked for)
 #pragma unroll
-            for (int nt = 0; nt < 8; nt += 2) st_partial2(o + 2 + 8 * i + nt, acc.O[nt][r], acc.O[nt + 1][r], device_scope);
-        if (i == 0) st_partial(o + 1, acc.O[8][r], device_scope);
+                for (int nt = 0; nt < 8; nt += 2) st_partial2(o + 2 + 8 * i + nt, acc.O[nt][r], acc.O[nt + 1][r]);
+            if (i == 0) st_partial(o + 1, acc.O[8][r]);
+        }
     }
-    if (blk == 0 && tile.valid(i)) st_partial(ws + (tile.row(i) * nparts + slot) * MF_PART, acc.m_run * LN2, device_scope);
+    if (blk == 0 && tab.off[i] >= 0) st_partial(base + tab.off[i] * step, acc.m_run * LN2);
 }
 
 // Combine the nparts partials of the tile's query rows into the output, in the order in which attend_merge_kernel
@@ -512,7 +528,7 @@ __device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const
 // RTP: rows of a tile at most.  lds: LDS_BYTES, the block's alone by now.
 constexpr int MERGE_MAX_CH = 36;
 template <int DH, int RTP, int WAVES, int LDS_BYTES, int CH>
-__device__ __forceinline__ void merge_rows_ch(const AttendCall &a, const RowTile &tile, int nparts, const float *ws,
+__device__ __forceinline__ void merge_rows_ch(const AttendCall &a, const RowTile &tile, const RowTable &tab, int nparts, const float *ws,
                                               int tid, int wave, uint64_t *lds) {
     constexpr int DD = MF_D * DH, PART = DD + 2;
     constexpr int VAL = DD / 2;                                     // channel pairs of a record
@@ -537,10 +553,12 @@ __device__ __forceinline__ void merge_rows_ch(const AttendCall &a, const RowTile
         float num0 = 0.f, num1 = 0.f, den = 0.f;
         float gm = -INFINITY;   // of the row the wave fetches
         const int j = r0 + my_row;
-        const bool mine = my_row < ROWS && tile.valid(j);
-        const int half = pairs && mine ? tile.pair_half(j) : 0;
-        const bool fetch = fp < PER_ROW && tile.valid(r0 + fr);
-        const uint64_t *row = reinterpret_cast<const uint64_t *>(ws + (fetch ? tile.row(r0 + fr) * nparts * PART : 0));
+        const int my_off = my_row < ROWS ? tab.off[j] : -1;
+        const bool mine = my_off >= 0;
+        const int half = my_row < ROWS ? tab.half[j] : 0;
+        const int f_off = __builtin_amdgcn_readfirstlane(tab.off[r0 + fr]);
+        const bool fetch = fp < PER_ROW && f_off >= 0;
+        const uint64_t *row = reinterpret_cast<const uint64_t *>(ws + (tile.base_row + (fetch ? f_off : 0)) * nparts * PART);
 #pragma unroll 1
         for (int s0 = 0; s0 < nparts; s0 += CH) {
             const int cnt = nparts - s0 < CH ? nparts - s0 : CH;
@@ -600,7 +618,7 @@ __device__ __forceinline__ void merge_rows_ch(const AttendCall &a, const RowTile
         }
         if (mine) {
             const float v0 = den > 0.f ? num0 / den : 0.f, v1 = den > 0.f ? num1 / den : 0.f;
-            const int64_t oi = pairs ? tile.io_row(j) * VAL + 2 * c2 : tile.row(j) * DD + 2 * c2;
+            const int64_t oi = pairs ? (tile.io_base + tab.io[j]) * VAL + 2 * c2 : (tile.base_row + my_off) * DD + 2 * c2;
             if (a.out_dtype == VQ_F16) { ((f16 *)a.out)[oi] = (f16)v0; ((f16 *)a.out)[oi + 1] = (f16)v1; }
             else if (a.out_dtype == VQ_BF16) { ((u16 *)a.out)[oi] = f32_to_bf16(v0); ((u16 *)a.out)[oi + 1] = f32_to_bf16(v1); }
             else { ((float *)a.out)[oi] = v0; ((float *)a.out)[oi + 1] = v1; }
@@ -608,13 +626,13 @@ __device__ __forceinline__ void merge_rows_ch(const AttendCall &a, const RowTile
     }
 }
 template <int DH, int RTP, int WAVES, int LDS_BYTES>
-__device__ __forceinline__ void merge_rows(const AttendCall &a, const RowTile &tile, int nparts, const float *ws,
+__device__ __forceinline__ void merge_rows(const AttendCall &a, const RowTile &tile, const RowTable &tab, int nparts, const float *ws,
                                            int tid, int wave, void *lds) {
     uint64_t *l = reinterpret_cast<uint64_t *>(lds);
     // (the round sizes of merge_records)
-    if (nparts <= 8) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, 8>(a, tile, nparts, ws, tid, wave, l);
-    else if (nparts <= 16) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, 16>(a, tile, nparts, ws, tid, wave, l);
-    else merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_MAX_CH>(a, tile, nparts, ws, tid, wave, l);
+    if (nparts <= 8) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, 8>(a, tile, tab, nparts, ws, tid, wave, l);
+    else if (nparts <= 16) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, 16>(a, tile, tab, nparts, ws, tid, wave, l);
+    else merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_MAX_CH>(a, tile, tab, nparts, ws, tid, wave, l);
 }
 
 // launchers of the packed-prefix kernel (it also runs the fp16 tail and, given sync counters,

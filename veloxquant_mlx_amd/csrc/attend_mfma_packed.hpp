@@ -775,6 +775,8 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
     const int RT = tile.RT;
 
     const bool single_launch = a.sync_counters != nullptr;
+    __shared__ RowTable tab;
+    if (tid < MF_ROWS) tab.fill(tile, tid);
     stage_query<RTP, PK_THREADS, DH>(a, tile, tid, s_qraw);
     if (DH == 1 && sp == 0 && newest >= 0 && tid < 32) {
         // the newest token's key and value rows become the last tail row: 16 pieces of 16 bytes each
@@ -791,8 +793,8 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
     if constexpr (DH == 1) {
         const int tail_waves = nparts - nsplit;
         if (sp == 0 && wave >= PK_WAVES - tail_waves)
-            tail_wave(a, bh, tile, c, nsplit + wave - (PK_WAVES - tail_waves), nparts, ws, s_qraw, PK_QROW, lane,
-                      wave - (PK_WAVES - tail_waves), tail_waves, single_launch, newest);
+            tail_wave(a, bh, tile, tab, c, nsplit + wave - (PK_WAVES - tail_waves), nparts, ws, s_qraw, PK_QROW, lane,
+                      wave - (PK_WAVES - tail_waves), tail_waves, newest);
     }
     // what the unit loop derives from the lane number is formed from here on, not ahead of the tail: the tail
     // needs its 168 registers to itself
@@ -811,10 +813,10 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
     for (int r = 0; r < 4; ++r) acc.nm[r] = (float)(SB::EV - SB::pos(r));
 
     // packed tokens the rows of the tile see: all of them up to full_vis, none from max_vis on
-    int64_t full_vis = tile.visible(0), max_vis = tile.visible(RT - 1);
+    int64_t full_vis = tab.vis[0], max_vis = tab.vis[RT - 1];
     if (full_vis > a.n_packed) full_vis = a.n_packed;
     if (max_vis > a.n_packed) max_vis = a.n_packed;
-    int64_t lane_vis = tile.visible(n % RTP < RT ? n % RTP : 0);
+    int64_t lane_vis = tab.vis[n % RTP];   // (row 0's past the last row)
     if (lane_vis > a.n_packed) lane_vis = a.n_packed;
 
     int64_t t_begin = (int64_t)sp * split_len - tail_equiv;
@@ -827,14 +829,14 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
     const int lane_rel = (int)(lane_vis - t_begin < 0 ? 0 : lane_vis - t_begin > rel_cap ? rel_cap : lane_vis - t_begin);
     const int full_rel = (int)(full_vis - t_begin < 0 ? 0 : full_vis - t_begin > rel_cap ? rel_cap : full_vis - t_begin);
     // sliding window: first token the lane's row sees, and the first token every row sees
-    const int64_t lane_first = tile.first(n % RTP < RT ? n % RTP : 0) - t_begin, edge_first = tile.first(RT - 1) - t_begin;
+    const int64_t lane_first = tab.first[n % RTP] - t_begin, edge_first = tab.first[RT - 1] - t_begin;
     const int lo_rel = (int)(lane_first < 0 ? 0 : lane_first > rel_cap ? rel_cap : lane_first);
     const int edge_rel = (int)(edge_first < 0 ? 0 : edge_first > rel_cap ? rel_cap : edge_first);
     packed_units<BITS, M, GV, RTP, DH>(a, bh, c, t_begin, n_units, lane_rel, full_rel, lo_rel, edge_rel, lane_u, wave, acc, s_qraw, s_const,
                                    s_ring, &s_next, order);
     if (n_units == 0 && single_launch && a.sink_k == nullptr) {
         // a block of the tail alone (split 0 of a short context): its packed partial saw nothing, which the merge reads from its maximum
-        if (tid < RT && tile.valid(tid)) st_partial2(ws + (tile.row(tid) * nparts + sp) * PART, -INFINITY, 0.f, true);
+        if (tid < RT && tab.off[tid] >= 0) st_partial2(ws + ((tile.base_row + tab.off[tid]) * nparts + sp) * PART, -INFINITY, 0.f);
     } else {
         __syncthreads();   // every wave has read its last slot
 
@@ -864,7 +866,8 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
         // a thread takes two neighbouring channels; every LDS read of the waves' sums is issued before the first use
         for (int e = tid; e < RT * (DD / 2); e += PK_THREADS) {
             const int row = e / (DD / 2), d = 2 * (e % (DD / 2)), g = d / (DD / GV);
-            if (!tile.valid(row)) continue;
+            const int off = tab.off[row];
+            if (off < 0) continue;
             float m[PK_WAVES], l[PK_WAVES], z[PK_WAVES];
             float2 o2[PK_WAVES];
 #pragma unroll
@@ -887,9 +890,9 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
                 num1 += seen ? (o2[w].y + z[w]) * f : 0.f;
                 den += seen ? l[w] * f : 0.f;
             }
-            float *o = ws + (tile.row(row) * nparts + sp) * PART;
-            if (DH != 1 || tile.pair_R == 0 || tile.pair_half(row) == d / (DD / 2)) st_partial2(o + 2 + d, num0, num1, single_launch);
-            if (d == 0) st_partial2(o, gm * LN2, den, single_launch);
+            float *o = ws + ((tile.base_row + off) * nparts + sp) * PART;
+            if (DH != 1 || tile.pair_R == 0 || tab.half[row] == d / (DD / 2)) st_partial2(o + 2 + d, num0, num1);
+            if (d == 0) st_partial2(o, gm * LN2, den);
         }
     }
 
@@ -912,7 +915,7 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
         __syncthreads();
         if (s_ticket != nsplit - 1) return;
     }
-    merge_rows<DH, RTP, PK_WAVES, RG::BYTES>(a, tile, nparts, ws, tid, wave, s_ring);
+    merge_rows<DH, RTP, PK_WAVES, RG::BYTES>(a, tile, tab, nparts, ws, tid, wave, s_ring);
     if (nsplit > 1 && tid == 0) __hip_atomic_store(a.sync_counters + by, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
