@@ -132,3 +132,27 @@ def test_units_dealt_over_the_waves_of_one_block(D, Hq, H, bits, g, meta, dtype,
     assert float((got.float() - want).abs().max()) <= eps * float(want.abs().max()) + 1e-3
     free = c.fused_sdpa(q, D ** -0.5)
     assert float((free.float() - want).abs().max()) <= eps * float(want.abs().max()) + 1e-3
+
+
+@pytest.mark.parametrize("Hq,H,bits,g,B,ctx,dtype,meta", [(12, 4, 2, 32, 3, 700, torch.bfloat16, "float16"), (8, 4, 4, 64, 1, 193, torch.float16, "float32"),
+                                                          (10, 1, 3, 128, 2, 1100, torch.float16, "float16")])
+def test_step_of_256_channels_brings_its_token_along(Hq, H, bits, g, B, ctx, dtype, meta):
+    """The newest token's rows read by the tail's launch from where the caller holds them and stored by it, against a cache
+    that stores them first: the same bits, token after token across a flush."""
+    require_gpu()
+    a, new, rand = _cache(256, bits, g, B, H, ctx, dtype, Hq + ctx, meta)
+    b, _, _ = _cache(256, bits, g, B, H, ctx, dtype, Hq + ctx, meta)
+    deferred = 0
+    for step in range(g + 2):
+        k, v = new()
+        for c in (a, b):
+            c.update_and_fetch(k, v)
+        b._store_pending()
+        deferred += a._pending is not None
+        q = rand(B, Hq, 1, 256).to(dtype)
+        kw = dict(fixed_order=True, sliding_window=0 if step % 3 else 150)
+        assert torch.equal(a.fused_sdpa(q, 0.0625, **kw), b.fused_sdpa(q, 0.0625, **kw)), step
+        n = a.offset - a._n_quantized
+        assert a._pending is None
+        assert torch.equal(a._tail_k[:, :, :n], b._tail_k[:, :, :n]) and torch.equal(a._tail_v[:, :, :n], b._tail_v[:, :, :n])
+    assert deferred >= g - 1
