@@ -88,11 +88,13 @@ AttendPlan plan_attend(const AttendCall &a) {
     p.nsplit = (int)ns;
     p.split_len = len;
     // MFMA decode path: the tail is run by up to eight waves of split 0, every wave into a partial of
-    // its own.  A launch with many blocks is bound by throughput: one wave takes eight units of 32
-    // tokens (the other waves stream meanwhile); a launch with few is bound by latency: one unit a wave.
+    // its own.  A launch of many long blocks is bound by throughput: one wave takes eight units of 32
+    // tokens (the other waves stream meanwhile); one of few or short blocks by latency: one unit a wave.  Measured, 8 kv heads of
+    // 128, eight units a wave / one: blocks of 2200 tokens (16 x 4000 at 2 and 4 bits, 8 x 8000) 24.9 / 22.9, 24.6 / 23.4, 23.9 / 22.4
+    // us, of 600 (16 x 1000) 15.1 / 13.2, of 4200 (16 x 8000, 8 x 16000) 31.4 / 33.2, 31.9 / 34.2; the line is drawn between.
     p.nparts = p.nsplit;
     if (p.path == 1 && a.n_tail > 0) {
-        int64_t tw = cdiv(cdiv(a.n_tail, 32), units >= 64 ? 8 : 1);
+        int64_t tw = cdiv(cdiv(a.n_tail, 32), units >= 64 && len > 3072 ? 8 : 1);
         // (a head of 256 channels: the tail launch of the vector kernel, up to four runs of at least 16 tokens)
         const int64_t tr = cdiv(a.n_tail, 16);
         p.nparts += a.D == 128 ? (int)(tw < 1 ? 1 : tw > 8 ? 8 : tw) : (int)(tr > 4 ? 4 : tr);
