@@ -421,7 +421,7 @@ __device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const
     // memory latency: a row's ADDRESS is chosen (the newest token's rows, when the call brings them, are read from where the
     // caller holds them: row `newest` of the tail is being written by this block at the same time), never a
     // loaded value, and a conversion of the whole unit follows the last load (a unit from loads to stored partial: 7.0 us
-    // with a choice between two loads and 64-bit comparisons, 5.0 us now).
+    // with a choice between two loads, 64-bit comparisons and each row worked out again for its stores, 4.0 us now).
     struct TUnit { uint4 kr[2][4], vr[8]; };
     const int64_t new_base = new_row_base(a, bh);
     const int new_cols = new_row_cols(a, bh);
@@ -524,7 +524,7 @@ __device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const
 // once, a wave a record, into `lds`, and summed from there, a thread two neighbouring channels of a row.  The
 // wave that has a row's maxima and sums turns them into factors while the accumulators are on their way (28 records of
 // four rows: 3.7 us where every thread fetched its channel of every record, 4.6; eight records of eight rows 4.3 of 5.5).
-// The whole launch, 32 / 8 heads at 2 bits: 8320 tokens of 128 channels 17.1 -> 15.1 us, 700 of 64 channels 16.4 -> 13.7.
+// The whole launch, 32 / 8 heads at 2 bits: 8320 tokens of 128 channels 17.1 -> 14.5 us, 700 of 64 channels 16.4 -> 12.9.
 // RTP: rows of a tile at most.  lds: LDS_BYTES, the block's alone by now.
 constexpr int MERGE_MAX_CH = 36;
 template <int DH, int RTP, int WAVES, int LDS_BYTES, int CH>
