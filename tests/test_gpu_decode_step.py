@@ -115,7 +115,7 @@ def test_units_dealt_over_the_waves_of_one_block(D, Hq, H, bits, g, meta, dtype,
     """One block a kv head (num_splits=1) over numbers of 32-token units around one chunk a wave, where they are dealt out
     evenly, and beyond, where waves draw chunks: against the general kernel, which sums token by token in float32.  Output
     rounding is 2^-11 (fp16) or 2^-8 (bf16) of values of order one, the products' remainder terms 2^-21; the
-    three-step call of a cache is the same bits as the general wrapper's."""
+    cache's own call is the same bits as the general wrapper's."""
     require_gpu()
     ctx = 128 + -(-32 * units // g) * g
     c, new, rand = _cache(D, bits, g, 2, H, ctx, dtype, units, meta)
