@@ -409,7 +409,8 @@ int vq_kivi_prefill_tiles(const vq_attend_args *a, int64_t first_unit, int64_t n
 int vq_kivi_attend_fixed_order(int enable);
 
 /* Bytes of scratch vq_kivi_attend needs for these shapes (fields other than the shapes, pack_bits,
- * group, num_splits, sliding_window and sink_k are ignored).  0 for a launch that writes its output
+ * group, num_splits, sliding_window, sink_k and whether packed_lens is given are ignored; for a call with
+ * vq_attend_ext: vq_kivi_attend_workspace_ext).  0 for a launch that writes its output
  * itself (a prefill whose row tiles fill the GPU, one run per row, no protected rows): workspace may
  * then be NULL.  A call with several query positions (fewer than 256 rows a kv head) and a GQA group of 3, 5, 6 or 7 heads runs as
  * the next group size the matrix-unit kernels tile (4 or 8: every group filled up with heads of
@@ -449,6 +450,9 @@ typedef struct vq_attend_ext {
      * end of those).  k_new / v_new go to row n_tail - 1 of every sequence's tail, live or not. */
     const int64_t *seq_lens;
 } vq_attend_ext;
+/* Bytes of scratch vq_kivi_attend_ext needs (x may be NULL).  vq_kivi_attend_workspace(a) may answer with less: a batch
+ * with lengths of its own is not cut at the sliding window and takes other kernels over plain rows. */
+size_t vq_kivi_attend_workspace_ext(const vq_attend_args *a, const vq_attend_ext *x);
 int vq_kivi_attend_ext(const vq_attend_args *a, const vq_attend_ext *x);
 
 /* vq_kivi_attend for callers that cannot allocate device memory (code under HIP graph capture,

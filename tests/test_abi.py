@@ -77,3 +77,36 @@ def test_packed_argument_block_is_the_structure():
     values = [0.5 if t is _lib.f32 else i + 1 for i, (_, t) in enumerate(_lib.AttendArgs._fields_)]
     a = _lib.AttendArgs.from_buffer_copy(_lib.ATTEND_PACK.pack(*values))
     assert [getattr(a, n) for n, _ in _lib.AttendArgs._fields_] == values
+
+
+@pytest.mark.parametrize("lens", [None, "seq_lens", "packed_lens"])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,D,n_packed,n_tail,window,pairs", [
+    (1, 64, 8, 1, 128, 32768, 128, 1024, 0), (2, 64, 8, 1, 128, 32768, 128, 4096, 0),      # a window far below the context
+    (7, 12, 4, 1, 256, 20000, 140, 1024, 0), (8, 40, 10, 1, 128, 8192, 130, 512, 0),
+    (2, 32, 8, 4, 128, 8192, 128, 1024, 0), (2, 12, 4, 4, 128, 8192, 128, 1024, 0),        # several positions; groups filled up
+    (2, 14, 2, 16, 64, 4096, 7, 100, 0), (3, 40, 2, 32, 128, 4096, 50, 64, 0),             # vector kernel; groups of more than eight
+    (16, 32, 8, 128, 128, 0, 128, 0, 0), (2, 32, 32, 700, 128, 0, 700, 99, 0),             # a right-padded prompt over plain rows
+    (3, 32, 4, 1, 128, 8192, 33, 200, 8), (2, 12, 2, 1, 128, 2048, 64, 0, 3)])             # heads of 64 channels in pairs
+def test_workspace_query_covers_the_call_that_runs(B, Hq, Hkv, Sq, D, n_packed, n_tail, window, pairs, lens):
+    """What the query answers is what the call asks for, with lengths a sequence and without (the call is refused for want of
+    any workspace, before a launch)."""
+    lib = _lib.load()
+    a = _lib.AttendArgs()
+    a.B, a.Hq, a.Hkv, a.Sq, a.D, a.n_packed, a.n_tail, a.sliding_window = B, Hq, Hkv, Sq, D, n_packed, n_tail, window
+    a.pack_bits, a.group, a.meta_dtype, a.v_layout, a.cap_tokens, a.tail_cap = 4, 32, 0, 1, 32768, 768
+    a.q_dtype = a.out_dtype = a.tail_dtype = 0
+    a.scale, a.causal = 0.1, int(Sq > 1)
+    for f in ("q", "out", "sync_counters") + (("k_packed", "k_scale", "k_zero", "v_packed", "v_scale", "v_zero") if n_packed else ()):
+        setattr(a, f, 4096)
+    a.k_tail = a.v_tail = 4096
+    if lens == "packed_lens":
+        a.packed_lens = a.tail_lens = 4096
+    x = _lib.AttendExt(pairs, 4096 if lens == "seq_lens" else None) if pairs or lens == "seq_lens" else None
+    need = lib.vq_kivi_attend_workspace_ext(a, x)
+    assert need == lib.attend_packed_workspace(bytes(a), None if x is None else bytes(x))
+    if x is None:
+        assert need == lib.vq_kivi_attend_workspace(a)
+    if need == 0:
+        return   # the launch writes its output itself: nothing refuses the call
+    assert lib.vq_kivi_attend_ext(a, x) == _lib.VQ_ERR_WORKSPACE
+    assert int(re.search(r"workspace of (\d+) bytes required", _lib.last_error()).group(1)) == need

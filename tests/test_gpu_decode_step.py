@@ -89,6 +89,39 @@ def test_lengths_of_a_batch_in_the_launch(D, Hq, H, bits, dtype):
     got = c.fused_sdpa(q, scale, lengths=some, fixed_order=True)
     alone = [c.fused_sdpa(q, scale, lengths=torch.full((B,), int(n), device="cuda"), fixed_order=True)[i] for i, n in enumerate(some)]
     assert torch.equal(got, torch.stack(alone))
+    want = _clamped_lists(c, pad_queries_for_paired_heads(q, H) if pairs else q, some, scale)
+    assert torch.equal(got, own_half_of_paired_output(want, H) if pairs else want)
+
+
+def _clamped_lists(c, q, lens, scale, window=0):
+    """The call with two clamped lists of lengths in place of one length a sequence."""
+    nq, n_tail = c._n_quantized, c.offset - c._n_quantized
+    kw = dict(k_packed=c._kp, k_scale=c._ks, k_zero=c._kz, v_packed=c._vp, v_scale=c._vs, v_zero=c._vz, n_packed=nq, bits=c._field,
+              group_size=c._group_size, v_layout=c._v_layout) if nq else {}
+    return K.kivi_packed_attend(q, k_tail=c._tail_k, v_tail=c._tail_v, n_tail=n_tail, scale=scale, causal=q.shape[2] > 1,
+                                out_dtype=q.dtype, fixed_order=True, sliding_window=window, tiles=False,
+                                packed_lens=torch.clamp(lens, max=nq), tail_lens=torch.clamp(lens - nq, min=0, max=n_tail), **kw)
+
+
+@pytest.mark.parametrize("B,Hq,H,D,Sq,window,ctx,dtype", [
+    (2, 64, 8, 128, 1, 1024, 16400, torch.float16), (7, 12, 4, 256, 1, 1024, 9000, torch.bfloat16), (2, 32, 8, 128, 4, 1024, 8200, torch.float16),
+    (3, 12, 4, 128, 5, 300, 4100, torch.float16), (16, 32, 8, 128, 64, 0, 128, torch.float16), (5, 8, 2, 128, 40, 30, 100, torch.bfloat16)])
+def test_lengths_and_a_window_from_an_empty_workspace(B, Hq, H, D, Sq, window, ctx, dtype):
+    """Lengths a sequence beside a window, and a right-padded prompt over plain rows: the call finds the scratch of the launch that
+    runs with no workspace left from earlier calls, and gives the bits of the two clamped lists."""
+    require_gpu()
+    c, new, rand = _cache(D, 4, 32, B, H, ctx, dtype, ctx + Sq)
+    q, scale = rand(B, Hq, Sq, D).to(dtype), D ** -0.5
+    lens = torch.tensor([max(Sq, c.offset - 37 * i) for i in range(B)], device="cuda")
+    K._workspaces.clear()
+    got = c.fused_sdpa(q, scale, lengths=lens, sliding_window=window, fixed_order=True)
+    assert torch.equal(got, _clamped_lists(c, q, lens, scale, window))
+    k, v = new()
+    c.update_and_fetch(k, v)   # a step on top, its token brought along where that is done
+    q, lens = rand(B, Hq, 1, D).to(dtype), lens + 1
+    K._workspaces.clear()
+    got = c.fused_sdpa(q, scale, lengths=lens, sliding_window=window, fixed_order=True)
+    assert torch.equal(got, _clamped_lists(c, q, lens, scale, window))
 
 
 def test_pair_heads_refusals():

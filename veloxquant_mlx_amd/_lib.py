@@ -145,6 +145,7 @@ _SIGNATURES = {
     "vq_kivi_attend_workspace": (sz, [C.POINTER(AttendArgs)]),
     "vq_kivi_attend_plan": (i32, [C.POINTER(AttendArgs), C.POINTER(i32), C.POINTER(i32)]),
     "vq_kivi_attend": (i32, [C.POINTER(AttendArgs)]),
+    "vq_kivi_attend_workspace_ext": (sz, [C.POINTER(AttendArgs), C.POINTER(AttendExt)]),
     "vq_kivi_attend_ext": (i32, [C.POINTER(AttendArgs), C.POINTER(AttendExt)]),
     "vq_kivi_attend_static": (i32, [C.POINTER(AttendArgs)]),
     "vq_kivi_prefill_tiles": (i32, [C.POINTER(AttendArgs), i64, i64]),
@@ -172,8 +173,9 @@ def load():
                 fn = getattr(lib, name)
                 fn.restype = res
                 fn.argtypes = args
-            # the same entry point over a packed argument block (ATTEND_PACK), and its extension or None
+            # the same entry points over a packed argument block (ATTEND_PACK), and its extension or None
             lib.attend_packed = C.CFUNCTYPE(i32, C.c_char_p, C.c_char_p)(("vq_kivi_attend_ext", lib))
+            lib.attend_packed_workspace = C.CFUNCTYPE(sz, C.c_char_p, C.c_char_p)(("vq_kivi_attend_workspace_ext", lib))
             _lib = lib
             return _lib
         except (OSError, AttributeError) as e:  # missing file or symbol

@@ -258,9 +258,11 @@ static size_t attend_workspace(const AttendCall *a) {
     return (size_t)(a->B * a->Hq * a->Sq) * (size_t)p.nparts * (size_t)(a->D + 2) * sizeof(float);
 }
 
-extern "C" size_t vq_kivi_attend_workspace(const vq_attend_args *a) {
+extern "C" size_t vq_kivi_attend_workspace(const vq_attend_args *a) { return vq_kivi_attend_workspace_ext(a, nullptr); }
+
+extern "C" size_t vq_kivi_attend_workspace_ext(const vq_attend_args *a, const vq_attend_ext *x) {
     if (a == nullptr) return 0;
-    const AttendCall call(*a);
+    const AttendCall call(*a, x);
     return attend_workspace(&call);
 }
 

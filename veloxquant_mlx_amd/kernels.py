@@ -1227,14 +1227,12 @@ def kivi_packed_attend(q: torch.Tensor, *, k_packed=None, k_scale=None, k_zero=N
     if static_scratch:
         _lib.check(lib.vq_kivi_attend_static(a))
         return out
-    need = lib.vq_kivi_attend_workspace(a)
+    ext = _lib.AttendExt(pair_heads, None if seq_lens is None else seq_lens.data_ptr()) if pair_heads or seq_lens is not None else None
+    need = lib.vq_kivi_attend_workspace_ext(a, ext)   # of the call that runs: lengths change its plan
     ws = _workspace(q.device, need)
     a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
     a.sync_counters = _counters(q.device).data_ptr() if _single_launch else None
-    if pair_heads or seq_lens is not None:
-        _lib.check(lib.vq_kivi_attend_ext(a, _lib.AttendExt(pair_heads, None if seq_lens is None else seq_lens.data_ptr())))
-    else:
-        _lib.check(lib.vq_kivi_attend(a))
+    _lib.check(lib.vq_kivi_attend_ext(a, ext))
     return out
 
 
@@ -1298,7 +1296,7 @@ def kivi_decode_attend(q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero, 
             return out
         if rc != _lib.VQ_ERR_WORKSPACE:
             break
-        ws = _workspace(device, lib.vq_kivi_attend_workspace(AttendArgs.from_buffer_copy(args)), stream)
+        ws = _workspace(device, lib.attend_packed_workspace(args, ext), stream)
     if rc != _lib.VQ_ERR_INVALID and rc != _lib.VQ_ERR_UNSUPPORTED:
         _lib.check(rc)
     return None
