@@ -167,25 +167,23 @@ def test_units_dealt_over_the_waves_of_one_block(D, Hq, H, bits, g, meta, dtype,
     assert float((free.float() - want).abs().max()) <= eps * float(want.abs().max()) + 1e-3
 
 
-@pytest.mark.parametrize("Hq,H,bits,g,B,ctx,dtype,meta", [(12, 4, 2, 32, 3, 700, torch.bfloat16, "float16"), (8, 4, 4, 64, 1, 193, torch.float16, "float32"),
-                                                          (10, 1, 3, 128, 2, 1100, torch.float16, "float16")])
-def test_step_of_256_channels_brings_its_token_along(Hq, H, bits, g, B, ctx, dtype, meta):
-    """The newest token's rows read by the tail's launch from where the caller holds them and stored by it, against a cache
-    that stores them first: the same bits, token after token across a flush."""
+@pytest.mark.parametrize("D,Hq,H,bits,g,B,ctx,dtype,meta", [
+    (256, 12, 4, 2, 32, 3, 700, torch.bfloat16, "float16"), (256, 8, 4, 4, 64, 1, 193, torch.float16, "float32"),
+    (256, 10, 1, 3, 128, 2, 1100, torch.float16, "float16")])
+def test_step_takes_its_token_at_once(D, Hq, H, bits, g, B, ctx, dtype, meta):
+    """A caller that writes its key and value buffers again between a step's update and its attention: the same bits as with
+    tensors of its own a step, token after token across a flush."""
     require_gpu()
-    a, new, rand = _cache(256, bits, g, B, H, ctx, dtype, Hq + ctx, meta)
-    b, _, _ = _cache(256, bits, g, B, H, ctx, dtype, Hq + ctx, meta)
-    deferred = 0
+    a, new, rand = _cache(D, bits, g, B, H, ctx, dtype, Hq + ctx, meta)
+    b, _, _ = _cache(D, bits, g, B, H, ctx, dtype, Hq + ctx, meta)
+    kbuf, vbuf = (torch.empty(B, H, 1, D, dtype=dtype, device="cuda") for _ in range(2))
     for step in range(g + 2):
         k, v = new()
-        for c in (a, b):
-            c.update_and_fetch(k, v)
-        b._store_pending()
-        deferred += a._pending is not None
-        q = rand(B, Hq, 1, 256).to(dtype)
+        b.update_and_fetch(k, v)
+        a.update_and_fetch(kbuf.copy_(k), vbuf.copy_(v))
+        kbuf.fill_(55.0), vbuf.fill_(-77.0)
+        q = rand(B, Hq, 1, D).to(dtype)
         kw = dict(fixed_order=True, sliding_window=0 if step % 3 else 150)
-        assert torch.equal(a.fused_sdpa(q, 0.0625, **kw), b.fused_sdpa(q, 0.0625, **kw)), step
+        assert torch.equal(a.fused_sdpa(q, D ** -0.5, **kw), b.fused_sdpa(q, D ** -0.5, **kw)), step
         n = a.offset - a._n_quantized
-        assert a._pending is None
         assert torch.equal(a._tail_k[:, :, :n], b._tail_k[:, :, :n]) and torch.equal(a._tail_v[:, :, :n], b._tail_v[:, :, :n])
-    assert deferred >= g - 1

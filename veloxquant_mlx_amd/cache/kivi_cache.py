@@ -312,8 +312,7 @@ class KIVIKVCache(FP16KVCache):
         self._store_pending()
         n_tail, dtype = self.offset - self._n_quantized, keys.dtype
         if not (n_tail < self._tail_k.shape[2] and keys.shape == values.shape and dtype == self._tail_k.dtype
-                and values.dtype == dtype
-                and (keys.shape[3] == 128 or self._pair or (keys.shape[3] == 256 and self._pairs_attend_direct()))
+                and values.dtype == dtype and (keys.shape[3] == 128 or self._pair)
                 and keys.is_contiguous() and values.is_contiguous() and keys.data_ptr() % 16 == 0
                 and values.data_ptr() % 16 == 0
                 and (max(0, self.offset + 1 - self._residual_length) // self._group_size) * self._group_size
@@ -441,8 +440,7 @@ class KIVIKVCache(FP16KVCache):
                             num_splits=num_splits)
 
     def _pairs_attend_direct(self) -> bool:
-        """Whether a decode step over kv heads kept in pairs, or of 256 channels, takes the matrix-unit decode launch (its gate on the
-        cache's side)."""
+        """Whether a decode step over kv heads kept in pairs takes the matrix-unit decode launch (its gate on the cache's side)."""
         return (self._n_quantized > 0 and self._field in (2, 4) and self._group_size >= 32 and self._v_layout == "token"
                 and (self._tail_k is None or self._tail_k.dtype in (torch.float16, torch.bfloat16)))
 

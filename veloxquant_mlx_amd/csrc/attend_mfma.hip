@@ -21,12 +21,9 @@ int mfma_row_tiles(const AttendCall &a) {
 
 bool mfma_decode_supported(const AttendCall &a) {
     if ((a.D != MF_D && a.D != 2 * MF_D) || a.n_packed <= 0) return false;
-    // A head of 256 channels: packed prefix only, its tail goes through the vector kernel, one more launch, which also
-    // stores a token brought along by the call where it reads whole 16-byte pieces of 16-bit rows.
-    if (a.D == 2 * MF_D && !rows_kernel_supported(a)) return false;
-    if (a.D == 2 * MF_D && a.k_new != nullptr &&
-        (!(a.tail_dtype == VQ_F16 || a.tail_dtype == VQ_BF16) || (((uintptr_t)a.k_tail | (uintptr_t)a.v_tail) & 15u)))
-        return false;
+    // a head of 256 channels: packed prefix only (its tail goes through the vector kernel, one more launch), no
+    // token brought along by the call
+    if (a.D == 2 * MF_D && (a.k_new != nullptr || !rows_kernel_supported(a))) return false;
     if (a.Hq % a.Hkv != 0) return false;
     const int64_t R = a.Hq / a.Hkv;
     // a tile has eight rows (a high and a remainder column each): the whole group at one position, a

@@ -85,11 +85,7 @@ __global__ __launch_bounds__(256) void attend_rows_kernel(AttendCall a, int64_t 
     // (32-bit divisions: the tail's launch is a few microseconds of latency, and a 64-bit division a hundred instructions of it)
     const int bh32 = tiles == 1 ? by : by / tiles, b32 = bh32 / (int)a.Hkv;
     const int64_t bh = bh32, hkv = bh32 - b32 * (int)a.Hkv, b = b32;
-    const int64_t n_tail_all = a.n_tail;
     take_sequence_lengths(a, b);
-    // a launch over the tail alone may bring the newest token's rows along (k_new): the last tail row of the whole batch under
-    // seq_lens, of the sequence's own under tail_lens; read from where the caller holds them, stored by one block of the head
-    const int64_t newest = part0 < 0 || a.k_new == nullptr ? -1 : (a.seq_lens != nullptr ? n_tail_all : a.n_tail) - 1;
     const int D = (int)a.D, g = a.k_packed != nullptr && a.group >= 1 ? (int)a.group : (1 << 30);   // plain rows: one group
     const int W = (D + PER - 1) / PER, WL = (D + CPL - 1) / CPL;   // words, lanes of a token row
     int lpt = 4;
@@ -291,17 +287,14 @@ __global__ __launch_bounds__(256) void attend_rows_kernel(AttendCall a, int64_t 
                 const u16 *kt = (const u16 *)a.k_tail, *vt = (const u16 *)a.v_tail;
                 for (int64_t t = q0 + gslot; t < t1; t += 2 * nslots) {
                     const bool two = t + nslots < t1;   // the same for the lanes of a slot
-                    const int64_t row = t - a.n_packed, ti = (bh * a.tail_cap + row) * D + d0;
-                    const u16 *ka = kt + ti, *va = vt + ti, *kb2 = ka + (int64_t)nslots * D, *vb2 = va + (int64_t)nslots * D;
-                    if (row == newest) { ka = (const u16 *)a.k_new + bh * D + d0; va = (const u16 *)a.v_new + bh * D + d0; }
-                    if (row + nslots == newest) { kb2 = (const u16 *)a.k_new + bh * D + d0; vb2 = (const u16 *)a.v_new + bh * D + d0; }
+                    const int64_t ti = (bh * a.tail_cap + (t - a.n_packed)) * D + d0;
                     uint4 k0 = make_uint4(0, 0, 0, 0), v0 = k0, k1 = k0, v1 = k0;
                     if (live) {
-                        k0 = *reinterpret_cast<const uint4 *>(ka);
-                        v0 = *reinterpret_cast<const uint4 *>(va);
+                        k0 = *reinterpret_cast<const uint4 *>(kt + ti);
+                        v0 = *reinterpret_cast<const uint4 *>(vt + ti);
                         if (two) {
-                            k1 = *reinterpret_cast<const uint4 *>(kb2);
-                            v1 = *reinterpret_cast<const uint4 *>(vb2);
+                            k1 = *reinterpret_cast<const uint4 *>(kt + ti + (int64_t)nslots * D);
+                            v1 = *reinterpret_cast<const uint4 *>(vt + ti + (int64_t)nslots * D);
                         }
                     }
                     float kc[8], vc[8];
@@ -328,12 +321,6 @@ __global__ __launch_bounds__(256) void attend_rows_kernel(AttendCall a, int64_t 
                 token(t, kc, vc, 1.f, 0.f, 1.f, 0.f);
             }
         }
-    }
-
-    if (newest >= 0 && sp == 0 && t_in_bh == 0 && tid < D / 4) {   // D / 8 pieces of 16 bytes each of keys and values
-        const int piece = tid < D / 8 ? tid : tid - D / 8;
-        const uint4 x = reinterpret_cast<const uint4 *>(tid < D / 8 ? a.k_new : a.v_new)[bh * (D / 8) + piece];
-        reinterpret_cast<uint4 *>(const_cast<void *>(tid < D / 8 ? a.k_tail : a.v_tail))[(bh * a.tail_cap + newest) * (D / 8) + piece] = x;
     }
 
     // ---- zero points in, then the slots of the wave, then the waves of the block
