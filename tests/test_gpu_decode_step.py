@@ -105,14 +105,14 @@ def _clamped_lists(c, q, lens, scale, window=0):
 
 @pytest.mark.parametrize("B,Hq,H,D,Sq,window,ctx,dtype", [
     (2, 64, 8, 128, 1, 1024, 16400, torch.float16), (7, 12, 4, 256, 1, 1024, 9000, torch.bfloat16), (2, 32, 8, 128, 4, 1024, 8200, torch.float16),
-    (3, 12, 4, 128, 5, 300, 4100, torch.float16), (16, 32, 8, 128, 64, 0, 128, torch.float16), (5, 8, 2, 128, 40, 30, 100, torch.bfloat16)])
+    (3, 12, 4, 128, 5, 300, 4100, torch.float16), (32, 32, 8, 128, 64, 0, 128, torch.float16), (5, 8, 2, 128, 40, 30, 100, torch.bfloat16)])
 def test_lengths_and_a_window_from_an_empty_workspace(B, Hq, H, D, Sq, window, ctx, dtype):
     """Lengths a sequence beside a window, and a right-padded prompt over plain rows: the call finds the scratch of the launch that
     runs with no workspace left from earlier calls, and gives the bits of the two clamped lists."""
     require_gpu()
     c, new, rand = _cache(D, 4, 32, B, H, ctx, dtype, ctx + Sq)
     q, scale = rand(B, Hq, Sq, D).to(dtype), D ** -0.5
-    lens = torch.tensor([max(Sq, c.offset - 37 * i) for i in range(B)], device="cuda")
+    lens = torch.tensor([max(Sq, c.offset - 37 * (i % 4)) for i in range(B)], device="cuda")
     K._workspaces.clear()
     got = c.fused_sdpa(q, scale, lengths=lens, sliding_window=window, fixed_order=True)
     assert torch.equal(got, _clamped_lists(c, q, lens, scale, window))
@@ -169,7 +169,8 @@ def test_units_dealt_over_the_waves_of_one_block(D, Hq, H, bits, g, meta, dtype,
 
 @pytest.mark.parametrize("D,Hq,H,bits,g,B,ctx,dtype,meta", [
     (256, 12, 4, 2, 32, 3, 700, torch.bfloat16, "float16"), (256, 8, 4, 4, 64, 1, 193, torch.float16, "float32"),
-    (256, 10, 1, 3, 128, 2, 1100, torch.float16, "float16")])
+    (256, 10, 1, 3, 128, 2, 1100, torch.float16, "float16"), (64, 9, 3, 2, 32, 3, 700, torch.bfloat16, "float16"),
+    (64, 10, 5, 4, 64, 1, 193, torch.float16, "float32")])
 def test_step_takes_its_token_at_once(D, Hq, H, bits, g, B, ctx, dtype, meta):
     """A caller that writes its key and value buffers again between a step's update and its attention: the same bits as with
     tensors of its own a step, token after token across a flush."""

@@ -255,7 +255,11 @@ class KIVIKVCache(FP16KVCache):
     def update_and_fetch(self, keys: torch.Tensor, values: torch.Tensor):
         """Append ``[B,H,S,D]`` keys/values and quantise whatever aged out of the
         fp16 residual window, in ``kivi_group_size``-aligned blocks
-        (kivi_cache.py:230-262)."""
+        (kivi_cache.py:230-262).
+
+        Memory-bound mode: of a single token of heads of 128 channels, or of an even number of heads of 64, the cache may hold
+        ``keys`` and ``values`` themselves until the next call on it (the attention call of the step stores them in its own
+        launch); a caller that writes those buffers again before then passes clones."""
         B, H, S, D = keys.shape
         if self._memory_bound:
             if self.offset == 0 and self._n_quantized == 0:
@@ -305,8 +309,8 @@ class KIVIKVCache(FP16KVCache):
 
     def _defer_token(self, keys: torch.Tensor, values: torch.Tensor) -> bool:
         """A plain decode step with no flush due: the attention launch of this step stores the token (kv heads kept in pairs: the
-        caller's own rows of 64 channels).  Until then the cache holds the caller's tensors, not a copy: a caller that
-        reuses its key / value buffers between update_and_fetch and fused_sdpa must pass clones."""
+        caller's own rows of 64 channels).  Until then the cache holds the caller's tensors, not a copy (see update_and_fetch); of an odd
+        number of heads a copy, as the rows beside zeros that are stored otherwise would be."""
         if keys.shape[2] != 1 or self._n_quantized == 0 or self._tail_k is None:
             return False
         self._store_pending()
@@ -319,6 +323,8 @@ class KIVIKVCache(FP16KVCache):
                 == self._n_quantized):
             return False
         self._drop_tiles()   # decoding has begun: the prefill scratch goes back
+        if self._pair and keys.shape[1] % 2:   # (one launch for both copies)
+            keys, values = torch.stack((keys, values)).unbind()
         self._pending = (keys, values)
         self.offset += 1
         B, H, D = self._shape_bhd
