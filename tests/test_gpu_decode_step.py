@@ -8,7 +8,7 @@ import torch
 
 from tests._gpu import gpu, require_gpu
 from veloxquant_mlx_amd import kernels as K
-from veloxquant_mlx_amd.cache import KVCacheConfig, KVCacheFactory
+from veloxquant_mlx_amd.cache import KVCacheConfig, KVCacheFactory, LayerStackedKIVICache
 from veloxquant_mlx_amd.cache.kivi_cache import own_half_of_paired_output, pad_queries_for_paired_heads
 
 pytestmark = gpu
@@ -188,3 +188,39 @@ def test_step_takes_its_token_at_once(D, Hq, H, bits, g, B, ctx, dtype, meta):
         assert torch.equal(a.fused_sdpa(q, D ** -0.5, **kw), b.fused_sdpa(q, D ** -0.5, **kw)), step
         n = a.offset - a._n_quantized
         assert torch.equal(a._tail_k[:, :, :n], b._tail_k[:, :, :n]) and torch.equal(a._tail_v[:, :, :n], b._tail_v[:, :, :n])
+
+
+@pytest.mark.parametrize("how", ["attend", "general", "trim", "stack"])
+def test_attention_on_another_stream_keeps_the_tokens_memory(how, monkeypatch):
+    """A token handed over on one stream and read by a launch on another: its memory is held for that stream; on the same
+    stream nothing is recorded."""
+    require_gpu()
+    held = []
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda t, s: held.append((t.data_ptr(), s.cuda_stream)))
+    H, D, ctx = 4, 128, 400
+    if how == "stack":
+        cfg = KVCacheConfig(method="kivi", head_dim=D, bit_width_inlier=4, kivi_group_size=32, fused_sdpa=True, fused_sdpa_memory_bound=True)
+        c = LayerStackedKIVICache(cfg, 2)
+        layers = c.layers
+        for l in layers:
+            l.update_and_fetch(*(torch.randn(1, H, ctx, D, device="cuda").half() for _ in range(2)))
+        c.fused_sdpa_all(torch.randn(2, 1, 8, 1, D, device="cuda").half(), 0.1)
+    else:
+        c, _, _ = _cache(D, 4, 32, 1, H, ctx, torch.float16, 1)
+        layers = [c]
+    use = {"attend": lambda: c.fused_sdpa(torch.randn(1, 8, 1, D, device="cuda").half(), 0.1),
+           "general": lambda: c.fused_sdpa(torch.randn(1, 8, 2, D, device="cuda").half(), 0.1),
+           "trim": lambda: c.trim(0), "stack": lambda: c.fused_sdpa_all(torch.randn(2, 1, 8, 1, D, device="cuda").half(), 0.1)}[how]
+    other = torch.cuda.Stream()
+    for stream in (torch.cuda.current_stream(), other):
+        tokens = [[torch.randn(1, H, 1, D, device="cuda").half() for _ in range(2)] for _ in layers]
+        for l, (k, v) in zip(layers, tokens):
+            l.update_and_fetch(k, v)
+            assert l._pending is not None
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            use()
+        assert all(l._pending is None for l in layers)
+        want = [(t.data_ptr(), other.cuda_stream) for kv in tokens for t in kv] if stream is other else []
+        assert sorted(held) == sorted(want)
+        torch.cuda.synchronize()

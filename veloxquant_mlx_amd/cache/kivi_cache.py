@@ -176,6 +176,7 @@ class KIVIKVCache(FP16KVCache):
         # memory-bound decode: the newest token's (keys, values), counted in ``offset`` but not yet in the
         # tail; the next fused_sdpa stores them in the same launch that attends, anything else stores them first
         self._pending = None
+        self._pending_stream = 0   # the stream it was handed over on
         self._zero_scalar = None
         # memory-bound prefill: the slots once more as ready-made fp16 tiles for prefill-sized attention calls
         # (scratch of the prefill phase, given back at the first decode step); the first _tiles_packed units
@@ -302,10 +303,19 @@ class KIVIKVCache(FP16KVCache):
         """Write a deferred newest token into the tail (see ``_pending``)."""
         if self._pending is not None:
             k, v = self._pending
-            self._pending = None
             if self._pair:
                 k, v = pair_heads(k), pair_heads(v)
             K.kv_tail_append(k, v, self._tail_k, self._tail_v, self.offset - self._n_quantized - 1)
+            self._release_pending()
+
+    def _release_pending(self) -> None:
+        """The launch that reads the deferred token is enqueued: let go of it.  On another stream than it was handed over on,
+        its memory must not be given out again before that launch has run."""
+        pending, self._pending = self._pending, None
+        device = pending[0].device
+        if K._stream_of(device) != self._pending_stream:
+            for t in pending:
+                t.record_stream(torch.cuda.current_stream(device))
 
     def _defer_token(self, keys: torch.Tensor, values: torch.Tensor) -> bool:
         """A plain decode step with no flush due: the attention launch of this step stores the token (kv heads kept in pairs: the
@@ -326,6 +336,7 @@ class KIVIKVCache(FP16KVCache):
         if self._pair and keys.shape[1] % 2:   # (one launch for both copies)
             keys, values = torch.stack((keys, values)).unbind()
         self._pending = (keys, values)
+        self._pending_stream = K._stream_of(keys.device)
         self.offset += 1
         B, H, D = self._shape_bhd
         self._account_bytes(B, H, 1, D, 0)
@@ -472,7 +483,8 @@ class KIVIKVCache(FP16KVCache):
                                        self._v_layout, self._tail_k, self._tail_v, n_tail, float(scale), max(0, int(num_splits)),
                                        fixed_order, int(sliding_window or 0), k_new, v_new, pair_heads, lengths)
             if out is not None:
-                self._pending = None
+                if k_new is not None:
+                    self._release_pending()
                 return out
         if self._memory_bound:
             tk, tv = self._tail_k, self._tail_v
@@ -494,7 +506,7 @@ class KIVIKVCache(FP16KVCache):
         if self._pending is not None:
             try:   # append and attend in one launch (single-query MFMA decode path)
                 out = K.kivi_packed_attend(q, k_new=self._pending[0], v_new=self._pending[1], **kw)
-                self._pending = None
+                self._release_pending()
                 return out
             except ValueError:   # a shape that path does not take: store the token, then attend
                 self._store_pending()

@@ -258,7 +258,7 @@ class LayerStackedKIVICache:
             try:
                 out = K.kivi_packed_attend(qf, k_new=k_new, v_new=v_new, **kw)
                 for c in self.layers:
-                    c._pending = None
+                    c._release_pending()
                 return out.view((NL, B) + tuple(out.shape[1:]))
             except ValueError:   # a shape the append-and-attend launch does not take
                 for c in self.layers:
