@@ -646,3 +646,25 @@ def test_step_indices_go_into_the_store(B, H, S, D, kn, ks, vn, vs, dtype, rows)
     # what does not fit the store is refused by the library before any launch
     assert not K.vecinfer_encode_step(keys, values, kcb, ks, vcb, vs, Hm, smooth, ks_store, vs_store, cap - S + 1)
     assert torch.equal(ks_store, want_k) and torch.equal(vs_store, want_v)
+
+
+def test_factors_of_another_width_are_refused():
+    """Smoothing factors whose rows are not as wide as a head: not taken by the step's launch, refused by the cache at the update
+    and by the fused encode, and nothing stored."""
+    require_gpu()
+    r = lambda *s: torch.randn(s, device="cuda")
+    B, H, D = 1, 4, 128
+    keys, values, kcb, vcb = r(B, H, 1, D).half(), r(B, H, 1, D).half(), r(256, 8), r(256, 8)
+    Hm = walsh_hadamard_matrix(D, device="cuda")
+    stores = [torch.full((B, H, 4, D // 8), 77, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    for smooth in (r(64).exp(), r(H, 64).exp(), r(1, 96).exp(), r(1, 1, D).exp(), torch.ones((), device="cuda")):
+        assert not K.vecinfer_encode_step(keys, values, kcb, 8, vcb, 8, Hm, smooth, *stores, 1)
+    assert all(bool((s == 77).all()) for s in stores)
+    for smooth in (r(64).exp(), r(H, 64).exp()):
+        with pytest.raises(RuntimeError):
+            K.vecinfer_encode_decode_metal(keys, kcb, 8, Hm, smooth)
+        c = KVCacheFactory.create(KVCacheConfig(method="vecinfer", head_dim=D, key_codebook_bits=8, key_sub_dim=8, key_codebook=kcb, value_codebook=vcb,
+                                                smooth_factors=smooth, fused_sdpa=True, fused_sdpa_memory_bound=True))
+        with pytest.raises(RuntimeError):
+            c.update_and_fetch(keys, values)
+        assert c.offset == 0 and c._stored_S_kv == 0

@@ -858,7 +858,9 @@ def vecinfer_encode_decode_metal(keys: torch.Tensor, k_codebook: torch.Tensor, s
         sm = sm.contiguous()
     n_sub = D // sub_dim
     h = _sylvester_scale(H_mat)
-    fused = h > 0 and sub_dim in (4, 8) and n_sub in (8, 16, 32, 64) and cb.shape[0] * sub_dim <= 16384
+    # (factors of another width: the composition broadcasts or refuses them, the kernel would read past their end)
+    fused = (h > 0 and sub_dim in (4, 8) and n_sub in (8, 16, 32, 64) and cb.shape[0] * sub_dim <= 16384
+             and (sm is None or sm.shape[-1] == D))
     if fused and cb.shape[0] > 256:   # the composition's products carry gradients and tangents: a caller who asks for them keeps them
         fused = _forward_ad._current_level < 0 and not (
             (H_mat.requires_grad or (sm is not None and sm.requires_grad) or (want_k_tilde and keys.requires_grad)) and torch.is_grad_enabled())
@@ -913,7 +915,8 @@ def vecinfer_encode_step(keys, values, k_codebook, k_sub_dim, v_codebook, v_sub_
         return False   # the composition's transform, as in vecinfer_encode_decode_metal
     sm = smooth
     if sm is not None:
-        if sm.dtype != torch.float32 or not sm.is_cuda or not sm.is_contiguous() or (sm.ndim == 2 and sm.shape[0] not in (1, Hh)):
+        if (sm.dtype != torch.float32 or not sm.is_cuda or not sm.is_contiguous() or sm.ndim not in (1, 2) or sm.shape[-1] != D
+                or (sm.ndim == 2 and sm.shape[0] not in (1, Hh))):
             return False
     h = _sylvester_scale(H_mat)
     if not h > 0:
