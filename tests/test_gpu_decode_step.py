@@ -224,3 +224,28 @@ def test_attention_on_another_stream_keeps_the_tokens_memory(how, monkeypatch):
         want = [(t.data_ptr(), other.cuda_stream) for kv in tokens for t in kv] if stream is other else []
         assert sorted(held) == sorted(want)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("D,bits,g,dtype,more,deferred", [
+    (128, 4, 32, torch.float16, {}, True), (128, 1, 64, torch.bfloat16, {}, True), (64, 2, 32, torch.float16, {}, True),
+    (128, 8, 32, torch.float16, {}, False), (128, 3, 32, torch.float16, dict(kivi_code_field="tight"), False),
+    (128, 4, 32, torch.float16, dict(kivi_value_layout="channel"), False), (128, 4, 32, torch.float32, {}, False),
+    (128, 4, 16, torch.bfloat16, {}, False), (64, 8, 32, torch.float16, {}, False), (64, 4, 32, torch.float16, dict(kivi_pair_heads=False), False)])
+def test_only_a_launch_that_stores_the_token_is_left_it(D, bits, g, dtype, more, deferred, monkeypatch):
+    """A step's token waits for the attention launch only where that launch stores it, and the step is one library call either way:
+    none is refused and made again."""
+    require_gpu()
+    B, H, Hq = 2, 4, 8
+    c = KVCacheFactory.create(KVCacheConfig(method="kivi", head_dim=D, bit_width_inlier=bits, kivi_group_size=g, residual_length=64,
+                                            fused_sdpa=True, fused_sdpa_memory_bound=True, **more))
+    r = lambda *s: torch.randn(s, device="cuda").to(dtype)
+    c.update_and_fetch(r(B, H, 64 + 2 * g + 3, D), r(B, H, 64 + 2 * g + 3, D))
+    taken, real = [], K.kivi_decode_attend
+    monkeypatch.setattr(K, "kivi_decode_attend", lambda *a: taken.append(real(*a)) or taken[-1])
+    k, v = r(B, H, 1, D), r(B, H, 1, D)
+    c.update_and_fetch(k, v)
+    assert (c._pending is not None) == deferred
+    out = c.fused_sdpa(r(B, Hq, 1, D), 0.1)
+    assert c._pending is None and out.shape == (B, Hq, 1, D) and len(taken) == 1 and taken[0] is not None
+    row = c._tail_k[:, :, c.offset - c._n_quantized - 1]
+    assert torch.equal(row.reshape(B, H, D), k[:, :, 0])

@@ -326,7 +326,7 @@ class KIVIKVCache(FP16KVCache):
         self._store_pending()
         n_tail, dtype = self.offset - self._n_quantized, keys.dtype
         if not (n_tail < self._tail_k.shape[2] and keys.shape == values.shape and dtype == self._tail_k.dtype
-                and values.dtype == dtype and (keys.shape[3] == 128 or self._pair)
+                and values.dtype == dtype and (keys.shape[3] == 128 or self._pair) and self._attends_in_one_launch()
                 and keys.is_contiguous() and values.is_contiguous() and keys.data_ptr() % 16 == 0
                 and values.data_ptr() % 16 == 0
                 and (max(0, self.offset + 1 - self._residual_length) // self._group_size) * self._group_size
@@ -441,7 +441,7 @@ class KIVIKVCache(FP16KVCache):
             if q.shape[1] % H:
                 raise ValueError(f"KIVIKVCache.fused_sdpa: {q.shape[1]} query heads over {H} kv heads")
             opts = dict(causal=causal, sliding_window=sliding_window, fixed_order=fixed_order, lengths=lengths, num_splits=num_splits)
-            if q.shape[2] == 1 and self._pairs_attend_direct():
+            if q.shape[2] == 1 and self._attends_in_one_launch():
                 try:   # a launch that reads queries and writes outputs by halves
                     return self._attend(q, scale, pair_heads=H, **opts)
                 except ValueError:   # a shape it does not take
@@ -456,9 +456,10 @@ class KIVIKVCache(FP16KVCache):
         return self._attend(q, scale, causal=causal, sliding_window=sliding_window, fixed_order=fixed_order, lengths=lengths,
                             num_splits=num_splits)
 
-    def _pairs_attend_direct(self) -> bool:
-        """Whether a decode step over kv heads kept in pairs takes the matrix-unit decode launch (its gate on the cache's side)."""
-        return (self._n_quantized > 0 and self._field in (2, 4) and self._group_size >= 32 and self._v_layout == "token"
+    def _attends_in_one_launch(self) -> bool:
+        """Whether a decode step over heads of 128 channels, or of 64 kept in pairs, takes the matrix-unit decode launch, the one
+        that stores a deferred token (its gate on the cache's side: a token deferred for any other launch is refused twice a step)."""
+        return (self._n_quantized > 0 and self._field in (2, 4) and self._group_size in (32, 64, 128) and self._v_layout == "token"
                 and (self._tail_k is None or self._tail_k.dtype in (torch.float16, torch.bfloat16)))
 
     def _attend(self, q: torch.Tensor, scale: float, *, causal: bool, sliding_window: int, fixed_order: bool | None, lengths,

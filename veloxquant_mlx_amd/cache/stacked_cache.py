@@ -194,7 +194,7 @@ class LayerStackedKIVICache:
             if q.shape[2] % H:
                 raise ValueError(f"LayerStackedKIVICache.fused_sdpa_all: {q.shape[2]} query heads over {H} kv heads")
             opts = dict(causal=causal, sliding_window=sliding_window, fixed_order=fixed_order, num_splits=num_splits)
-            if q.shape[3] == 1 and all(c._pairs_attend_direct() for c in self.layers):
+            if q.shape[3] == 1 and all(c._attends_in_one_launch() for c in self.layers):
                 try:   # a launch that reads queries and writes outputs by halves
                     return self._attend_all(q, scale, pair_heads=H, **opts)
                 except ValueError:   # a shape it does not take
