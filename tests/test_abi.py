@@ -110,3 +110,20 @@ def test_workspace_query_covers_the_call_that_runs(B, Hq, Hkv, Sq, D, n_packed, 
         return   # the launch writes its output itself: nothing refuses the call
     assert lib.vq_kivi_attend_ext(a, x) == _lib.VQ_ERR_WORKSPACE
     assert int(re.search(r"workspace of (\d+) bytes required", _lib.last_error()).group(1)) == need
+
+
+def test_half_a_pair_of_length_lists_is_refused():
+    """packed_lens and tail_lens go together, with the extension and without: one list alone is the library's own form of
+    one length a sequence and never a caller's."""
+    lib = _lib.load()
+    a = _lib.AttendArgs()
+    a.B, a.Hq, a.Hkv, a.Sq, a.D, a.n_tail, a.tail_cap, a.scale = 2, 4, 4, 1, 128, 64, 64, 0.1
+    a.q = a.out = a.k_tail = a.v_tail = 4096
+    for field in ("packed_lens", "tail_lens"):
+        setattr(a, field, 4096)
+        for x in (None, _lib.AttendExt(0, 4096)):
+            assert lib.vq_kivi_attend_ext(a, x) == lib.vq_kivi_attend(a) == _lib.VQ_ERR_INVALID
+            assert "go together" in _lib.last_error()
+        setattr(a, field, None)
+    a.packed_lens = a.tail_lens = 4096
+    assert lib.vq_kivi_attend_ext(a, _lib.AttendExt(0, 4096)) == _lib.VQ_ERR_INVALID and "exclude" in _lib.last_error()

@@ -110,7 +110,7 @@ static int64_t gcd64(int64_t x, int64_t y) { while (y) { const int64_t t = x % y
 // and heads stay those of cap_tokens, so the kernels address the rest as before.  What is left
 // below the window inside the first stretch is masked in the kernels.
 static AttendCall skip_below_window(const AttendCall &a) {
-    if (a.sliding_window <= 0 || a.own_lengths() || a.n_packed <= 0) return a;
+    if (a.sliding_window <= 0 || a.packed_lens != nullptr || a.n_packed <= 0) return a;
     int64_t first = a.n_packed + a.n_tail - a.Sq + 1 - a.sliding_window;   // first slot of the first query
     if (first > a.n_packed) first = a.n_packed;
     const int64_t per = 32 / a.pack_bits;
@@ -308,8 +308,6 @@ static int attend(const AttendCall *a_in) {
         VQ_REQUIRE(a->k_packed && a->v_packed && a->k_scale && a->k_zero && a->v_scale && a->v_zero, VQ_ERR_INVALID,
                    "%s: null packed-cache pointer", fn);
     if (a->n_tail > 0) VQ_REQUIRE(a->k_tail && a->v_tail, VQ_ERR_INVALID, "%s: null tail pointer", fn);
-    VQ_REQUIRE((a->packed_lens == nullptr) == (a->tail_lens == nullptr), VQ_ERR_INVALID,
-               "%s: packed_lens and tail_lens go together", fn);
     VQ_REQUIRE((a->k_new == nullptr) == (a->v_new == nullptr), VQ_ERR_INVALID, "%s: k_new and v_new go together", fn);
     if (a->k_new != nullptr) {
         VQ_REQUIRE(a->n_tail >= 1, VQ_ERR_INVALID, "%s: k_new / v_new fill the last tail row, so n_tail must be >= 1", fn);
@@ -420,15 +418,16 @@ static int attend(const AttendCall *a_in) {
 }
 
 extern "C" int vq_kivi_attend(const vq_attend_args *a) {
-    VQ_REQUIRE(a != nullptr, VQ_ERR_INVALID, "%s: null argument block", "vq_kivi_attend");
-    const AttendCall call(*a);
-    return attend(&call);
+    return vq_kivi_attend_ext(a, nullptr);
 }
 
 extern "C" int vq_kivi_attend_ext(const vq_attend_args *a, const vq_attend_ext *x) {
-    VQ_REQUIRE(a != nullptr, VQ_ERR_INVALID, "%s: null argument block", "vq_kivi_attend_ext");
+    const char *fn = "vq_kivi_attend";
+    VQ_REQUIRE(a != nullptr, VQ_ERR_INVALID, "%s: null argument block", fn);
+    VQ_REQUIRE((a->packed_lens == nullptr) == (a->tail_lens == nullptr), VQ_ERR_INVALID,
+               "%s: packed_lens and tail_lens go together", fn);
     VQ_REQUIRE(x == nullptr || x->seq_lens == nullptr || a->packed_lens == nullptr, VQ_ERR_INVALID,
-               "%s: seq_lens and packed_lens exclude each other", "vq_kivi_attend_ext");
+               "%s: seq_lens and packed_lens exclude each other", fn);
     const AttendCall call(*a, x);
     return attend(&call);
 }

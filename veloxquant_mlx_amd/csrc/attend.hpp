@@ -4,32 +4,43 @@
 
 namespace vq {
 
-// A call as the kernels take it: the caller's argument block and what vq_attend_ext adds to it.
+// A call as the library runs it: the caller's argument block and what vq_attend_ext adds to it.  One length a sequence travels in
+// the block's own fields -- packed_lens the int64 list, tail_lens null, a form that no caller's block has -- and the kernels
+// that know nothing of pairs take the block alone: two more fields in every kernel's arguments made the sixteen launches of an 8k
+// prefill 3 us longer in all.
 struct AttendCall : vq_attend_args {
     int64_t pair_heads;          // > 0: kv heads of 64 channels, kept in pairs; the caller's kv head count
-    const int64_t *seq_lens;     // live slots of every sequence, prefix and tail together
     AttendCall() = default;
-    explicit AttendCall(const vq_attend_args &a, const vq_attend_ext *x = nullptr)
-        : vq_attend_args(a), pair_heads(x ? x->pair_heads : 0), seq_lens(x ? x->seq_lens : nullptr) {}
-    __host__ __device__ bool own_lengths() const { return packed_lens != nullptr || seq_lens != nullptr; }
+    explicit AttendCall(const vq_attend_args &a, const vq_attend_ext *x = nullptr) : vq_attend_args(a), pair_heads(x ? x->pair_heads : 0) {
+        if (x != nullptr && x->seq_lens != nullptr) {
+            packed_lens = reinterpret_cast<const int32_t *>(x->seq_lens);
+            tail_lens = nullptr;
+        }
+    }
 };
+
+// live slots of every sequence, prefix and tail together (null: none, or two lists of lengths)
+__device__ __host__ __forceinline__ const int64_t *seq_lens(const vq_attend_args &a) {
+    return a.tail_lens == nullptr ? reinterpret_cast<const int64_t *>(a.packed_lens) : nullptr;
+}
 
 // a batch whose sequences differ in length: the block's copy of the arguments takes the lengths
 // of its own sequence
-__device__ __forceinline__ void take_sequence_lengths(AttendCall &a, int64_t b) {
-    if (a.packed_lens != nullptr) {
-        a.n_packed = a.packed_lens[b];
-        a.n_tail = a.tail_lens[b];
-    } else if (a.seq_lens != nullptr) {
-        const int64_t n = a.seq_lens[b], tail = n - a.n_packed;
+__device__ __forceinline__ void take_sequence_lengths(vq_attend_args &a, int64_t b) {
+    if (a.packed_lens == nullptr) return;
+    if (const int64_t *lens = seq_lens(a)) {
+        const int64_t n = lens[b], tail = n - a.n_packed;
         if (tail < a.n_tail) a.n_tail = tail < 0 ? 0 : tail;
         if (n < a.n_packed) a.n_packed = n;
+    } else {
+        a.n_packed = a.packed_lens[b];
+        a.n_tail = a.tail_lens[b];
     }
 }
 
 // first slot a query at position `pos` (of Sq, aligned to the end of n_total slots) sees under a
 // sliding window; 0 without one
-__device__ __host__ __forceinline__ int64_t window_first(const AttendCall &a, int64_t n_total, int64_t pos) {
+__device__ __host__ __forceinline__ int64_t window_first(const vq_attend_args &a, int64_t n_total, int64_t pos) {
     const int64_t lo = n_total - a.Sq + pos + 1 - a.sliding_window;
     return a.sliding_window > 0 && lo > 0 ? lo : 0;
 }

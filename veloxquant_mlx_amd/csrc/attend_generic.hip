@@ -31,7 +31,7 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-__global__ __launch_bounds__(256) void attend_generic_kernel(AttendCall a, int nsplit, int64_t split_len,
+__global__ __launch_bounds__(256) void attend_generic_kernel(vq_attend_args a, int nsplit, int64_t split_len,
                                                              float *__restrict__ ws) {
     const int lane = threadIdx.x & 63;
     const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(MS_THREADS) void attend_merge_splits_kernel(const f
 // apart, takes the weight of every visible stand-in out of the softmax sum (its values are stored
 // as zeros, so the numerators never saw it; its key is rebuilt from the packed store as
 // code * scale + zero), then folds the exact rows in with a running maximum and writes the row.
-__global__ __launch_bounds__(256) void attend_sink_patch_kernel(AttendCall a, int nparts, const float *__restrict__ ws) {
+__global__ __launch_bounds__(256) void attend_sink_patch_kernel(vq_attend_args a, int nparts, const float *__restrict__ ws) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int64_t rows = a.B * a.Hq * a.Sq;

@@ -752,7 +752,7 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
     take_sequence_lengths(a, b);
     // the newest token of the call (k_new) is the last row of the tail: of the whole batch's under seq_lens, of the sequence's
     // own under tail_lens
-    const int64_t newest = a.k_new == nullptr ? -1 : (a.seq_lens != nullptr ? n_tail_all : a.n_tail) - 1;
+    const int64_t newest = a.k_new == nullptr ? -1 : (seq_lens(a) != nullptr ? n_tail_all : a.n_tail) - 1;
     const float c = a.scale * LOG2E;
 
     RowTile tile;

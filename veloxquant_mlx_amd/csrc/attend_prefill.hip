@@ -99,7 +99,7 @@ __device__ __forceinline__ int pf_krow(int t) { return (t >> 1) + 16 * (t & 1); 
 // Scale / zero are fp16 (GV = channel groups per value row).
 template <int BITS, int GV>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void attend_prefill_kernel(AttendCall a, int qp, int nparts, float *__restrict__ ws) {
+void attend_prefill_kernel(vq_attend_args a, int qp, int nparts, float *__restrict__ ws) {
     __shared__ __align__(16) f16 s_k[2][32 * PF_KSTRIDE];
     __shared__ __align__(16) f16 s_v[2][MF_D * PF_VSTRIDE];
     // What turns the unit's tile into keys and values, staged with it: keys [scale | zero |
@@ -488,7 +488,7 @@ __device__ __forceinline__ f16x8 recon8(f16x8 c, const Meta8<float> &s, const Me
 }
 
 // one run per row, nothing to patch afterwards, 256-row blocks: the kernel writes `out`, no merge launch follows
-__host__ __device__ inline bool mfma_prefill_writes_output(const AttendCall &a, int nparts) {
+__host__ __device__ inline bool mfma_prefill_writes_output(const vq_attend_args &a, int nparts) {
     return nparts == 1 && a.sink_k == nullptr && (a.Hq / a.Hkv) * a.Sq >= (a.D == 2 * MF_D ? 128 : 256);
 }
 
@@ -504,7 +504,7 @@ template <int BITS, typename M> struct PrStage {
 // on the vector unit and holds no staging registers.  BITS, GV and M play no part then.
 template <int BITS, int GV, typename M, bool TILES = false>
 __global__ __launch_bounds__(PR_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void attend_prefill_rows_kernel(AttendCall a, int qp, int nparts, float *__restrict__ ws) {
+void attend_prefill_rows_kernel(vq_attend_args a, int qp, int nparts, float *__restrict__ ws) {
     __shared__ __align__(16) f16 s_k[TILES ? 1 : 3][32 * PF_KSTRIDE];
     __shared__ __align__(16) f16 s_v[TILES ? 1 : 3][MF_D * PF_VSTRIDE];
     __shared__ __align__(16) char s_ring[TILES ? 4 * PF_TILE_BYTES : 16];
@@ -909,7 +909,7 @@ void attend_prefill_rows_kernel(AttendCall a, int qp, int nparts, float *__restr
 // (sequence, kv head): packed units are reconstructed exactly as the 256-row blocks do it (c s + z rounded once
 // to fp16), tail units are the plain rows; the thread-to-piece assignment is that of the blocks' producer.
 template <int BITS, int GV, typename M>
-__global__ __launch_bounds__(PR_THREADS) void prefill_tiles_kernel(AttendCall a, int first_unit) {
+__global__ __launch_bounds__(PR_THREADS) void prefill_tiles_kernel(vq_attend_args a, int first_unit) {
     constexpr int PER = 32 / BITS;
     constexpr int KW = MF_D / PER;
     constexpr int gshift = GV == 4 ? 5 : GV == 2 ? 6 : 7;
@@ -986,7 +986,7 @@ template <typename M> struct PrStage2 {
 
 template <int BITS, int GV, typename M>
 __global__ __launch_bounds__(PR_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void attend_prefill_rows_d256_kernel(AttendCall a, int qp, int nparts, int v_half, float *__restrict__ ws) {
+void attend_prefill_rows_d256_kernel(vq_attend_args a, int qp, int nparts, int v_half, float *__restrict__ ws) {
     constexpr int DH = 2 * MF_D;          // channels of a head
     constexpr int KST = DH + 8;           // fp16 per token row of the key tile (528 B: conflict-free b128 reads)
     __shared__ __align__(16) f16 s_k[3][32 * KST];
@@ -1371,7 +1371,7 @@ bool mfma_prefill_supported(const AttendCall &a) {
     } else {
         // plain keys and values only (the tail units of the same kernels): worth the matrix unit
         // from a few hundred tokens on
-        if (a.n_tail < 64 || a.own_lengths()) return false;
+        if (a.n_tail < 64 || a.packed_lens != nullptr) return false;
     }
     if (!(a.scale > 0.f)) return false;
     if (a.n_tail > 0 && (!(a.tail_dtype == VQ_F16 || a.tail_dtype == VQ_BF16) || (((uintptr_t)a.k_tail | (uintptr_t)a.v_tail) & 15u))) return false;
@@ -1393,13 +1393,13 @@ bool mfma_prefill_direct_output(const AttendCall &a, int nparts) {
 }
 
 bool mfma_prefill_uses_tiles(const AttendCall &a) {
-    return a.kv_tiles != nullptr && !a.own_lengths() && a.D == MF_D && mfma_prefill_block_rows(a) == 256 &&
+    return a.kv_tiles != nullptr && a.packed_lens == nullptr && a.D == MF_D && mfma_prefill_block_rows(a) == 256 &&
            ((uintptr_t)a.kv_tiles & 15u) == 0 && a.tile_cap * 32 >= a.n_packed + a.n_tail && a.n_packed % 32 == 0;
 }
 
 int launch_prefill_tiles(const AttendCall &a, int64_t first_unit, int64_t n_units) {
     const char *fn = "vq_kivi_prefill_tiles";
-    VQ_REQUIRE(a.D == MF_D && !a.own_lengths(), VQ_ERR_UNSUPPORTED, "%s: head_dim 128 and one length for the batch only", fn);
+    VQ_REQUIRE(a.D == MF_D && a.packed_lens == nullptr, VQ_ERR_UNSUPPORTED, "%s: head_dim 128 and one length for the batch only", fn);
     VQ_REQUIRE(a.B * a.Hkv <= 65535 && n_units <= 0x7fffffff, VQ_ERR_UNSUPPORTED, "%s: too many (sequence, kv head) pairs or units", fn);
     if (a.n_packed > 0) {
         VQ_REQUIRE((a.pack_bits == 2 || a.pack_bits == 4) && (a.group == 32 || a.group == 64 || a.group == 128) &&

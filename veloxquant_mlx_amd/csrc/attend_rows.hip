@@ -73,7 +73,7 @@ bool rows_kernel_supported(const AttendCall &a) {
 
 // NR: the rows a tile can hold (1 .. AR_NR): the per-row loops of a launch whose tiles are smaller shrink with it
 template <int BITS, int NR>
-__global__ __launch_bounds__(256) void attend_rows_kernel(AttendCall a, int64_t split_len, int pq, int tiles,
+__global__ __launch_bounds__(256) void attend_rows_kernel(vq_attend_args a, int64_t split_len, int pq, int tiles,
                                                           float *__restrict__ ws, int part0, int nparts) {
     constexpr int PER = 32 / BITS, CPL = ar_cpl(PER), SUBW = PER / CPL;   // SUBW lanes share a word
     constexpr uint32_t MASK = (1u << BITS) - 1u;

@@ -448,7 +448,7 @@ bool wide_kernel_supported(const AttendCall &a) {
     const int64_t blocks = a.B * a.Hkv * (int64_t)tiles;
     if (a.num_splits == 0 && blocks > 256 && a.n_packed * a.D <= (blocks > 1536 ? 8192 : 4608)) return false;
     return a.num_splits >= 0 && a.n_packed > 0 && a.n_tail == 0 && a.pack_bits == 8 && a.v_layout == VQ_V_CHANNEL_PACKED &&
-           a.meta_dtype == VQ_F32 && wide_head(a.D) && a.group % 32 == 0 && !a.own_lengths() && a.k_new == nullptr &&
+           a.meta_dtype == VQ_F32 && wide_head(a.D) && a.group % 32 == 0 && a.packed_lens == nullptr && a.k_new == nullptr &&
            a.sink_k == nullptr && a.scale > 0.f && blocks <= 65535 &&
            (((uintptr_t)a.k_packed | (uintptr_t)a.v_packed | (uintptr_t)a.k_scale | (uintptr_t)a.k_zero) & 15u) == 0;
 }
