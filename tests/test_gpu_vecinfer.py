@@ -668,3 +668,31 @@ def test_factors_of_another_width_are_refused():
         with pytest.raises(RuntimeError):
             c.update_and_fetch(keys, values)
         assert c.offset == 0 and c._stored_S_kv == 0
+
+
+@pytest.mark.parametrize("nc", [1, 3, 16, 17, 31, 32, 33, 64])
+@pytest.mark.parametrize("odd", ["plain", "nan", "all nan", "inf", "equal"])
+def test_step_over_codebooks_of_a_tile_or_two(nc, odd):
+    """A codebook of one tile, whose two cells are all there is, and the first of two: the indices of the two launches, with
+    centroids and sub-vectors that are no numbers, infinite ones and equal ones."""
+    require_gpu()
+    g = torch.Generator(device="cuda").manual_seed(nc)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda")
+    B, H, D = 3, 4, 128
+    keys, values = rand(B, H, 1, D).half(), rand(B, H, 1, D).half()
+    values[0, 0, 0, 5], values[0, 1, 0, 17], values[0, 2, 0] = float("nan"), float("inf"), 0.0
+    kcb, vcb = rand(nc, 4), rand(nc, 8)
+    for cb in (kcb, vcb):
+        if odd == "nan":
+            cb[nc // 2, 1] = float("nan")
+        elif odd == "all nan":
+            cb[:] = float("nan")
+        elif odd == "inf":
+            cb[nc - 1, 0] = float("inf")
+        elif odd == "equal":
+            cb[:] = cb[0].clone()
+    Hm = walsh_hadamard_matrix(D, device="cuda")
+    ks, vs = (torch.full((B, H, 2, D // n), 99, dtype=torch.uint8, device="cuda") for n in (4, 8))
+    assert K.vecinfer_encode_step(keys, values, kcb, 4, vcb, 8, Hm, None, ks, vs, 1)
+    assert torch.equal(ks[:, :, 1:], K.vecinfer_encode_decode_metal(keys, kcb, 4, Hm, index_dtype=torch.uint8, want_k_hat=False)[1])
+    assert torch.equal(vs[:, :, 1:], K.vecinfer_quantize_metal(values, vcb, 8, index_dtype=torch.uint8))

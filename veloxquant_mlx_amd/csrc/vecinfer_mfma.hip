@@ -749,7 +749,8 @@ __device__ __forceinline__ void assign_split(const AssignJob &j, int64_t block, 
             xs[e] = t.x; xs[e + 1] = t.y; xs[e + 2] = t.z; xs[e + 3] = t.w;
         }
         const float lim = __uint_as_float(f1) + margin<SUB>(v, f1);
-        const bool second = !(__uint_as_float(f2) > lim), all = far || !(__uint_as_float(bound) > lim);
+        // (a codebook of one tile is its two cells: nothing was dropped that a bound stands for)
+        const bool second = !(__uint_as_float(f2) > lim), all = far || (ntiles > 1 && !(__uint_as_float(bound) > lim));
         float d = INFINITY;
         int i = 0x7fffffff;
         // sixteen rows of a cell, 16 / WAVES a lane
@@ -773,7 +774,8 @@ __device__ __forceinline__ void assign_split(const AssignJob &j, int64_t block, 
         }
 #pragma unroll
         for (int o = 1; o < WAVES; o <<= 1) take_nearer(d, i, __shfl_xor(d, o), __shfl_xor(i, o));
-        const unsigned long long m = __ballot(all && l == 0);   // one lane of each group
+        // one lane of each group (a cell without a distance below infinity decides nothing)
+        const unsigned long long m = __ballot((all || !(d < INFINITY)) && l == 0);
         if (m != 0) scan_all<SUB>(m, xs, j.cb, j.ct, aligned, j.nc, lane, i);
         if (l == 0) lds.idx[g] = i;
     }
@@ -791,7 +793,9 @@ __global__ __launch_bounds__(64 * WAVES) void vq_assign_split_kernel(AssignJob j
 // A decode step's keys and values, SPLIT both, in one launch that writes into the index store: the first key_blocks blocks take the
 // keys, the others the values beside them.  What bounds a few tokens is one block's latency, then launches and the
 // host: apart it was a launch each and two strided copies (2 tokens, 8 heads of 128, 4096 x 4 and 256 x 8 centroids:
-// 10.8 + 5.0 + 2 + 1.9 us and their gaps, now 11.3).
+// 10.8 + 5.0 + 2 + 1.9 us and their gaps, now 11.3).  Codebooks of every size take it, though alone SPLIT is the form for more
+// than kSplitC centroids: 1 to 32 tokens, apart with the copies / here, in one graph, 256 x 8 keys and values 13.8-16.9 / 8.9-9.2
+// us, 1024 x 8 keys 20-24 / 9.3-9.8, 32 x 8 keys and values 11.7-14.9 / 8.7-9.0.
 template <int SUB, int LT>
 __global__ __launch_bounds__(1024) void vq_encode_step_kernel(AssignJob jk, AssignJob jv, int key_blocks, int v_sub) {
     __shared__ SplitLds<16> lds;
