@@ -249,3 +249,15 @@ def test_only_a_launch_that_stores_the_token_is_left_it(D, bits, g, dtype, more,
     assert c._pending is None and out.shape == (B, Hq, 1, D) and len(taken) == 1 and taken[0] is not None
     row = c._tail_k[:, :, c.offset - c._n_quantized - 1]
     assert torch.equal(row.reshape(B, H, D), k[:, :, 0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,Hq,H,S", [(64, 8, 4, 1), (64, 9, 3, 1), (128, 8, 2, 1), (128, 4, 1, 3), (256, 12, 4, 1)])
+@pytest.mark.parametrize("off", [1, 3, 4, 8])
+def test_queries_between_sixteen_byte_boundaries(D, Hq, H, S, dtype, off):
+    """Queries that are a contiguous view at an odd place: the bits that aligned ones give."""
+    require_gpu()
+    c, new, rand = _cache(D, 4, 32, 2, H, 300, torch.float16, D + off)
+    q = rand(2, Hq, S, D).to(dtype)
+    moved = torch.zeros(q.numel() + off, dtype=dtype, device="cuda")[off:].view(q.shape).copy_(q)
+    assert moved.is_contiguous() and torch.equal(c.fused_sdpa(moved, 0.1, fixed_order=True), c.fused_sdpa(q, 0.1, fixed_order=True))

@@ -357,9 +357,8 @@ static int attend(const AttendCall *a_in) {
                    "%s: pair_heads = %lld goes with %lld kv heads of 128 channels, query heads in multiples of twice that and one "
                    "query position", fn, (long long)H, (long long)((H + 1) / 2));
         // the launch that merges inside the kernel is the one that reads queries and writes outputs by halves
-        VQ_REQUIRE(p.path == 1 && a->sync_counters != nullptr && a->sink_k == nullptr &&
-                       (a->q_dtype == VQ_F32 || ((uintptr_t)a->q & 15u) == 0),
-                   VQ_ERR_UNSUPPORTED, "%s: pair_heads needs the single-launch decode path and 16-byte aligned queries", fn);
+        VQ_REQUIRE(p.path == 1 && a->sync_counters != nullptr && a->sink_k == nullptr, VQ_ERR_UNSUPPORTED,
+                   "%s: pair_heads needs the single-launch decode path", fn);
     }
     size_t need = attend_workspace(a);
     VQ_REQUIRE(need == 0 || (a->workspace != nullptr && a->workspace_bytes >= need), VQ_ERR_WORKSPACE,

@@ -185,7 +185,13 @@ __device__ __forceinline__ void stage_query(const AttendCall &a, const RowTile &
         const bool pairs = DH == 1 && tile.pair_R != 0;   // a query head's channels in its kv head's half, zeros in the other
         if (tile.valid(row) && (!pairs || tile.pair_half(row) == d / (DD / 2))) {
             const int64_t i = pairs ? tile.io_row(row) * (DD / 2) + d % (DD / 2) : tile.row(row) * DD + d;
-            // (whole pieces in every type: element by element, eight dependent loads stood ahead of everything else)
+            // (whole pieces in every type: element by element, eight dependent loads stood ahead of everything else; queries that
+            // start between 16-byte boundaries -- a view into something larger -- take those)
+            if (((uintptr_t)a.q & 15u) != 0) {
+#pragma unroll 1
+                for (int j = 0; j < 8; ++j) s_qraw[row * PK_QROW + d + j] = (f16)ldq(a.q, a.q_dtype, i + j);
+                continue;
+            }
             if (a.q_dtype == VQ_F16) v = *reinterpret_cast<const f16x8 *>((const f16 *)a.q + i);
             else if (a.q_dtype == VQ_BF16) {
                 const uint4 x = *reinterpret_cast<const uint4 *>((const u16 *)a.q + i);
