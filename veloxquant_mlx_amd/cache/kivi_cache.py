@@ -30,6 +30,7 @@ from .. import kernels as K
 from ..core.exceptions import QuantizerConfigError
 from ._fp16_cache import FP16KVCache
 
+_SIXTEEN_BIT = frozenset((torch.float16, torch.bfloat16))
 _META = {"float16": torch.float16, "float32": torch.float32}
 
 
@@ -150,6 +151,9 @@ class KIVIKVCache(FP16KVCache):
                 f"KIVIKVCache: token-packed values need kivi_group_size % {per} == 0 at {self._field} bits a code.")
         self._v_layout = layout
         self._per = per
+        # the store is one that the matrix-unit decode launch takes, which stores a deferred token (a token deferred for any
+        # other launch would be refused twice a step)
+        self._launch_stores = self._field in (2, 4) and self._group_size in (32, 64, 128) and layout == "token"
         # heads of 64 channels, memory-bound mode: kv heads 2m and 2m+1 are kept side by side as one head of 128
         # channels (same codes, scale and zero; queries zero-padded into their own half), the head size the
         # matrix-unit kernels and the one-launch append take; decided at the first tokens (an even head count)
@@ -312,31 +316,31 @@ class KIVIKVCache(FP16KVCache):
         """The launch that reads the deferred token is enqueued: let go of it.  On another stream than it was handed over on,
         its memory must not be given out again before that launch has run."""
         pending, self._pending = self._pending, None
-        device = pending[0].device
-        if K._stream_of(device) != self._pending_stream:
+        if K._stream(pending[0]) != self._pending_stream:
             for t in pending:
-                t.record_stream(torch.cuda.current_stream(device))
+                t.record_stream(torch.cuda.current_stream(t.device))
 
     def _defer_token(self, keys: torch.Tensor, values: torch.Tensor) -> bool:
         """A plain decode step with no flush due: the attention launch of this step stores the token (kv heads kept in pairs: the
         caller's own rows of 64 channels).  Until then the cache holds the caller's tensors, not a copy (see update_and_fetch); of an odd
         number of heads a copy, as the rows beside zeros that are stored otherwise would be."""
-        if keys.shape[2] != 1 or self._n_quantized == 0 or self._tail_k is None:
+        shape, tail = keys.shape, self._tail_k
+        if shape[2] != 1 or self._n_quantized == 0 or tail is None:
             return False
-        self._store_pending()
-        n_tail, dtype = self.offset - self._n_quantized, keys.dtype
-        if not (n_tail < self._tail_k.shape[2] and keys.shape == values.shape and dtype == self._tail_k.dtype
-                and values.dtype == dtype and (keys.shape[3] == 128 or self._pair) and self._attends_in_one_launch()
-                and keys.is_contiguous() and values.is_contiguous() and keys.data_ptr() % 16 == 0
-                and values.data_ptr() % 16 == 0
+        if self._pending is not None:
+            self._store_pending()
+        dtype = keys.dtype
+        if not (self._launch_stores and (shape[3] == 128 or self._pair) and self.offset - self._n_quantized < tail.shape[2]
+                and values.shape == shape and dtype == tail.dtype and values.dtype == dtype and dtype in _SIXTEEN_BIT
+                and keys.is_contiguous() and values.is_contiguous() and (keys.data_ptr() | values.data_ptr()) & 15 == 0
                 and (max(0, self.offset + 1 - self._residual_length) // self._group_size) * self._group_size
                 == self._n_quantized):
             return False
         self._drop_tiles()   # decoding has begun: the prefill scratch goes back
-        if self._pair and keys.shape[1] % 2:   # (one launch for both copies)
+        if self._pair and shape[1] % 2:   # (one launch for both copies)
             keys, values = torch.stack((keys, values)).unbind()
         self._pending = (keys, values)
-        self._pending_stream = K._stream_of(keys.device)
+        self._pending_stream = K._stream(keys)
         self.offset += 1
         B, H, D = self._shape_bhd
         self._account_bytes(B, H, 1, D, 0)
@@ -457,18 +461,18 @@ class KIVIKVCache(FP16KVCache):
                             num_splits=num_splits)
 
     def _attends_in_one_launch(self) -> bool:
-        """Whether a decode step over heads of 128 channels, or of 64 kept in pairs, takes the matrix-unit decode launch, the one
-        that stores a deferred token (its gate on the cache's side: a token deferred for any other launch is refused twice a step)."""
-        return (self._n_quantized > 0 and self._field in (2, 4) and self._group_size in (32, 64, 128) and self._v_layout == "token"
-                and (self._tail_k is None or self._tail_k.dtype in (torch.float16, torch.bfloat16)))
+        """Whether a decode step over heads of 128 channels, or of 64 kept in pairs, takes the matrix-unit decode launch (its gate
+        on the cache's side)."""
+        return self._launch_stores and self._n_quantized > 0 and (self._tail_k is None or self._tail_k.dtype in _SIXTEEN_BIT)
 
     def _attend(self, q: torch.Tensor, scale: float, *, causal: bool, sliding_window: int, fixed_order: bool | None, lengths,
                 num_splits: int, pair_heads: int = 0):
         nq = self._n_quantized
         n_tail = self.offset - nq
-        if q.shape[2] == 1:
+        step = q.shape[2] == 1
+        if step:
             self._drop_tiles()   # a decode step, with or without per-sequence lengths
-        if self._pending is not None and q.shape[2] != 1:
+        elif self._pending is not None:
             self._store_pending()
         extra = self._extra_attend_args()
         if lengths is not None:
@@ -478,7 +482,7 @@ class KIVIKVCache(FP16KVCache):
             if n.numel() != q.shape[0]:
                 raise ValueError(f"KIVIKVCache.fused_sdpa: lengths has {n.numel()} entries for a batch of {q.shape[0]}")
             lengths = n
-        if q.ndim == 4 and q.shape[2] == 1 and self._memory_bound and nq > 0 and n_tail > 0 and not extra:
+        if step and q.ndim == 4 and self._memory_bound and nq > 0 and n_tail > 0 and not extra:
             k_new, v_new = self._pending if self._pending is not None else (None, None)
             out = K.kivi_decode_attend(q, self._kp, self._ks, self._kz, self._vp, self._vs, self._vz, nq, self._field, self._group_size,
                                        self._v_layout, self._tail_k, self._tail_v, n_tail, float(scale), max(0, int(num_splits)),
