@@ -261,3 +261,13 @@ def test_queries_between_sixteen_byte_boundaries(D, Hq, H, S, dtype, off):
     q = rand(2, Hq, S, D).to(dtype)
     moved = torch.zeros(q.numel() + off, dtype=dtype, device="cuda")[off:].view(q.shape).copy_(q)
     assert moved.is_contiguous() and torch.equal(c.fused_sdpa(moved, 0.1, fixed_order=True), c.fused_sdpa(q, 0.1, fixed_order=True))
+
+
+def test_numbers_that_the_packed_block_does_not_hold():
+    """A scale past float32 and a split count past 32 bits go the general way, as they did before steps had a block of their own."""
+    require_gpu()
+    c, new, rand = _cache(128, 4, 32, 1, 2, 300, torch.float16, 5)
+    q = rand(1, 4, 1, 128).half()
+    assert c.fused_sdpa(q, 1e39).shape == q.shape
+    # (kept as its low 32 bits: one run)
+    assert torch.equal(c.fused_sdpa(q, 0.1, num_splits=(1 << 32) + 1, fixed_order=True), c.fused_sdpa(q, 0.1, num_splits=1, fixed_order=True))

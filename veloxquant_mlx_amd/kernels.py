@@ -1287,13 +1287,16 @@ def kivi_decode_attend(q, k_packed, k_scale, k_zero, v_packed, v_scale, v_zero, 
     if order is None:
         return None
     for _ in range(2):
-        args = _lib.ATTEND_PACK.pack(
-            q.data_ptr(), out.data_ptr(), tag, tag, B, Hq, Hkv, 1, D,
-            k_packed.data_ptr(), k_scale.data_ptr(), k_zero.data_ptr(), v_packed.data_ptr(), v_scale.data_ptr(), v_zero.data_ptr(),
-            bits, group_size, VQ_F16 if meta == torch.float16 else VQ_F32, _V_LAYOUT[v_layout], n_packed, cap,
-            k_tail.data_ptr(), v_tail.data_ptr(), tail_tag, n_tail, k_tail.shape[2], scale, 0, num_splits,
-            ws.data_ptr(), ws.numel(), stream, _counters(device, stream).data_ptr(), 0, 0, new_k, new_v, order, sliding_window,
-            0, 0, 0, 0, 0, 0, 0, 0)
+        try:
+            args = _lib.ATTEND_PACK.pack(
+                q.data_ptr(), out.data_ptr(), tag, tag, B, Hq, Hkv, 1, D,
+                k_packed.data_ptr(), k_scale.data_ptr(), k_zero.data_ptr(), v_packed.data_ptr(), v_scale.data_ptr(), v_zero.data_ptr(),
+                bits, group_size, VQ_F16 if meta == torch.float16 else VQ_F32, _V_LAYOUT[v_layout], n_packed, cap,
+                k_tail.data_ptr(), v_tail.data_ptr(), tail_tag, n_tail, k_tail.shape[2], scale, 0, num_splits,
+                ws.data_ptr(), ws.numel(), stream, _counters(device, stream).data_ptr(), 0, 0, new_k, new_v, order, sliding_window,
+                0, 0, 0, 0, 0, 0, 0, 0)
+        except (_lib.struct.error, OverflowError):   # a number that the block's fields do not hold as it is
+            return None
         rc = lib.attend_packed(args, ext)
         if rc == 0:
             return out
