@@ -69,13 +69,8 @@ struct AttendPlan {
 // One output element from the split partials of its query row: p points at nparts records
 // of `stride` floats (max in natural-log units, sum, accumulator[D]).  CH records are
 // fetched at a time with independent loads (a round costs one memory latency, so callers with
-// many records pick a large CH); DEVICE_SCOPE reads partials that other blocks
-// of the same launch wrote.
-template <bool DEVICE_SCOPE> __device__ __forceinline__ float ld_part(const float *p) {
-    if (DEVICE_SCOPE) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return *p;
-}
-template <bool DEVICE_SCOPE, int CH = 8>
+// many records pick a large CH).
+template <int CH>
 __device__ __forceinline__ float merge_partials(const float *p, int nparts, int64_t stride, int64_t d) {
     float gm = -INFINITY, num = 0.f, den = 0.f;
     for (int s0 = 0; s0 < nparts; s0 += CH) {
@@ -83,9 +78,9 @@ __device__ __forceinline__ float merge_partials(const float *p, int nparts, int6
 #pragma unroll
         for (int j = 0; j < CH; ++j) {
             const float *q = p + (int64_t)(s0 + j < nparts ? s0 + j : s0) * stride;
-            m[j] = ld_part<DEVICE_SCOPE>(q);
-            l[j] = ld_part<DEVICE_SCOPE>(q + 1);
-            o[j] = ld_part<DEVICE_SCOPE>(q + 2 + d);
+            m[j] = q[0];
+            l[j] = q[1];
+            o[j] = q[2 + d];
         }
         // every load of the round is issued before the first use: left to itself the scheduler
         // weaves the maxima between the loads and waits for each record in turn
@@ -109,14 +104,14 @@ __device__ __forceinline__ float merge_partials(const float *p, int nparts, int6
     }
     return den > 0.f ? num / den : 0.f;
 }
-// the round size by the number of records: one round of loads when they fit (the decode kernel's own merge and the launch
-// that does it otherwise both go through here, so they add in the same order; launch_merge_splits, of the vector kernels, has
-// an order of its own)
-template <bool DEVICE_SCOPE>
+// The round size by the number of records: one round of loads when they fit.  The decode kernel that merges inside its launch
+// (merge_rows) fetches whole records through LDS and adds them in rounds of the same sizes, in the same order;
+// launch_merge_splits, of the vector kernels, has an order of its own.
+constexpr int MERGE_FEW = 8, MERGE_SOME = 16, MERGE_MANY = 36;
 __device__ __forceinline__ float merge_records(const float *p, int nparts, int64_t stride, int64_t d) {
-    return nparts <= 8 ? merge_partials<DEVICE_SCOPE, 8>(p, nparts, stride, d)
-           : nparts <= 16 ? merge_partials<DEVICE_SCOPE, 16>(p, nparts, stride, d)
-                          : merge_partials<DEVICE_SCOPE, 36>(p, nparts, stride, d);
+    return nparts <= MERGE_FEW ? merge_partials<MERGE_FEW>(p, nparts, stride, d)
+           : nparts <= MERGE_SOME ? merge_partials<MERGE_SOME>(p, nparts, stride, d)
+                                  : merge_partials<MERGE_MANY>(p, nparts, stride, d);
 }
 
 

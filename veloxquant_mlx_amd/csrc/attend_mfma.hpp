@@ -519,21 +519,20 @@ __device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const
 }
 
 // Combine the nparts partials of the tile's query rows into the output, in the order in which attend_merge_kernel
-// adds them (merge_partials: rounds of CH records).  Partials written by other blocks of this launch are read with
+// adds them (merge_records: rounds of CH records).  Partials written by other blocks of this launch are read with
 // device-scope loads, which come from beyond this XCD's L2: a round's records are fetched by the whole block at
 // once, a wave a record, into `lds`, and summed from there, a thread two neighbouring channels of a row.  The
 // wave that has a row's maxima and sums turns them into factors while the accumulators are on their way (28 records of
 // four rows: 3.7 us where every thread fetched its channel of every record, 4.6; eight records of eight rows 4.3 of 5.5).
 // The whole launch, 32 / 8 heads at 2 bits: 8320 tokens of 128 channels 17.1 -> 14.5 us, 700 of 64 channels 16.4 -> 12.9.
 // RTP: rows of a tile at most.  lds: LDS_BYTES, the block's alone by now.
-constexpr int MERGE_MAX_CH = 36;
 template <int DH, int RTP, int WAVES, int LDS_BYTES, int CH>
 __device__ __forceinline__ void merge_rows_ch(const AttendCall &a, const RowTile &tile, const RowTable &tab, int nparts, const float *ws,
                                               int tid, int wave, uint64_t *lds) {
     constexpr int DD = MF_D * DH, PART = DD + 2;
     constexpr int VAL = DD / 2;                                     // channel pairs of a record
     // rows at a time: what the threads cover at two channels each and the records' places hold, a power of two
-    constexpr int ROOM = LDS_BYTES / (MERGE_MAX_CH * 8 * (VAL + 1)), COVER = WAVES / DH;
+    constexpr int ROOM = LDS_BYTES / (MERGE_MANY * 8 * (VAL + 1)), COVER = WAVES / DH;
     constexpr int FIT = ROOM < COVER ? ROOM : COVER, POW = FIT >= 8 ? 8 : FIT >= 4 ? 4 : FIT >= 2 ? 2 : 1;
     constexpr int ROWS = RTP < POW ? RTP : POW, PER_ROW = WAVES / ROWS;   // waves that fetch a row's records
     static_assert(ROOM >= 1 && ROWS * VAL <= 64 * WAVES, "a row's records fit the rings, a thread a channel pair");
@@ -629,10 +628,9 @@ template <int DH, int RTP, int WAVES, int LDS_BYTES>
 __device__ __forceinline__ void merge_rows(const AttendCall &a, const RowTile &tile, const RowTable &tab, int nparts, const float *ws,
                                            int tid, int wave, void *lds) {
     uint64_t *l = reinterpret_cast<uint64_t *>(lds);
-    // (the round sizes of merge_records)
-    if (nparts <= 8) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, 8>(a, tile, tab, nparts, ws, tid, wave, l);
-    else if (nparts <= 16) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, 16>(a, tile, tab, nparts, ws, tid, wave, l);
-    else merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_MAX_CH>(a, tile, tab, nparts, ws, tid, wave, l);
+    if (nparts <= MERGE_FEW) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_FEW>(a, tile, tab, nparts, ws, tid, wave, l);
+    else if (nparts <= MERGE_SOME) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_SOME>(a, tile, tab, nparts, ws, tid, wave, l);
+    else merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_MANY>(a, tile, tab, nparts, ws, tid, wave, l);
 }
 
 // launchers of the packed-prefix kernel (it also runs the fp16 tail and, given sync counters,

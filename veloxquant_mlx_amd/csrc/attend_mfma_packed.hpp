@@ -792,7 +792,7 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
         uint4 *dst = reinterpret_cast<uint4 *>(const_cast<void *>(val ? a.v_tail : a.k_tail)) +
                      (bh * a.tail_cap + newest) * (MF_D / 8) + piece;
         *dst = 8 * piece < new_row_cols(a, bh) ? *src : make_uint4(0u, 0u, 0u, 0u);
-        }
+    }
     __syncthreads();
     // the launch has nparts - nsplit tail slots (filled even when this sequence's tail is empty): the
     // last waves of split 0 run the tail first, each into a slot of its own, while the others stream
