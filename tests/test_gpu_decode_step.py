@@ -271,3 +271,21 @@ def test_numbers_that_the_packed_block_does_not_hold():
     assert c.fused_sdpa(q, 1e39).shape == q.shape
     # (kept as its low 32 bits: one run)
     assert torch.equal(c.fused_sdpa(q, 0.1, num_splits=(1 << 32) + 1, fixed_order=True), c.fused_sdpa(q, 0.1, num_splits=1, fixed_order=True))
+
+
+def test_a_tail_unit_without_a_number_counts_for_nothing():
+    """32 tail tokens whose fp16 keys are no numbers, one unit of a wave of its own: the attention over all other slots (values of
+    order one; weights in fp16 and the output's rounding, 2^-11)."""
+    require_gpu()
+    B, Hq, H, D, scale, dtype = 1, 8, 2, 128, 128 ** -0.5, torch.float16
+    c, new, rand = _cache(D, 4, 32, B, H, 300, dtype, 11)
+    nq, n_tail = c._n_quantized, c.offset - c._n_quantized
+    q = rand(B, Hq, 1, D).to(dtype)
+    c._tail_k[:, :, 32:64] = float("nan")
+    keep = [i for i in range(c.offset) if not nq + 32 <= i < nq + 64]
+    deq = lambda p, s, z, axis, kw: K.kivi_dequant(p, s, z, axis, 32, c._field, nq, D, out_dtype=torch.float32, **kw)
+    k = torch.cat([deq(c._kp, c._ks, c._kz, -2, {}), c._tail_k[:, :, :n_tail].float()], 2)[:, :, keep].repeat_interleave(Hq // H, 1)
+    v = torch.cat([deq(c._vp, c._vs, c._vz, -1, dict(v_layout=c._v_layout)), c._tail_v[:, :, :n_tail].float()], 2)[:, :, keep].repeat_interleave(Hq // H, 1)
+    want = torch.softmax((q.float() * k).sum(-1) * scale, -1)[..., None].mul(v).sum(2, keepdim=True)
+    got = c.fused_sdpa(q, scale).float()
+    assert float((got - want).abs().max()) <= 2.0 ** -11 * float(want.abs().max()) + 2e-3

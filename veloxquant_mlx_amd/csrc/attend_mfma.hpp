@@ -323,7 +323,7 @@ __device__ __forceinline__ f16x8 tail_softmax_unit(const f32x4 (&S)[2], float c,
     mx = fmaxf(mx, __shfl_xor(mx, 16));
     mx = fmaxf(mx, __shfl_xor(mx, 32));
     const float m_seen = mx * c;
-    if (first) acc.m_run = m_seen;   // nothing accumulated yet
+    if (first) acc.m_run = fmaxf(-INFINITY, m_seen);   // nothing accumulated yet (a unit whose scores are all no numbers: as if it saw nothing)
     else if (__any(m_seen > acc.m_run + RESCALE_SLACK)) {
         const float m_new = fmaxf(acc.m_run, m_seen);
         const float alpha = m_new == -INFINITY ? 1.f : exp2f(acc.m_run - m_new);   // 0 on the first unit
