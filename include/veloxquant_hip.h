@@ -319,7 +319,7 @@ typedef struct vq_attend_args {
                      * reconstructed key and value rounded to fp16 first, the form in which the
                      * reference's cache holds them (cache/kivi_cache.py:198-201) and the
                      * 256-row prefill blocks attend over them */
-    void *workspace;
+    void *workspace;   /* aligned as floats are, to 256 bytes where vq_kivi_attend_workspace says so */
     size_t workspace_bytes;
     void *stream;
     /* Optional: int32 counters, one per (sequence, kv head, row tile of the decode path) -- B*Hkv for

@@ -289,3 +289,21 @@ def test_a_tail_unit_without_a_number_counts_for_nothing():
     want = torch.softmax((q.float() * k).sum(-1) * scale, -1)[..., None].mul(v).sum(2, keepdim=True)
     got = c.fused_sdpa(q, scale).float()
     assert float((got - want).abs().max()) <= 2.0 ** -11 * float(want.abs().max()) + 2e-3
+
+
+@pytest.mark.parametrize("D,Hq,H,ctx", [(128, 32, 8, 1500), (64, 8, 4, 700), (256, 8, 2, 900)])
+def test_workspace_aligned_as_floats_are(D, Hq, H, ctx, monkeypatch):
+    """A workspace four bytes off a boundary of eight: the bits of an aligned one, with the merge in the launch and after it."""
+    require_gpu()
+    c, new, rand = _cache(D, 4, 32, 1, H, ctx, torch.float16, ctx)
+    q = rand(1, Hq, 1, D).half()
+    want = c.fused_sdpa(q, 0.1, fixed_order=True)
+    room = torch.empty(8 << 20, dtype=torch.uint8, device="cuda")[4:]
+    assert room.data_ptr() % 8 == 4
+    monkeypatch.setattr(K, "_workspace", lambda *a: room)
+    assert torch.equal(c.fused_sdpa(q, 0.1, fixed_order=True), want)
+    if D != 64:
+        kw = dict(k_packed=c._kp, k_scale=c._ks, k_zero=c._kz, v_packed=c._vp, v_scale=c._vs, v_zero=c._vz, n_packed=c._n_quantized,
+                  bits=c._field, group_size=32, v_layout=c._v_layout, k_tail=c._tail_k, v_tail=c._tail_v, n_tail=c.offset - c._n_quantized,
+                  scale=0.1, fixed_order=True)
+        assert torch.equal(K.kivi_packed_attend(q, _single_launch=False, **kw), want)

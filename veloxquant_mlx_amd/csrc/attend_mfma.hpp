@@ -349,7 +349,8 @@ __device__ __forceinline__ f16x8 tail_softmax_unit(const f32x4 (&S)[2], float c,
 // Partials another block will read in this launch go out as device-scope stores (written
 // through to where every compute die sees them); where a launch of their own merges them, plain ones would do as well.
 __device__ __forceinline__ void st_partial(float *p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-// two neighbouring floats at an even offset of a record (records start on 8 bytes)
+// two neighbouring floats at an even offset of a record (records start on 8 bytes from the workspace on; a workspace that is aligned
+// to 4 only is as good: a two-dword access asks for dword alignment)
 __device__ __forceinline__ void st_partial2(float *p, float v0, float v1) {
     const uint64_t u = (uint64_t)__float_as_uint(v0) | ((uint64_t)__float_as_uint(v1) << 32);
     __hip_atomic_store(reinterpret_cast<uint64_t *>(p), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
