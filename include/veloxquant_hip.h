@@ -459,7 +459,8 @@ int vq_kivi_attend_ext(const vq_attend_args *a, const vq_attend_ext *x);
  * tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The
  * split partials and the sync counters come from a device array built into the library (8 MiB +
  * 64 KiB per GPU, held until the process ends); a->workspace, a->workspace_bytes and
- * a->sync_counters are ignored.  Shapes whose partials exceed 8 MiB (vq_kivi_attend_workspace) or
+ * a->sync_counters are ignored.  Shapes whose partials exceed 8 MiB (vq_kivi_attend_workspace; a decode call over short
+ * contexts of many sequences makes do with one for eight times as many tail tokens where that figure is past it) or
  * with more than 16384 (sequence, kv head, row tile) triples return VQ_ERR_WORKSPACE.  The call
  * itself allocates and frees nothing.  All calls on one GPU share that GPU's array: calls that
  * overlap on one GPU (two streams, two threads) race -- serialise them, or use vq_kivi_attend

@@ -66,6 +66,20 @@ def test_static_scratch_entry_point_equals_the_workspace_entry_point():
         K.kivi_packed_attend(q512, static_scratch=True, **{**big[1], "causal": True})
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,n_packed,n_tail", [(64, 64, 8, 256, 128), (50, 40, 10, 96, 250)])
+def test_static_scratch_over_short_contexts_of_many_sequences(B, Hq, Hkv, n_packed, n_tail):
+    """A partial for every 32 tail tokens would not fit the built-in scratch here, one for 256 does: the call runs with
+    those, in agreement with the other plan (weights rounded to fp16 against another maximum, output fp16)."""
+    require_gpu()
+    q, kw = _case(B, Hq, Hkv, n_packed, n_tail, 4, 32, seed=B)
+    plan = {}
+    ref = K.kivi_packed_attend(q, _plan_out=plan, **kw)
+    assert plan["path"] == 1 and B * Hq * plan["nparts"] * 130 * 4 > 8 << 20
+    got = K.kivi_packed_attend(q, static_scratch=True, **kw)
+    assert float((got.float() - ref.float()).abs().max()) <= 2e-3 * max(1.0, float(ref.abs().max()))
+    assert torch.equal(got, K.kivi_packed_attend(q, static_scratch=True, **kw))
+
+
 def test_static_scratch_makes_no_tile_scratch_for_long_plain_prefill():
     """A causal call over plain keys and values with thousands of query rows per kv head: the ordinary call
     writes the input once as tiles into a scratch it keeps; with ``static_scratch=True`` nothing may be

@@ -94,7 +94,7 @@ AttendPlan plan_attend(const AttendCall &a) {
     // us, of 600 (16 x 1000) 15.1 / 13.2, of 4200 (16 x 8000, 8 x 16000) 31.4 / 33.2, 31.9 / 34.2; the line is drawn between.
     p.nparts = p.nsplit;
     if (p.path == 1 && a.n_tail > 0) {
-        int64_t tw = cdiv(cdiv(a.n_tail, 32), units >= 64 && len > 3072 ? 8 : 1);
+        int64_t tw = cdiv(cdiv(a.n_tail, 32), units >= 64 && (len > 3072 || a.few_parts != 0) ? 8 : 1);
         // (a head of 256 channels: the tail launch of the vector kernel, up to four runs of at least 16 tokens)
         const int64_t tr = cdiv(a.n_tail, 16);
         p.nparts += a.D == 128 ? (int)(tw < 1 ? 1 : tw > 8 ? 8 : tw) : (int)(tr > 4 ? 4 : tr);
@@ -455,11 +455,16 @@ extern "C" int vq_kivi_attend_static(const vq_attend_args *a) {
     const char *fn = "vq_kivi_attend_static";
     int rc = validate(a, fn);
     if (rc != VQ_OK) return rc;
-    const size_t need = vq_kivi_attend_workspace(a);
+    VQ_REQUIRE((a->packed_lens == nullptr) == (a->tail_lens == nullptr), VQ_ERR_INVALID,
+               "%s: packed_lens and tail_lens go together", fn);
+    AttendCall call(*a);
+    // (short contexts of many sequences: a partial for every unit of 32 tail tokens is the faster plan where there is room for it)
+    if (attend_workspace(&call) > STATIC_WS_BYTES) call.few_parts = 1;
+    const size_t need = attend_workspace(&call);
     VQ_REQUIRE(need <= STATIC_WS_BYTES, VQ_ERR_WORKSPACE,
                "%s: these shapes need %zu bytes of split partials, the built-in scratch holds %zu; use vq_kivi_attend "
                "with a workspace of its own", fn, need, STATIC_WS_BYTES);
-    AttendCall w = skip_below_window(AttendCall(*a));
+    AttendCall w = skip_below_window(call);
     if (const int64_t Rp = padded_group(w)) {   // the call that runs: its GQA groups filled up
         w.Hq = w.Hkv * Rp;
         w.q = nullptr;
@@ -483,16 +488,15 @@ extern "C" int vq_kivi_attend_static(const vq_attend_args *a) {
         }
         ptr = g_scratch_ptr[dev];
     }
-    vq_attend_args b = *a;
-    b.workspace = ptr;
-    b.workspace_bytes = STATIC_WS_BYTES;
+    call.workspace = ptr;
+    call.workspace_bytes = STATIC_WS_BYTES;
     // the counters start at zero (static storage) and every finished call leaves them at zero; a call that
     // failed half-way (a launch error) may not have, and a later call would then never reach its last ticket
     // and leave `out` unwritten: the counters are cleared again behind a failed call
-    b.sync_counters = reinterpret_cast<int32_t *>(ptr + STATIC_WS_BYTES);
-    rc = vq_kivi_attend(&b);
+    call.sync_counters = reinterpret_cast<int32_t *>(ptr + STATIC_WS_BYTES);
+    rc = attend(&call);
     if (rc != VQ_OK) {
-        hipLaunchKernelGGL(zero_counters_kernel, dim3(16), dim3(256), 0, (hipStream_t)a->stream, b.sync_counters,
+        hipLaunchKernelGGL(zero_counters_kernel, dim3(16), dim3(256), 0, (hipStream_t)a->stream, call.sync_counters,
                            (int)STATIC_COUNTERS);
         (void)hipGetLastError();   // the error reported is the call's own (already recorded)
     }

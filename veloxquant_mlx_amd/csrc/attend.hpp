@@ -9,9 +9,11 @@ namespace vq {
 // that know nothing of pairs take the block alone: two more fields in every kernel's arguments made the sixteen launches of an 8k
 // prefill 3 us longer in all.
 struct AttendCall : vq_attend_args {
-    int64_t pair_heads;          // > 0: kv heads of 64 channels, kept in pairs; the caller's kv head count
+    int32_t pair_heads;   // > 0: kv heads of 64 channels, kept in pairs; the caller's kv head count (negative: not one)
+    int32_t few_parts;    // 1: the plan with the fewest partials (scratch of a fixed size)
     AttendCall() = default;
-    explicit AttendCall(const vq_attend_args &a, const vq_attend_ext *x = nullptr) : vq_attend_args(a), pair_heads(x ? x->pair_heads : 0) {
+    explicit AttendCall(const vq_attend_args &a, const vq_attend_ext *x = nullptr)
+        : vq_attend_args(a), pair_heads(x == nullptr ? 0 : x->pair_heads == (int32_t)x->pair_heads ? (int32_t)x->pair_heads : -1), few_parts(0) {
         if (x != nullptr && x->seq_lens != nullptr) {
             packed_lens = reinterpret_cast<const int32_t *>(x->seq_lens);
             tail_lens = nullptr;
