@@ -29,7 +29,7 @@ __device__ __host__ __forceinline__ const int64_t *seq_lens(const vq_attend_args
 // a batch whose sequences differ in length: the block's copy of the arguments takes the lengths
 // of its own sequence
 __device__ __forceinline__ void take_sequence_lengths(vq_attend_args &a, int64_t b) {
-    if (a.packed_lens == nullptr) return;
+    if (__builtin_expect(a.packed_lens == nullptr, 1)) return;
     if (const int64_t *lens = seq_lens(a)) {
         const int64_t n = lens[b], tail = n - a.n_packed;
         if (tail < a.n_tail) a.n_tail = tail < 0 ? 0 : tail;
