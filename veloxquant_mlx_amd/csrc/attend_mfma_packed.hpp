@@ -369,7 +369,9 @@ __device__ __forceinline__ void packed_units(const AttendCall &a, int64_t bh, fl
     // A block with no more than a chunk a wave deals its units out evenly, whole token groups in one (shorter) chunk a
     // wave, and draws nothing: with chunks of CHUNK units, DEPTH of them in a row, 384 tokens kept three waves of twelve busy
     // for five units each, one after the other (700 tokens at 2 bits, 8 kv heads of 128: the waves are through after 4.6 us
-    // of the launch instead of 6.6).
+    // of the launch instead of 6.6).  A wave's weights are rounded to fp16 against the maximum of other units than before, so the last
+    // bits of such a call are others (2-norm up to 6e-4 in bf16, 2e-4 in fp16); against float64, 36 steps over heads of 64 / 128 / 256,
+    // 2 to 4 bits and 439 to 29180 tokens: 1.0152e-3 rms with chunks, 1.0144e-3 so, no case further off by more than 1 in 1000.
     const bool dealt_out = n_units <= RG::WAVES * RG::CHUNK;
     constexpr int DEAL = RG::WAVES * RG::UPG;
     const int CH = dealt_out ? (n_units + DEAL - 1) / DEAL * RG::UPG : RG::CHUNK;
