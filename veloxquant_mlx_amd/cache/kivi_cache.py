@@ -30,6 +30,7 @@ from .. import kernels as K
 from ..core.exceptions import QuantizerConfigError
 from ._fp16_cache import FP16KVCache
 
+_raw_stream = K._raw_stream
 _SIXTEEN_BIT = frozenset((torch.float16, torch.bfloat16))
 _META = {"float16": torch.float16, "float32": torch.float32}
 
@@ -312,11 +313,13 @@ class KIVIKVCache(FP16KVCache):
             K.kv_tail_append(k, v, self._tail_k, self._tail_v, self.offset - self._n_quantized - 1)
             self._release_pending()
 
-    def _release_pending(self) -> None:
+    def _release_pending(self, stream: int | None = None) -> None:
         """The launch that reads the deferred token is enqueued: let go of it.  On another stream than it was handed over on,
         its memory must not be given out again before that launch has run."""
         pending, self._pending = self._pending, None
-        if K._stream(pending[0]) != self._pending_stream:
+        if stream is None:
+            stream = K._stream(pending[0])
+        if stream != self._pending_stream:
             for t in pending:
                 t.record_stream(torch.cuda.current_stream(t.device))
 
@@ -340,7 +343,7 @@ class KIVIKVCache(FP16KVCache):
         if self._pair and shape[1] % 2:   # (one launch for both copies)
             keys, values = torch.stack((keys, values)).unbind()
         self._pending = (keys, values)
-        self._pending_stream = K._stream(keys)
+        self._pending_stream = _raw_stream(keys.get_device()) if _raw_stream is not None else K._stream(keys)
         self.offset += 1
         B, H, D = self._shape_bhd
         self._account_bytes(B, H, 1, D, 0)
@@ -489,7 +492,10 @@ class KIVIKVCache(FP16KVCache):
                                        fixed_order, int(sliding_window or 0), k_new, v_new, pair_heads, lengths)
             if out is not None:
                 if k_new is not None:
-                    self._release_pending()
+                    if _raw_stream is not None and _raw_stream(q.get_device()) == self._pending_stream:
+                        self._pending = None
+                    else:
+                        self._release_pending()
                 return out
         if self._memory_bound:
             tk, tv = self._tail_k, self._tail_v

@@ -257,8 +257,12 @@ class LayerStackedKIVICache:
         if k_new is not None:
             try:
                 out = K.kivi_packed_attend(qf, k_new=k_new, v_new=v_new, **kw)
+                stream = K._stream(q)
                 for c in self.layers:
-                    c._release_pending()
+                    if c._pending_stream == stream:
+                        c._pending = None
+                    else:
+                        c._release_pending(stream)
                 return out.view((NL, B) + tuple(out.shape[1:]))
             except ValueError:   # a shape the append-and-attend launch does not take
                 for c in self.layers:
