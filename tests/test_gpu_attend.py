@@ -179,6 +179,25 @@ def test_flash_prefill_on_the_matrix_unit(BH, Sq, Skv):
     assert err < TOL
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,D", [(1, 3, 3, 600, 128), (1, 12, 12, 520, 128), (2, 24, 8, 300, 128), (1, 5, 5, 1030, 128), (1, 3, 3, 300, 256)])
+def test_causal_tiles_of_any_number_of_heads_land_once_each(B, Hq, Hkv, Sq, D):
+    """Longest tiles first over all heads: head counts that are and are not multiples or divisors of the eight XCDs, several
+    row tiles, one run and several; every row against the oracle, same bar as the other plain-row cases."""
+    require_gpu()
+    rng = np.random.default_rng(Hq + Sq)
+    q = rng.standard_normal((B, Hq, Sq, D)).astype(np.float16)
+    k, v = (rng.standard_normal((B, Hkv, Sq, D)).astype(np.float16) for _ in range(2))
+    ref = oa.sdpa(q, k, v, D ** -0.5, causal=True)
+    for splits in (0, 1):
+        plan = {}
+        out = K.kivi_packed_attend(to_dev(q), k_tail=to_dev(k), v_tail=to_dev(v), n_tail=Sq, scale=D ** -0.5, causal=True,
+                                   out_dtype=torch.float32, num_splits=splits, _plan_out=plan)
+        assert plan["path"] == 2, plan
+        err = float(np.max(np.abs(host(out) - ref)))
+        print(f"max-abs err {err:.2e}")
+        assert err < TOL
+
+
 def test_flash_prefill_large_logits_bf16_and_future_keys():
     """test_flash_prefill.py:141-151: logits three times as wide (score std ~ 9) stay within the
     reference's 2e-2 -- here within 4e-3, the scores being accumulated in float32; bf16 keys and

@@ -499,6 +499,30 @@ template <int BITS, typename M> struct PrStage {
                      // raw key and value pieces travel in the first piece of each
 };
 
+// Which (row tile, (sequence, kv head), run) a block of a (tiles, heads, runs) grid is.  Workgroups go to the eight
+// XCDs in turn by their linear number, start in that order, and every XCD has its own L2: with the launch's own
+// numbering the row tiles and runs of one kv head land on all eight, and each fetches that head's keys and values from
+// HBM for itself (68 MB per launch at config 4 for 15 MB of input).  A head's blocks share an XCD (a multiple of eight
+// heads) or 8 / heads of them (1, 2 or 4 heads).
+// Under a causal mask a tile's work grows with its number, so all heads' longest tiles (numbered from the end) come first
+// and the short ones fill what is left: 4096 tokens of 32 heads, two rounds of blocks, 179
+// us against 253 with one head's tiles after the other's (the last head's longest tile then starts when the chip is half
+// done); chunks of 2048 of 2 x 40 heads 1081 against 1236 a pass of three.
+// Without one all blocks are alike and a head's stay together.
+struct BlockPlace { unsigned tile, bh, run; };
+__device__ __forceinline__ BlockPlace place_block(bool causal) {
+    const unsigned lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    if (causal || 8 % gridDim.y == 0) {
+        const unsigned within = lin / gridDim.y;
+        const unsigned bh = lin - within * gridDim.y;
+        if (causal) return {within / gridDim.z, bh, within % gridDim.z};
+        return {within % gridDim.x, bh, within / gridDim.x};
+    }
+    if (gridDim.y % 8 != 0) return {blockIdx.x, blockIdx.y, blockIdx.z};
+    const unsigned per_head = gridDim.x * gridDim.z, slot = lin / 8, within = slot % per_head;
+    return {within % gridDim.x, lin % 8 + 8 * (slot / per_head), within / gridDim.x};
+}
+
 // TILES: every unit comes ready-made from a.kv_tiles (the packed prefix and the tail alike) and is copied from
 // global memory straight into a ring of four LDS buffers, four units ahead; the block then has no producer work
 // on the vector unit and holds no staging registers.  BITS, GV and M play no part then.
@@ -527,28 +551,9 @@ void attend_prefill_rows_kernel(vq_attend_args a, int qp, int nparts, float *__r
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, blk = lane >> 4;
-    // Which (row tile, (sequence, kv head), run) this block is.  Workgroups go to the eight XCDs in turn by
-    // their linear number, and every XCD has its own L2: with the launch's own numbering the row tiles and runs
-    // of one kv head land on all eight, and each fetches that head's keys and values from HBM for itself (68 MB
-    // per launch at config 4 for 15 MB of input).  The blocks are renumbered so that a head's tiles and runs share
-    // an XCD (a multiple of eight heads) or 8 / heads of them (1, 2 or 4 heads); other counts keep the launch's
-    // numbering.
-    unsigned tile_x = blockIdx.x, bh_y = blockIdx.y, run_z = blockIdx.z;
-    if (gridDim.y % 8 == 0 || 8 % gridDim.y == 0) {
-        const unsigned lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-        const unsigned per_head = gridDim.x * gridDim.z, xcd = lin % 8, slot = lin / 8;
-        unsigned within;
-        if (gridDim.y % 8 == 0) {
-            bh_y = xcd + 8 * (slot / per_head);
-            within = slot % per_head;
-        } else {
-            bh_y = xcd % gridDim.y;
-            within = xcd / gridDim.y + (8 / gridDim.y) * slot;
-        }
-        tile_x = within % gridDim.x;
-        run_z = within / gridDim.x;
-    }
-    const int64_t bh = bh_y;
+    const BlockPlace place = place_block(a.causal != 0);
+    const unsigned tile_x = place.tile, run_z = place.run;
+    const int64_t bh = place.bh;
     const int64_t hkv = bh % a.Hkv, b = bh / a.Hkv;
     if constexpr (TILES) {   // one length for the batch (mfma_prefill_uses_tiles), one kind of unit: all slots count as tail slots
         a.n_tail += a.n_packed;
@@ -1003,28 +1008,9 @@ void attend_prefill_rows_d256_kernel(vq_attend_args a, int qp, int nparts, int v
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, blk = lane >> 4;
-    // Which (row tile, (sequence, kv head), run) this block is.  Workgroups go to the eight XCDs in turn by
-    // their linear number, and every XCD has its own L2: with the launch's own numbering the row tiles and runs
-    // of one kv head land on all eight, and each fetches that head's keys and values from HBM for itself (68 MB
-    // per launch at config 4 for 15 MB of input).  The blocks are renumbered so that a head's tiles and runs share
-    // an XCD (a multiple of eight heads) or 8 / heads of them (1, 2 or 4 heads); other counts keep the launch's
-    // numbering.
-    unsigned tile_x = blockIdx.x, bh_y = blockIdx.y, run_z = blockIdx.z;
-    if (gridDim.y % 8 == 0 || 8 % gridDim.y == 0) {
-        const unsigned lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-        const unsigned per_head = gridDim.x * gridDim.z, xcd = lin % 8, slot = lin / 8;
-        unsigned within;
-        if (gridDim.y % 8 == 0) {
-            bh_y = xcd + 8 * (slot / per_head);
-            within = slot % per_head;
-        } else {
-            bh_y = xcd % gridDim.y;
-            within = xcd / gridDim.y + (8 / gridDim.y) * slot;
-        }
-        tile_x = within % gridDim.x;
-        run_z = within / gridDim.x;
-    }
-    const int64_t bh = bh_y;
+    const BlockPlace place = place_block(a.causal != 0);
+    const unsigned tile_x = place.tile, run_z = place.run;
+    const int64_t bh = place.bh;
     const int64_t hkv = bh % a.Hkv, b = bh / a.Hkv;
     take_sequence_lengths(a, b);
     const int R = (int)(a.Hq / a.Hkv);
