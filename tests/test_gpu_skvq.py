@@ -249,6 +249,9 @@ def test_reorder_beats_identity_on_heterogeneous_channels():   # test_skvq_cache
     (1, 2, 37, 50, 3, 16),       # channels that do not move as 16-byte pieces, a ragged last group
     (3, 2, 21, 80, 2, 32),
     (1, 2, 9, 2056, 4, 64),      # more channels than a block has threads
+    (8, 2, 123, 128, 4, 32),     # more rows than one round of requests takes, the last round not full
+    (2, 1, 71, 600, 3, 32),      # fewer than two threads a channel
+    (1, 2, 45, 256, 2, 64),      # half a wave a row
 ])
 def test_channel_orders_match_the_stated_rule(dtype, B, H, r, D, bits, g):
     """Channels by range (stable), kept where the mean squared error of the float32 round trip is lower; heads whose two

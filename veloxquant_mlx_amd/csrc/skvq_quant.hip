@@ -361,6 +361,9 @@ void skvq_roundtrip_kernel(SkSides sides, double *__restrict__ err, int64_t n_bh
     __syncthreads();
 
     if constexpr (ERR) {
+        // `place` names the words of channels (without `inv`: of places in the order); looking the order up again for each row
+        // cost 2.9 of 22.5 us
+        const bool staged = scatter || !perm;
         for (int lr = lr_base; lr < rows_pb && lr_base < rpp; lr += rpp) {
             if (row0 + lr >= n_rows) continue;
             const Where w = where(lr);
@@ -371,11 +374,12 @@ void skvq_roundtrip_kernel(SkSides sides, double *__restrict__ err, int64_t n_bh
             for (int c0 = cq * 8; c0 < (int)D; c0 += tpr * 8) {
                 float v[8];
                 if (vec) Vec8<T>::ld(src + c0, v);
+                if (staged) place(w.head, c0);
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
                     const int c = c0 + k;
                     if (c >= (int)D) continue;
-                    const double d = (double)__fsub_rn(srcl[pos(iv ? iv[c] : c)], vec ? v[k] : Elem<T>::ld(src + c));
+                    const double d = (double)__fsub_rn(srcl[staged ? off[k] : pos(iv ? iv[c] : c)], vec ? v[k] : Elem<T>::ld(src + c));
                     sum += d * d;
                 }
             }
@@ -422,74 +426,120 @@ __device__ __forceinline__ uint32_t sk_key(float f) {
 __device__ __forceinline__ float sk_unkey(uint32_t k) { return __uint_as_float(k & 0x80000000u ? k & 0x7fffffffu : ~k); }
 
 // One block per head; W channels (8 where rows move as 16-byte pieces, else 1) a thread, so that the block reads
-// SK_ORD_THREADS / (D / W) rows at a time.  LDS: smallest, largest, NaN mark of every channel, then the ranges.
+// SK_ORD_THREADS / (D / W) rows at a time.  LDS: smallest, largest, NaN mark of every channel, then ranges and places; channel c's
+// words lie at slot(c), piece after piece for equal c % W, so that the pieces of a wave meet different banks.
+// Few blocks, so a block's own instructions are what it waits for (8 heads of 8 x 123 rows of 128 channels, two tensors: 26.8 -> 15.2 us): two
+// rows an operation and one comparison for a NaN in either (eight operations a value and row before, now two and a half), up to
+// AHEAD rows requested at once, the lanes of a wave with the same channels reduced before the LDS atomics, and
+// SK_ORD_THREADS / D threads to a channel's comparisons (128 in a row by an eighth of the threads before).
+
+// smallest and largest of the two halves (rows) of a wave, in every lane
+template <int HALF> __device__ __forceinline__ void sk_fold_lanes(float &mn, float &mx, uint32_t &nan) {
+    mn = fminf(mn, __shfl_xor(mn, HALF));
+    mx = fmaxf(mx, __shfl_xor(mx, HALF));
+    nan |= __shfl_xor(nan, HALF);
+}
 template <typename T, int W>
 __global__ __launch_bounds__(SK_ORD_THREADS)
 void skvq_order_kernel(SkSides sides, int64_t B, int64_t H, int64_t r, int D, int64_t x_stride_bh) {
     const T *__restrict__ x = (const T *)sides.t[blockIdx.z].x;
     int32_t *__restrict__ perm = sides.t[blockIdx.z].perm, *__restrict__ inv = sides.t[blockIdx.z].inv;
+    constexpr int AHEAD = W == 8 ? 16 / (int)sizeof(T) : 16;   // (twice as many pieces of 16 bytes spill)
     extern __shared__ uint32_t s_ord[];
     uint32_t *s_mn = s_ord, *s_mx = s_ord + D, *s_nan = s_ord + 2 * D;
     float *s_rng = reinterpret_cast<float *>(s_ord);
+    int32_t *s_place = reinterpret_cast<int32_t *>(s_ord + D);
     const int tid = threadIdx.x;
     const int64_t h = blockIdx.x, n = B * r;
     for (int c = tid; c < D; c += SK_ORD_THREADS) { s_mn[c] = ~0u; s_mx[c] = 0u; s_nan[c] = 0u; }
     __syncthreads();
     const int pieces = D / W, width = pieces < SK_ORD_THREADS ? pieces : SK_ORD_THREADS, rows = SK_ORD_THREADS / width;
+    auto slot = [&](int c) { return W == 1 ? c : c % W * pieces + c / W; };
     const int p0 = tid % width, row0 = tid / width;
+    // a wave holds whole rows, and the number of its lanes between equal channels is a power of two
+    const bool fold = width < 64 && 64 % width == 0;
     for (int p = p0; p < pieces && row0 < rows; p += width) {
         float mn[W], mx[W];
-        uint32_t nan = 0u;
+        bool bad[W];
 #pragma unroll
-        for (int k = 0; k < W; ++k) { mn[k] = INFINITY; mx[k] = -INFINITY; }
-        int64_t b = row0 / r, t = row0 - b * r;   // the thread's next row, carried along: no division in the loop
+        for (int k = 0; k < W; ++k) { mn[k] = INFINITY; mx[k] = -INFINITY; bad[k] = false; }
+        int b = row0 / (int)r, t = row0 - b * (int)r;   // the thread's next row, carried along: no division in the loop
 #pragma unroll 1
-        for (int64_t i = row0; i < n; i += SK_AHEAD * rows) {
-            typename Vec8<T>::Raw raw[SK_AHEAD];
-            float one[SK_AHEAD];
+        for (int64_t i = row0; i < n; i += AHEAD * rows) {
+            typename Vec8<T>::Raw raw[AHEAD];
+            float one[AHEAD];
 #pragma unroll
-            for (int j = 0; j < SK_AHEAD; ++j) {
-                if (i + j * rows >= n) continue;
-                const T *src = x + (b * H + h) * x_stride_bh + t * D + (int64_t)p * W;
+            for (int j = 0; j < AHEAD; ++j) {   // past the end the last row comes again
+                const T *src = x + (b * H + h) * x_stride_bh + (int64_t)t * D + (int64_t)p * W;
                 if constexpr (W == 8) raw[j] = Vec8<T>::request(src);
                 else one[j] = Elem<T>::ld(src);
-                for (t += rows; t >= r; t -= r) ++b;
+                if (i + (j + 1) * rows < n)
+                    for (t += rows; t >= (int)r; t -= (int)r) ++b;
             }
 #pragma unroll
-            for (int j = 0; j < SK_AHEAD; ++j) {
-                if (i + j * rows >= n) continue;
-                float v[8];
-                if constexpr (W == 8) Vec8<T>::unpack(raw[j], v);
-                else v[0] = one[j];
+            for (int j = 0; j < AHEAD; j += 2) {   // two rows an operation: min3, max3, one comparison for a NaN in either
+                float v[8], u[8];
+                if constexpr (W == 8) {
+                    Vec8<T>::unpack(raw[j], v);
+                    Vec8<T>::unpack(raw[j + 1], u);
+                } else {
+                    v[0] = one[j];
+                    u[0] = one[j + 1];
+                }
 #pragma unroll
                 for (int k = 0; k < W; ++k) {
-                    mn[k] = fminf(mn[k], v[k]);
-                    mx[k] = fmaxf(mx[k], v[k]);
-                    nan |= v[k] != v[k] ? 1u << k : 0u;
+                    mn[k] = fminf(fminf(mn[k], v[k]), u[k]);
+                    mx[k] = fmaxf(fmaxf(mx[k], v[k]), u[k]);
+                    bad[k] = bad[k] | (bool)__builtin_isunordered(v[k], u[k]);
                 }
             }
         }
+        uint32_t nan = 0u;
+#pragma unroll
+        for (int k = 0; k < W; ++k) nan |= bad[k] ? 1u << k : 0u;
+        if (fold) {   // (one pass of the loop over p, every lane in it)
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+                uint32_t none = 0u, &mark = k == 0 ? nan : none;
+                if (width <= 32) sk_fold_lanes<32>(mn[k], mx[k], mark);
+                if (width <= 16) sk_fold_lanes<16>(mn[k], mx[k], mark);
+                if (width <= 8) sk_fold_lanes<8>(mn[k], mx[k], mark);
+            }
+        }
+        if (fold && (tid & 63) >= (width < 8 ? 8 : width)) continue;
 #pragma unroll
         for (int k = 0; k < W; ++k) {
-            atomicMin(&s_mn[p * W + k], sk_key(mn[k]));
-            atomicMax(&s_mx[p * W + k], sk_key(mx[k]));
-            if (nan >> k & 1u) s_nan[p * W + k] = 1u;
+            atomicMin(&s_mn[k * (W == 1 ? 0 : pieces) + p], sk_key(mn[k]));
+            atomicMax(&s_mx[k * (W == 1 ? 0 : pieces) + p], sk_key(mx[k]));
+            if (nan >> k & 1u) s_nan[k * (W == 1 ? 0 : pieces) + p] = 1u;
         }
     }
     __syncthreads();
-    for (int c = tid; c < D; c += SK_ORD_THREADS)   // each thread its own words: the range takes the place of the smallest value
+    for (int c = tid; c < D; c += SK_ORD_THREADS) {   // each thread its own words: range and place take the values' place
         s_rng[c] = s_nan[c] ? NAN : __fsub_rn(sk_unkey(s_mx[c]), sk_unkey(s_mn[c]));
+        s_place[c] = 0;
+    }
     __syncthreads();
-    for (int c = tid; c < D; c += SK_ORD_THREADS) {   // place = channels before this one; a NaN comes after every number
-        const float mine = s_rng[c];
+    // place = channels before this one; a NaN comes after every number.  `share` threads a channel, a run of the others each.
+    const int share = D < SK_ORD_THREADS ? SK_ORD_THREADS / D : 1, run = (D + share - 1) / share;
+    const int part = D < SK_ORD_THREADS ? tid / D : 0;
+    for (int c = D < SK_ORD_THREADS ? tid % D : tid; c < D && part < share; c += SK_ORD_THREADS) {
+        const float mine = s_rng[slot(c)];
         const bool mine_nan = mine != mine;
+        const int to = (part + 1) * run < D ? (part + 1) * run : D;
         int place = 0;
-        for (int j = 0; j < D; ++j) {
-            const float o = s_rng[j];
+#pragma unroll 8
+        for (int j = part * run; j < to; ++j) {
+            const float o = s_rng[slot(j)];
             const bool o_nan = o != o;
             const bool before = mine_nan ? !o_nan : o < mine, same = mine_nan ? o_nan : o == mine;
             place += (before || (same && j < c)) ? 1 : 0;
         }
+        atomicAdd(&s_place[slot(c)], place);
+    }
+    __syncthreads();
+    for (int c = tid; c < D; c += SK_ORD_THREADS) {
+        const int place = s_place[slot(c)];
         perm[h * D + place] = c;
         inv[h * D + c] = place;
     }
