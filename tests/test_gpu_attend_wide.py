@@ -25,6 +25,8 @@ def _visible(Sq, n, causal, window, device):
     (1, 8, 2, 64, 1, 32, 1, False, 0, 31), (2, 7, 1, 64, 129, 32, 1, False, 0, 0), (1, 4, 4, 128, 33, 64, 1, False, 0, 63),
     (2, 28, 4, 128, 1037, 32, 1, False, 0, 3), (1, 12, 4, 256, 517, 128, 1, False, 0, 0), (1, 2, 1, 256, 95, 32, 3, True, 0, 0),
     (1, 8, 2, 128, 700, 32, 2, True, 0, 4), (1, 4, 2, 128, 900, 32, 1, False, 77, 0), (3, 16, 1, 128, 4099, 96, 1, False, 0, 0),
+    # a last tile of one head; positions of one and of three heads in a tile, the last tile short
+    (1, 9, 1, 128, 300, 32, 1, False, 0, 0), (2, 3, 3, 64, 200, 32, 6, True, 50, 0), (1, 3, 1, 128, 260, 32, 2, True, 0, 5),
 ])
 def test_byte_codes_against_the_general_kernel(B, Hq, Hkv, D, n, group, Sq, causal, window, extra):
     require_gpu()

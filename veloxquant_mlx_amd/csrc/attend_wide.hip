@@ -3,9 +3,9 @@
 // codebook indices (VecInferKVCache.fused_sdpa, veloxquant_mlx/cache/vecinfer_cache.py:670-731).  Everything is computed in
 // float32 on the vector unit; keys and values are rebuilt in registers.
 //
-// 32 / 8 heads of 128 channels, one query: byte codes of 2 x 8192 tokens 77 -> 24.6 us with the merge (42 MB, 1.7 TB/s);
+// 32 / 8 heads of 128 channels, one query: byte codes of 2 x 8192 tokens 77 -> 23 us with the merge (42 MB, 1.8 TB/s);
 // 4096 x 4 / 256 x 8 codebooks over 2 x 9001 tokens 203 us (copy of the indices, gather to float32, general kernel, merge) ->
-// 24.6 us.  What bounds it is latency: a decode call reads a few tens of MB, so every wave has two or three units of tokens to do and
+// 22.5 us.  What bounds it is latency: a decode call reads a few tens of MB, so every wave has two or three units of tokens to do and
 // waits for each.  Hence
 //   * sixteen channels a lane: D / 16 lanes hold a token, a wave 64 / (D / 16) tokens at once, and the sums over a token's lanes
 //     take two to four DPP adds a row (the general kernel in attend_rows.hip owns four channels a lane for byte codes: five);
@@ -17,6 +17,11 @@
 //   * the query transform of VecInfer, (q * smooth) @ Hadamard, is a fast transform of the block's rows in LDS.
 // The slots' sums are added by halving exchanges (56 a wave for 4 x 16 sums over 8 slots; adding every sum over every slot
 // takes 192).
+// What is left is issue: with two waves a SIMD, 1300 instructions a unit and two or three units a wave, the instructions that run once
+// count.  Row coordinates by comparison instead of division, exchanges by lane swaps instead of LDS permutes (80 waits in a
+// row) and one pass over the block's partials took 4140 instructions to 3100: byte codes of 2 x 8192 tokens 20.5 -> 18.8 us a launch,
+// 2 x 9001 indices 20.9 -> 18.4 (without the merge, 4 us).  Asking for the first unit ahead of tables and queries, eight pieces of the
+// codebooks in flight, or a stretch of whole steps for every wave did not help (21.2, 21.9, 22.4 us): the waits are the other wave's turn.
 #include <atomic>
 
 #include "attend_rows.hpp"
@@ -40,7 +45,7 @@ struct WideArgs {
     int smooth_rows;
     float hscale;                    // > 0: rows are multiplied by the Hadamard matrix of this magnitude
     int64_t split_len;
-    int pq, tiles;
+    int pq, tiles, group;            // group: query heads of a kv head
     float *ws;
 };
 
@@ -156,6 +161,46 @@ template <int KSUB, int VSUB> struct IndexRows {
     static __device__ __forceinline__ float vzero(const Raw &) { return 0.f; }
 };
 
+// The wave's lanes OFF apart, without a trip through LDS: what both of them hold (in every lane, the lower one's first) ...
+struct Both { float lo, hi; };
+template <int OFF> __device__ __forceinline__ Both lanes_apart(float x) {
+    if constexpr (OFF == 32 || OFF == 16) {
+        const uint32_t u = __float_as_uint(x);
+        const auto r = [&] {
+            if constexpr (OFF == 32) return __builtin_amdgcn_permlane32_swap(u, u, false, false);
+            else return __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        }();
+        return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+    } else if constexpr (OFF == 8) {
+        return {x, ar_dpp<0x128>(x)};   // row_ror 8
+    } else {
+        return {x, __shfl_xor(x, OFF)};
+    }
+}
+// ... and a half-exchange: lanes with the bit OFF clear get the sum of both lanes' x, those with it set that of both lanes' y.
+template <int OFF> __device__ __forceinline__ float exchange_add(float x, float y, bool upper) {
+    if constexpr (OFF == 32 || OFF == 16) {
+        const uint32_t u = __float_as_uint(x), v = __float_as_uint(y);
+        const auto r = [&] {
+            if constexpr (OFF == 32) return __builtin_amdgcn_permlane32_swap(u, v, false, false);
+            else return __builtin_amdgcn_permlane16_swap(u, v, false, false);
+        }();
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else {
+        const float keep = upper ? y : x, give = upper ? x : y;
+        return keep + (OFF == 8 ? ar_dpp<0x128>(give) : __shfl_xor(give, OFF));
+    }
+}
+template <int OFF> __device__ __forceinline__ float slots_max(float x) {   // over the lanes OFF, 2 OFF, .. 32 apart
+    const Both b = lanes_apart<OFF>(x);
+    if constexpr (OFF == 32) return fmaxf(b.lo, b.hi);
+    else return slots_max<2 * OFF>(fmaxf(b.lo, b.hi));
+}
+template <int OFF> __device__ __forceinline__ float slots_add(float x) {
+    const Both b = lanes_apart<OFF>(x);
+    if constexpr (OFF == 32) return b.lo + b.hi;
+    else return slots_add<2 * OFF>(b.lo + b.hi);
+}
 // Sums a[0 .. T) over the 64 / LPT slots of a wave: at every exchange a lane keeps half of its sums and gives the other
 // half away.  Returns the first of the T / (64 / LPT) sums that are left in a[0 ..].
 template <int T, int OFF, int LPT> __device__ __forceinline__ int slots_reduce(float *a, int lane) {
@@ -164,13 +209,22 @@ template <int T, int OFF, int LPT> __device__ __forceinline__ int slots_reduce(f
     } else {
         const bool upper = (lane & OFF) != 0;
 #pragma unroll
-        for (int j = 0; j < T / 2; ++j) {
-            const float keep = upper ? a[j + T / 2] : a[j], give = upper ? a[j] : a[j + T / 2];
-            a[j] = keep + __shfl_xor(give, OFF);
-        }
+        for (int j = 0; j < T / 2; ++j) a[j] = exchange_add<OFF>(a[j], a[j + T / 2], upper);
         return (upper ? T / 2 : 0) + slots_reduce<T / 2, OFF / 2, LPT>(a, lane);
     }
 }
+
+// The query rows of a block: `heads` heads of the group from h0 on, at consecutive positions from pos0 on.  At most AR_NR rows, so head
+// and position of one take comparisons; as divisions, by every wave and for every row, they were a fifth of the instructions
+// of a short run.
+struct WideRows {
+    int64_t base_row, Sq;   // row of (sequence, first head of the group, position 0); query positions
+    int heads, h0, pos0, n;
+    __device__ __forceinline__ int at(int r) const { return (r >= heads) + (r >= 2 * heads) + (r >= 3 * heads); }
+    __device__ __forceinline__ bool valid(int r) const { return r < n && pos0 + at(r) < Sq; }
+    __device__ __forceinline__ int64_t row(int r) const { return base_row + (int64_t)(h0 + r - at(r) * heads) * Sq + pos0 + at(r); }
+};
+static_assert(AR_NR <= 4, "WideRows::at");
 
 template <int D, int NR, class Rows>
 __global__ __launch_bounds__(WD_THREADS) void attend_wide_kernel(WideArgs a, Rows rows) {
@@ -181,23 +235,20 @@ __global__ __launch_bounds__(WD_THREADS) void attend_wide_kernel(WideArgs a, Row
     __shared__ float s_q[NR][D];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int sp = (int)blockIdx.x, nsplit = (int)gridDim.x, by = (int)blockIdx.y;
-    const int64_t bh = by / a.tiles, hkv = bh % a.Hkv, b = bh / a.Hkv;
+    const int sp = (int)blockIdx.x, nsplit = (int)gridDim.x;
+    const uint32_t by = blockIdx.y, bh32 = by / (uint32_t)a.tiles, b = bh32 / (uint32_t)a.Hkv;   // (fewer than 65536 blocks)
+    const int64_t bh = bh32, hkv = bh32 - b * (uint32_t)a.Hkv;
     const int w = lane % LPT, slot = lane / LPT;
 
-    RowTile tile;
-    const int group = (int)(a.Hq / a.Hkv);
-    const int htiles = group > AR_NR ? (group + AR_NR - 1) / AR_NR : 1;
-    const int t_in_bh = by % a.tiles;
-    tile.h0 = (t_in_bh % htiles) * AR_NR;
-    tile.R = htiles > 1 ? (group - tile.h0 < AR_NR ? group - tile.h0 : AR_NR) : group;
-    tile.RT = tile.R * a.pq;
-    tile.pos0 = (t_in_bh / htiles) * a.pq;
+    const int htiles = a.group > AR_NR ? (a.group + AR_NR - 1) / AR_NR : 1;
+    const int t_in_bh = (int)(by - bh32 * (uint32_t)a.tiles);
+    WideRows tile;
+    tile.h0 = htiles > 1 ? (t_in_bh % htiles) * AR_NR : 0;
+    tile.heads = htiles > 1 ? (a.group - tile.h0 < AR_NR ? a.group - tile.h0 : AR_NR) : a.group;
+    tile.n = tile.heads * a.pq;
+    tile.pos0 = (htiles > 1 ? t_in_bh / htiles : t_in_bh) * a.pq;
     tile.Sq = a.Sq;
-    tile.n_total = a.n;
-    tile.causal = a.causal;
-    tile.window = a.window;
-    tile.base_row = (b * a.Hq + hkv * group) * a.Sq;
+    tile.base_row = ((int64_t)b * a.Hq + hkv * a.group) * a.Sq;
 
     rows.template block_init<D>(s_dyn, tid);
     for (int e = tid; e < NR * D; e += WD_THREADS) {
@@ -227,8 +278,10 @@ __global__ __launch_bounds__(WD_THREADS) void attend_wide_kernel(WideArgs a, Row
     const float mul = a.scale * WD_LOG2E * (a.hscale > 0.f ? a.hscale : 1.f);   // scores in log2 units
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
-        vis[r] = tile.valid(r) ? tile.visible(r) : 0;
-        fst[r] = tile.valid(r) ? tile.first(r) : 0;
+        // queries align to the end of the tokens
+        const int64_t upto = a.n - a.Sq + tile.pos0 + tile.at(r) + 1, from = upto - a.window;
+        vis[r] = !tile.valid(r) ? 0 : a.causal ? upto : a.n;
+        fst[r] = tile.valid(r) && a.window > 0 && from > 0 ? from : 0;
         if (tile.valid(r)) {
             t_lo = fst[r] < t_lo ? fst[r] : t_lo;
             t_hi = vis[r] > t_hi ? vis[r] : t_hi;
@@ -323,13 +376,9 @@ __global__ __launch_bounds__(WD_THREADS) void attend_wide_kernel(WideArgs a, Row
     // ---- the slots of the wave, then the waves of the block (a lane's probabilities are those of its token's other lanes)
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
-        float mw = m[r];
-#pragma unroll
-        for (int off = LPT; off < 64; off <<= 1) mw = fmaxf(mw, __shfl_xor(mw, off));
+        const float mw = slots_max<LPT>(m[r]);
         const float f = m[r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[r] - mw);
-        l[r] *= f;
-#pragma unroll
-        for (int off = LPT; off < 64; off <<= 1) l[r] += __shfl_xor(l[r], off);
+        l[r] = slots_add<LPT>(l[r] * f);
 #pragma unroll
         for (int j = 0; j < 16; ++j) acc[r * 16 + j] = Rows::SCALED ? (acc[r * 16 + j] + oz[r]) * f : acc[r * 16 + j] * f;
         m[r] = mw;
@@ -350,22 +399,27 @@ __global__ __launch_bounds__(WD_THREADS) void attend_wide_kernel(WideArgs a, Row
         }
     }
     __syncthreads();
-    for (int e = tid; e < NR * (D + 2); e += WD_THREADS) {
-        const int r = e / (D + 2), c = e % (D + 2);
+    for (int e = tid; e < NR * D; e += WD_THREADS) {   // a thread a sum; the first of a row also writes its maximum and weight
+        const int r = e / D, c = e % D;
         if (!tile.valid(r)) continue;
-        float gm = -INFINITY;
+        float mv[WD_WAVES], gm = -INFINITY, x = 0.f, den = 0.f;
 #pragma unroll
-        for (int v = 0; v < WD_WAVES; ++v) gm = fmaxf(gm, s_dyn[(v * NR + r) * (D + 2)]);
-        float x = gm;
-        if (c >= 1) {
-            x = 0.f;
+        for (int v = 0; v < WD_WAVES; ++v) {
+            mv[v] = s_dyn[(v * NR + r) * (D + 2)];
+            gm = fmaxf(gm, mv[v]);
+        }
 #pragma unroll
-            for (int v = 0; v < WD_WAVES; ++v) {
-                const float *p = s_dyn + (v * NR + r) * (D + 2);
-                if (p[0] != -INFINITY) x += p[c] * __expf(p[0] - gm);
+        for (int v = 0; v < WD_WAVES; ++v) {
+            const float *p = s_dyn + (v * NR + r) * (D + 2);
+            const float f = mv[v] == -INFINITY ? 0.f : __expf(mv[v] - gm);
+            if (mv[v] != -INFINITY) {
+                x += p[2 + c] * f;
+                den += p[1] * f;
             }
         }
-        a.ws[(tile.row(r) * nsplit + sp) * (D + 2) + c] = x;
+        float *o = a.ws + (tile.row(r) * nsplit + sp) * (D + 2);
+        o[2 + c] = x;
+        if (c == 0) { o[0] = gm; o[1] = den; }
     }
 }
 
@@ -461,7 +515,7 @@ void plan_attend_wide(const AttendCall &a, AttendPlan &p) {
 
 void launch_attend_wide(const AttendCall &a, const AttendPlan &p) {
     const WideArgs w = {a.q, a.q_dtype, a.Hq, a.Hkv, a.Sq, a.n_packed, a.cap_tokens, a.scale, a.causal, a.sliding_window,
-                        nullptr, 1, 0.f, p.split_len, p.pq, p.tiles, (float *)a.workspace};
+                        nullptr, 1, 0.f, p.split_len, p.pq, p.tiles, (int)(a.Hq / a.Hkv), (float *)a.workspace};
     const ByteRows rows = {(const uint8_t *)a.k_packed, (const uint8_t *)a.v_packed, (const float *)a.k_scale, (const float *)a.k_zero,
                            (const float *)a.v_scale, (const float *)a.v_zero, a.group, a.cap_tokens};
     launch_wide(w, rows, a.B, a.D, p.nsplit, 0, (hipStream_t)a.stream);
@@ -536,7 +590,7 @@ extern "C" int vq_vecinfer_attend_indices(const vq_index_attend_args *a) {
                a->workspace_bytes);
     hipStream_t st = (hipStream_t)a->stream;
     const WideArgs w = {a->q, a->q_dtype, a->Hq, a->Hkv, a->Sq, a->n_tokens, a->cap_tokens, a->scale, a->causal, a->sliding_window,
-                        a->smooth, a->smooth_rows, a->hadamard_scale, len, pq, tiles, (float *)a->workspace};
+                        a->smooth, a->smooth_rows, a->hadamard_scale, len, pq, tiles, (int)(a->Hq / a->Hkv), (float *)a->workspace};
     auto run = [&](auto r) {
         r.k = a->k_idx; r.v = a->v_idx;
         r.k_u8 = a->k_idx_dtype == VQ_U8; r.v_u8 = a->v_idx_dtype == VQ_U8;
