@@ -30,6 +30,7 @@
 // with one lane a centroid.  SPLIT spends twice the vector work a sub-vector (every wave forms its operands from float
 // rows) but fills the chip from a few dozen blocks on.  Where the line lies: see kSplitMax.
 #include <atomic>
+#include <type_traits>
 
 #include "vecinfer.hpp"
 
@@ -640,6 +641,21 @@ void vq_assign_image_kernel(AssignJob j) {
     }
 }
 
+// The partner of a reduction over 16 lanes at step O = 1, 2, 4, 8, without a trip through LDS: 4 and 8 mirror the lanes of eight and
+// sixteen, which after the steps before them hold the same in fours and eights.
+template <int O, typename V> __device__ __forceinline__ V near_lane(V x) {
+    static_assert(sizeof(V) == 4 && (O == 1 || O == 2 || O == 4 || O == 8), "a word, one of four steps");
+    constexpr int CTRL = O == 1 ? 0xB1 : O == 2 ? 0x4E : O == 4 ? 0x141 : 0x140;
+    const int i = __builtin_bit_cast(int, x);
+    return __builtin_bit_cast(V, __builtin_amdgcn_update_dpp(i, i, CTRL, 0xF, 0xF, false));
+}
+template <class F> __device__ __forceinline__ void over_16_lanes(const F &step) {
+    step(std::integral_constant<int, 1>{});
+    step(std::integral_constant<int, 2>{});
+    step(std::integral_constant<int, 4>{});
+    step(std::integral_constant<int, 8>{});
+}
+
 // ---- SPLIT: one block for 64 sub-vectors, the tiles shared out over its waves -------------------
 
 template <int WAVES> struct SplitLds {
@@ -669,8 +685,8 @@ __device__ __forceinline__ void assign_split(const AssignJob &j, int64_t block, 
     load_centroids<SUB, TW>(j.cb, j.ct, aligned, rc, row);
 #pragma unroll
     for (int i = 0; i < TW; ++i) cmax2 = fmaxf(cmax2, norm2<SUB>(row[i]));
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) cmax2 = fmaxf(cmax2, __shfl_xor(cmax2, o));
+    over_16_lanes([&](auto o) { cmax2 = fmaxf(cmax2, near_lane<o()>(cmax2)); });
+    cmax2 = fmaxf(cmax2, __shfl_xor(cmax2, 16));
     if (lane == 0) lds.red[wave] = cmax2;
     SubVec<SUB> s;
     take_subvec<SUB, LT>(s, j.x, j.xt, raw, sv, live, lane, j.kx);
@@ -723,11 +739,11 @@ __device__ __forceinline__ void assign_split(const AssignJob &j, int64_t block, 
         // a tracker is (wave, half); of its two cells the first can lead, the second bounds what it dropped
         u32 f1 = min(e.x, e.z), f2 = max(e.x, e.z), bound = min(e.y, e.w);
         int o1 = 2 * l + (e.z < e.x), o2 = 2 * l + !(e.z < e.x);
-#pragma unroll
-        for (int o = 1; o < WAVES; o <<= 1) {
-            const u32 g1 = __shfl_xor(f1, o), g2 = __shfl_xor(f2, o);
-            const int p1 = __shfl_xor(o1, o), p2 = __shfl_xor(o2, o);
-            bound = min(bound, (u32)__shfl_xor(bound, o));
+        static_assert(WAVES == 16, "the lanes of a sub-vector");
+        over_16_lanes([&](auto o) {
+            const u32 g1 = near_lane<o()>(f1), g2 = near_lane<o()>(f2);
+            const int p1 = near_lane<o()>(o1), p2 = near_lane<o()>(o2);
+            bound = min(bound, near_lane<o()>(bound));
             const bool mine = f1 < g1 || (f1 == g1 && o1 < p1);
             // the second of the pair, and what falls out joins the bound
             const u32 a = mine ? f2 : g2, b = mine ? g1 : f1, c = mine ? g2 : f2;
@@ -738,7 +754,7 @@ __device__ __forceinline__ void assign_split(const AssignJob &j, int64_t block, 
             f2 = keep ? a : b;
             o2 = keep ? pa : pb;
             bound = min(bound, min(keep ? b : a, c));
-        }
+        });
         SubVec<SUB> v;
         v.x2 = lds.x2[g];
         const bool far = v.x2 < 0.f;
@@ -772,8 +788,7 @@ __device__ __forceinline__ void assign_split(const AssignJob &j, int64_t block, 
                 }
             }
         }
-#pragma unroll
-        for (int o = 1; o < WAVES; o <<= 1) take_nearer(d, i, __shfl_xor(d, o), __shfl_xor(i, o));
+        over_16_lanes([&](auto o) { take_nearer(d, i, near_lane<o()>(d), near_lane<o()>(i)); });
         // one lane of each group (a cell without a distance below infinity decides nothing)
         const unsigned long long m = __ballot((all || !(d < INFINITY)) && l == 0);
         if (m != 0) scan_all<SUB>(m, xs, j.cb, j.ct, aligned, j.nc, lane, i);
@@ -793,7 +808,7 @@ __global__ __launch_bounds__(64 * WAVES) void vq_assign_split_kernel(AssignJob j
 // A decode step's keys and values, SPLIT both, in one launch that writes into the index store: the first key_blocks blocks take the
 // keys, the others the values beside them.  What bounds a few tokens is one block's latency, then launches and the
 // host: apart it was a launch each and two strided copies (2 tokens, 8 heads of 128, 4096 x 4 and 256 x 8 centroids:
-// 10.8 + 5.0 + 2 + 1.9 us and their gaps, now 11.3).  Codebooks of every size take it, though alone SPLIT is the form for more
+// 10.8 + 5.0 + 2 + 1.9 us and their gaps, now 10.8; 11.4 with the reductions over a sub-vector's lanes as LDS permutes).  Codebooks of every size take it, though alone SPLIT is the form for more
 // than kSplitC centroids: 1 to 32 tokens, apart with the copies / here, in one graph, 256 x 8 keys and values 13.8-16.9 / 8.9-9.2
 // us, 1024 x 8 keys 20-24 / 9.3-9.8, 32 x 8 keys and values 11.7-14.9 / 8.7-9.0.
 template <int SUB, int LT>
