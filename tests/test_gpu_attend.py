@@ -778,3 +778,21 @@ def test_sliding_window_without_packed_tokens_and_not_causal():
             ref = oa.sdpa(q, k, v, 0.09, causal=causal, sliding_window=w)
             assert float(np.max(np.abs(host(out) - ref))) < TOL, (Sq, Skv, causal)
     _packed_case(1, 8, 2, 512, 40, 128, 4, 32, "token", torch.float16, Sq=4, causal=False, seed=9, window=100)
+
+
+@pytest.mark.parametrize("B,Hkv,n,nparts", [(1, 10, 16384, 22), (3, 8, 4096, 8), (7, 8, 1024, 4), (13, 10, 512, 1), (16, 16, 256, 1), (17, 16, 256, 1), (13, 10, 16512, 3)])
+def test_a_decode_launch_takes_the_splits_of_one_round(B, Hkv, n, nparts):
+    """Numbers of (sequence, kv head) tiles that do not divide the chip's 256 CUs: splits rounded down to one round of blocks (three where
+    half the chip would idle over a long run), against the general kernel."""
+    require_gpu()
+    D, gen = 128, torch.Generator(device="cuda").manual_seed(n + Hkv)
+    k, v = (torch.randn((B, Hkv, n, D), generator=gen, device="cuda").half() for _ in range(2))
+    q = torch.randn((B, Hkv, 1, D), generator=gen, device="cuda").half()
+    kp, ks, kz = K.kivi_quant_pack(k, -2, 32, 4, meta_dtype=torch.float16)
+    vp, vs, vz = K.kivi_quant_pack(v, -1, 32, 4, meta_dtype=torch.float16, v_layout="token")
+    kw = dict(k_packed=kp, k_scale=ks, k_zero=kz, v_packed=vp, v_scale=vs, v_zero=vz, n_packed=n, bits=4, group_size=32, v_layout="token",
+              scale=D ** -0.5, out_dtype=torch.float32)
+    plan = {}
+    out = K.kivi_packed_attend(q, _plan_out=plan, **kw)
+    assert plan["path"] == 1 and plan["nparts"] == nparts, plan
+    assert float((out - K.kivi_packed_attend(q, num_splits=-1, **kw)).abs().max()) < TOL

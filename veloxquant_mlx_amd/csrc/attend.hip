@@ -12,6 +12,20 @@ static std::atomic<int> g_fixed_order{0};
 // what a tail token costs the block of split 0, in packed tokens, when the plan balances the splits
 constexpr int64_t TAIL_EQUIV = 4;
 
+// Splits of a decode launch over `units` tiles of (sequence, kv head).  A CU holds one block and the blocks take equally long, so a few
+// blocks more than the chip's 256 CUs run as a second round: as many splits as fit one round, rounded down.  Rounded up they took, us for
+// two steps (splits rounded up / down, 32 / 8 and 40 / 10 heads of 128, 12 / 4 of 256): 5 sequences of 8320 tokens at 4 bits 57.1 / 39.4, 7 of
+// 2000 at 2 bits 46.5 / 30.7, 13 of 32900 215 / 170, 1 x 10 heads of 32900 alike; heads of 256, 7 x 20011 149 / 109, 3 x 8320 92 / 75.
+// More splits over two and three rounds lose (104 tiles of 32900 tokens, 2 / 4 / 7 splits: 170 / 178 / 187 us; of 8320 60 / 82 / 98): the CUs
+// that a round leaves idle cost less than another round's start.  The exception is a chip half idle over long runs: 130 tiles
+// of 20011 tokens 165 us as one split, 148 as three (160 tiles 196 / 193); of 8320 88 / 91.
+// A batch with lengths keeps the rounded-up number: its shorter sequences leave blocks without work.
+static int64_t decode_splits(const AttendCall &a, int64_t units, int64_t n) {
+    if (a.packed_lens != nullptr) return cdiv(256, units);
+    if (units > 128 && units <= 170 && n > 16384) return 3;
+    return units < 256 ? 256 / units : 1;
+}
+
 AttendPlan plan_attend(const AttendCall &a) {
     AttendPlan p;
     // bit 0: fixed chunk order; bit 1 (fixed_order == 3): the decode kernel also waits for every copy in flight
@@ -76,8 +90,8 @@ AttendPlan plan_attend(const AttendCall &a) {
     // units of parallel work before splitting: a wave per query row (generic)
     // or an eight-wave block per kv head (MFMA)
     const int64_t units = p.path == 1 ? a.B * a.Hkv * p.tiles : a.B * a.Hq * a.Sq;
-    const int64_t target = p.path == 1 ? 256 : 4096;   // MFMA path: one eight-wave block per CU
-    int64_t ns = a.num_splits > 0 ? a.num_splits : cdiv(target, units > 0 ? units : 1);   // < 0: choose as well
+    int64_t ns = a.num_splits;   // < 0: choose as well
+    if (ns <= 0) ns = p.path == 1 ? decode_splits(a, units > 0 ? units : 1, n_split) : cdiv(4096, units > 0 ? units : 1);
     if (ns > max_splits) ns = max_splits;
     if (ns > 512) ns = 512;
     if (ns < 1) ns = 1;
