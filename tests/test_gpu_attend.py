@@ -796,3 +796,27 @@ def test_a_decode_launch_takes_the_splits_of_one_round(B, Hkv, n, nparts):
     out = K.kivi_packed_attend(q, _plan_out=plan, **kw)
     assert plan["path"] == 1 and plan["nparts"] == nparts, plan
     assert float((out - K.kivi_packed_attend(q, num_splits=-1, **kw)).abs().max()) < TOL
+
+
+@pytest.mark.parametrize("lens", [(4352, 0, 31, 4351, 2000, 128, 4000), (4352,) * 7, (4352, 0, 0, 0, 0, 0, 0), (0, 0, 0, 0, 0, 0, 96)])
+@pytest.mark.parametrize("Hq,Hkv,D,n_tail", [(16, 8, 128, 40), (16, 8, 128, 0), (12, 4, 256, 40)])
+def test_blocks_even_themselves_out_over_sequences_of_different_lengths(lens, Hq, Hkv, D, n_tail):
+    """Batches whose blocks work their split out from all lengths: an empty sequence, lengths off every boundary, all alike and one
+    sequence alone, against the general kernel on the same lengths."""
+    require_gpu()
+    B, n, gen = len(lens), 4352, torch.Generator(device="cuda").manual_seed(sum(lens) + D)
+    k, v = (torch.randn((B, Hkv, n, D), generator=gen, device="cuda").half() for _ in range(2))
+    q = torch.randn((B, Hq, 1, D), generator=gen, device="cuda").half()
+    kp, ks, kz = K.kivi_quant_pack(k, -2, 32, 2, meta_dtype=torch.float16)
+    vp, vs, vz = K.kivi_quant_pack(v, -1, 32, 2, meta_dtype=torch.float16, v_layout="token")
+    kw = dict(k_packed=kp, k_scale=ks, k_zero=kz, v_packed=vp, v_scale=vs, v_zero=vz, n_packed=n, bits=2, group_size=32, v_layout="token",
+              scale=D ** -0.5, out_dtype=torch.float32, packed_lens=torch.tensor(lens, dtype=torch.int32, device="cuda"))
+    tails = [0 if m == 0 else min(n_tail, 7 * i + 1) for i, m in enumerate(lens)]
+    if n_tail:
+        kw.update(k_tail=k[:, :, :n_tail].contiguous(), v_tail=v[:, :, :n_tail].contiguous(), n_tail=n_tail)
+    kw["tail_lens"] = torch.tensor(tails, dtype=torch.int32, device="cuda")
+    plan = {}
+    out = K.kivi_packed_attend(q, _plan_out=plan, **kw)
+    assert plan["path"] == 1 and plan["nparts"] >= 6, plan
+    ref = K.kivi_packed_attend(q, num_splits=-1, **kw)
+    assert torch.isfinite(out).all() and float((out - ref).abs().max()) < TOL

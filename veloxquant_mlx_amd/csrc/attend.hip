@@ -19,10 +19,27 @@ constexpr int64_t TAIL_EQUIV = 4;
 // More splits over two and three rounds lose (104 tiles of 32900 tokens, 2 / 4 / 7 splits: 170 / 178 / 187 us; of 8320 60 / 82 / 98): the CUs
 // that a round leaves idle cost less than another round's start.  The exception is a chip half idle over long runs: 130 tiles
 // of 20011 tokens 165 us as one split, 148 as three (160 tiles 196 / 193); of 8320 88 / 91.
-// A batch with lengths keeps the rounded-up number: its shorter sequences leave blocks without work.
+//
+// A batch with lengths: the splits are cut by the longest sequence, shorter ones leave blocks without work.  Where rounding up gives more
+// blocks than one round, over more than 4096 tokens of many tiles, the launch takes half as many blocks again and they
+// even themselves out by the lengths (even_split): two steps over sequences of a third to the whole of the length, rounded up / evened,
+// 13 x 20011 tokens of 40 / 10 heads 178 / 107 us, 7 x 32900 154 / 85, 13 x 8320 of 32 / 8 74 / 62, 11 x 32900 of 28 / 4 107 / 80, heads
+// of 256 channels 7 x 20011 120 / 94, 11 x 20011 168 / 111.  The evening costs a launch 1 to 2 us and the merge more records: fewer tiles stay
+// rounded up (20 tiles of 20011 tokens 49 / 55, 30 47 / 54, heads of 256 20 tiles of 8320 78 / 81), and short contexts are rounded down (7 x 2000 tokens of
+// 40 / 10 heads 47 / 32, 13 x 2000 51 / 39; 7 of 32 / 8, five splits of 56 tiles, 32 / 37).
+enum class RaggedSplits { UP, DOWN, EVEN };
+static RaggedSplits ragged_splits(const AttendCall &a, int64_t units, int64_t n) {
+    const int64_t up = cdiv(256, units), blocks = cdiv(n, cdiv(cdiv(n > 0 ? n : 1, up), 128) * 128) * units;
+    if (units < (a.D == 128 ? 44 : 28) || units > 170 || blocks <= 256 || a.B < 2 || a.B > 64) return RaggedSplits::UP;
+    if (n > 4096 && a.few_parts == 0) return RaggedSplits::EVEN;
+    // an odd number of splits spreads the blocks without work over the XCDs, so that a few blocks too many find room
+    return blocks <= 288 && blocks / units % 2 != 0 ? RaggedSplits::UP : RaggedSplits::DOWN;
+}
 static int64_t decode_splits(const AttendCall &a, int64_t units, int64_t n) {
-    if (a.packed_lens != nullptr) return cdiv(256, units);
-    if (units > 128 && units <= 170 && n > 16384) return 3;
+    const RaggedSplits r = a.packed_lens != nullptr ? ragged_splits(a, units, n) : RaggedSplits::DOWN;
+    if (r == RaggedSplits::EVEN) return 384 / units;
+    if (r == RaggedSplits::UP) return cdiv(256, units);
+    if (a.packed_lens == nullptr && units > 128 && units <= 170 && n > 16384) return 3;
     return units < 256 ? 256 / units : 1;
 }
 
@@ -107,6 +124,7 @@ AttendPlan plan_attend(const AttendCall &a) {
     // 128, eight units a wave / one: blocks of 2200 tokens (16 x 4000 at 2 and 4 bits, 8 x 8000) 24.9 / 22.9, 24.6 / 23.4, 23.9 / 22.4
     // us, of 600 (16 x 1000) 15.1 / 13.2, of 4200 (16 x 8000, 8 x 16000) 31.4 / 33.2, 31.9 / 34.2; the line is drawn between.
     p.nparts = p.nsplit;
+    p.even = p.path == 1 && a.num_splits == 0 && a.packed_lens != nullptr && ragged_splits(a, units, n_split) == RaggedSplits::EVEN;
     if (p.path == 1 && a.n_tail > 0) {
         int64_t tw = cdiv(cdiv(a.n_tail, 32), units >= 64 && (len > 3072 || a.few_parts != 0) ? 8 : 1);
         // (a head of 256 channels: the tail launch of the vector kernel, up to four runs of at least 16 tokens)

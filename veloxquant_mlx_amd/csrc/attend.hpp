@@ -64,6 +64,8 @@ struct AttendPlan {
     // MFMA decode path: deal token chunks to the waves round robin instead of on demand, so that
     // results are identical from run to run
     int fixed_order;
+    // MFMA decode path, sequences of different lengths: the blocks work split_len out from all lengths (at least the one above)
+    int even = 0;
     // rows kernel over the tail only: first partial it writes (-1: the whole context, partials 0 .. nsplit - 1)
     int part0 = -1;
 };

@@ -713,9 +713,59 @@ __device__ __forceinline__ void packed_units(const AttendCall &a, int64_t bh, fl
     }
 }
 
+__device__ __forceinline__ u32 wave_sum_u32(u32 x) {
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, true);    // quad_perm [1,0,3,2]
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, true);    // quad_perm [2,3,0,1]
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x141, 0xF, 0xF, true);   // row_half_mirror
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x140, 0xF, 0xF, true);   // row_mirror
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    x = r[0] + r[1];
+    const auto h = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return uniform(h[0] + h[1]);
+}
+// sum over lanes 0 .. lane
+__device__ __forceinline__ u32 wave_scan_u32(u32 x, int lane) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const u32 y = (u32)__shfl_up((int)x, o);
+        x += lane >= o ? y : 0u;
+    }
+    return x;
+}
+// Which tile and split a block takes in a batch whose sequences differ in length (up to 64 of them), and the tokens of a split: the
+// fewest, in whole 128s, with which the splits that hold tokens are one round of blocks.  The host knows the longest sequence
+// only: cut by that length every block of it is as long as if all sequences were.  The launch has half as many blocks again as CUs;
+// those with tokens come first in the order the chip starts them (XCDs in turn), the others end at once.
+struct EvenSplit { int by, sp; int64_t len; };
+__device__ __forceinline__ EvenSplit even_split(const AttendCall &a, int64_t split_len, int64_t tail_equiv, int lane) {
+    u32 n = 0;   // tokens of sequence `lane`, in 128s
+    const bool there = lane < (int)a.B;
+    if (there) {
+        const int64_t *lens = seq_lens(a);
+        int64_t t = lens != nullptr ? lens[lane] : a.packed_lens[lane];
+        if (t > a.n_packed) t = a.n_packed;
+        n = (u32)(((t < 0 ? 0 : t) + tail_equiv + 127) / 128);
+    }
+    const u32 per = gridDim.y / (u32)a.B;   // tiles of a sequence
+    u32 len = (u32)(((uint64_t)wave_sum_u32(n) * per + 255) / 256), splits;
+    if (len < (u32)(split_len / 128)) len = (u32)(split_len / 128);
+    for (;; len += (len + 15) / 16) {   // (at one split a sequence there are at most 170)
+        splits = (n + len - 1) / len;
+        if (wave_sum_u32(splits) * per <= 256) break;
+    }
+    const u32 lin = blockIdx.x + gridDim.x * blockIdx.y, live = wave_sum_u32(splits) * per;
+    const bool empty = lin >= live;
+    const u32 mine = !there ? 0u : empty ? gridDim.x - splits : splits;   // blocks of a tile of the lane's sequence, of this kind
+    const u32 upto = wave_scan_u32(mine * per, lane), at = empty ? lin - live : lin;
+    const int b = uniform((u32)__popcll(__ballot(there && upto <= at)));
+    const u32 of_tile = (u32)__builtin_amdgcn_readlane((int)mine, b), before = (u32)__builtin_amdgcn_readlane((int)upto, b) - of_tile * per;
+    const u32 t = (at - before) / of_tile, i = (at - before) - t * of_tile;
+    return {(int)((u32)b * per + t), (int)(empty ? (u32)__builtin_amdgcn_readlane((int)splits, b) + i : i), (int64_t)len * 128};
+}
+
 // grid (nsplit, B*Hkv*tiles), Ring<...>::THREADS threads.  A block works on one tile of query rows (the GQA
 // group at pq consecutive positions; of a group of more than eight heads, eight at one position) and on packed tokens
-// [max(0, x*split_len - tail_equiv), min(n_packed, (x+1)*split_len - tail_equiv)), cut to what the
+// [max(0, x*split_len - tail_equiv), min(n_packed, (x+1)*split_len - tail_equiv)) (order, bit 2: split_len from the sequences' lengths), cut to what the
 // tile sees; in the block of split 0 the last nparts - nsplit waves first run the fp16 tail, each
 // into a partial slot of its own.  With sync counters the block that finishes last for its tile
 // merges the nparts partials into the output.
@@ -750,8 +800,14 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
         if (sizeof(M) == 2) reinterpret_cast<u32 *>(s_const)[tid] = tid < 16 ? 0x3C003C00u : 0u;
         else reinterpret_cast<u32 *>(s_const)[tid] = tid < 32 ? __float_as_uint(1.f) : 0u;
     }
-    const int by = blockIdx.y;
-    const int sp = (int)blockIdx.x, nsplit = (int)gridDim.x;
+    int by = blockIdx.y, sp = (int)blockIdx.x;
+    const int nsplit = (int)gridDim.x;
+    if (order & 4) {
+        const EvenSplit e = even_split(a, split_len, tail_equiv, lane);
+        by = e.by;
+        sp = e.sp;
+        split_len = e.len;
+    }
     // A short context's launch is bound by the instructions on its way, most of them fetched for the first time (~10 ns
     // each at one wave a SIMD), not by bytes: 32-bit divisions, and none where there is one tile.
     const int bh32 = tiles == 1 ? by : by / tiles, b32 = bh32 / (int)a.Hkv;
@@ -946,7 +1002,7 @@ static void launch_mfma_packed(const AttendCall &a, const AttendPlan &p, float *
         }                                                                                                              \
         hipLaunchKernelGGL((attend_mfma_packed_kernel<BITS, M, GV, RTP, DH>), grid, dim3(RGL::THREADS),                \
                            ring_bytes, st, a, p.split_len,                                                             \
-                           p.tail_equiv, p.nparts, p.pq, p.tiles, p.fixed_order, ws);                                  \
+                           p.tail_equiv, p.nparts, p.pq, p.tiles, p.fixed_order | (p.even ? 4 : 0), ws);                                  \
     } while (0)
     if (a.pack_bits == 4) {
         if (gv == DH) VQ_LAUNCH(4, DH); else if (gv == 2 * DH) VQ_LAUNCH(4, 2 * DH); else VQ_LAUNCH(4, 4 * DH);
