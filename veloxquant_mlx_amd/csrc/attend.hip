@@ -39,7 +39,8 @@ static int64_t decode_splits(const AttendCall &a, int64_t units, int64_t n) {
     const RaggedSplits r = a.packed_lens != nullptr ? ragged_splits(a, units, n) : RaggedSplits::DOWN;
     if (r == RaggedSplits::EVEN) return 384 / units;
     if (r == RaggedSplits::UP) return cdiv(256, units);
-    if (a.packed_lens == nullptr && units > 128 && units <= 170 && n > 16384) return 3;
+    // (scratch of a fixed size held two splits of these, and may not hold three)
+    if (a.packed_lens == nullptr && units > 128 && units <= 170 && n > 16384 && a.few_parts == 0) return 3;
     return units < 256 ? 256 / units : 1;
 }
 
