@@ -349,7 +349,9 @@ typedef struct vq_attend_args {
     const void *v_new;
     /* Order in which the decode kernel's waves take token chunks, for this call:
      * 0 = the process default (vq_kivi_attend_fixed_order), 1 = a fixed order (identical bits
-     * from run to run), 2 = on demand (fastest; the last bits can differ between runs). */
+     * from run to run, and the context cut by the shapes alone: a sequence's bits do not depend on the
+     * lengths beside it), 2 = on demand (fastest; the last bits can differ between runs, and with
+     * num_splits = 0 the launch may cut the contexts by all lengths of the batch). */
     int32_t fixed_order;
     /* > 0: a query at position p of the sequence (queries align to the end of the slots) sees
      * only the slots (p - sliding_window, p], with or without `causal` -- the window of

@@ -93,6 +93,25 @@ def test_lengths_of_a_batch_in_the_launch(D, Hq, H, bits, dtype):
     assert torch.equal(got, own_half_of_paired_output(want, H) if pairs else want)
 
 
+@pytest.mark.parametrize("D,Hq,H,B,ctx,bits,dtype", [(128, 32, 8, 9, 4700, 2, torch.float16), (128, 14, 2, 26, 9000, 4, torch.bfloat16),
+                                                     (64, 16, 16, 7, 6000, 2, torch.float16), (256, 12, 4, 7, 8700, 2, torch.bfloat16)])
+def test_a_sequences_bits_do_not_depend_on_the_lengths_beside_it(D, Hq, H, B, ctx, bits, dtype):
+    """Under a fixed order, of batches whose blocks are cut by all lengths otherwise: sequences of different lengths against batches
+    whose sequences all have one of these lengths, bit for bit, and the cut by all lengths against the oracle's bar."""
+    require_gpu()
+    c, _, rand = _cache(D, bits, 32, B, H, ctx, dtype, D + B)
+    q, scale = rand(B, Hq, 1, D).to(dtype), D ** -0.5
+    lens = torch.tensor([c.offset - (i * 997) % (ctx - 1) for i in range(B)], device="cuda")
+    got = c.fused_sdpa(q, scale, lengths=lens, fixed_order=True)
+    for i, n in enumerate(lens.tolist()):
+        alike = torch.full((B,), n, device="cuda")
+        assert torch.equal(got[i], c.fused_sdpa(q, scale, lengths=alike, fixed_order=True)[i]), (i, n)
+    lists = _clamped_lists(c, pad_queries_for_paired_heads(q, H) if D == 64 else q, lens, scale)
+    assert torch.equal(got, own_half_of_paired_output(lists, H) if D == 64 else lists)
+    on_demand = c.fused_sdpa(q, scale, lengths=lens, fixed_order=False)
+    assert float((on_demand.float() - got.float()).abs().max()) < (2e-3 if dtype == torch.float16 else 1.6e-2)
+
+
 def _clamped_lists(c, q, lens, scale, window=0):
     """The call with two clamped lists of lengths in place of one length a sequence."""
     nq, n_tail = c._n_quantized, c.offset - c._n_quantized

@@ -435,7 +435,8 @@ class KIVIKVCache(FP16KVCache):
         device or the host) gives every sequence of a right-padded batch its own number of live
         tokens: sequence ``b`` attends over its first ``lengths[b]`` slots, its queries aligned to
         the end of those.  ``num_splits`` > 0 fixes into how many runs the context is cut (0: chosen from the
-        shapes; two calls that are to agree bit for bit need the same cut as well as ``fixed_order``)."""
+        shapes, without ``fixed_order`` also by all ``lengths`` of the batch; two calls that are to agree bit for
+        bit need the same cut as well as ``fixed_order``)."""
         if not self._fused_enabled:
             raise RuntimeError("KIVIKVCache.fused_sdpa called but fused_sdpa was not enabled via "
                                "KVCacheConfig.fused_sdpa=True.")

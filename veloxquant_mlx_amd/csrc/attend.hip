@@ -27,16 +27,17 @@ constexpr int64_t TAIL_EQUIV = 4;
 // of 256 channels 7 x 20011 120 / 94, 11 x 20011 168 / 111.  The evening costs a launch 1 to 2 us and the merge more records: fewer tiles stay
 // rounded up (20 tiles of 20011 tokens 49 / 55, 30 47 / 54, heads of 256 20 tiles of 8320 78 / 81), and short contexts are rounded down (7 x 2000 tokens of
 // 40 / 10 heads 47 / 32, 13 x 2000 51 / 39; 7 of 32 / 8, five splits of 56 tiles, 32 / 37).
+// Not under a fixed order, whose cut is that of the shapes: a sequence's bits do not depend on the lengths beside it.
 enum class RaggedSplits { UP, DOWN, EVEN };
-static RaggedSplits ragged_splits(const AttendCall &a, int64_t units, int64_t n) {
+static RaggedSplits ragged_splits(const AttendCall &a, int fixed_order, int64_t units, int64_t n) {
     const int64_t up = cdiv(256, units), blocks = cdiv(n, cdiv(cdiv(n > 0 ? n : 1, up), 128) * 128) * units;
     if (units < (a.D == 128 ? 44 : 28) || units > 170 || blocks <= 256 || a.B < 2 || a.B > 64) return RaggedSplits::UP;
-    if (n > 4096 && a.few_parts == 0) return RaggedSplits::EVEN;
+    if (n > 4096 && a.few_parts == 0) return fixed_order != 0 ? RaggedSplits::UP : RaggedSplits::EVEN;
     // an odd number of splits spreads the blocks without work over the XCDs, so that a few blocks too many find room
     return blocks <= 288 && blocks / units % 2 != 0 ? RaggedSplits::UP : RaggedSplits::DOWN;
 }
-static int64_t decode_splits(const AttendCall &a, int64_t units, int64_t n) {
-    const RaggedSplits r = a.packed_lens != nullptr ? ragged_splits(a, units, n) : RaggedSplits::DOWN;
+static int64_t decode_splits(const AttendCall &a, int fixed_order, int64_t units, int64_t n) {
+    const RaggedSplits r = a.packed_lens != nullptr ? ragged_splits(a, fixed_order, units, n) : RaggedSplits::DOWN;
     if (r == RaggedSplits::EVEN) return 384 / units;
     if (r == RaggedSplits::UP) return cdiv(256, units);
     // (scratch of a fixed size held two splits of these, and may not hold three)
@@ -109,7 +110,7 @@ AttendPlan plan_attend(const AttendCall &a) {
     // or an eight-wave block per kv head (MFMA)
     const int64_t units = p.path == 1 ? a.B * a.Hkv * p.tiles : a.B * a.Hq * a.Sq;
     int64_t ns = a.num_splits;   // < 0: choose as well
-    if (ns <= 0) ns = p.path == 1 ? decode_splits(a, units > 0 ? units : 1, n_split) : cdiv(4096, units > 0 ? units : 1);
+    if (ns <= 0) ns = p.path == 1 ? decode_splits(a, p.fixed_order, units > 0 ? units : 1, n_split) : cdiv(4096, units > 0 ? units : 1);
     if (ns > max_splits) ns = max_splits;
     if (ns > 512) ns = 512;
     if (ns < 1) ns = 1;
@@ -125,7 +126,7 @@ AttendPlan plan_attend(const AttendCall &a) {
     // 128, eight units a wave / one: blocks of 2200 tokens (16 x 4000 at 2 and 4 bits, 8 x 8000) 24.9 / 22.9, 24.6 / 23.4, 23.9 / 22.4
     // us, of 600 (16 x 1000) 15.1 / 13.2, of 4200 (16 x 8000, 8 x 16000) 31.4 / 33.2, 31.9 / 34.2; the line is drawn between.
     p.nparts = p.nsplit;
-    p.even = p.path == 1 && a.num_splits == 0 && a.packed_lens != nullptr && ragged_splits(a, units, n_split) == RaggedSplits::EVEN;
+    p.even = p.path == 1 && a.num_splits == 0 && a.packed_lens != nullptr && ragged_splits(a, p.fixed_order, units, n_split) == RaggedSplits::EVEN;
     if (p.path == 1 && a.n_tail > 0) {
         int64_t tw = cdiv(cdiv(a.n_tail, 32), units >= 64 && (len > 3072 || a.few_parts != 0) ? 8 : 1);
         // (a head of 256 channels: the tail launch of the vector kernel, up to four runs of at least 16 tokens)
@@ -276,7 +277,8 @@ static size_t attend_workspace(const AttendCall *a) {
     if (!a || a->B < 1 || a->Hq < 1 || a->Hkv < 1 || a->Sq < 1 || a->D < 1 || a->Hq % a->Hkv != 0 ||
         a->n_packed < 0 || a->n_tail < 0 || (a->n_packed > 0 && (a->pack_bits < 1 || a->pack_bits > 8 || a->group < 1)))
         return 0;
-    const AttendCall w = skip_below_window(*a);
+    AttendCall w = skip_below_window(*a);
+    w.fixed_order = 2;   // the order that takes the most partials: the process default may change between this query and the launch
     if (const int64_t Rp = padded_group(w)) {
         // the padded call's own workspace, then its queries and its outputs
         AttendCall b = *a;

@@ -119,8 +119,8 @@ __device__ __forceinline__ float merge_records(const float *p, int nparts, int64
 }
 
 
-// Decides kernel and split count from shapes only, so that the workspace query
-// and the launch agree.
+// Decides kernel and split count from shapes, whether there are lengths and the order, so that the workspace query (which
+// takes the order with the most partials) covers the launch.
 AttendPlan plan_attend(const AttendCall &a);
 
 int launch_attend_generic(const AttendCall &a, int nsplit, int64_t split_len);
