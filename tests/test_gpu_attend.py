@@ -198,6 +198,25 @@ def test_causal_tiles_of_any_number_of_heads_land_once_each(B, Hq, Hkv, Sq, D):
         assert err < TOL
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,window", [(7, 64, 8, 1024, 0), (7, 64, 8, 1000, 77), (6, 64, 8, 1024, 0), (9, 64, 8, 992, 0)])
+def test_causal_tiles_over_many_rounds_of_blocks(B, Hq, Hkv, Sq, window):
+    """Around the line from which on a head's tiles stay together (32 tiles a head, six rounds of 32 blocks an XCD): every sequence has the
+    bits of the launch over it alone, and those are within the bar of float32 attention."""
+    require_gpu()
+    D, gen = 128, torch.Generator(device="cuda").manual_seed(B + Sq)
+    q = torch.randn((B, Hq, Sq, D), generator=gen, device="cuda").half()
+    k, v = (torch.randn((B, Hkv, Sq, D), generator=gen, device="cuda").half() for _ in range(2))
+    ref = oa.sdpa(host(q[:1, :8]), host(k[:1, :1]), host(v[:1, :1]), D ** -0.5, causal=True, sliding_window=window)
+    for splits in (1, 3):
+        kw = dict(n_tail=Sq, scale=D ** -0.5, causal=True, out_dtype=torch.float32, num_splits=splits, sliding_window=window)
+        plan = {}
+        out = K.kivi_packed_attend(q, k_tail=k, v_tail=v, _plan_out=plan, **kw)
+        assert plan == {"path": 2, "nparts": splits}
+        for b in range(B):
+            assert torch.equal(out[b], K.kivi_packed_attend(q[b:b + 1], k_tail=k[b:b + 1], v_tail=v[b:b + 1], **kw)[0]), b
+        assert float(np.max(np.abs(host(out[:1, :8]) - ref))) < TOL
+
+
 def test_flash_prefill_large_logits_bf16_and_future_keys():
     """test_flash_prefill.py:141-151: logits three times as wide (score std ~ 9) stay within the
     reference's 2e-2 -- here within 4e-3, the scores being accumulated in float32; bf16 keys and

@@ -505,13 +505,23 @@ template <int BITS, typename M> struct PrStage {
 // HBM for itself (68 MB per launch at config 4 for 15 MB of input).  A head's blocks share an XCD (a multiple of eight
 // heads) or 8 / heads of them (1, 2 or 4 heads).
 // Under a causal mask a tile's work grows with its number, so all heads' longest tiles (numbered from the end) come first
-// and the short ones fill what is left: 4096 tokens of 32 heads, two rounds of blocks, 179
-// us against 253 with one head's tiles after the other's (the last head's longest tile then starts when the chip is half
+// and the short ones fill what is left: 4096 tokens of 32 heads, two rounds of blocks, 174
+// us against 251 with one head's tiles after the other's (the last head's longest tile then starts when the chip is half
 // done); chunks of 2048 of 2 x 40 heads 1081 against 1236 a pass of three.
-// Without one all blocks are alike and a head's stay together.
+// An XCD then reads the rows of all its heads at once (4096 tokens of 32 heads: 66 MB fetched against 49, 8192: 497 against 190), and over many
+// rounds of blocks that costs more than the even end gives.  Where a head alone fills an XCD (32 tiles for its 32 CUs) and the XCD has
+// more than PR_ROUNDS rounds, a head's tiles stay together, longest first: causal rows of 128 channels, all heads at once / head after head,
+// 32 heads of 8192 (4 rounds) 609 / 618 us, 12288 (6) 1295 / 1297, 14000 (7) 1702 / 1671, 16384 (8) 2315 / 2224 (2.1 GB fetched / 455 MB), 40 of 16384
+// (10) 2944 / 2791, 64 of 8192 (8) 1290 / 1272, of 12288 (12) 2790 / 2637; but 128 heads of 4096, 16 tiles each (8 rounds), 714 / 803, and 32 heads of 256
+// channels of 8192 (a block takes twice as long for the same rows) 3383 / 3706.  Head counts that are no multiple of eight
+// have every head on all XCDs either way and keep this order (20 heads of 16384 1400 / 1778).
+// Without a mask all blocks are alike and a head's stay together.
+constexpr unsigned PR_ROUNDS = 6, PR_XCD_CUS = 32;
 struct BlockPlace { unsigned tile, bh, run; };
-__device__ __forceinline__ BlockPlace place_block(bool causal) {
+template <unsigned ROUNDS> __device__ __forceinline__ BlockPlace place_block(bool causal) {
     const unsigned lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const unsigned per_head = gridDim.x * gridDim.z;
+    if (gridDim.y % 8 == 0 && per_head >= PR_XCD_CUS && gridDim.y / 8 * per_head > ROUNDS * PR_XCD_CUS) causal = false;
     if (causal || 8 % gridDim.y == 0) {
         const unsigned within = lin / gridDim.y;
         const unsigned bh = lin - within * gridDim.y;
@@ -519,7 +529,7 @@ __device__ __forceinline__ BlockPlace place_block(bool causal) {
         return {within % gridDim.x, bh, within / gridDim.x};
     }
     if (gridDim.y % 8 != 0) return {blockIdx.x, blockIdx.y, blockIdx.z};
-    const unsigned per_head = gridDim.x * gridDim.z, slot = lin / 8, within = slot % per_head;
+    const unsigned slot = lin / 8, within = slot % per_head;
     return {within % gridDim.x, lin % 8 + 8 * (slot / per_head), within / gridDim.x};
 }
 
@@ -551,7 +561,7 @@ void attend_prefill_rows_kernel(vq_attend_args a, int qp, int nparts, float *__r
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, blk = lane >> 4;
-    const BlockPlace place = place_block(a.causal != 0);
+    const BlockPlace place = place_block<PR_ROUNDS>(a.causal != 0);
     const unsigned tile_x = place.tile, run_z = place.run;
     const int64_t bh = place.bh;
     const int64_t hkv = bh % a.Hkv, b = bh / a.Hkv;
@@ -1008,7 +1018,7 @@ void attend_prefill_rows_d256_kernel(vq_attend_args a, int qp, int nparts, int v
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, blk = lane >> 4;
-    const BlockPlace place = place_block(a.causal != 0);
+    const BlockPlace place = place_block<~0u / PR_XCD_CUS>(a.causal != 0);
     const unsigned tile_x = place.tile, run_z = place.run;
     const int64_t bh = place.bh;
     const int64_t hkv = bh % a.Hkv, b = bh / a.Hkv;
