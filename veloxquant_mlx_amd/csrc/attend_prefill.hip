@@ -539,10 +539,11 @@ template <unsigned ROUNDS> __device__ __forceinline__ BlockPlace place_block(boo
 template <int BITS, int GV, typename M, bool TILES = false>
 __global__ __launch_bounds__(PR_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attend_prefill_rows_kernel(vq_attend_args a, int qp, int nparts, float *__restrict__ ws) {
-    // The loop over units is 13.5 KB of straight code, and where it lies modulo the 32 bytes of an instruction fetch moves a launch by
-    // up to 3 %: 4096 causal tokens of 32 heads, 250.5 to 254.9 us over eight places.  Two instructions ahead of everything put
-    // that of the instantiation for plain fp16 rows on a boundary of 32 (251.4; without them 24 bytes past one, 253.5).
-    if constexpr (!TILES) asm volatile("s_nop 0\n\ts_nop 0");
+    // The loop over units is 13.5 KB of straight code, and where it lies modulo an instruction fetch moves a launch by 1 to 3 %.  Any change
+    // of the code ahead of it moves it.  Plain fp16 rows, 4096 causal tokens of 32 heads, by the number of
+    // instructions put here (0 to 7: the loop 40, 44, .. 60, 0, 4 bytes past a multiple of 64): 169.6, 170.5, 170.2, 170.5, 171.7, 169.1, 170.7,
+    // 169.8 us, the same order at 2048 to 5000 tokens.  The tile form shows no such differences (16384 tokens 2155 to 2209 us at any).
+    if constexpr (!TILES) asm volatile("s_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
     __shared__ __align__(16) f16 s_k[TILES ? 1 : 3][32 * PF_KSTRIDE];
     __shared__ __align__(16) f16 s_v[TILES ? 1 : 3][MF_D * PF_VSTRIDE];
     __shared__ __align__(16) char s_ring[TILES ? 4 * PF_TILE_BYTES : 16];
