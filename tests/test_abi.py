@@ -129,19 +129,20 @@ def test_half_a_pair_of_length_lists_is_refused():
     assert lib.vq_kivi_attend_ext(a, _lib.AttendExt(0, 4096)) == _lib.VQ_ERR_INVALID and "exclude" in _lib.last_error()
 
 
-@pytest.mark.parametrize("D,Hq,Hkv,B,n_packed,n_tail", [
-    (128, 32, 8, 6, 4224, 140), (128, 32, 8, 9, 8192, 0), (128, 40, 10, 9, 20000, 150), (128, 28, 4, 15, 32768, 129), (128, 8, 1, 50, 4096, 33),
-    (256, 12, 4, 7, 8960, 140), (256, 12, 4, 10, 20000, 0), (256, 8, 4, 10, 20000, 1)])
-def test_a_fixed_order_cuts_by_shapes_alone(D, Hq, Hkv, B, n_packed, n_tail):
+@pytest.mark.parametrize("D,Hq,Hkv,B,n_packed,n_tail,splits", [
+    (128, 40, 10, 2, 32000, 100, 13), (128, 28, 4, 9, 8192, 150, 7), (128, 32, 8, 6, 4224, 140, 5), (128, 32, 8, 9, 8192, 0, 3),
+    (128, 40, 10, 9, 20000, 150, 3), (128, 28, 4, 15, 32768, 129, 4), (128, 8, 1, 50, 4096, 33, 5), (256, 12, 4, 6, 20000, 140, 11),
+    (256, 12, 4, 7, 8960, 140, 9), (256, 12, 4, 10, 20000, 0, 7), (256, 8, 4, 10, 20000, 1, 7)])
+def test_a_fixed_order_cuts_by_shapes_alone(D, Hq, Hkv, B, n_packed, n_tail, splits):
     """Sequences of different lengths: on demand the blocks cut every sequence by all lengths of the batch; under a fixed order, asked
-    for by the call or the process, the launch has the splits of the shapes (as many as give every CU a block).  The workspace is
-    the larger of the two, whichever order the query or the process names."""
+    for by the call or the process, or where another launch merges, the launch has the splits of the shapes.  The workspace is the larger of the two, whichever order the query or the process names."""
     lib = _lib.load()
     a = _lib.AttendArgs()
     a.B, a.Hq, a.Hkv, a.Sq, a.D, a.n_packed, a.n_tail = B, Hq, Hkv, 1, D, n_packed, n_tail
     a.pack_bits, a.group, a.meta_dtype, a.v_layout, a.cap_tokens, a.tail_cap = 2, 32, 0, 1, 32768, 768
     a.scale = 0.1
-    for f in ("q", "out", "k_packed", "k_scale", "k_zero", "v_packed", "v_scale", "v_zero", "k_tail", "v_tail", "packed_lens", "tail_lens"):
+    for f in ("q", "out", "k_packed", "k_scale", "k_zero", "v_packed", "v_scale", "v_zero", "k_tail", "v_tail", "packed_lens", "tail_lens",
+              "sync_counters"):
         setattr(a, f, 4096)
 
     def nparts(order, num_splits=0):
@@ -150,9 +151,14 @@ def test_a_fixed_order_cuts_by_shapes_alone(D, Hq, Hkv, B, n_packed, n_tail):
         assert lib.vq_kivi_attend_plan(a, ctypes.byref(path), ctypes.byref(n)) == 0 and path.value == 1
         return n.value
 
-    by_shapes = nparts(1, -(-256 // (B * Hkv)))
+    by_shapes = nparts(1, splits)
     assert nparts(2) > by_shapes   # (a shape that is evened)
     assert nparts(1) == nparts(3) == by_shapes
+    for field in ("sync_counters", "sink_k"):   # another launch reads the partials: cut by the shapes
+        was, a.sink_v, a.sink_pos, a.sink_cap = getattr(a, field), 4096, 4096, 1
+        setattr(a, field, None if was else 4096)
+        assert nparts(2) == by_shapes
+        setattr(a, field, was)
     before = lib.vq_kivi_attend_fixed_order(1)
     try:
         assert nparts(0) == by_shapes and nparts(2) > by_shapes

@@ -817,13 +817,15 @@ def test_a_decode_launch_takes_the_splits_of_one_round(B, Hkv, n, nparts):
     assert float((out - K.kivi_packed_attend(q, num_splits=-1, **kw)).abs().max()) < TOL
 
 
-@pytest.mark.parametrize("lens", [(4352, 0, 31, 4351, 2000, 128, 4000), (4352,) * 7, (4352, 0, 0, 0, 0, 0, 0), (0, 0, 0, 0, 0, 0, 96)])
-@pytest.mark.parametrize("Hq,Hkv,D,n_tail", [(16, 8, 128, 40), (16, 8, 128, 0), (12, 4, 256, 40)])
-def test_blocks_even_themselves_out_over_sequences_of_different_lengths(lens, Hq, Hkv, D, n_tail):
+@pytest.mark.parametrize("lens", [(1., 0, 31, 1 - 1e-9, .46, 128, .92), (1.,) * 7, (1., 0, 0, 0, 0, 0, 0), (0, 0, 0, 0, 0, 0, 96)])
+@pytest.mark.parametrize("Hq,Hkv,D,n,n_tail,nparts", [(16, 8, 128, 4352, 40, 8), (16, 8, 128, 4352, 0, 6), (12, 4, 256, 8960, 40, 15),
+                                                      (8, 4, 256, 8960, 0, 12), (80, 10, 128, 8192, 300, 13)])
+def test_blocks_even_themselves_out_over_sequences_of_different_lengths(lens, Hq, Hkv, D, n, n_tail, nparts):
     """Batches whose blocks work their split out from all lengths: an empty sequence, lengths off every boundary, all alike and one
-    sequence alone, against the general kernel on the same lengths."""
+    sequence alone, against the general kernel on the same lengths.  nparts is the evened launch's; the cut by the shapes has another."""
     require_gpu()
-    B, n, gen = len(lens), 4352, torch.Generator(device="cuda").manual_seed(sum(lens) + D)
+    lens = [int(x * n) if isinstance(x, float) else x for x in lens]   # (fractions of the longest, or tokens)
+    B, gen = len(lens), torch.Generator(device="cuda").manual_seed(sum(lens) + D)
     k, v = (torch.randn((B, Hkv, n, D), generator=gen, device="cuda").half() for _ in range(2))
     q = torch.randn((B, Hq, 1, D), generator=gen, device="cuda").half()
     kp, ks, kz = K.kivi_quant_pack(k, -2, 32, 2, meta_dtype=torch.float16)
@@ -834,8 +836,11 @@ def test_blocks_even_themselves_out_over_sequences_of_different_lengths(lens, Hq
     if n_tail:
         kw.update(k_tail=k[:, :, :n_tail].contiguous(), v_tail=v[:, :, :n_tail].contiguous(), n_tail=n_tail)
     kw["tail_lens"] = torch.tensor(tails, dtype=torch.int32, device="cuda")
-    plan = {}
+    plan, shapes = {}, {}
     out = K.kivi_packed_attend(q, _plan_out=plan, **kw)
-    assert plan["path"] == 1 and plan["nparts"] >= 6, plan
+    assert plan == {"path": 1, "nparts": nparts}
     ref = K.kivi_packed_attend(q, num_splits=-1, **kw)
     assert torch.isfinite(out).all() and float((out - ref).abs().max()) < TOL
+    other = K.kivi_packed_attend(q, _plan_out=shapes, _single_launch=False, **kw)   # merged by another launch: cut by the shapes
+    assert shapes["nparts"] < nparts and float((other - ref).abs().max()) < TOL
+    assert int(K._counters(q.device).abs().sum()) == 0

@@ -112,14 +112,111 @@ def test_a_sequences_bits_do_not_depend_on_the_lengths_beside_it(D, Hq, H, B, ct
     assert float((on_demand.float() - got.float()).abs().max()) < (2e-3 if dtype == torch.float16 else 1.6e-2)
 
 
-def _clamped_lists(c, q, lens, scale, window=0):
+@pytest.mark.parametrize("D,Hq,H,B,ctx,bits,Sq,window,dtype", [
+    (128, 32, 8, 7, 5100, 2, 1, 0, torch.float16),         # a token brought along by the launch
+    (128, 14, 2, 30, 4700, 4, 1, 0, torch.bfloat16),
+    (64, 16, 16, 6, 5100, 2, 1, 0, torch.float16),         # heads of 64 channels in pairs
+    (64, 9, 3, 26, 8300, 2, 1, 700, torch.bfloat16),       # an odd number of them, under a window
+    (256, 12, 4, 7, 8700, 2, 1, 0, torch.bfloat16),
+    (128, 8, 2, 13, 4800, 2, 4, 0, torch.float16),         # several positions, two row tiles a kv head
+    (128, 32, 8, 2, 6000, 4, 6, 1000, torch.float16),      # and a window
+    (128, 4, 1, 64, 4500, 2, 2, 0, torch.float16),         # as many sequences as one wave holds
+    (256, 4, 1, 64, 4500, 2, 1, 0, torch.float16)])
+def test_steps_over_evened_blocks(D, Hq, H, B, ctx, bits, Sq, window, dtype):
+    """The cut by all lengths through the cache's own entry point: one int64 length a sequence, spread over the whole context, two steps
+    with their tokens brought along where that is done, against the general kernel over the two clamped lists."""
+    require_gpu()
+    c, new, rand = _cache(D, bits, 32, B, H, ctx, dtype, D + B)
+    scale = D ** -0.5
+    lens = torch.tensor([c.offset - (i * 1009) % (ctx - Sq) for i in range(B)], device="cuda")
+    for step in range(2):
+        c.update_and_fetch(*new())
+        lens += 1
+        q = rand(B, Hq, Sq, D).to(dtype)
+        got = c.fused_sdpa(q, scale, lengths=lens, sliding_window=window)
+        wide = pad_queries_for_paired_heads(q, H) if D == 64 else q
+        plan, shapes = {}, {}
+        for single, out in ((True, plan), (False, shapes)):
+            _clamped_lists(c, wide, lens, scale, window, fixed_order=False, _single_launch=single, _plan_out=out)
+        assert plan["path"] == 1 and plan["nparts"] >= shapes["nparts"]
+        want = _clamped_lists(c, wide, lens, scale, window, fixed_order=None, num_splits=-1)
+        want = own_half_of_paired_output(want, H) if D == 64 else want
+        # (two roundings of an output of up to 4: half a unit in the last place each)
+        assert float((got.float() - want.float()).abs().max()) < (4e-3 if dtype == torch.float16 else 3.2e-2), step
+    assert int(K._counters(q.device).abs().sum()) == 0
+
+
+def test_a_stack_of_layers_of_different_lengths_over_evened_blocks():
+    """Layers whose contexts differ in length as the sequences of one launch, on demand."""
+    require_gpu()
+    NL, B, H, D, dtype = 6, 1, 8, 128, torch.float16
+    cfg = KVCacheConfig(method="kivi", head_dim=D, bit_width_inlier=2, kivi_group_size=32, residual_length=128, fused_sdpa=True,
+                        fused_sdpa_memory_bound=True, fused_sdpa_max_ctx=8192)
+    stack, gen = LayerStackedKIVICache(cfg, NL), torch.Generator(device="cuda").manual_seed(5)
+    rand = lambda *s: torch.randn(s, generator=gen, device="cuda").to(dtype)
+    for l in range(NL):
+        n = 8000 - 1303 * l
+        stack[l].update_and_fetch(rand(B, H, n, D), rand(B, H, n, D))
+    q = rand(NL, B, 32, 1, D)
+    out = stack.fused_sdpa_all(q, 0.09)
+    for l in range(NL):
+        assert float((out[l].float() - stack[l].fused_sdpa(q[l], 0.09).float()).abs().max()) < 2e-3, l
+
+
+def test_evened_blocks_in_a_graph_read_the_lengths_of_the_replay():
+    """A captured step over uneven sequences, replayed after the lengths changed, between eager steps."""
+    require_gpu()
+    B, H, D, dtype = 7, 8, 128, torch.float16
+    c, _, rand = _cache(D, 2, 32, B, H, 5100, dtype, 3)
+    q, lens, out = rand(B, 32, 1, D).to(dtype), torch.full((B,), c.offset, device="cuda"), torch.empty(B, 32, 1, D, dtype=dtype, device="cuda")
+    nq, n_tail = c._n_quantized, c.offset - c._n_quantized
+    kw = dict(k_packed=c._kp, k_scale=c._ks, k_zero=c._kz, v_packed=c._vp, v_scale=c._vs, v_zero=c._vz, n_packed=nq, bits=c._field, group_size=32,
+              v_layout=c._v_layout, k_tail=c._tail_k, v_tail=c._tail_v, n_tail=n_tail, scale=0.09)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            K.kivi_packed_attend(q, seq_lens=lens, out=out, **kw)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        K.kivi_packed_attend(q, seq_lens=lens, out=out, **kw)
+    for step in range(4):
+        lens.copy_(torch.tensor([max(1, c.offset - (i + step) * 811 * (step > 0)) for i in range(B)]))
+        out.zero_()
+        graph.replay()
+        got = out.clone()
+        eager = c.fused_sdpa(q, 0.09, lengths=lens)
+        torch.cuda.synchronize()
+        want = _clamped_lists(c, q, lens, 0.09, fixed_order=None, num_splits=-1)
+        assert float((got.float() - want.float()).abs().max()) < 2e-3 and float((eager.float() - want.float()).abs().max()) < 2e-3, step
+
+
+def test_uneven_lengths_in_the_built_in_scratch():
+    """Shapes whose evened partials exceed the built-in scratch fall back to the cut with fewer; smaller ones are evened there as well."""
+    require_gpu()
+    for B, Hq, H, D, n in ((34, 40, 5, 256, 4128), (7, 16, 8, 128, 4352)):
+        gen = torch.Generator(device="cuda").manual_seed(B)
+        k, v = (torch.randn((B, H, n, D), generator=gen, device="cuda").half() for _ in range(2))
+        q = torch.randn((B, Hq, 1, D), generator=gen, device="cuda").half()
+        kp, ks, kz = K.kivi_quant_pack(k, -2, 32, 2, meta_dtype=torch.float16)
+        vp, vs, vz = K.kivi_quant_pack(v, -1, 32, 2, meta_dtype=torch.float16, v_layout="token")
+        lens = torch.tensor([n - (i * 613) % n for i in range(B)], dtype=torch.int32, device="cuda")
+        kw = dict(k_packed=kp, k_scale=ks, k_zero=kz, v_packed=vp, v_scale=vs, v_zero=vz, n_packed=n, bits=2, group_size=32, v_layout="token",
+                  k_tail=k[:, :, :70].contiguous(), v_tail=v[:, :, :70].contiguous(), n_tail=70, scale=D ** -0.5, out_dtype=torch.float32,
+                  packed_lens=lens // 32 * 32, tail_lens=lens % 71)
+        got = K.kivi_packed_attend(q, static_scratch=True, **kw)
+        assert float((got - K.kivi_packed_attend(q, num_splits=-1, **kw)).abs().max()) < 2e-3
+
+
+def _clamped_lists(c, q, lens, scale, window=0, **more):
     """The call with two clamped lists of lengths in place of one length a sequence."""
     nq, n_tail = c._n_quantized, c.offset - c._n_quantized
     kw = dict(k_packed=c._kp, k_scale=c._ks, k_zero=c._kz, v_packed=c._vp, v_scale=c._vs, v_zero=c._vz, n_packed=nq, bits=c._field,
               group_size=c._group_size, v_layout=c._v_layout) if nq else {}
     return K.kivi_packed_attend(q, k_tail=c._tail_k, v_tail=c._tail_v, n_tail=n_tail, scale=scale, causal=q.shape[2] > 1,
-                                out_dtype=q.dtype, fixed_order=True, sliding_window=window, tiles=False,
-                                packed_lens=torch.clamp(lens, max=nq), tail_lens=torch.clamp(lens - nq, min=0, max=n_tail), **kw)
+                                out_dtype=q.dtype, sliding_window=window, tiles=False, packed_lens=torch.clamp(lens, max=nq),
+                                tail_lens=torch.clamp(lens - nq, min=0, max=n_tail), **{"fixed_order": True, **kw, **more})
 
 
 @pytest.mark.parametrize("B,Hq,H,D,Sq,window,ctx,dtype", [

@@ -21,23 +21,29 @@ constexpr int64_t TAIL_EQUIV = 4;
 // of 20011 tokens 165 us as one split, 148 as three (160 tiles 196 / 193); of 8320 88 / 91.
 //
 // A batch with lengths: the splits are cut by the longest sequence, shorter ones leave blocks without work.  Where rounding up gives more
-// blocks than one round, over more than 4096 tokens of many tiles, the launch takes half as many blocks again and they
-// even themselves out by the lengths (even_split): two steps over sequences of a third to the whole of the length, rounded up / evened,
-// 13 x 20011 tokens of 40 / 10 heads 178 / 107 us, 7 x 32900 154 / 85, 13 x 8320 of 32 / 8 74 / 62, 11 x 32900 of 28 / 4 107 / 80, heads
-// of 256 channels 7 x 20011 120 / 94, 11 x 20011 168 / 111.  The evening costs a launch 1 to 2 us and the merge more records: fewer tiles stay
-// rounded up (20 tiles of 20011 tokens 49 / 55, 30 47 / 54, heads of 256 20 tiles of 8320 78 / 81), and short contexts are rounded down (7 x 2000 tokens of
-// 40 / 10 heads 47 / 32, 13 x 2000 51 / 39; 7 of 32 / 8, five splits of 56 tiles, 32 / 37).
-// Not under a fixed order, whose cut is that of the shapes: a sequence's bits do not depend on the lengths beside it.
+// blocks than one round, over more than 4096 tokens, one round of blocks evens itself out by the lengths (even_split).  Two steps
+// over sequences of a third to the whole of the length, three draws each, at 2 bits, rounded up / rounded down / evened, us:
+//   32 / 8 heads of 128:   5 x 8700 (40 tiles)  49 39 39 / 35 34 35 / 34 33 33,  7 x 8700 (56)  41 57 41 / 40 42 41 / 36 39 36,
+//     9 x 8700 (72)  74 72 72 / 47 46 46 / 47 43 42,  9 x 20011  108 / 75 / 59 66 59,  12 x 4600 (96)  51 41 55 / 41 43 43 / 39 38 41;
+//   28 / 4 heads:   7 x 4600 (28)  39 40 36 / 34 33 33 / 33 33 32,  9 x 20011 (36)  90 / 54 / 51 53 53,  13 x 8700 (52)  48 46 60 / 48 / 40 41 41;
+//   40 / 10 heads:   2 x 32900 (20)  47 / 47 / 42 44 39,  13 x 20011 (130)  178 165 162 / 160 155 151 / 98;
+//   12 / 4 heads of 256:   6 x 20011 (24)  90 91 88 / 88 87 87 / 83 83 76,  7 x 20011 (28)  119 112 107 / 90 / 86,  10 x 8700 (40)  83 76 91 / 78 / 74 72 75,
+//     33 x 4600 (132)  162 154 152 / 138 / 108.
+// Of 12 to 16 tiles the forms are alike (0.98 to 1.02), and up to 4096 tokens evening gains and loses (48 and 50 tiles of 2000 to 3000 tokens 3 to 5 % over
+// rounding down): these are cut by the shapes.  So is a launch under a fixed order (a sequence's bits do not depend on the lengths beside it), and one
+// whose partials another launch reads (no counters, protected rows: evened tiles leave some unwritten).  The shapes round down, as without lengths, but
+// for an odd number of splits a few blocks over one round, which spreads the blocks without work over the XCDs: 88 to 96 tiles of 20011 tokens, three splits / two,
+// 81 to 101 / 95, of 8700 51 to 72 / 57; up to 4096 tokens five splits (52 and 56 tiles of 1200 28 / 30, 27 / 27, of 2000 34 / 32, 31 / 27), not
+// three (88 to 96 tiles of 2000 31 to 45 / 30 to 33), but of heads of 256 channels three as well (88 tiles of 1200 to 2000 at 4 bits 79 92 / 86 98).
 enum class RaggedSplits { UP, DOWN, EVEN };
-static RaggedSplits ragged_splits(const AttendCall &a, int fixed_order, int64_t units, int64_t n) {
-    const int64_t up = cdiv(256, units), blocks = cdiv(n, cdiv(cdiv(n > 0 ? n : 1, up), 128) * 128) * units;
-    if (units < (a.D == 128 ? 44 : 28) || units > 170 || blocks <= 256 || a.B < 2 || a.B > 64) return RaggedSplits::UP;
-    if (n > 4096 && a.few_parts == 0) return fixed_order != 0 ? RaggedSplits::UP : RaggedSplits::EVEN;
-    // an odd number of splits spreads the blocks without work over the XCDs, so that a few blocks too many find room
-    return blocks <= 288 && blocks / units % 2 != 0 ? RaggedSplits::UP : RaggedSplits::DOWN;
+static RaggedSplits ragged_splits(const AttendCall &a, bool may_even, int64_t units, int64_t n) {
+    const int64_t up = cdiv(256, units), splits = cdiv(n, cdiv(cdiv(n > 0 ? n : 1, up), 128) * 128), blocks = splits * units;
+    if (units < 20 || units > 170 || blocks <= 256 || a.B < 2 || a.B > 64) return RaggedSplits::UP;
+    if (n > 4096 && may_even && a.few_parts == 0) return RaggedSplits::EVEN;
+    return blocks <= 288 && splits % 2 != 0 && (n > 4096 || splits >= 5 || a.D != 128) ? RaggedSplits::UP : RaggedSplits::DOWN;
 }
-static int64_t decode_splits(const AttendCall &a, int fixed_order, int64_t units, int64_t n) {
-    const RaggedSplits r = a.packed_lens != nullptr ? ragged_splits(a, fixed_order, units, n) : RaggedSplits::DOWN;
+static int64_t decode_splits(const AttendCall &a, bool may_even, int64_t units, int64_t n) {
+    const RaggedSplits r = a.packed_lens != nullptr ? ragged_splits(a, may_even, units, n) : RaggedSplits::DOWN;
     if (r == RaggedSplits::EVEN) return 384 / units;
     if (r == RaggedSplits::UP) return cdiv(256, units);
     // (scratch of a fixed size held two splits of these, and may not hold three)
@@ -45,7 +51,7 @@ static int64_t decode_splits(const AttendCall &a, int fixed_order, int64_t units
     return units < 256 ? 256 / units : 1;
 }
 
-AttendPlan plan_attend(const AttendCall &a) {
+AttendPlan plan_attend(const AttendCall &a, bool widest) {
     AttendPlan p;
     // bit 0: fixed chunk order; bit 1 (fixed_order == 3): the decode kernel also waits for every copy in flight
     p.fixed_order = a.fixed_order == 1 ? 1 : a.fixed_order == 3 ? 3 : a.fixed_order == 2 ? 0 : g_fixed_order.load(std::memory_order_relaxed);
@@ -110,7 +116,8 @@ AttendPlan plan_attend(const AttendCall &a) {
     // or an eight-wave block per kv head (MFMA)
     const int64_t units = p.path == 1 ? a.B * a.Hkv * p.tiles : a.B * a.Hq * a.Sq;
     int64_t ns = a.num_splits;   // < 0: choose as well
-    if (ns <= 0) ns = p.path == 1 ? decode_splits(a, p.fixed_order, units > 0 ? units : 1, n_split) : cdiv(4096, units > 0 ? units : 1);
+    const bool may_even = widest || (p.fixed_order == 0 && a.sync_counters != nullptr && a.sink_k == nullptr);
+    if (ns <= 0) ns = p.path == 1 ? decode_splits(a, may_even, units > 0 ? units : 1, n_split) : cdiv(4096, units > 0 ? units : 1);
     if (ns > max_splits) ns = max_splits;
     if (ns > 512) ns = 512;
     if (ns < 1) ns = 1;
@@ -126,7 +133,7 @@ AttendPlan plan_attend(const AttendCall &a) {
     // 128, eight units a wave / one: blocks of 2200 tokens (16 x 4000 at 2 and 4 bits, 8 x 8000) 24.9 / 22.9, 24.6 / 23.4, 23.9 / 22.4
     // us, of 600 (16 x 1000) 15.1 / 13.2, of 4200 (16 x 8000, 8 x 16000) 31.4 / 33.2, 31.9 / 34.2; the line is drawn between.
     p.nparts = p.nsplit;
-    p.even = p.path == 1 && a.num_splits == 0 && a.packed_lens != nullptr && ragged_splits(a, p.fixed_order, units, n_split) == RaggedSplits::EVEN;
+    p.even = p.path == 1 && a.num_splits == 0 && a.packed_lens != nullptr && ragged_splits(a, may_even, units, n_split) == RaggedSplits::EVEN;
     if (p.path == 1 && a.n_tail > 0) {
         int64_t tw = cdiv(cdiv(a.n_tail, 32), units >= 64 && (len > 3072 || a.few_parts != 0) ? 8 : 1);
         // (a head of 256 channels: the tail launch of the vector kernel, up to four runs of at least 16 tokens)
@@ -277,8 +284,7 @@ static size_t attend_workspace(const AttendCall *a) {
     if (!a || a->B < 1 || a->Hq < 1 || a->Hkv < 1 || a->Sq < 1 || a->D < 1 || a->Hq % a->Hkv != 0 ||
         a->n_packed < 0 || a->n_tail < 0 || (a->n_packed > 0 && (a->pack_bits < 1 || a->pack_bits > 8 || a->group < 1)))
         return 0;
-    AttendCall w = skip_below_window(*a);
-    w.fixed_order = 2;   // the order that takes the most partials: the process default may change between this query and the launch
+    const AttendCall w = skip_below_window(*a);
     if (const int64_t Rp = padded_group(w)) {
         // the padded call's own workspace, then its queries and its outputs
         AttendCall b = *a;
@@ -288,7 +294,7 @@ static size_t attend_workspace(const AttendCall *a) {
         return round256(attend_workspace(&b)) + round256(rows * (a->q_dtype == VQ_F32 ? 4 : 2)) +
                round256(rows * (a->out_dtype == VQ_F32 ? 4 : 2));
     }
-    AttendPlan p = plan_attend(w);
+    const AttendPlan p = plan_attend(w, true);   // (the process's order may change between the query and the launch)
     if (p.path == 2 && mfma_prefill_direct_output(w, p.nparts)) return 0;   // the kernel writes `out` itself
     return (size_t)(a->B * a->Hq * a->Sq) * (size_t)p.nparts * (size_t)(a->D + 2) * sizeof(float);
 }
@@ -408,8 +414,8 @@ static int attend(const AttendCall *a_in) {
         return VQ_OK;
     };
     if (p.path == 1) {
-        if (a->D != 128 && a->n_tail > 0) {   // the tail as partial p.nsplit of every row, from the vector kernel
-            rc = launch_attend_rows_tail(*a, p.nsplit, p.nparts);
+        if (a->D != 128 && a->n_tail > 0) {   // the tail as partials of every row, behind the splits' (evened: ahead), from the vector kernel
+            rc = launch_attend_rows_tail(*a, p.even ? 0 : p.nsplit, p.nparts - p.nsplit, p.nparts);
             if (rc != VQ_OK) return rc;
             VQ_HIP_CHECK_LAUNCH(fn);
         }

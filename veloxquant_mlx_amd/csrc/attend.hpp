@@ -47,6 +47,8 @@ __device__ __host__ __forceinline__ int64_t window_first(const vq_attend_args &a
     return a.sliding_window > 0 && lo > 0 ? lo : 0;
 }
 
+constexpr int EVEN_BLOCKS = 256;   // one to a CU
+
 struct AttendPlan {
     int path;           // 0 generic waves, 1 MFMA decode (row tiles of <= 8), 2 MFMA prefill (LDS-staged, 64-row blocks),
                         // 3 vector-unit rows kernel (any head_dim / bit width, four query rows a block),
@@ -64,7 +66,8 @@ struct AttendPlan {
     // MFMA decode path: deal token chunks to the waves round robin instead of on demand, so that
     // results are identical from run to run
     int fixed_order;
-    // MFMA decode path, sequences of different lengths: the blocks work split_len out from all lengths (at least the one above)
+    // MFMA decode path, sequences of different lengths: a launch of EVEN_BLOCKS blocks that work split_len (at least the one above)
+    // and the splits of every tile (at most nsplit) out from all lengths
     int even = 0;
     // rows kernel over the tail only: first partial it writes (-1: the whole context, partials 0 .. nsplit - 1)
     int part0 = -1;
@@ -119,9 +122,9 @@ __device__ __forceinline__ float merge_records(const float *p, int nparts, int64
 }
 
 
-// Decides kernel and split count from shapes, whether there are lengths and the order, so that the workspace query (which
-// takes the order with the most partials) covers the launch.
-AttendPlan plan_attend(const AttendCall &a);
+// Decides kernel and split count from shapes, whether there are lengths, the order and whether the launch merges by itself, so that the
+// workspace query (`widest`: the order and the merge with the most partials) covers the launch.
+AttendPlan plan_attend(const AttendCall &a, bool widest = false);
 
 int launch_attend_generic(const AttendCall &a, int nsplit, int64_t split_len);
 // vector-unit kernel with the kv head's bytes shared by its query heads (attend_rows.hip): whether it takes the
@@ -129,8 +132,8 @@ int launch_attend_generic(const AttendCall &a, int nsplit, int64_t split_len);
 bool rows_kernel_supported(const AttendCall &a);
 void rows_tiling(const AttendCall &a, int &pq, int &tiles);
 int launch_attend_rows(const AttendCall &a, const AttendPlan &p);
-// the same kernel over the tail tokens only, into partial `part0` of `nparts` per query row
-int launch_attend_rows_tail(const AttendCall &a, int part0, int nparts);
+// the same kernel over the tail tokens only, in `runs` runs into partials `part0` on of `nparts` per query row
+int launch_attend_rows_tail(const AttendCall &a, int part0, int runs, int nparts);
 // byte codes, sixteen channels a lane (attend_wide.hip): whether it takes the shapes, its splits, the launch
 bool wide_kernel_supported(const AttendCall &a);
 void plan_attend_wide(const AttendCall &a, AttendPlan &p);

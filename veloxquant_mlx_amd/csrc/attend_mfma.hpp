@@ -519,7 +519,7 @@ __device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const
     if (blk == 0 && tab.off[i] >= 0) st_partial(base + tab.off[i] * step, acc.m_run * LN2);
 }
 
-// Combine the nparts partials of the tile's query rows into the output, in the order in which attend_merge_kernel
+// Combine the first nrec of the nparts partials of the tile's query rows into the output, in the order in which attend_merge_kernel
 // adds them (merge_records: rounds of CH records).  Partials written by other blocks of this launch are read with
 // device-scope loads, which come from beyond this XCD's L2: a round's records are fetched by the whole block at
 // once, a wave a record, into `lds`, and summed from there, a thread two neighbouring channels of a row.  The
@@ -528,7 +528,7 @@ __device__ __forceinline__ void tail_wave(const AttendCall &a, int64_t bh, const
 // The whole launch, 32 / 8 heads at 2 bits: 8320 tokens of 128 channels 17.1 -> 14.5 us, 700 of 64 channels 16.4 -> 12.9.
 // RTP: rows of a tile at most.  lds: LDS_BYTES, the block's alone by now.
 template <int DH, int RTP, int WAVES, int LDS_BYTES, int CH>
-__device__ __forceinline__ void merge_rows_ch(const AttendCall &a, const RowTile &tile, const RowTable &tab, int nparts, const float *ws,
+__device__ __forceinline__ void merge_rows_ch(const AttendCall &a, const RowTile &tile, const RowTable &tab, int nrec, int nparts, const float *ws,
                                               int tid, int wave, uint64_t *lds) {
     constexpr int DD = MF_D * DH, PART = DD + 2;
     constexpr int VAL = DD / 2;                                     // channel pairs of a record
@@ -560,8 +560,8 @@ __device__ __forceinline__ void merge_rows_ch(const AttendCall &a, const RowTile
         const bool fetch = fp < PER_ROW && f_off >= 0;
         const uint64_t *row = reinterpret_cast<const uint64_t *>(ws + (tile.base_row + (fetch ? f_off : 0)) * nparts * PART);
 #pragma unroll 1
-        for (int s0 = 0; s0 < nparts; s0 += CH) {
-            const int cnt = nparts - s0 < CH ? nparts - s0 : CH;
+        for (int s0 = 0; s0 < nrec; s0 += CH) {
+            const int cnt = nrec - s0 < CH ? nrec - s0 : CH;
             if (fetch) {
                 const uint64_t *rec = row + (int64_t)s0 * (PART / 2);
                 uint64_t hdr = 0;
@@ -614,7 +614,7 @@ __device__ __forceinline__ void merge_rows_ch(const AttendCall &a, const RowTile
                     num1 += seen ? hi(vk) * lo(fk) : 0.f;
                 }
             }
-            if (s0 + CH < nparts || r0 + ROWS < tile.RT) __syncthreads();   // the records' places are filled again
+            if (s0 + CH < nrec || r0 + ROWS < tile.RT) __syncthreads();   // the records' places are filled again
         }
         if (mine) {
             const float v0 = den > 0.f ? num0 / den : 0.f, v1 = den > 0.f ? num1 / den : 0.f;
@@ -626,12 +626,12 @@ __device__ __forceinline__ void merge_rows_ch(const AttendCall &a, const RowTile
     }
 }
 template <int DH, int RTP, int WAVES, int LDS_BYTES>
-__device__ __forceinline__ void merge_rows(const AttendCall &a, const RowTile &tile, const RowTable &tab, int nparts, const float *ws,
+__device__ __forceinline__ void merge_rows(const AttendCall &a, const RowTile &tile, const RowTable &tab, int nrec, int nparts, const float *ws,
                                            int tid, int wave, void *lds) {
     uint64_t *l = reinterpret_cast<uint64_t *>(lds);
-    if (nparts <= MERGE_FEW) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_FEW>(a, tile, tab, nparts, ws, tid, wave, l);
-    else if (nparts <= MERGE_SOME) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_SOME>(a, tile, tab, nparts, ws, tid, wave, l);
-    else merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_MANY>(a, tile, tab, nparts, ws, tid, wave, l);
+    if (nrec <= MERGE_FEW) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_FEW>(a, tile, tab, nrec, nparts, ws, tid, wave, l);
+    else if (nrec <= MERGE_SOME) merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_SOME>(a, tile, tab, nrec, nparts, ws, tid, wave, l);
+    else merge_rows_ch<DH, RTP, WAVES, LDS_BYTES, MERGE_MANY>(a, tile, tab, nrec, nparts, ws, tid, wave, l);
 }
 
 // launchers of the packed-prefix kernel (it also runs the fp16 tail and, given sync counters,

@@ -723,56 +723,68 @@ __device__ __forceinline__ u32 wave_sum_u32(u32 x) {
     const auto h = __builtin_amdgcn_permlane32_swap(x, x, false, false);
     return uniform(h[0] + h[1]);
 }
-// sum over lanes 0 .. lane
-__device__ __forceinline__ u32 wave_scan_u32(u32 x, int lane) {
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const u32 y = (u32)__shfl_up((int)x, o);
-        x += lane >= o ? y : 0u;
-    }
+// sum over lanes 0 .. lane: within rows of sixteen, then a row's last lane to the row after it, then the first half's to the second
+__device__ __forceinline__ u32 wave_scan_u32(u32 x) {
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, false);   // row_shr 1
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, false);   // row_shr 2
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, false);   // row_shr 4
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, false);   // row_shr 8
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, false);   // row_bcast 15, into rows 1 and 3
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xC, 0xF, false);   // row_bcast 31, into rows 2 and 3
     return x;
 }
-// Which tile and split a block takes in a batch whose sequences differ in length (up to 64 of them), and the tokens of a split: the
-// fewest, in whole 128s, with which the splits that hold tokens are one round of blocks.  The host knows the longest sequence
-// only: cut by that length every block of it is as long as if all sequences were.  The launch has half as many blocks again as CUs;
-// those with tokens come first in the order the chip starts them (XCDs in turn), the others end at once.
-struct EvenSplit { int by, sp; int64_t len; };
-__device__ __forceinline__ EvenSplit even_split(const AttendCall &a, int64_t split_len, int64_t tail_equiv, int lane) {
+// x / y rounded up, for 1 <= y and x below 2^21 (the product with the reciprocal is then off by less than 1 / x of itself)
+__device__ __forceinline__ u32 div_up_small(u32 x, u32 y) {
+    const u32 q = (u32)((float)x * __builtin_amdgcn_rcpf((float)y));
+    return q + (q * y < x ? 1u : 0u);
+}
+// Which tile and split a block takes in a batch whose sequences differ in length (up to 64 of them), how many splits its tile has, and the
+// tokens of a split.  The host knows the longest sequence only: cut by that length every block of it is as long as if all sequences were.
+// Here the splits that hold tokens (one at least a tile) are one round of blocks: their length is the first of those that grow by a sixteenth, from
+// the larger of the average and the host's, with which there are at most EVEN_BLOCKS, in whole 128s (up to a
+// sixteenth longer than need be).  The launch has EVEN_BLOCKS blocks, dealt to the splits in the order the chip starts them (XCDs in turn); what is
+// left over ends at once (splits 0).  (A launch of half as many blocks again, whose empty ones wrote empty partials: a CU holds one block, so those
+// began when others ended, and every merge waited for its tile's: two steps over 6 x 8320 tokens of 32 / 8 heads
+// 41 to 45 us, now 33 to 36, 7 x 20011 of 12 / 4 heads of 256 92 and 86.)
+struct EvenSplit { int by, sp, splits, len; };
+__device__ __forceinline__ EvenSplit even_split(const AttendCall &a, int64_t split_len, int64_t tail_equiv, int tiles, int lane) {
     u32 n = 0;   // tokens of sequence `lane`, in 128s
-    const bool there = lane < (int)a.B;
-    if (there) {
+    if (lane < (int)a.B) {
         const int64_t *lens = seq_lens(a);
         int64_t t = lens != nullptr ? lens[lane] : a.packed_lens[lane];
         if (t > a.n_packed) t = a.n_packed;
         n = (u32)(((t < 0 ? 0 : t) + tail_equiv + 127) / 128);
+        n = n < 1 ? 1 : n;
     }
-    const u32 per = gridDim.y / (u32)a.B;   // tiles of a sequence
-    u32 len = (u32)(((uint64_t)wave_sum_u32(n) * per + 255) / 256), splits;
+    const u32 per = (u32)a.Hkv * (u32)tiles, lin = blockIdx.x;   // tiles of a sequence
+    u32 len = (u32)(((uint64_t)wave_sum_u32(n) * per + EVEN_BLOCKS - 1) / EVEN_BLOCKS), splits, live;
     if (len < (u32)(split_len / 128)) len = (u32)(split_len / 128);
-    for (;; len += (len + 15) / 16) {   // (at one split a sequence there are at most 170)
-        splits = (n + len - 1) / len;
-        if (wave_sum_u32(splits) * per <= 256) break;
+    for (;; len += (len + 15) / 16) {   // (at one split a sequence there are fewer: ragged_splits)
+        splits = div_up_small(n, len);
+        live = wave_sum_u32(splits) * per;
+        if (live <= EVEN_BLOCKS) break;
     }
-    const u32 lin = blockIdx.x + gridDim.x * blockIdx.y, live = wave_sum_u32(splits) * per;
-    const bool empty = lin >= live;
-    const u32 mine = !there ? 0u : empty ? gridDim.x - splits : splits;   // blocks of a tile of the lane's sequence, of this kind
-    const u32 upto = wave_scan_u32(mine * per, lane), at = empty ? lin - live : lin;
-    const int b = uniform((u32)__popcll(__ballot(there && upto <= at)));
-    const u32 of_tile = (u32)__builtin_amdgcn_readlane((int)mine, b), before = (u32)__builtin_amdgcn_readlane((int)upto, b) - of_tile * per;
-    const u32 t = (at - before) / of_tile, i = (at - before) - t * of_tile;
-    return {(int)((u32)b * per + t), (int)(empty ? (u32)__builtin_amdgcn_readlane((int)splits, b) + i : i), (int64_t)len * 128};
+    if (lin >= live) return {0, 0, 0, 0};
+    const u32 upto = wave_scan_u32(splits) * per;
+    const int b = uniform((u32)__popcll(__ballot(upto <= lin)));   // lanes past the batch hold the total
+    const u32 of_tile = (u32)__builtin_amdgcn_readlane((int)splits, b);
+    const u32 at = lin - ((u32)__builtin_amdgcn_readlane((int)upto, b) - of_tile * per);
+    const u32 t = uniform(div_up_small(at + 1, of_tile)) - 1;   // at / of_tile
+    return {(int)((u32)b * per + t), (int)(at - t * of_tile), (int)of_tile, (int)len};
 }
 
 // grid (nsplit, B*Hkv*tiles), Ring<...>::THREADS threads.  A block works on one tile of query rows (the GQA
 // group at pq consecutive positions; of a group of more than eight heads, eight at one position) and on packed tokens
-// [max(0, x*split_len - tail_equiv), min(n_packed, (x+1)*split_len - tail_equiv)) (order, bit 2: split_len from the sequences' lengths), cut to what the
+// [max(0, x*split_len - tail_equiv), min(n_packed, (x+1)*split_len - tail_equiv)), cut to what the
 // tile sees; in the block of split 0 the last nparts - nsplit waves first run the fp16 tail, each
 // into a partial slot of its own.  With sync counters the block that finishes last for its tile
 // merges the nparts partials into the output.
+// EVEN: EVEN_BLOCKS blocks, whose tile, split and split_len follow from the lengths of all sequences (even_split); the host's nsplit comes in the
+// bits of `order` from 8 on, and the launch merges by itself.  A form of its own: as a branch of the one kernel it cost every launch 0.2 to 0.4 us.
 // DH = 2: a head of 256 channels, worked as two halves of 128 in the first product (eight k-steps into the same
 // scores) and as sixteen value tiles in the second; GV counts the groups of the whole head.  Such a launch runs no
 // tail waves (the fp16 tail comes as a partial of its own from the vector kernel) and takes no k_new / v_new.
-template <int BITS, typename M, int GV, int RTP, int DH = 1, int WAVES = Ring<BITS, M, GV, RTP, DH>::WAVES>
+template <int BITS, typename M, int GV, int RTP, int DH = 1, bool EVEN = false, int WAVES = Ring<BITS, M, GV, RTP, DH>::WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES / 4, WAVES / 4)))
 void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equiv, int nparts, int pq, int tiles,
                                int order, float *__restrict__ ws) {
@@ -801,12 +813,18 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
         else reinterpret_cast<u32 *>(s_const)[tid] = tid < 32 ? __float_as_uint(1.f) : 0u;
     }
     int by = blockIdx.y, sp = (int)blockIdx.x;
-    const int nsplit = (int)gridDim.x;
-    if (order & 4) {
-        const EvenSplit e = even_split(a, split_len, tail_equiv, lane);
+    // splits of the tile, its records (nparts are kept of a row), where the tail's and the splits' begin
+    int nsplit = (int)gridDim.x, nrec = nparts, tail0 = nsplit, sp0 = 0;
+    if constexpr (EVEN) {   // (the records of the tail come first: what follows those of the tile's splits is not written)
+        const EvenSplit e = even_split(a, split_len, tail_equiv, tiles, lane);
+        if (e.splits == 0) return;
         by = e.by;
         sp = e.sp;
-        split_len = e.len;
+        split_len = (int64_t)e.len * 128;
+        tail0 = 0;
+        sp0 = nparts - (order >> 8);
+        nsplit = e.splits;
+        nrec = sp0 + nsplit;
     }
     // A short context's launch is bound by the instructions on its way, most of them fetched for the first time (~10 ns
     // each at one wave a SIMD), not by bytes: 32-bit divisions, and none where there is one tile.
@@ -852,12 +870,12 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
         *dst = 8 * piece < new_row_cols(a, bh) ? *src : make_uint4(0u, 0u, 0u, 0u);
     }
     __syncthreads();
-    // the launch has nparts - nsplit tail slots (filled even when this sequence's tail is empty): the
+    // the launch has tail_waves tail slots (filled even when this sequence's tail is empty): the
     // last waves of split 0 run the tail first, each into a slot of its own, while the others stream
     if constexpr (DH == 1) {
-        const int tail_waves = nparts - nsplit;
+        const int tail_waves = EVEN ? sp0 : nparts - nsplit;
         if (sp == 0 && wave >= PK_WAVES - tail_waves)
-            tail_wave(a, bh, tile, tab, c, nsplit + wave - (PK_WAVES - tail_waves), nparts, ws, s_qraw, PK_QROW, lane,
+            tail_wave(a, bh, tile, tab, c, tail0 + wave - (PK_WAVES - tail_waves), nparts, ws, s_qraw, PK_QROW, lane,
                       wave - (PK_WAVES - tail_waves), tail_waves, newest);
     }
     // what the unit loop derives from the lane number is formed from here on, not ahead of the tail: the tail
@@ -900,7 +918,7 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
                                    s_ring, &s_next, order);
     if (n_units == 0 && single_launch && a.sink_k == nullptr) {
         // a block of the tail alone (split 0 of a short context): its packed partial saw nothing, which the merge reads from its maximum
-        if (tid < RT && tab.off[tid] >= 0) st_partial2(ws + ((tile.base_row + tab.off[tid]) * nparts + sp) * PART, -INFINITY, 0.f);
+        if (tid < RT && tab.off[tid] >= 0) st_partial2(ws + ((tile.base_row + tab.off[tid]) * nparts + sp0 + sp) * PART, -INFINITY, 0.f);
     } else {
         __syncthreads();   // every wave has read its last slot
 
@@ -954,7 +972,7 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
                 num1 += seen ? (o2[w].y + z[w]) * f : 0.f;
                 den += seen ? l[w] * f : 0.f;
             }
-            float *o = ws + ((tile.base_row + off) * nparts + sp) * PART;
+            float *o = ws + ((tile.base_row + off) * nparts + sp0 + sp) * PART;
             if (DH != 1 || tile.pair_R == 0 || tab.half[row] == d / (DD / 2)) st_partial2(o + 2 + d, num0, num1);
             if (d == 0) st_partial2(o, gm * LN2, den);
         }
@@ -979,16 +997,15 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
         __syncthreads();
         if (s_ticket != nsplit - 1) return;
     }
-    merge_rows<DH, RTP, PK_WAVES, RG::BYTES>(a, tile, tab, nparts, ws, tid, wave, s_ring);
+    merge_rows<DH, RTP, PK_WAVES, RG::BYTES>(a, tile, tab, nrec, nparts, ws, tid, wave, s_ring);
     if (nsplit > 1 && tid == 0) __hip_atomic_store(a.sync_counters + by, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <typename M, int RTP, int DH = 1>
 static void launch_mfma_packed(const AttendCall &a, const AttendPlan &p, float *ws, hipStream_t st) {
-    const dim3 grid((unsigned)p.nsplit, (unsigned)(a.B * a.Hkv * p.tiles));
     const int gv = (int)(MF_D * DH / a.group);   // groups of the whole head
     // more than 64 KB of block-shared memory has to be allowed per kernel and device, once
-#define VQ_LAUNCH(BITS, GV)                                                                                            \
+#define VQ_LAUNCH_FORM(BITS, GV, EVEN, GRID, ORDER)                                                                    \
     do {                                                                                                               \
         using RGL = Ring<BITS, M, GV, RTP, DH>;                                                                        \
         constexpr int ring_bytes = RGL::BYTES;                                                                         \
@@ -996,13 +1013,18 @@ static void launch_mfma_packed(const AttendCall &a, const AttendPlan &p, float *
         int dev = 0;                                                                                                   \
         (void)hipGetDevice(&dev);                                                                                      \
         if (dev < 0 || dev >= 64 || !allowed[dev].load(std::memory_order_acquire)) {                                   \
-            (void)hipFuncSetAttribute((const void *)attend_mfma_packed_kernel<BITS, M, GV, RTP, DH>,                   \
+            (void)hipFuncSetAttribute((const void *)attend_mfma_packed_kernel<BITS, M, GV, RTP, DH, EVEN>,             \
                                       hipFuncAttributeMaxDynamicSharedMemorySize, ring_bytes);                         \
             if (dev >= 0 && dev < 64) allowed[dev].store(true, std::memory_order_release);                             \
         }                                                                                                              \
-        hipLaunchKernelGGL((attend_mfma_packed_kernel<BITS, M, GV, RTP, DH>), grid, dim3(RGL::THREADS),                \
+        hipLaunchKernelGGL((attend_mfma_packed_kernel<BITS, M, GV, RTP, DH, EVEN>), GRID, dim3(RGL::THREADS),          \
                            ring_bytes, st, a, p.split_len,                                                             \
-                           p.tail_equiv, p.nparts, p.pq, p.tiles, p.fixed_order | (p.even ? 4 : 0), ws);                                  \
+                           p.tail_equiv, p.nparts, p.pq, p.tiles, ORDER, ws);                                          \
+    } while (0)
+#define VQ_LAUNCH(BITS, GV)                                                                                            \
+    do {                                                                                                               \
+        if (p.even) VQ_LAUNCH_FORM(BITS, GV, true, dim3(EVEN_BLOCKS), p.nsplit << 8);                                  \
+        else VQ_LAUNCH_FORM(BITS, GV, false, dim3((unsigned)p.nsplit, (unsigned)(a.B * a.Hkv * p.tiles)), p.fixed_order); \
     } while (0)
     if (a.pack_bits == 4) {
         if (gv == DH) VQ_LAUNCH(4, DH); else if (gv == 2 * DH) VQ_LAUNCH(4, 2 * DH); else VQ_LAUNCH(4, 4 * DH);
@@ -1010,6 +1032,7 @@ static void launch_mfma_packed(const AttendCall &a, const AttendPlan &p, float *
         if (gv == DH) VQ_LAUNCH(2, DH); else if (gv == 2 * DH) VQ_LAUNCH(2, 2 * DH); else VQ_LAUNCH(2, 4 * DH);
     }
 #undef VQ_LAUNCH
+#undef VQ_LAUNCH_FORM
 }
 
 }  // namespace vq

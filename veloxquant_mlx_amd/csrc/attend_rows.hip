@@ -388,11 +388,11 @@ static void launch_rows_bits(const AttendCall &a, const AttendPlan &p, dim3 grid
     }
 }
 
-int launch_attend_rows_tail(const AttendCall &a, int part0, int nparts) {
+int launch_attend_rows_tail(const AttendCall &a, int part0, int runs, int nparts) {
     AttendPlan p = {};
     p.path = 3;
     rows_tiling(a, p.pq, p.tiles);
-    p.nsplit = nparts - part0 > 1 ? nparts - part0 : 1;   // the partials past part0 are this launch's runs
+    p.nsplit = runs;
     p.split_len = a.n_tail > 0 ? cdiv(a.n_tail, p.nsplit) : 1;
     p.nparts = nparts;
     p.part0 = part0;
