@@ -108,6 +108,8 @@ def test_search_narrowed_by_bounds_takes_the_stated_winner(group, bits, alphas):
         np.where(rng.random((n, D)) < 0.03, base * np.float32(50), base),
         np.where(rng.random((n, D)) < 0.03, np.float32(1e15), base),
         np.where(rng.random((n, D)) < 0.03, np.float32(9e14), np.float32(-9e14)) + base,
+        np.float32(1000) + base * np.float32(1e-4), np.float32(-1e6) + base * np.float32(0.1),   # a few last places of the magnitude: codes
+        np.float32(3e4) - np.abs(base) * np.float32(4e-3), np.float32(7) + base * np.float32(1e-6),   # far outside the range before the clamp
     ]
     x = np.concatenate(kinds).reshape(1, 1, -1, D).astype(np.float32)
     with np.errstate(all="ignore"):

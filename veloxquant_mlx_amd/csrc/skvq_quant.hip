@@ -106,15 +106,21 @@ template <typename T> struct Vec8 {
 // rounded, squares added left to right -- costs ten operations a value and a division where a code is near a tie; five give r = sc * sqrt(sum((t - q)^2)) with
 // t = (x - lo) / sc in one fma and q = clamp(rint(t)), which is close enough to rule out
 // all factors but one in 99.6 % of the groups at 4 bits (a 4100-token prompt of 8 x 8 heads, both tensors with their orders: 243 ->
-// 230 us, 222 now; what is left is vector issue, 93 % of the SIMD-busy cycles).
+// 230 us, 206 now; what is left is vector issue, 93 % of the SIMD-busy cycles).
 // How close (u = 2^-24, W = levels * sc, M the largest |x|, so |lo| <= M and |x - lo| <= rng to within a few u * M):
 //   * the stated difference d = q * sc + lo - x of a code has an error of u (3 W + 3 M);
 //   * t has an error of u (2 rng + M) / sc (1 / sc is good to u after the Newton step), the stated quotient one of 2 u rng / sc;
-//   * codes that differ for that stand on either side of a tie, so their |d| differ by twice the sum of both;
+//   * the stated code is the nearest of 0 .. levels to its quotient, q the nearest to t, and the distance to the nearest of a set of
+//     numbers changes by no more than the number does: sc |t - q| and the stated |d| differ by u (4 rng + M) for the two errors above;
 //   * t - q is rounded where the clamp moved q: u rng.
-// So every |d| is within u (3 W + 6 M + 11 rng) of sc |t - q|, and by the triangle inequality the roots of the two sums differ
-// by at most sqrt(GROUP) times that; the sums' own rounding and the root cost (GROUP + 6) u relative.  The bounds below are these
-// with a fourth to spare.  Errors below 1e-15, where squares lose bits, stay open, and so does everything at magnitudes
+// So every |d| is within u (3 W + 4 M + 5 rng) of sc |t - q|.  The factor 1 clips nothing, and its q stays unclamped.  That is another number only where t
+// lies half a code outside [0, levels] or further, and then both distances are at most that of t to the end.  How far out: mid, the range, lo and the
+// scale are rounded, u M, u rng, u (M + rng / 2) and u W, so x - lo lies within u (2 M + 1.5 rng + W) of [0, W] (a scale raised to 1e-8: W is longer than
+// the range, and only 0 is passed), and t by its own error, u (2 rng + M), further -- over many codes where the range is a few last places of
+// M.  With it the distance is u (4 W + 7 M + 8 rng) at most.
+// By the triangle inequality the roots of the two sums differ by at most sqrt(GROUP) times these; the sums' own rounding and the root cost (GROUP + 6) u
+// relative.  The bounds below are these with a seventh of M and 6 u rng to spare (over groups of magnitudes 1e-3 to 1e5 and ranges down to 1e-9 of
+// them the roots differ by a quarter of the bound at most).  Errors below 1e-15, where squares lose bits, stay open, and so does everything at magnitudes
 // whose squares could overflow and for values that are not numbers.  `low` is the group's own memory, read before.
 // best_lo / best_sc: of the one factor that is open, if it is one.
 template <int GROUP, class Factor>
@@ -129,7 +135,7 @@ __device__ __forceinline__ uint32_t sk_open_factors(const float *xv, float *low,
         float rs = __builtin_amdgcn_rcpf(sc);
         rs = __builtin_fmaf(__builtin_fmaf(-sc, rs, 1.f), rs, rs);
         const float c = -lo * rs;
-        if (al.a[k] == 1.f) {   // nothing is clipped: a code outside [0, levels] is one that differs from the stated one at a tie (207.2 -> 205.9 us)
+        if (al.a[k] == 1.f) {   // nothing is clipped, see above (207.2 -> 205.9 us)
 #pragma unroll
             for (int j = 0; j < GROUP; ++j) {
                 const float t = __builtin_fmaf(xv[j], rs, c);
