@@ -1004,27 +1004,27 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
 template <typename M, int RTP, int DH = 1>
 static void launch_mfma_packed(const AttendCall &a, const AttendPlan &p, float *ws, hipStream_t st) {
     const int gv = (int)(MF_D * DH / a.group);   // groups of the whole head
-    // more than 64 KB of block-shared memory has to be allowed per kernel and device, once
-#define VQ_LAUNCH_FORM(BITS, GV, EVEN, GRID, ORDER)                                                                    \
+    // more than 64 KB of block-shared memory has to be allowed per kernel and device, once: for both forms at the first launch of
+    // either, so that a caller's warm-up without lengths serves a capture with them
+#define VQ_LAUNCH(BITS, GV)                                                                                            \
     do {                                                                                                               \
-        using RGL = Ring<BITS, M, GV, RTP, DH>;                                                                        \
-        constexpr int ring_bytes = RGL::BYTES;                                                                         \
-        static std::atomic<bool> allowed[64] = {};   /* set once per device; a second setter repeats the same call */ \
+        constexpr int ring_bytes = Ring<BITS, M, GV, RTP, DH>::BYTES, threads = Ring<BITS, M, GV, RTP, DH>::THREADS;   \
+        const auto plain = attend_mfma_packed_kernel<BITS, M, GV, RTP, DH, false>;                                     \
+        const auto evened = attend_mfma_packed_kernel<BITS, M, GV, RTP, DH, true>;                                     \
+        static std::atomic<bool> allowed[64] = {};   /* set once per device; a second setter repeats the same calls */ \
         int dev = 0;                                                                                                   \
         (void)hipGetDevice(&dev);                                                                                      \
         if (dev < 0 || dev >= 64 || !allowed[dev].load(std::memory_order_acquire)) {                                   \
-            (void)hipFuncSetAttribute((const void *)attend_mfma_packed_kernel<BITS, M, GV, RTP, DH, EVEN>,             \
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, ring_bytes);                         \
+            (void)hipFuncSetAttribute((const void *)plain, hipFuncAttributeMaxDynamicSharedMemorySize, ring_bytes);    \
+            (void)hipFuncSetAttribute((const void *)evened, hipFuncAttributeMaxDynamicSharedMemorySize, ring_bytes);   \
             if (dev >= 0 && dev < 64) allowed[dev].store(true, std::memory_order_release);                             \
         }                                                                                                              \
-        hipLaunchKernelGGL((attend_mfma_packed_kernel<BITS, M, GV, RTP, DH, EVEN>), GRID, dim3(RGL::THREADS),          \
-                           ring_bytes, st, a, p.split_len,                                                             \
-                           p.tail_equiv, p.nparts, p.pq, p.tiles, ORDER, ws);                                          \
-    } while (0)
-#define VQ_LAUNCH(BITS, GV)                                                                                            \
-    do {                                                                                                               \
-        if (p.even) VQ_LAUNCH_FORM(BITS, GV, true, dim3(EVEN_BLOCKS), p.nsplit << 8);                                  \
-        else VQ_LAUNCH_FORM(BITS, GV, false, dim3((unsigned)p.nsplit, (unsigned)(a.B * a.Hkv * p.tiles)), p.fixed_order); \
+        if (p.even)                                                                                                    \
+            hipLaunchKernelGGL(evened, dim3(EVEN_BLOCKS), dim3(threads), ring_bytes, st, a, p.split_len, p.tail_equiv, \
+                               p.nparts, p.pq, p.tiles, p.nsplit << 8, ws);                                            \
+        else                                                                                                           \
+            hipLaunchKernelGGL(plain, dim3((unsigned)p.nsplit, (unsigned)(a.B * a.Hkv * p.tiles)), dim3(threads),      \
+                               ring_bytes, st, a, p.split_len, p.tail_equiv, p.nparts, p.pq, p.tiles, p.fixed_order, ws); \
     } while (0)
     if (a.pack_bits == 4) {
         if (gv == DH) VQ_LAUNCH(4, DH); else if (gv == 2 * DH) VQ_LAUNCH(4, 2 * DH); else VQ_LAUNCH(4, 4 * DH);
@@ -1032,7 +1032,6 @@ static void launch_mfma_packed(const AttendCall &a, const AttendPlan &p, float *
         if (gv == DH) VQ_LAUNCH(2, DH); else if (gv == 2 * DH) VQ_LAUNCH(2, 2 * DH); else VQ_LAUNCH(2, 4 * DH);
     }
 #undef VQ_LAUNCH
-#undef VQ_LAUNCH_FORM
 }
 
 }  // namespace vq
