@@ -3,7 +3,7 @@
 // codebook indices (VecInferKVCache.fused_sdpa, veloxquant_mlx/cache/vecinfer_cache.py:670-731).  Everything is computed in
 // float32 on the vector unit; keys and values are rebuilt in registers.
 //
-// 32 / 8 heads of 128 channels, one query: byte codes of 2 x 8192 tokens 77 -> 23 us with the merge (42 MB, 1.8 TB/s);
+// 32 / 8 heads of 128 channels, one query: byte codes of 2 x 8192 tokens 77 -> 21.2 us with the merge (42 MB, 2.0 TB/s);
 // 4096 x 4 / 256 x 8 codebooks over 2 x 9001 tokens 203 us (copy of the indices, gather to float32, general kernel, merge) ->
 // 22.5 us.  What bounds it is latency: a decode call reads a few tens of MB, so every wave has two or three units of tokens to do and
 // waits for each.  Hence
@@ -19,8 +19,8 @@
 // takes 192).
 // What is left is issue: with two waves a SIMD, 1300 instructions a unit and two or three units a wave, the instructions that run once
 // count.  Row coordinates by comparison instead of division, exchanges by lane swaps instead of LDS permutes (80 waits in a
-// row) and one pass over the block's partials took 4140 instructions to 3100: byte codes of 2 x 8192 tokens 20.5 -> 18.8 us a launch,
-// 2 x 9001 indices 20.9 -> 18.4 (without the merge, 4 us).  Asking for the first unit ahead of tables and queries, eight pieces of the
+// row) and one pass over the block's partials took 3970 executed instructions a wave to 3520 (indices 3880 to 3435): byte codes of 2 x 8192 tokens
+// 20.5 -> 18.7 us a launch, a call 22.9 -> 21.2, 2 x 9001 indices 20.9 -> 18.4 a launch (without the merge, 4 us).  Asking for the first unit ahead of tables and queries, eight pieces of the
 // codebooks in flight, or a stretch of whole steps for every wave did not help (21.2, 21.9, 22.4 us): the waits are the other wave's turn.
 #include <atomic>
 
