@@ -134,8 +134,8 @@ def test_half_a_pair_of_length_lists_is_refused():
     (128, 40, 10, 9, 20000, 150, 3), (128, 28, 4, 15, 32768, 129, 4), (128, 8, 1, 50, 4096, 33, 5), (256, 12, 4, 6, 20000, 140, 11),
     (256, 12, 4, 7, 8960, 140, 9), (256, 12, 4, 10, 20000, 0, 7), (256, 8, 4, 10, 20000, 1, 7)])
 def test_a_fixed_order_cuts_by_shapes_alone(D, Hq, Hkv, B, n_packed, n_tail, splits):
-    """Sequences of different lengths: on demand the blocks cut every sequence by all lengths of the batch; under a fixed order, asked
-    for by the call or the process, or where another launch merges, the launch has the splits of the shapes.  The workspace is the larger of the two, whichever order the query or the process names."""
+    """Sequences of different lengths: on demand the blocks cut every sequence by all lengths of the batch, also where another launch
+    reads the partials; under a fixed order, asked for by the call or the process, the launch has the splits of the shapes.  The workspace is the larger of the two, whichever order the query or the process names."""
     lib = _lib.load()
     a = _lib.AttendArgs()
     a.B, a.Hq, a.Hkv, a.Sq, a.D, a.n_packed, a.n_tail = B, Hq, Hkv, 1, D, n_packed, n_tail
@@ -152,12 +152,13 @@ def test_a_fixed_order_cuts_by_shapes_alone(D, Hq, Hkv, B, n_packed, n_tail, spl
         return n.value
 
     by_shapes = nparts(1, splits)
-    assert nparts(2) > by_shapes   # (a shape that is evened)
+    evened = nparts(2)
+    assert evened > by_shapes   # (a shape that is evened)
     assert nparts(1) == nparts(3) == by_shapes
-    for field in ("sync_counters", "sink_k"):   # another launch reads the partials: cut by the shapes
+    for field in ("sync_counters", "sink_k"):   # another launch reads the partials
         was, a.sink_v, a.sink_pos, a.sink_cap = getattr(a, field), 4096, 4096, 1
         setattr(a, field, None if was else 4096)
-        assert nparts(2) == by_shapes
+        assert nparts(2) == evened and nparts(1) == by_shapes
         setattr(a, field, was)
     before = lib.vq_kivi_attend_fixed_order(1)
     try:

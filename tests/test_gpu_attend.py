@@ -841,6 +841,9 @@ def test_blocks_even_themselves_out_over_sequences_of_different_lengths(lens, Hq
     assert plan == {"path": 1, "nparts": nparts}
     ref = K.kivi_packed_attend(q, num_splits=-1, **kw)
     assert torch.isfinite(out).all() and float((out - ref).abs().max()) < TOL
-    other = K.kivi_packed_attend(q, _plan_out=shapes, _single_launch=False, **kw)   # merged by another launch: cut by the shapes
-    assert shapes["nparts"] < nparts and float((other - ref).abs().max()) < TOL
+    K._workspace(q.device, B * Hq * nparts * (D + 2) * 4).fill_(0xff)   # (NaN: a record that nothing writes must not be read as one)
+    other = K.kivi_packed_attend(q, _single_launch=False, **kw)   # merged by another launch
+    assert float((other - ref).abs().max()) < TOL
+    K.kivi_packed_attend(q, _plan_out=shapes, fixed_order=True, **kw)
+    assert shapes["nparts"] < nparts
     assert int(K._counters(q.device).abs().sum()) == 0

@@ -136,13 +136,35 @@ def test_steps_over_evened_blocks(D, Hq, H, B, ctx, bits, Sq, window, dtype):
         got = c.fused_sdpa(q, scale, lengths=lens, sliding_window=window)
         wide = pad_queries_for_paired_heads(q, H) if D == 64 else q
         plan, shapes = {}, {}
-        for single, out in ((True, plan), (False, shapes)):
-            _clamped_lists(c, wide, lens, scale, window, fixed_order=False, _single_launch=single, _plan_out=out)
+        for fixed, out in ((False, plan), (True, shapes)):
+            _clamped_lists(c, wide, lens, scale, window, fixed_order=fixed, _plan_out=out)
         assert plan["path"] == 1 and plan["nparts"] >= shapes["nparts"]
         want = _clamped_lists(c, wide, lens, scale, window, fixed_order=None, num_splits=-1)
         want = own_half_of_paired_output(want, H) if D == 64 else want
         # (two roundings of an output of up to 4: half a unit in the last place each)
         assert float((got.float() - want.float()).abs().max()) < (4e-3 if dtype == torch.float16 else 3.2e-2), step
+    assert int(K._counters(q.device).abs().sum()) == 0
+
+
+@pytest.mark.parametrize("D,Hq,H,B,ctx,bits", [(128, 32, 8, 7, 5100, 2), (128, 10, 2, 64, 4500, 4), (256, 12, 4, 7, 8700, 2)])
+def test_protected_rows_over_evened_blocks(D, Hq, H, B, ctx, bits):
+    """Protected rows are put in by a launch that reads all partials of a row: the cut by all lengths of the batch, whose shorter sequences
+    have fewer of them, against the cut by the shapes, with NaN in the workspace beforehand."""
+    require_gpu()
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    rand = lambda *s: torch.randn(s, generator=gen, device="cuda").half()
+    c = KVCacheFactory.create(KVCacheConfig(method="kivi_sink", head_dim=D, bit_width_inlier=bits, kivi_group_size=32, residual_length=128,
+                                            n_sink_tokens=3, fused_sdpa=True))
+    k = rand(B, H, ctx, D)
+    k[:, :, [40, 3111]] *= 9
+    c.update_and_fetch(k, rand(B, H, ctx, D))
+    assert c._extra_attend_args()
+    q, scale = rand(B, Hq, 1, D), D ** -0.5
+    lens = torch.tensor([ctx - (i * 1009) % (ctx - 1) for i in range(B)], device="cuda")
+    want = c.fused_sdpa(q, scale, lengths=lens, fixed_order=True)
+    K._workspace(q.device, 1 << 20).fill_(0xff)
+    got = c.fused_sdpa(q, scale, lengths=lens, fixed_order=False)
+    assert torch.isfinite(want).all() and float((got.float() - want.float()).abs().max()) < 4e-3   # (two roundings of an output of up to 4)
     assert int(K._counters(q.device).abs().sum()) == 0
 
 

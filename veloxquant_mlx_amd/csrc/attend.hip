@@ -30,8 +30,7 @@ constexpr int64_t TAIL_EQUIV = 4;
 //   12 / 4 heads of 256:   6 x 20011 (24)  90 91 88 / 88 87 87 / 83 83 76,  7 x 20011 (28)  119 112 107 / 90 / 86,  10 x 8700 (40)  83 76 91 / 78 / 74 72 75,
 //     33 x 4600 (132)  162 154 152 / 138 / 108.
 // Of 12 to 16 tiles the forms are alike (0.98 to 1.02), and up to 4096 tokens evening gains and loses (48 and 50 tiles of 2000 to 3000 tokens 3 to 5 % over
-// rounding down): these are cut by the shapes.  So is a launch under a fixed order (a sequence's bits do not depend on the lengths beside it), and one
-// whose partials another launch reads (no counters, protected rows: evened tiles leave some unwritten).  The shapes round down, as without lengths, but
+// rounding down): these are cut by the shapes.  So is a launch under a fixed order (a sequence's bits do not depend on the lengths beside it).  The shapes round down, as without lengths, but
 // for an odd number of splits a few blocks over one round, which spreads the blocks without work over the XCDs: 88 to 96 tiles of 20011 tokens, three splits / two,
 // 81 to 101 / 95, of 8700 51 to 72 / 57; up to 4096 tokens five splits (52 and 56 tiles of 1200 28 / 30, 27 / 27, of 2000 34 / 32, 31 / 27), not
 // three (88 to 96 tiles of 2000 31 to 45 / 30 to 33), but of heads of 256 channels three as well (88 tiles of 1200 to 2000 at 4 bits 79 92 / 86 98).
@@ -116,7 +115,7 @@ AttendPlan plan_attend(const AttendCall &a, bool widest) {
     // or an eight-wave block per kv head (MFMA)
     const int64_t units = p.path == 1 ? a.B * a.Hkv * p.tiles : a.B * a.Hq * a.Sq;
     int64_t ns = a.num_splits;   // < 0: choose as well
-    const bool may_even = widest || (p.fixed_order == 0 && a.sync_counters != nullptr && a.sink_k == nullptr);
+    const bool may_even = widest || p.fixed_order == 0;
     if (ns <= 0) ns = p.path == 1 ? decode_splits(a, may_even, units > 0 ? units : 1, n_split) : cdiv(4096, units > 0 ? units : 1);
     if (ns > max_splits) ns = max_splits;
     if (ns > 512) ns = 512;

@@ -122,8 +122,8 @@ __device__ __forceinline__ float merge_records(const float *p, int nparts, int64
 }
 
 
-// Decides kernel and split count from shapes, whether there are lengths, the order and whether the launch merges by itself, so that the
-// workspace query (`widest`: the order and the merge with the most partials) covers the launch.
+// Decides kernel and split count from shapes, whether there are lengths and the order, so that the workspace query (`widest`: the order
+// with the most partials) covers the launch.
 AttendPlan plan_attend(const AttendCall &a, bool widest = false);
 
 int launch_attend_generic(const AttendCall &a, int nsplit, int64_t split_len);

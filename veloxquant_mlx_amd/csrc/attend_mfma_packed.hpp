@@ -780,7 +780,8 @@ __device__ __forceinline__ EvenSplit even_split(const AttendCall &a, int64_t spl
 // into a partial slot of its own.  With sync counters the block that finishes last for its tile
 // merges the nparts partials into the output.
 // EVEN: EVEN_BLOCKS blocks, whose tile, split and split_len follow from the lengths of all sequences (even_split); the host's nsplit comes in the
-// bits of `order` from 8 on, and the launch merges by itself.  A form of its own: as a branch of the one kernel it cost every launch 0.2 to 0.4 us.
+// bits of `order` from 8 on.  Records past those of a tile's splits are written (as empty) only where another launch reads them: one
+// that merges, or the one that puts protected rows in (13 x 20011 tokens of 40 / 10 heads of which four are protected 118 us cut by the shapes, 89 evened).  A form of its own: as a branch of the one kernel it cost every launch 0.2 to 0.4 us.
 // DH = 2: a head of 256 channels, worked as two halves of 128 in the first product (eight k-steps into the same
 // scores) and as sixteen value tiles in the second; GV counts the groups of the whole head.  Such a launch runs no
 // tail waves (the fp16 tail comes as a partial of its own from the vector kernel) and takes no k_new / v_new.
@@ -988,6 +989,13 @@ void attend_mfma_packed_kernel(AttendCall a, int64_t split_len, int64_t tail_equ
     // accesses, of which none passes between the blocks (the ticket took 1.3 to 3.3 us, now 0.5 to 1).
     // A tile with a single run has no other block to count: the barrier has collected its own partials (the
     // packed one and the tail waves'; the tail launch of a 256-channel head ended before this one began).
+    if constexpr (EVEN) {   // another launch reads all nparts records of a row
+        if (sp == 0 && (!single_launch || a.sink_k != nullptr))
+            for (int e = tid; e < RT * (nparts - nrec); e += PK_THREADS) {
+                const int row = e / (nparts - nrec), rec = nrec + e - row * (nparts - nrec);
+                if (tab.off[row] >= 0) st_partial2(ws + ((tile.base_row + tab.off[row]) * nparts + rec) * PART, -INFINITY, 0.f);
+            }
+    }
     if (!single_launch) return;
     wait_copies<0>();
     __syncthreads();

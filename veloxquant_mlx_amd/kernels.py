@@ -1221,8 +1221,6 @@ def kivi_packed_attend(q: torch.Tensor, *, k_packed=None, k_scale=None, k_zero=N
                 raise ValueError(f"{name}: {nm} must be a contiguous [{B}, {Hkv}, 1, {D}] device tensor in the dtype of the tail")
         a.k_new, a.v_new = k_new.data_ptr(), v_new.data_ptr()
     lib = _lib.load()
-    # (ahead of the plan, which asks for them; vq_kivi_attend_static has its own, and such a call allocates none)
-    a.sync_counters = _counters(q.device).data_ptr() if _single_launch and not static_scratch else None
     if _plan_out is not None:
         import ctypes
         pth, npt = ctypes.c_int(0), ctypes.c_int(0)
@@ -1236,6 +1234,7 @@ def kivi_packed_attend(q: torch.Tensor, *, k_packed=None, k_scale=None, k_zero=N
     need = lib.vq_kivi_attend_workspace_ext(a, ext)   # of the call that runs: lengths change its plan
     ws = _workspace(q.device, need)
     a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+    a.sync_counters = _counters(q.device).data_ptr() if _single_launch else None
     _lib.check(lib.vq_kivi_attend_ext(a, ext))
     return out
 
